@@ -1,0 +1,552 @@
+"""The work that users of this package have it do, as a list of cases to time.
+
+Every case is one call, or one short run, through the public entry points
+(``Solver``, ``run_with_grad``, ``Ensemble``) at a size of one of the package's
+workloads: the Sod tube, the isentropic vortex, the relaxation channel and its
+gradient, the fluctuating ensemble, the 13-moment Taylor-Green vortex and its
+gradient, and ideal-gas and relaxation flows with the other bases and with
+boundaries.  A case is a plain dict; ``kind`` names the entry point, ``flow``
+the physics, the rest are sizes and options.
+
+``exact`` computes a case's outputs with the operator written out in plain
+torch float64 (the DG right-hand side, the limiter, the SSP-RK steps, and
+autograd through them for the gradients).  The ensembles have no such value:
+their stochastic stress is the package's own generator.
+"""
+import math
+
+import numpy as np
+import torch
+
+from hermeshd_amd.adjoint import AdjointRunner, run_with_grad
+from hermeshd_amd.config import HDConfig, fluct_ensemble, poiseuille_2d, sod_1d, taylor_green_3d, vortex_3d
+from hermeshd_amd.ensemble import Ensemble
+from hermeshd_amd.solver import Solver
+
+RH, MX, MY, MZ, EN = 0, 1, 2, 3, 4
+
+
+def listed():
+    return [
+        # the smallest call: one step of a 1D shock tube, all launches and latency
+        dict(name="sod_256", kind="step", flow="sod", nx=256, ny=1, nz=1),
+        # one fixed-dt step of the 2D relaxation channel with no-slip walls
+        dict(name="channel_64x128", kind="update", flow="channel", nx=64, ny=128, nz=1),
+        # gradient of a short channel run (forward, recompute, transposed stages)
+        dict(name="channel_grad_64x128", kind="grad", flow="channel", nx=64, ny=128, nz=1, nsteps=10, every=5),
+        # the flagship grid: quadratic basis, HLLC, SSP-RK3
+        dict(name="vortex_128x128x32", kind="step", flow="vortex", nx=128, ny=128, nz=32),
+        # the same flow on a ragged grid, as a resolution study has it
+        dict(name="vortex_75x61x27", kind="step", flow="vortex", nx=75, ny=61, nz=27),
+        # production-size linear-basis gas dynamics: outflow in x, walls in y
+        dict(name="linear_256x256x128", kind="step", flow="gas", nx=256, ny=256, nz=128, nbasis=4, open=True),
+        # trilinear basis, all periodic
+        dict(name="trilinear_120x80x64", kind="step", flow="gas", nx=120, ny=80, nz=64, nbasis=8, open=False),
+        # viscous relaxation model on the quadratic basis, no-slip walls in y
+        dict(name="viscous_64x64x48", kind="step", flow="viscous", nx=64, ny=64, nz=48, nbasis=10, walls=True),
+        # a few fluctuating boxes, as a first look at a structure factor
+        dict(name="ensemble_20", kind="ensemble", n16=8, n24=8, n32=4, nsteps=4),
+        # the full ensemble of 256 uneven boxes
+        dict(name="ensemble_256", kind="ensemble", n16=96, n24=96, n32=64, nsteps=2),
+        # one step of the 13-moment Taylor-Green vortex
+        dict(name="tgv_96", kind="step", flow="tgv", nx=96, ny=96, nz=96),
+        # gradient of the final state of a short 13-moment run
+        dict(name="tgv_grad_40", kind="grad", flow="tgv", nx=40, ny=40, nz=40, nsteps=2, every=1),
+    ]
+
+
+def draw(rng):
+    def n(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    f = rng.randrange(9)
+    if f == 0:
+        return dict(kind="step", flow="sod", nx=n(64, 2048), ny=1, nz=1)
+    if f == 1:
+        return dict(kind="update", flow="channel", nx=n(24, 160), ny=n(32, 256), nz=1)
+    if f == 2:
+        return dict(kind="grad", flow="channel", nx=n(24, 96), ny=n(32, 160), nz=1, nsteps=rng.randint(4, 10),
+                    every=rng.randint(2, 5))
+    if f == 3:
+        return dict(kind="step", flow="vortex", nx=n(24, 144), ny=n(24, 144), nz=n(3, 25))
+    if f == 4:
+        return dict(kind="step", flow="gas", nx=n(32, 300), ny=n(32, 256), nz=n(16, 100),
+                    nbasis=rng.choice([4, 4, 8]), open=rng.random() < 0.5)
+    if f == 5:
+        return dict(kind="step", flow="viscous", nx=n(16, 72), ny=n(16, 72), nz=n(8, 36),
+                    nbasis=rng.choice([4, 10]), walls=rng.random() < 0.5)
+    if f == 6:
+        return dict(kind="ensemble", n16=n(2, 96), n24=n(2, 96), n32=n(1, 60), nsteps=rng.randint(1, 2))
+    if f == 7:
+        return dict(kind="step", flow="tgv", nx=n(20, 96), ny=n(20, 96), nz=n(20, 96))
+    m = n(12, 40)
+    return dict(kind="grad", flow="tgv", nx=m, ny=n(12, 40), nz=n(12, 40), nsteps=rng.randint(1, 2), every=1)
+
+
+# ---------------------------------------------------------------- inputs ----
+def config(case):
+    flow, nx, ny, nz = case["flow"], case["nx"], case["ny"], case["nz"]
+    if flow == "sod":
+        return sod_1d(nx)
+    if flow == "channel":
+        return poiseuille_2d(nx, ny)
+    if flow == "vortex":
+        return vortex_3d(nx, ny, nz)
+    if flow == "tgv":
+        c = taylor_green_3d(nx)
+        return c.replace(ny=ny, nz=nz, ly=c.lx * ny / nx, lz=c.lx * nz / nx)
+    nb = case["nbasis"]
+    box = dict(nx=nx, ny=ny, nz=nz, lx=float(nx), ly=float(ny), lz=float(nz), nbasis=nb, iquad=3 if nb == 10 else 2)
+    if flow == "gas":
+        bc = ("outflow", "outflow", "wall", "wall") if case["open"] else ("periodic",) * 4
+        return HDConfig(nQ=5, riemann="hllc", limiter=True, integrator="heun", bc=bc + ("periodic",) * 2, gamma=1.4,
+                        T_floor=1e-4, **box)
+    vis = 0.05
+    bc = ("periodic", "periodic") + (("noslip", "noslip") if case["walls"] else ("periodic", "periodic"))
+    return HDConfig(nQ=11, ivis=1, riemann="hllc", limiter=True, integrator="shu-osher",
+                    bc=bc + ("periodic", "periodic"), gamma=5.0 / 3.0, T_floor=1e-4, coll=1.0 / vis, colvis=1.0,
+                    body_force=(1e-3, 0.0, 0.0), **box)
+
+
+def smooth(shape, scale, gen, dev):
+    """Unit-variance Gaussian field correlated over `scale` cells, periodic."""
+    w = torch.fft.rfftn(torch.randn(shape, generator=gen, dtype=torch.float64, device=dev))
+    for ax, n in enumerate(shape):
+        k = torch.fft.rfftfreq(n, dtype=torch.float64, device=dev) if ax == 2 else \
+            torch.fft.fftfreq(n, dtype=torch.float64, device=dev)
+        g = torch.exp(-0.5 * (2 * math.pi * scale * k) ** 2) if n > 1 else torch.ones_like(k)
+        w = w * g.reshape([-1 if a == ax else 1 for a in range(3)])
+    f = torch.fft.irfftn(w, s=shape)
+    return (f - f.mean()) / f.std().clamp_min(1e-300)
+
+
+def conserved(rho, u, v, w, p, gamma):
+    return torch.stack([rho, rho * u, rho * v, rho * w, p / (gamma - 1.0) + 0.5 * rho * (u * u + v * v + w * w)])
+
+
+def with_slopes(m0, cfg):
+    """A state whose higher modes are those of the field sampled by the cell
+    averages m0 (nQ, nz, ny, nx): central differences, one-sided at a
+    boundary, zero along an axis of one cell."""
+    def two(a, ax):
+        axis = 3 - ax
+        if a.shape[axis] == 1:
+            return a, a
+        up, dn = torch.roll(a, -1, axis), torch.roll(a, 1, axis)
+        if cfg.bc[2 * ax] != "periodic":
+            n = a.shape[axis]
+            up.narrow(axis, n - 1, 1).copy_(a.narrow(axis, n - 1, 1))
+            dn.narrow(axis, 0, 1).copy_(a.narrow(axis, 0, 1))
+        return up, dn
+
+    def d1(a, ax):
+        up, dn = two(a, ax)
+        return (up - dn) / 4.0
+
+    q = torch.zeros(cfg.shape, dtype=torch.float64, device=m0.device)
+    q[0] = m0
+    for ax in range(3):
+        q[1 + ax] = d1(m0, ax)
+    if cfg.nbasis > 4:
+        q[4], q[5], q[6] = d1(q[2], 2), d1(q[3], 0), d1(q[1], 1)
+    if cfg.nbasis == 8:
+        q[7] = d1(q[6], 2)
+    if cfg.nbasis == 10:
+        for ax in range(3):
+            up, dn = two(m0, ax)
+            q[7 + ax] = (up - 2.0 * m0 + dn) / 12.0
+    return q
+
+
+def initial(case, cfg, seed, dev):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    shape = (cfg.nz, cfg.ny, cfg.nx)
+    one = torch.ones(shape, dtype=torch.float64, device=dev)
+
+    def axis(n, length, ax):
+        x = (torch.arange(n, dtype=torch.float64, device=dev) + 0.5) * (length / n) - 0.5 * length
+        return x.reshape([-1 if a == 2 - ax else 1 for a in range(3)])
+
+    def noise():
+        return torch.randn(shape, generator=gen, dtype=torch.float64, device=dev)
+
+    x, y, z = axis(cfg.nx, cfg.lx, 0), axis(cfg.ny, cfg.ly, 1), axis(cfg.nz, cfg.lz, 2)
+    flow = case["flow"]
+    if flow == "sod":
+        left = (x <= 0) & (one > 0)
+        rho = torch.where(left, one, 0.125 * one) * (1.0 + 1e-3 * noise())
+        p = torch.where(left, one, 0.1 * one)
+        q = torch.zeros(cfg.shape, dtype=torch.float64, device=dev)
+        q[0] = conserved(rho, 1e-3 * noise(), 0.0 * one, 0.0 * one, p, cfg.gamma)
+        return q
+    if flow == "vortex":
+        beta, g = 5.0, cfg.gamma
+        r2 = x * x + y * y
+        e = torch.exp(0.5 * (1.0 - r2))
+        T = 1.0 - (g - 1.0) * beta ** 2 / (8.0 * g * math.pi ** 2) * e * e * one
+        rho = T ** (1.0 / (g - 1.0))
+        m0 = conserved(rho * (1.0 + 1e-6 * noise()), 1.0 - beta / (2 * math.pi) * e * y * one,
+                       1.0 + beta / (2 * math.pi) * e * x * one, 1e-6 * noise(), rho ** g, g)
+        return with_slopes(m0, cfg)
+    if flow == "tgv":
+        x, y, z = x + 0.5 * cfg.lx, y + 0.5 * cfg.ly, z + 0.5 * cfg.lz
+        kx, ky, kz = 1.0, 2 * math.pi / cfg.ly, 2 * math.pi / cfg.lz
+        u = torch.sin(kx * x) * torch.cos(ky * y) * torch.cos(kz * z) + 1e-4 * noise()
+        v = -torch.cos(kx * x) * torch.sin(ky * y) * torch.cos(kz * z) + 1e-4 * noise()
+        m0 = torch.zeros((13,) + shape, dtype=torch.float64, device=dev)
+        p = 100.0 / cfg.gamma + (torch.cos(2 * kx * x) + torch.cos(2 * ky * y)) * (torch.cos(2 * kz * z) + 2) / 16.0
+        m0[:5] = conserved(one, u, v, 1e-4 * noise(), p * one, cfg.gamma)
+        return with_slopes(m0, cfg)
+
+    def s(scale):
+        return smooth(shape, scale, gen, dev)
+
+    if flow == "gas":
+        m0 = conserved(1.0 + 0.1 * s(4.0), 0.2 + 0.2 * s(5.0), 0.2 * s(5.0), 0.2 * s(5.0), 1.0 + 0.1 * s(4.0),
+                       cfg.gamma)
+        return with_slopes(m0, cfg)
+    m0 = torch.zeros((11,) + shape, dtype=torch.float64, device=dev)
+    if flow == "channel":
+        m0[:5] = conserved(one, 0.1 * s(8.0), 0.1 * s(8.0), 0.0 * one, one, cfg.gamma)
+    else:
+        m0[:5] = conserved(1.0 + 0.02 * s(4.0), 0.1 * s(5.0), 0.1 * s(5.0), 0.1 * s(5.0), 1.0 + 0.02 * s(4.0),
+                           cfg.gamma)
+        for f in range(5, 11):
+            m0[f] = 1e-3 * s(4.0)
+    return with_slopes(m0, cfg)
+
+
+FIXED_DT = {"channel": 0.05}
+
+
+def grad_dt(case, cfg):
+    # the 13-moment vortex has sound speed 10 and |u| <= 1
+    return FIXED_DT.get(case["flow"], 0.08 * (cfg.lx / cfg.nx) / 22.0)
+
+
+def boxes(case):
+    return ((case["n16"], 16), (case["n24"], 24), (case["n32"], 32))
+
+
+def prepare(case, seed):
+    dev = torch.device("cuda")
+    if case["kind"] == "ensemble":
+        base, dims = fluct_ensemble(sizes=boxes(case), seed=1000 + seed)
+        ens = Ensemble(base, dims)
+        gen = torch.Generator(device=dev)
+        gen.manual_seed(seed)
+        q = ens.zeros()
+        for v in ens.views(q):
+            # rest plus velocities of the fluctuation amplitude
+            v[0, RH] = 1.0
+            v[0, MX:MZ + 1] = 0.01 * torch.randn(v[0, MX:MZ + 1].shape, generator=gen, dtype=torch.float64, device=dev)
+            v[0, EN] = 1.0 / (base.gamma - 1.0) + 0.5 * (v[0, MX:MZ + 1] ** 2).sum(0)
+        return dict(kind="ensemble", ens=ens, q=q, q1=ens.zeros(), nsteps=case["nsteps"])
+    cfg = config(case)
+    q = initial(case, cfg, seed, dev)
+    if case["kind"] == "grad":
+        gen = torch.Generator(device=dev)
+        gen.manual_seed(seed + 1)
+        runner = AdjointRunner(cfg, dt=grad_dt(case, cfg), nsteps=case["nsteps"], checkpoint_every=case["every"])
+        lam = torch.randn(cfg.shape, generator=gen, dtype=torch.float64, device=dev)
+        coll = torch.tensor(float(cfg.coll), dtype=torch.float64, device=dev, requires_grad=True)
+        return dict(kind="grad", runner=runner, q=q.requires_grad_(True), coll=coll, lam=lam)
+    s = Solver(cfg)
+    st = dict(kind=case["kind"], solver=s, q=q, q1=s.zeros(), t=torch.zeros_like(s.t), dt=torch.zeros_like(s.dt))
+    if case["kind"] == "update":
+        st["dt"].fill_(FIXED_DT[case["flow"]])
+    return st
+
+
+def run(state):
+    kind, q = state["kind"], state["q"]
+    if kind == "step":
+        state["solver"].step(q, state["q1"], None, t=state["t"], dt=state["dt"])
+        return {"q": q, "t": state["t"], "dt": state["dt"]}
+    if kind == "update":
+        state["solver"].update(q, state["q1"], None, state["dt"])
+        return {"q": q}
+    if kind == "ensemble":
+        state["ens"].run(q, state["q1"], None, 0.1, state["nsteps"])
+        return {"q": q}
+    out = run_with_grad(state["runner"], q, state["coll"])
+    gq, gc = torch.autograd.grad(out, (q, state["coll"]), state["lam"])
+    return {"q": out, "grad_q": gq, "grad_coll": gc}
+
+
+# ------------------------------------------------------------------ work ----
+def stage_work(cells, nb, nQ):
+    """FP64 operations of one stage of one cell, each face counted once: the
+    modes summed at the Gauss points of the volume and of three faces (both
+    sides), point fluxes, Riemann solves, and the projections back."""
+    q = 3 if nb == 10 else 2
+    npg, nf, nk = q ** 3, q ** 2, {4: 3, 8: 4, 10: 6}[nb]
+    nd = {4: 3, 8: 12, 10: 12}[nb]
+    volume = npg * nQ * (2 * (nb - 1) + 2 * nd) + npg * (16 + 10 * nQ)
+    face = nf * (2 * nQ * 2 * (nk - 1) + 2 * (16 + 3 * nQ) + 60 + nQ * 2 * nk) + 2 * nQ * 2 * nb
+    return cells * (volume + 3 * face + 4 * nQ * nb)
+
+
+def work(case):
+    if case["kind"] == "ensemble":
+        base, dims = fluct_ensemble(sizes=boxes(case))
+        cells = sum(a * b * c for a, b, c in dims)
+        state = 8.0 * cells * base.nQ * base.nbasis
+        points = sum(12 * (a + 1) * (b + 1) * (c + 1) + 8 * a * b * c for a, b, c in dims)
+        # per step: two stages (read the state, the second also the step's start; write) and the stress drawn once
+        return {"bytes": case["nsteps"] * (5 * state + 24.0 * points),
+                "flops": case["nsteps"] * (2 * stage_work(cells, base.nbasis, base.nQ) + 150.0 * points)}
+    cfg = config(case)
+    stages = 3 if cfg.integrator == "shu-osher" else 2
+    state = 8.0 * cfg.ncell * cfg.nQ * cfg.nbasis
+    ops = stage_work(cfg.ncell, cfg.nbasis, cfg.nQ)
+    step_bytes, step_ops = (3 * stages - 1) * state, stages * ops
+    if case["kind"] != "grad":
+        return {"bytes": step_bytes, "flops": step_ops}
+    # forward, recompute, and a transposed stage (state, cotangent in and out, about three times the operations)
+    return {"bytes": case["nsteps"] * (2 * step_bytes + stages * 4 * state), "flops": case["nsteps"] * 5 * step_ops}
+
+
+# ----------------------------------------------------------------- exact ----
+def legendre(a, x):
+    return torch.ones_like(x) if a == 0 else (x if a == 1 else 1.5 * x * x - 0.5)
+
+
+def dlegendre(a, x):
+    return torch.zeros_like(x) if a == 0 else (torch.ones_like(x) if a == 1 else 3.0 * x)
+
+
+class Exact:
+    """The DG operator, the limiter and the SSP-RK step in plain torch."""
+
+    def __init__(self, cfg, dev):
+        self.cfg, nb, n = cfg, cfg.nbasis, cfg.iquad
+        x1, w1 = np.polynomial.legendre.leggauss(n)
+        x, w = (torch.tensor(v, dtype=torch.float64, device=dev) for v in (x1, w1))
+        deg = [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (0, 1, 1), (1, 0, 1), (1, 1, 0)]
+        deg += {8: [(1, 1, 1)], 10: [(2, 0, 0), (0, 2, 0), (0, 0, 2)]}.get(nb, [])
+        deg = deg[:nb]
+        X, Y, Z = (a.reshape(-1) for a in torch.meshgrid(x, x, x, indexing="ij"))
+        W = torch.einsum("i,j,k->ijk", w, w, w).reshape(-1)
+        L, D = legendre, dlegendre
+        self.cb = torch.tensor([float((2 * a + 1) * (2 * b + 1) * (2 * c + 1)) for a, b, c in deg],
+                               dtype=torch.float64, device=dev)
+        self.phi = torch.stack([L(a, X) * L(b, Y) * L(c, Z) for a, b, c in deg], 1)
+        grads = [[D(a, X) * L(b, Y) * L(c, Z) for a, b, c in deg], [L(a, X) * D(b, Y) * L(c, Z) for a, b, c in deg],
+                 [L(a, X) * L(b, Y) * D(c, Z) for a, b, c in deg]]
+        self.wd = [W[:, None] * torch.stack(g, 1) for g in grads]
+        U, V = (a.reshape(-1) for a in torch.meshgrid(x, x, indexing="ij"))
+        self.wf = torch.einsum("i,j->ij", w, w).reshape(-1)
+        self.face = {}
+        for d in range(3):
+            for side, e in ((0, -torch.ones_like(U)), (1, torch.ones_like(U))):
+                P = [U, V]
+                P.insert(d, e)
+                self.face[d, side] = torch.stack([L(a, P[0]) * L(b, P[1]) * L(c, P[2]) for a, b, c in deg], 1)
+        self.dxi = (cfg.nx / cfg.lx, cfg.ny / cfg.ly, cfg.nz / cfg.lz)
+        self.gm1 = cfg.gamma - 1.0
+
+    def pressure(self, Q):
+        return self.gm1 * (Q[EN] - 0.5 * (Q[MX] ** 2 + Q[MY] ** 2 + Q[MZ] ** 2) / Q[RH])
+
+    def flux(self, Q, d):
+        c = self.cfg
+        u = [Q[MX] / Q[RH], Q[MY] / Q[RH], Q[MZ] / Q[RH]]
+        p = self.pressure(Q)
+        p = torch.where(p < c.P_floor, torch.full_like(p, c.P_floor), p)
+        zero = torch.zeros_like(p)
+        if c.nQ == 5:
+            S = [zero] * 3
+        elif c.nQ == 11:
+            S = [Q[i] for i in ((5, 8, 9), (8, 6, 10), (9, 10, 7))[d]]
+        else:
+            S = [(Q[5], Q[7], Q[8]), (Q[7], Q[6], Q[9]), (Q[8], Q[9], -(Q[5] + Q[6]))][d]
+        F = [Q[MX + d]] + [Q[MX + a] * u[d] + S[a] + (p if a == d else 0.0) for a in range(3)]
+        F.append((Q[EN] + p) * u[d] + S[0] * u[0] + S[1] * u[1] + S[2] * u[2])
+        if c.nQ > 5:
+            cv = c.colvis
+            diag = [cv * (4.0 if a == d else -2.0) / 3.0 * u[d] for a in range(3)]
+            off = [cv * u[b] if a == d else (cv * u[a] if b == d else zero) for a, b in ((0, 1), (0, 2), (1, 2))]
+            F += diag + off if c.nQ == 11 else diag[:2] + off
+        if c.nQ == 13:
+            F[EN] = F[EN] + Q[10 + d]
+            F += [c.col_q * p / Q[RH] if a == d else zero for a in range(3)]
+        return torch.stack(F)
+
+    def hllc(self, A, B, FA, FB, d):
+        c, n = self.cfg, MX + d
+        pa, pb, ua, ub = self.pressure(A), self.pressure(B), A[n] / A[RH], B[n] / B[RH]
+        ca, cb = torch.sqrt(c.gamma * pa / A[RH]), torch.sqrt(c.gamma * pb / B[RH])
+        # at a tie the slower speed is the first state's and the faster the second's (their derivatives differ)
+        sa = torch.where(ua - ca <= ub - cb, ua - ca, ub - cb)
+        sb = torch.where(ub + cb >= ua + ca, ub + cb, ua + ca)
+        ma, mb = A[RH] * (sa - ua), B[RH] * (sb - ub)
+        sm = (mb * ub - ma * ua + pa - pb) / (mb - ma)
+        ps = A[RH] * (ua - sa) * (ua - sm) + pa
+
+        def star(Q, F, s, u, p):
+            r = 1.0 / (s - sm)
+            rows = []
+            for f in range(5):
+                v = (s - u) * Q[f]
+                v = v + (ps - p) if f == n else (v - p * u + ps * sm if f == EN else v)
+                rows.append(F[f] + s * (v * r - Q[f]))
+            return torch.stack(rows)
+
+        out = torch.where(sm > 0, star(A, FA, sa, ua, pa), star(B, FB, sb, ub, pb))
+        return torch.where(sa > 0, FA[:5], torch.where(sb < 0, FB[:5], out))
+
+    def roe(self, A, B, FA, FB, d):
+        # Eulderink-Mellema form with half the thermal enthalpy, as the package documents it
+        gm1, cp = self.gm1, self.cfg.gamma / self.gm1
+        n, t1, t2 = MX + d, MX + (d + 1) % 3, MX + (d + 2) % 3
+
+        def roots(Q):
+            k = torch.sqrt(Q[RH])
+            v = [Q[f] / Q[RH] for f in (n, t1, t2)]
+            v2 = v[0] ** 2 + v[1] ** 2 + v[2] ** 2
+            return k, [k * a for a in v] + [0.5 * k * (v2 + cp * gm1 * (Q[EN] - 0.5 * Q[RH] * v2) / Q[RH])]
+
+        (ka, wa), (kb, wb) = roots(A), roots(B)
+        v0, v1, v2, h = ((a + b) / (ka + kb) for a, b in zip(wa, wb))
+        vv = v0 * v0 + v1 * v1 + v2 * v2
+        a2 = gm1 * (h - 0.5 * vv)
+        a = torch.sqrt(a2)
+        dr, dn, d1, d2, de = ((B[f] - A[f]) / A[RH] for f in (RH, n, t1, t2, EN))
+        vd = v0 * dn + v1 * d1 + v2 * d2 - de
+        even, odd = 0.5 * gm1 / a2 * (0.5 * vv * dr - vd), 0.5 * (dn - v0 * dr) / a
+        lo, hi = (even - odd) * (v0 - a).abs(), (even + odd) * (v0 + a).abs()
+        mid = gm1 / a2 * ((h - vv) * dr + vd) * v0.abs()
+        s1, s2 = (d1 - v1 * dr) * v0.abs(), (d2 - v2 * dr) * v0.abs()
+        diss = {RH: lo + hi + mid, n: lo * (v0 - a) + hi * (v0 + a) + mid * v0, t1: (lo + hi + mid) * v1 + s1,
+                t2: (lo + hi + mid) * v2 + s2,
+                EN: lo * (h - a * v0) + hi * (h + a * v0) + mid * 0.5 * vv + s1 * v1 + s2 * v2}
+        return torch.stack([0.5 * (FA[f] + FB[f] - diss[f] * A[RH]) for f in range(5)])
+
+    def ghost(self, own, d, side):
+        """Exterior states of a boundary; own: (points, nQ, ...) at its faces."""
+        kind, g, n = self.cfg.bc[2 * d + side], own.clone(), MX + d
+        if kind == "noslip":
+            g[:, MX:MZ + 1] = 0.0
+        elif kind == "wall":
+            g[:, n] = 0.0
+        elif (d, side) == (0, 1):
+            g[:, n] = torch.where(own[:, n] > 0, -own[:, n], own[:, n])
+        else:
+            back = own[:, n].amin(0) < 0 if side else own[:, n].amax(0) > 0
+            g[:, n] = torch.where(back, torch.zeros_like(own[:, n]), own[:, n])
+        return g
+
+    def rhs(self, q):
+        c, nb = self.cfg, self.cfg.nbasis
+        Qg = torch.matmul(self.phi, q.reshape(nb, -1)).reshape((-1,) + q.shape[1:]).transpose(0, 1)
+        out = 0.0
+        for d in range(3):
+            F = self.flux(Qg, d).transpose(0, 1).reshape(Qg.shape[1], -1)
+            out = out + self.dxi[d] * torch.matmul(self.wd[d].T, F).reshape(q.shape)
+            del F
+            ax = 4 - d
+            lo, hi = (torch.matmul(self.face[d, s], q.reshape(nb, -1)).reshape((-1,) + q.shape[1:]) for s in (0, 1))
+            n = q.shape[ax]
+            if c.bc[2 * d] == "periodic":
+                A = torch.cat([hi.narrow(ax, n - 1, 1), hi], ax)
+                B = torch.cat([lo, lo.narrow(ax, 0, 1)], ax)
+            else:
+                A = torch.cat([self.ghost(lo.narrow(ax, 0, 1), d, 0), hi], ax)
+                B = torch.cat([lo, self.ghost(hi.narrow(ax, n - 1, 1), d, 1)], ax)
+            A, B = A.transpose(0, 1), B.transpose(0, 1)
+            FA, FB = self.flux(A, d), self.flux(B, d)
+            solve = self.hllc if c.riemann == "hllc" else self.roe
+            G = torch.cat([solve(A, B, FA, FB, d), 0.5 * (FA[5:] + FB[5:])]).transpose(0, 1)
+            for s in (0, 1):
+                g = G.narrow(ax, s, n).reshape(G.shape[0], -1)
+                lift = torch.matmul((self.wf[:, None] * self.face[d, s]).T, g).reshape(q.shape)
+                out = out - self.dxi[d] * lift if s else out + self.dxi[d] * lift
+        out = 0.25 * self.cb.reshape(-1, 1, 1, 1, 1) * out
+        b = c.body_force
+        if any(b):
+            rows = list(out.unbind(1))
+            for a in range(3):
+                rows[MX + a] = rows[MX + a] + b[a] * q[:, RH]
+            rows[EN] = rows[EN] + sum(b[a] * q[:, MX + a] for a in range(3))
+            out = torch.stack(rows, 1)
+        return out
+
+    def limit(self, q):
+        """The positivity limiter; its factors are constants of the state (no gradient)."""
+        c = self.cfg
+        if not c.limiter:
+            return q
+        with torch.no_grad():
+            pts = torch.cat([self.face[k] for k in sorted(self.face)])
+            one, zero = torch.ones_like(q[0, RH]), torch.zeros_like(q[0, RH])
+
+            def trace(a):
+                return torch.matmul(pts, a.reshape(c.nbasis, -1)).reshape((-1,) + a.shape[1:])
+
+            floor = q[0, RH] < c.rh_floor
+            low = trace(q[:, RH]).amin(0)
+            th = torch.where(low < c.rh_floor, ((c.rh_floor - q[0, RH]) / (low - q[0, RH])).clamp(0, 1), one)
+            r = q[:, RH] * th
+            r[0] = q[0, RH]
+            pave = self.pressure(q[0])
+            eps = c.rh_floor * c.T_floor
+            e = trace(q[:, EN]) - 0.5 * (trace(q[:, MX]) ** 2 + trace(q[:, MY]) ** 2 + trace(q[:, MZ]) ** 2) / trace(r)
+            pmin = self.gm1 * e.amin(0)
+            tp = torch.where((pmin < eps) & (pave != pmin), ((pave - eps) / (pave - pmin)).clamp(0, 1), one)
+            tp = torch.where(floor | (pave < eps), zero, tp)
+        rows = [q[:, f] for f in range(c.nQ)]
+        for f in range(5):
+            rows[f] = torch.cat([rows[f][:1], rows[f][1:] * (tp * th if f == RH else tp)])
+        rows[RH] = torch.cat([torch.where(floor, torch.full_like(one, c.rh_floor), rows[RH][:1][0])[None],
+                              rows[RH][1:]])
+        return torch.stack(rows, 1)
+
+    def euler(self, m, dt, coll):
+        v = m + dt * self.rhs(m)
+        if self.cfg.ivis == 1 and self.cfg.nQ > 5:
+            v = torch.cat([v[:, :5], v[:, 5:10 if self.cfg.nQ == 13 else 11] / (1.0 + dt * coll)]
+                          + ([v[:, 10:] / (1.0 + dt * self.cfg.coll_q)] if self.cfg.nQ == 13 else []), 1)
+        return v
+
+    def step(self, q, dt, coll):
+        q0 = self.limit(q)
+        v = self.euler(q0, dt, coll)
+        if self.cfg.integrator == "heun":
+            return 0.5 * (q0 + self.euler(self.limit(v), dt, coll))
+        v = 0.75 * q0 + 0.25 * self.euler(self.limit(v), dt, coll)
+        return q0 / 3.0 + 2.0 / 3.0 * self.euler(self.limit(v), dt, coll)
+
+    def dt(self, q):
+        """cflm / (dxi (max wave speed + sound speed of the last cell)), on cell averages."""
+        m, c = q[0], self.cfg
+        u = m[MX:MZ + 1] / m[RH]
+        cs = torch.sqrt(c.gamma * (m[EN] / m[RH] - 0.5 * (u ** 2).sum(0)))
+        speed = u.abs().amax(0) + cs
+        speed = torch.where(m[RH] > 1.01 * c.rh_floor, speed, torch.zeros_like(speed)).max()
+        return c.cflm / ((speed + cs[-1, -1, -1]) * self.dxi[0])
+
+
+def exact(case, seed):
+    if case["kind"] == "ensemble":
+        return None
+    dev = torch.device("cuda" if torch.cuda.is_available() else "cpu")
+    cfg = config(case)
+    ex = Exact(cfg, dev)
+    q = initial(case, cfg, seed, dev)
+    if case["kind"] == "grad":
+        gen = torch.Generator(device=dev)
+        gen.manual_seed(seed + 1)
+        lam = torch.randn(cfg.shape, generator=gen, dtype=torch.float64, device=dev)
+        coll = torch.tensor(float(cfg.coll), dtype=torch.float64, device=dev, requires_grad=True)
+        q.requires_grad_(True)
+        out = q
+        for _ in range(case["nsteps"]):
+            out = ex.step(out, grad_dt(case, cfg), coll)
+        gq, gc = torch.autograd.grad(out, (q, coll), lam)
+        return {"q": out.detach(), "grad_q": gq, "grad_coll": gc}
+    if case["kind"] == "update":
+        return {"q": ex.step(q, FIXED_DT[case["flow"]], cfg.coll)}
+    dt = ex.dt(q)
+    return {"q": ex.step(q, dt, cfg.coll), "t": dt.clone(), "dt": dt}
