@@ -208,7 +208,8 @@ def initial(case, cfg, seed, dev):
         return with_slopes(m0, cfg)
     m0 = torch.zeros((11,) + shape, dtype=torch.float64, device=dev)
     if flow == "channel":
-        m0[:5] = conserved(one, 0.1 * s(8.0), 0.1 * s(8.0), 0.0 * one, one, cfg.gamma)
+        # a spanwise component too: with none, the HLLC branch of the z faces hangs on rounding
+        m0[:5] = conserved(one, 0.1 * s(8.0), 0.1 * s(8.0), 0.1 * s(8.0), one, cfg.gamma)
     else:
         m0[:5] = conserved(1.0 + 0.02 * s(4.0), 0.1 * s(5.0), 0.1 * s(5.0), 0.1 * s(5.0), 1.0 + 0.02 * s(4.0),
                            cfg.gamma)
