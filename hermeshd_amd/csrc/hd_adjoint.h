@@ -143,7 +143,7 @@ __device__ __forceinline__ void flux_vjp(const Phys& ph, const double* Q, const 
 }
 
 // ---------------------------------------------------------------- HLLC ----
-// reverse of pr::hllc<DIR> for the Euler fields: mu (cotangent of out[0..4])
+// reverse of the HLLC flux for the Euler fields: mu (cotangent of out[0..4])
 // -> bQL, bQR (+=, Euler fields), bFL, bFR (+=, Euler fields).  Returns false
 // when no branch applied (out kept the central flux).
 template <int DIR>
@@ -151,7 +151,7 @@ __device__ __forceinline__ bool hllc_vjp(const Phys& ph, const double* QL, const
                                          const pr::Prim& R, const double* mu, double* bQL, double* bQR, double* bFL,
                                          double* bFR) {
     constexpr int IP = MX + DIR, I1 = MX + (DIR + 1) % 3, I2 = MX + (DIR + 2) % 3;
-    // ---- forward, as pr::hllc
+    // ---- forward, as pr::face_flux
     const double rL = QL[RH], rR = QR[RH];
     const double uL = L.u[DIR], uR = R.u[DIR];
     const double v2L = L.u[0] * L.u[0] + L.u[1] * L.u[1] + L.u[2] * L.u[2];

@@ -3,6 +3,7 @@
 // All entry points are stream-ordered and return an error code; none aborts.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -112,7 +113,6 @@ StageParams stage_params(const hd_ctx* c, const double* dt_dev, int combine, int
     sp.noise[3] = c->noise_v;
     sp.nfb = c->nfb;
     sp.inflow = c->inflow;
-    sp.rows_zfast = c->rows_zfast;
     return sp;
 }
 
@@ -248,7 +248,7 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
     g.dzi = (double)cfg->nz / (cfg->lz / 2.0 - (-(cfg->lz / 2.0)));
     for (int s = 0; s < 6; s++) g.bc[s] = cfg->bc[s];
     Phys& ph = c->ph;
-    ph.gamma = cfg->gamma; ph.gm1 = cfg->gamma - 1.;
+    ph.gamma = cfg->gamma; ph.gm1 = cfg->gamma - 1.; ph.gm1i = 1. / ph.gm1;
     ph.P_floor = cfg->T_floor * cfg->rh_floor; ph.rh_floor = cfg->rh_floor;
     ph.colvis = cfg->colvis; ph.c2d3cv = (2. / 3.) * cfg->colvis; ph.c4d3cv = (4. / 3.) * cfg->colvis;
     ph.ivis = cfg->ivis;
@@ -316,22 +316,11 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
         hd_destroy(c);
         return fail(HD_ERR_HIP, "initialising context buffers failed");
     }
-    if (const char* ro = std::getenv("HD_STAGE_ROWS")) c->rows_zfast = std::strcmp(ro, "yz") != 0;
     if (const char* lm = std::getenv("HD_LIMITER")) c->table_limiter = std::strcmp(lm, "table") == 0;
     if (const char* fc = std::getenv("HD_FACES")) c->table_faces = std::strcmp(fc, "table") == 0;
     if (const char* vj = std::getenv("HD_VJP")) c->fused_vjp = std::strcmp(vj, "fused") == 0;
-    // workgroup size of the fused stage kernel: 64, 128 or 256 threads
-    if (const char* bs = std::getenv("HD_STAGE_BLOCK")) {
-        const int v = std::atoi(bs);
-        if (v == 64 || v == 128 || v == 256) c->stage_bs = v;
-    }
-    {
-        const size_t bytes = (size_t)c->nface * c->nQ * cfg->nx * sizeof(double);
-        const char* xs = std::getenv("HD_STAGE_XS");
-        const bool off = xs && std::strcmp(xs, "0") == 0;
-        if (!off && cfg->bc[0] == HD_BC_PERIODIC && cfg->nx % 64 == 0 && cfg->nx <= 256 && bytes <= 65536)
-            c->xs_bytes = (unsigned)bytes;
-    }
+    if (hipDeviceGetAttribute(&c->num_cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) c->num_cus = 256;
+    if (const char* sp = std::getenv("HD_STAGE_PLANES")) c->stage_planes = std::max(-1, std::atoi(sp));
     *out = c;
     return HD_OK;
 }

@@ -17,6 +17,10 @@
 #include "hd_adjoint.h"
 #include "hd_ensemble.h"
 
+namespace hd {
+constexpr int STAGE_AUTO = -2;
+}
+
 struct hd_ctx {
     hd_config cfg;
     int q, nb, nQ, nface;
@@ -52,17 +56,10 @@ struct hd_ctx {
     double rho_mask = 0.;
     double kap_f = 0., kap_v = 0.; // point amplitude factors of the face and volume rules
     bool generic = false;          // HD_KERNELS=generic selects the table-driven kernels
-    // threads per workgroup of the fused stage kernel (HD_STAGE_BLOCK): one
-    // wave per workgroup lets each SIMD start its next wave as soon as its
-    // last one ends (the waves' run times differ with the limiter's early-out)
-    int stage_bs = 64;
-    // LDS bytes of the row-shared x-face stage kernel, 0 when it does not apply
-    // (x not periodic, nx not a multiple of 64 up to 256, or too much LDS);
-    // HD_STAGE_XS=0 switches it off
-    unsigned xs_bytes = 0;
-    // workgroup order of the row-shared kernel: z fastest (HD_STAGE_ROWS=zy, the
-    // default) or y fastest (HD_STAGE_ROWS=yz)
-    int rows_zfast = 1;
+    int num_cus = 0;
+    // how the fused stage takes the grid (sg::stage_planes): chosen from its size,
+    // or set by HD_STAGE_PLANES: -1 five waves a tile, 0 equal runs, n items of n planes
+    int stage_planes = hd::STAGE_AUTO;
     // table-driven limiter kernel instead of fz::k_limit (HD_LIMITER=table)
     int table_limiter = 0;
     // one-thread-per-face k_face_flux for periodic 13-moment grids too (HD_FACES=table)
@@ -101,7 +98,7 @@ struct hd_ens {
     int* err = nullptr;
     unsigned long long* bad = nullptr;
     // launch shape (hd_ens_set_launch / hd_ens_tune)
-    int choice = -1, bs = 256, grid = 0, num_cus = 0;
+    int choice = -1, grid = 0, num_cus = 0;
     hd::ens::Launch launch{};
     // captured step (hd_ens_run)
     hipStream_t cap_stream = nullptr;

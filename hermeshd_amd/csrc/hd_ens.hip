@@ -22,16 +22,12 @@ namespace {
 using namespace hd;
 
 struct Candidate {
-    int bs, bx, by, bz, linear, wg_per_cu, xcd;
+    int zc, xcd;  // planes per workgroup (0: by march_planes' rule), XCD-contiguous chunks of the work list
 };
 
-// Launch shapes the tuner times: runs of consecutive cells or bricks, plain
-// grids (wg_per_cu 0: one workgroup per tile) or persistent grids.
+// Launch shapes the tuner times.
 const Candidate kCandidates[] = {
-    {256, 256, 1, 1, 1, 0, 0}, {256, 256, 1, 1, 1, 1, 1}, {256, 256, 1, 1, 1, 2, 1}, {256, 256, 1, 1, 1, 2, 0},
-    {128, 128, 1, 1, 1, 0, 0}, {128, 128, 1, 1, 1, 2, 1}, {64, 64, 1, 1, 1, 0, 0},    {64, 64, 1, 1, 1, 4, 1},
-    {256, 16, 4, 4, 0, 0, 0},  {256, 16, 4, 4, 0, 1, 1},  {256, 8, 8, 4, 0, 0, 0},    {256, 8, 8, 4, 0, 1, 1},
-    {128, 8, 4, 4, 0, 0, 0},   {128, 8, 4, 4, 0, 2, 1},   {64, 4, 4, 4, 0, 0, 0},     {64, 4, 4, 4, 0, 4, 1},
+    {0, 1}, {0, 0}, {1, 1}, {1, 0}, {2, 1}, {2, 0}, {3, 1}, {3, 0}, {4, 1}, {4, 0}, {8, 1}, {8, 0}, {16, 1}, {16, 0}, {32, 1}, {32, 0},
 };
 constexpr int kNumCandidates = (int)(sizeof(kCandidates) / sizeof(kCandidates[0]));
 
@@ -51,20 +47,28 @@ void drop_graph(hd_ens* e) {
 int set_launch(hd_ens* e, int choice) {
     if (choice < 0 || choice >= kNumCandidates) return fail(HD_ERR_INVALID, "launch choice out of range");
     const Candidate& k = kCandidates[choice];
+    // planes per workgroup: the shape's, or those of least cost
+    int zc = k.zc;
+    if (zc == 0) {
+        int nz = 1;
+        for (const ens::EnsReal& R : e->hreal) nz = std::max(nz, R.g.nz);
+        const long resident = (long)e->num_cus * sg::stage_occupancy(e->nb, e->nQ);
+        double best = 1e300;
+        for (int z = 1; z <= nz && z <= 32; z++) {
+            long items = 0;
+            for (const ens::EnsReal& R : e->hreal) items += (long)R.ntile * ((R.g.nz + z - 1) / z);
+            const double cost = sg::march_cost(items, z, resident);
+            if (cost < best) {
+                best = cost;
+                zc = z;
+            }
+        }
+    }
     e->hwork.clear();
     for (int r = 0; r < e->nreal; r++) {
-        ens::EnsReal& R = e->hreal[r];
-        long ntile;
-        if (k.linear) {
-            R.ntx = R.nty = R.ntz = 0;
-            ntile = (R.g.N + k.bs - 1) / k.bs;
-        } else {
-            R.ntx = (R.g.nx + k.bx - 1) / k.bx;
-            R.nty = (R.g.ny + k.by - 1) / k.by;
-            R.ntz = (R.g.nz + k.bz - 1) / k.bz;
-            ntile = (long)R.ntx * R.nty * R.ntz;
-        }
-        for (long t = 0; t < ntile; t++) e->hwork.push_back(make_int2(r, (int)t));
+        const ens::EnsReal& R = e->hreal[r];
+        const long n = (long)R.ntile * ((R.g.nz + zc - 1) / zc);
+        for (long t = 0; t < n; t++) e->hwork.push_back(make_int2(r, (int)t));
     }
     if (e->hwork.size() > (size_t)0x7fffffff) return fail(HD_ERR_INVALID, "work list too long");
     // launches in flight may still read the old tables
@@ -78,21 +82,10 @@ int set_launch(hd_ens* e, int choice) {
     }
     HIPCHK(hipMemcpy(e->dwork, e->hwork.data(), e->hwork.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(e->dreal, e->hreal.data(), e->hreal.size() * sizeof(ens::EnsReal), hipMemcpyHostToDevice));
-    e->launch.bx = k.bx; e->launch.by = k.by; e->launch.bz = k.bz;
-    e->launch.linear = k.linear;
+    e->launch.zc = zc;
     e->launch.nwork = (int)e->hwork.size();
-    e->bs = k.bs;
-    if (k.wg_per_cu == 0) {
-        e->grid = e->launch.nwork;
-        e->launch.xcd_chunk = 0;
-    } else {
-        // persistent: a multiple of 8 workgroups, at most one per work item
-        // rounded up to 8 (workgroups without items return at once)
-        long g = (long)k.wg_per_cu * e->num_cus;
-        g = std::min<long>(g, ((long)e->launch.nwork + 7) / 8 * 8);
-        e->grid = (int)std::max<long>(8, g / 8 * 8);
-        e->launch.xcd_chunk = k.xcd;
-    }
+    e->launch.xcd_chunk = k.xcd;
+    e->grid = (e->launch.nwork + 7) / 8 * 8;
     e->choice = choice;
     drop_graph(e);
     return HD_OK;
@@ -110,7 +103,6 @@ StageParams ens_params(const hd_ens* e, const double* dt_dev, int combine, int m
     sp.err = e->err;
     sp.bad = e->bad;
     sp.limit_out = 0;
-    sp.rows_zfast = 0;  // the ensemble kernels walk (realization, tile) work lists
     sp.lp = e->lp;
     for (int d = 0; d < 4; d++) sp.noise[d] = nullptr;  // set per realization by the kernel
     sp.nfb = 0;
@@ -233,7 +225,7 @@ int hd_ens_create(const hd_config* base, int32_t nreal, const int32_t* dims, con
     e->dyi = (double)base->ny / base->ly;
     e->dzi = (double)base->nz / base->lz;
     Phys& ph = e->ph;
-    ph.gamma = base->gamma; ph.gm1 = base->gamma - 1.;
+    ph.gamma = base->gamma; ph.gm1 = base->gamma - 1.; ph.gm1i = 1. / ph.gm1;
     ph.P_floor = base->T_floor * base->rh_floor; ph.rh_floor = base->rh_floor;
     ph.colvis = base->colvis; ph.c2d3cv = (2. / 3.) * base->colvis; ph.c4d3cv = (4. / 3.) * base->colvis;
     ph.ivis = base->ivis;
@@ -257,7 +249,7 @@ int hd_ens_create(const hd_config* base, int32_t nreal, const int32_t* dims, con
         R.cell0 = cell0;
         R.nfb = (long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
         R.noff = noff;
-        R.ntx = R.nty = R.ntz = 0;
+        R.ntile = (int)sg::stage_tiles(g);
         R.realization = realization_ids ? realization_ids[r] : base->realization + (uint32_t)r;
         qoff += g.N * e->nQ * e->nb;
         cell0 += g.N;
@@ -430,8 +422,9 @@ int32_t hd_ens_launch_count(void) { return kNumCandidates; }
 int hd_ens_launch_info(int32_t choice, int32_t info[6]) {
     if (!info || choice < 0 || choice >= kNumCandidates) return fail(HD_ERR_INVALID, "bad launch choice");
     const Candidate& k = kCandidates[choice];
-    info[0] = k.bs; info[1] = k.bx; info[2] = k.by; info[3] = k.bz; info[4] = k.linear ? 1 : 0;
-    info[5] = k.wg_per_cu * 2 + k.xcd;  // workgroups per CU (0: one per tile), times 2, plus the XCD flag
+    // 256 threads; a tile of 63 cells along x, zc planes (0: by rule); one workgroup per item
+    info[0] = 256; info[1] = 63; info[2] = 1; info[3] = k.zc; info[4] = 1;
+    info[5] = k.xcd;  // workgroups per CU (0: one per item), times 2, plus the XCD flag
     return HD_OK;
 }
 

@@ -3,17 +3,17 @@
 //
 // The reference runs one realization per process (src/main.f90 time loop,
 // src/random.f90 noise); here the realizations' states are packed back to
-// back, each in the reference layout Q(nx,ny,nz,nQ,nbasis), and a persistent
-// kernel walks a (realization, tile) work list.  A tile is blockDim.x cells:
-// either a run of consecutive cells (linear) or a bx*by*bz brick.  With
-// `xcd_chunk` the list is cut into 8 contiguous chunks, one per XCD, so that
-// a realization's tiles share one L2 (workgroup b runs on XCD b mod 8).
+// back, each in the reference layout Q(nx,ny,nz,nQ,nbasis), and the marching
+// stage kernel (hd_stage.h) takes a list of (realization, tile, planes) items,
+// one a workgroup.  With `xcd_chunk` each XCD takes a contiguous eighth of the
+// list, so that a realization's tiles share one L2 (workgroup b runs on XCD
+// b mod 8).
 // Noise is drawn per realization with the same counter layout as one
 // context, keyed by the realization id, so results do not depend on the
 // schedule.
 #pragma once
-#include "hd_fused.h"
 #include "hd_noise.h"
+#include "hd_stage.h"
 
 namespace hd {
 namespace ens {
@@ -24,101 +24,70 @@ struct EnsReal {
     long noff;     // offset of its noise block: 3 face families of 6*nface*nfb, then 6*npg*N volume
     long nfb;      // (nx+1)(ny+1)(nz+1)
     long cell0;    // first cell of the realization in the packed cell numbering
-    int ntx, nty, ntz;  // tiles per axis (brick tiles)
+    int ntile;     // tiles of a plane
     unsigned int realization;
 };
 
 struct Launch {
-    int bx, by, bz;   // brick shape; bx*by*bz = blockDim.x
-    int linear;       // 1: tiles are runs of blockDim.x consecutive cells
+    int zc;           // planes per item
     int xcd_chunk;    // 1: XCD-contiguous chunks of the work list
     int nwork;
 };
 
-// cell of thread threadIdx.x in tile t of realization R; false when outside
-__device__ __forceinline__ bool tile_cell(const EnsReal& R, const Launch& L, int t, fz::CellPos& cp) {
-    const Grid& g = R.g;
-    if (L.linear) {
-        const long c = (long)t * blockDim.x + threadIdx.x;
-        if (c >= g.N) return false;
-        cp.c = c;
-        cp.i = (int)(c % g.nx);
-        cp.j = (int)((c / g.nx) % g.ny);
-        cp.k = (int)(c / ((long)g.nx * g.ny));
-        return true;
-    }
-    const int tx = t % R.ntx, ty = (t / R.ntx) % R.nty, tz = t / (R.ntx * R.nty);
-    const int lx = threadIdx.x % L.bx, ly = (threadIdx.x / L.bx) % L.by, lz = threadIdx.x / (L.bx * L.by);
-    cp.i = tx * L.bx + lx;
-    cp.j = ty * L.by + ly;
-    cp.k = tz * L.bz + lz;
-    if (cp.i >= g.nx || cp.j >= g.ny || cp.k >= g.nz) return false;
-    cp.c = cp.i + (long)g.nx * (cp.j + (long)g.ny * cp.k);
-    return true;
-}
-
-// Walks the work list: plain striding, or 8 XCD-contiguous chunks.
-template <typename F>
-__device__ __forceinline__ void for_each_item(const Launch& L, F&& f) {
-    if (L.xcd_chunk) {
-        const int x = blockIdx.x & 7, per_xcd = (int)(gridDim.x >> 3), slot = (int)(blockIdx.x >> 3);
-        const int lo = (int)(((long)L.nwork * x) >> 3), hi = (int)(((long)L.nwork * (x + 1)) >> 3);
-        for (int w = lo + slot; w < hi; w += per_xcd) f(w);
-    } else {
-        for (int w = blockIdx.x; w < L.nwork; w += gridDim.x) f(w);
-    }
-}
-
 template <int NB, int QP, int NQ, int RM, bool NZ>
-__global__ __launch_bounds__(256) void k_ens_stage(const double* __restrict__ qin, const double* __restrict__ qn,
-                                                   double* __restrict__ qout, const EnsReal* __restrict__ reals,
-                                                   const int2* __restrict__ work, Launch L, Phys ph,
-                                                   StageParams sp, const float* __restrict__ noise,
-                                                   const unsigned long long* __restrict__ step, long nfloats) {
+__global__ __launch_bounds__(256, (sg::occupancy<NB, NQ>())) void k_ens_stage(
+    const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout,
+    const EnsReal* __restrict__ reals, const int2* __restrict__ work, Launch L, Phys ph, StageParams sp,
+    const float* __restrict__ noise, const unsigned long long* __restrict__ step, long nfloats) {
     constexpr int NF = QP * QP;
-    for_each_item(L, [&](int w) {
-        const int2 wk = work[w];
-        const EnsReal R = reals[wk.x];
-        fz::CellPos cp;
-        if (!tile_cell(R, L, wk.y, cp)) return;
-        StageParams s = sp;
-        if constexpr (NZ) {
-            const long fsz = 6L * NF * R.nfb;
-            // the field of the current step: buffer (step & 1)
-            const float* base = noise + ((*step & 1ull) ? nfloats : 0L) + R.noff;
-            s.noise[0] = base;
-            s.noise[1] = base + fsz;
-            s.noise[2] = base + 2 * fsz;
-            s.noise[3] = base + 3 * fsz;
-            s.nfb = R.nfb;
-        }
-        fz::stage_cell<NB, QP, NQ, RM, NZ>(qin + R.qoff, qn + R.qoff, qout + R.qoff, R.g, ph, s, cp, R.cell0 + cp.c);
-    });
+    __shared__ double lds[sg::lds_doubles<NB, NQ>()];
+    __shared__ int flags[2];
+    const int b = (int)(blockIdx.x >> 3);
+    const int t = L.xcd_chunk ? (int)(blockIdx.x & 7u) * (int)(gridDim.x >> 3) + b : (int)blockIdx.x;
+    if (t >= L.nwork) return;
+    const sg::Shared sh = sg::share<NB, NQ>(lds, flags);
+    const int2 wk = work[t];
+    const EnsReal& R = reals[wk.x];
+    const Grid g = R.g;
+    if constexpr (NZ) {
+        const long fsz = 6L * NF * R.nfb;
+        // the field of the current step: buffer (step & 1)
+        const float* base = noise + ((*step & 1ull) ? nfloats : 0L) + R.noff;
+        sp.noise[0] = base;
+        sp.noise[1] = base + fsz;
+        sp.noise[2] = base + 2 * fsz;
+        sp.noise[3] = base + 3 * fsz;
+        sp.nfb = R.nfb;
+    }
+    const int ch = wk.y / R.ntile, k0 = ch * L.zc, k1 = k0 + L.zc < g.nz ? k0 + L.zc : g.nz;
+    const int part = __builtin_amdgcn_readfirstlane(((int)(threadIdx.x >> 6) + b) & 3);
+    sg::stage_march<NB, QP, NQ, RM, NZ>(qin + R.qoff, qn + R.qoff, qout + R.qoff, g, ph, sp,
+                                        (unsigned)(wk.y - ch * R.ntile), k0, k1, 0, part, R.cell0, sh);
 }
 
+// The limiter, a cell a thread: realizations along y of the grid.
 template <int NB, int QP>
-__global__ __launch_bounds__(256) void k_ens_limit(double* __restrict__ q, const EnsReal* __restrict__ reals,
-                                                   const int2* __restrict__ work, Launch L, LimParams lp) {
-    for_each_item(L, [&](int w) {
-        const int2 wk = work[w];
-        const EnsReal R = reals[wk.x];
-        fz::CellPos cp;
-        if (!tile_cell(R, L, wk.y, cp)) return;
+__global__ __launch_bounds__(256) void k_ens_limit(double* __restrict__ q, const EnsReal* __restrict__ reals, int nreal,
+                                                   LimParams lp) {
+    for (int r = blockIdx.y; r < nreal; r += gridDim.y) {
+        const EnsReal& R = reals[r];
         double* qr = q + R.qoff;
         const long N = R.g.N;
         const int nQ = R.g.nQ;
-        double m[5][NB];
+        for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < N; c += (long)gridDim.x * blockDim.x) {
+            double m[5][NB];
 #pragma unroll
-        for (int r = 0; r < NB; r++)
+            for (int i = 0; i < NB; i++)
 #pragma unroll
-            for (int f = 0; f < 5; f++) m[f][r] = qr[((long)r * nQ + f) * N + cp.c];
-        if (fz::limit_cell<NB, QP, 5>(m, lp)) {
+                for (int f = 0; f < 5; f++) m[f][i] = qr[((long)i * nQ + f) * N + c];
+            if (fz::limit_cell<NB, QP, 5>(m, lp)) {
 #pragma unroll
-            for (int r = 0; r < NB; r++)
+                for (int i = 0; i < NB; i++)
 #pragma unroll
-                for (int f = 0; f < 5; f++) qr[((long)r * nQ + f) * N + cp.c] = m[f][r];
+                    for (int f = 0; f < 5; f++) qr[((long)i * nQ + f) * N + c] = m[f][i];
+            }
         }
-    });
+    }
 }
 
 // Noise of every realization for the current step: flat over all points;

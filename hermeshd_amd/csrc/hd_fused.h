@@ -1,6 +1,6 @@
-// hd_fused.h -- one fused HIP kernel per SSP-RK stage: volume integral, face
-// traces, Riemann fluxes on all six faces, surface lift, sources, update and
-// the SSP combination, for one cell per thread with the state in registers.
+// hd_fused.h -- what the fused kernels share: the basis and quadrature rules as
+// compile-time constants, face polynomials, mode loads, the limiter; and the
+// 13-moment face and cell kernels.
 //
 // Operator (the reference's glflux + innerintegral2 + source_calc +
 // advance_time_level, src/flux.f90:751-1022, src/sources.f90:12-84,
@@ -13,8 +13,6 @@
 // The basis is the Legendre product of src/basis_funcs.f90 with the mode order
 // of src/initialize.f90:126-194; quadrature nodes and weights are the
 // reference's values (1/sqrt(3); sqrt(15)/5, 5/9, 8/9) as exact hex literals.
-// Each interior face's flux is evaluated by both adjacent cells (same inputs,
-// same arithmetic, so both sides use the same value).
 #pragma once
 #include "hd_generic.h"
 #include "hd_prim.h"
@@ -79,6 +77,14 @@ HD_DEV constexpr double cvol(int d, int r, int i, int j, int k) {
     const double b = d == 1 ? Dval<QP>(deg<NB>(r, 1), j) : Lval<QP>(deg<NB>(r, 1), j);
     const double c = d == 2 ? Dval<QP>(deg<NB>(r, 2), k) : Lval<QP>(deg<NB>(r, 2), k);
     return 0.25 * cbasis<NB>(r) * Rule<QP>::w3(i, j, k) * (a * b * c);
+}
+// d(phi_r)/d(xi_d) at g
+template <int NB, int QP>
+HD_DEV constexpr double dphi(int d, int r, int i, int j, int k) {
+    const double a = d == 0 ? Dval<QP>(deg<NB>(r, 0), i) : Lval<QP>(deg<NB>(r, 0), i);
+    const double b = d == 1 ? Dval<QP>(deg<NB>(r, 1), j) : Lval<QP>(deg<NB>(r, 1), j);
+    const double c = d == 2 ? Dval<QP>(deg<NB>(r, 2), k) : Lval<QP>(deg<NB>(r, 2), k);
+    return a * b * c;
 }
 // face point p = (ii,jj), jj fastest: x faces (y=x[jj], z=x[ii]); y faces
 // (x=x[ii], z=x[jj]); z faces (x=x[jj], y=x[ii])  (src/basis_funcs.f90:346-567)
@@ -213,72 +219,6 @@ __device__ __forceinline__ void face_eval(const double (&K)[NQ][NK], const doubl
 // which would stretch live ranges past the register file.
 __device__ __forceinline__ void point_barrier() { __builtin_amdgcn_sched_barrier(0); }
 
-// ------------------------------------------------------------ volume -------
-// innerintegral2 (src/flux.f90:751-928): Q at every Gauss point, the three
-// directional fluxes from one set of primitives, and the projection onto
-// d(phi_r)/d(xi_d) with compile-time weights (zero weights drop out).
-template <int NB, int QP, int NQ, bool NZ>
-__device__ __forceinline__ void volume_term(const double (&m)[NQ][NB], double (&rhs)[NQ][NB], const Phys& ph,
-                                            double dxi, double dyi, double dzi, const StageParams& sp, long c,
-                                            long N) {
-#pragma unroll
-    for (int i = 0; i < QP; i++) {
-        // the stress of the plane's QP*QP points, loaded together so that
-        // the points do not each wait for memory
-        float Sv[QP * QP][6];
-        if constexpr (NZ) {
-            constexpr long npg = QP * QP * QP;
-#pragma unroll
-            for (int jk = 0; jk < QP * QP; jk++)
-#pragma unroll
-                for (int e = 0; e < 6; e++) Sv[jk][e] = sp.noise[3][((long)e * npg + i * QP * QP + jk) * N + c];
-        }
-#pragma unroll
-        for (int j = 0; j < QP; j++)
-#pragma unroll
-            for (int k = 0; k < QP; k++) {
-                double Qp[NQ];
-#pragma unroll
-                for (int f = 0; f < NQ; f++) {
-                    double s = 0.;
-#pragma unroll
-                    for (int r = 0; r < NB; r++) {
-                        const double b = phi_int<NB, QP>(r, i, j, k);
-                        if (b != 0.0) s += b * m[f][r];
-                    }
-                    Qp[f] = s;
-                }
-                const pr::Prim st = pr::prim<NQ>(ph, Qp);
-                double Fx[NQ], Fy[NQ], Fz[NQ];
-                double S[6];
-                const double* Sp = nullptr;
-                if constexpr (NZ) {
-                    // volume point (i,j,k) of the cell: stream id p*N + c
-#pragma unroll
-                    for (int e = 0; e < 6; e++) S[e] = Sv[j * QP + k][e];
-                    Sp = S;
-                }
-                pr::flux<NQ, 0>(ph, Qp, st, Fx, Sp);
-                pr::flux<NQ, 1>(ph, Qp, st, Fy, Sp);
-                pr::flux<NQ, 2>(ph, Qp, st, Fz, Sp);
-#pragma unroll
-                for (int f = 0; f < NQ; f++) {
-                    const double fx = dxi * Fx[f], fy = dyi * Fy[f], fz = dzi * Fz[f];
-#pragma unroll
-                    for (int r = 1; r < NB; r++) {
-                        const double cx = cvol<NB, QP>(0, r, i, j, k);
-                        const double cy = cvol<NB, QP>(1, r, i, j, k);
-                        const double cz = cvol<NB, QP>(2, r, i, j, k);
-                        if (cx != 0.0) rhs[f][r] += cx * fx;
-                        if (cy != 0.0) rhs[f][r] += cy * fy;
-                        if (cz != 0.0) rhs[f][r] += cz * fz;
-                    }
-                }
-                point_barrier();
-            }
-    }
-}
-
 // ------------------------------------------------------------- faces -------
 struct CellPos {
     int i, j, k;
@@ -319,170 +259,6 @@ __device__ __forceinline__ void inflow_ghost(const double* __restrict__ inflow, 
     oth[MY] = 0.0;
     oth[MZ] = 0.0;
     oth[EN] = inflow[base + fs * EN];
-}
-
-// One face of the cell: DIR 0/1/2, SIDE 0 (minus) / 1 (plus).
-// STORE: also write each point's scaled flux to xs[(p*NQ + f)*nx + i] for the
-// x-neighbour's lift (the row-shared x faces of k_stage_xs).
-// Modes of the neighbour across the DIR face on side SIDE (an interior or
-// periodic face).
-template <int NB, int NQ, int DIR, int SIDE>
-__device__ __forceinline__ void load_neighbor(const double* __restrict__ q, const Grid& g, const CellPos& cp,
-                                              double (&nm)[NQ][NB]) {
-    const int n_ax = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
-    const int a = DIR == 0 ? cp.i : DIR == 1 ? cp.j : cp.k;
-    int an = SIDE ? a + 1 : a - 1;
-    if (an < 0) an += n_ax;
-    if (an >= n_ax) an -= n_ax;
-    const long cn = DIR == 0 ? (cp.c - cp.i + an)
-                  : DIR == 1 ? (cp.c + (long)(an - cp.j) * g.nx)
-                             : (cp.c + (long)(an - cp.k) * g.nx * g.ny);
-    load_modes<NB, NQ>(q, g, cn, nm);
-}
-
-// PRE: the neighbour's modes were loaded earlier (pre), so that their
-// latency overlapped other work.
-template <int NB, int QP, int NQ, int RM, bool NZ, int DIR, int SIDE, bool STORE = false, bool PRE = false>
-__device__ __forceinline__ void face_term(const double* __restrict__ q, const Grid& g, const CellPos& cp,
-                                          const double (&m)[NQ][NB], double (&rhs)[NQ][NB], const Phys& ph,
-                                          double dxi_d, const StageParams& sp, double* xs = nullptr,
-                                          const double (*pre)[NB] = nullptr) {
-    constexpr int NF = QP * QP;
-    const auto& T = face_tab<NB>();
-    const int n_ax = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
-    const int a = DIR == 0 ? cp.i : DIR == 1 ? cp.j : cp.k;
-    const bool at_edge = SIDE ? (a == n_ax - 1) : (a == 0);
-    const int bc = g.bc[2 * DIR + SIDE];
-    const bool ext = at_edge && bc != BC_PERIODIC;
-    constexpr int NK = face_nk<NB>();
-    const auto& FP = face_poly<NB>();
-    double ko[NQ][NK], kn[NQ][NK];
-    face_coeffs<NB, NQ, DIR, SIDE, NK>(m, ko);
-    if (!ext) {
-        double nm[NQ][NB];
-        if constexpr (PRE) {
-#pragma unroll
-            for (int f = 0; f < NQ; f++)
-#pragma unroll
-                for (int r = 0; r < NB; r++) nm[f][r] = pre[f][r];
-        } else {
-            load_neighbor<NB, NQ, DIR, SIDE>(q, g, cp, nm);
-        }
-        face_coeffs<NB, NQ, DIR, 1 - SIDE, NK>(nm, kn);
-    }
-    // outflow boundaries decide on the whole face (src/boundary.f90:213-338)
-    bool zero_normal = false;
-    if (ext && bc == BC_OUTFLOW && !(DIR == 0 && SIDE == 1)) {
-        double v = 0.;
-        for (int p = 0; p < NF; p++) {
-            double s = 0.;
-#pragma unroll
-            for (int r = 0; r < NB; r++) s += T.bf[DIR][SIDE][p][r] * m[MX + DIR][r];
-            v = (p == 0) ? s : (SIDE ? fmin(v, s) : fmax(v, s));
-        }
-        zero_normal = SIDE ? (v < 0.0) : (v > 0.0);
-    }
-    long fid = 0;
-    if constexpr (NZ) {
-        // lattice id of this face; a periodic high face is the low face
-        int af = a + SIDE;
-        if (af == n_ax && bc == BC_PERIODIC) af = 0;
-        const int fi = DIR == 0 ? af : cp.i, fj = DIR == 1 ? af : cp.j, fk = DIR == 2 ? af : cp.k;
-        fid = (long)fi + (long)(g.nx + 1) * ((long)fj + (long)(g.ny + 1) * fk);
-    }
-    // the stress of all the face's points, loaded before the point loop
-    float Sf[NZ ? NF : 1][6];
-    if constexpr (NZ) {
-#pragma unroll
-        for (int p = 0; p < NF; p++)
-#pragma unroll
-            for (int e = 0; e < 6; e++) Sf[p][e] = sp.noise[DIR][((long)e * NF + p) * sp.nfb + fid];
-    }
-#pragma unroll 1
-    for (int p = 0; p < NF; p++) {
-        double own[NQ], oth[NQ];
-        face_eval<NQ, NK>(ko, FP.b[p], own);
-        if (!ext) {
-            face_eval<NQ, NK>(kn, FP.b[p], oth);
-        } else {
-#pragma unroll
-            for (int f = 0; f < NQ; f++) oth[f] = own[f];
-            if (bc == BC_NOSLIP) {
-                oth[MX] = oth[MY] = oth[MZ] = 0.0;
-            } else if (bc == BC_WALL) {
-                oth[MX + DIR] = 0.0;
-            } else if (bc == BC_OUTFLOW) {
-                if (DIR == 0 && SIDE == 1) {
-                    if (oth[MX] > 0.0) oth[MX] = -own[MX];
-                } else if (zero_normal) {
-                    oth[MX + DIR] = 0.0;
-                }
-            }
-            if constexpr (DIR == 0 && SIDE == 0) {
-                // x_bc_inflow (src/boundary.f90:571-592): prescribed rh, mx, en;
-                // no transverse momentum; the stress fields from the interior
-                if (bc == BC_INFLOW) inflow_ghost<NQ>(sp.inflow, g, cp, p, QP * QP, oth);
-            }
-        }
-        const double* QL = SIDE ? own : oth;
-        const double* QR = SIDE ? oth : own;
-        double S[6];
-        const double* Sp = nullptr;
-        if constexpr (NZ) {
-            // p is a loop counter (not unrolled): select rather than index,
-            // which keeps Sf in registers
-#pragma unroll
-            for (int e = 0; e < 6; e++) S[e] = Sf[0][e];
-#pragma unroll
-            for (int pp = 1; pp < NF; pp++)
-                if (pp == p)
-#pragma unroll
-                    for (int e = 0; e < 6; e++) S[e] = Sf[pp][e];
-            Sp = S;
-        }
-        double FL[NQ], FR[NQ], out[NQ];
-        if constexpr (RM == RIEMANN_ROE) {
-            flux_point<NQ, DIR>(ph, QL, FL, Sp);
-            flux_point<NQ, DIR>(ph, QR, FR, Sp);
-#pragma unroll
-            for (int f = 0; f < NQ; f++) out[f] = 0.5 * (FL[f] + FR[f]);
-            roe_point<DIR>(ph, QL, QR, FL, FR, out);
-        } else {
-            const pr::Prim sL = pr::prim<NQ>(ph, QL), sR = pr::prim<NQ>(ph, QR);
-            pr::flux<NQ, DIR>(ph, QL, sL, FL, Sp);
-            pr::flux<NQ, DIR>(ph, QR, sR, FR, Sp);
-#pragma unroll
-            for (int f = 0; f < NQ; f++) out[f] = 0.5 * (FL[f] + FR[f]);
-            if constexpr (RM == RIEMANN_HLLC) pr::hllc<DIR>(ph, QL, sL, QR, sR, FL, FR, out);
-        }
-#pragma unroll
-        for (int f = 0; f < NQ; f++) {
-            const double v = dxi_d * out[f];
-            if constexpr (STORE) xs[(long)(p * NQ + f) * g.nx + cp.i] = v;
-#pragma unroll
-            for (int r = 0; r < NB; r++) rhs[f][r] += T.cf[DIR][SIDE][p][r] * v;
-        }
-    }
-}
-
-// The -x face of a cell is the +x face of its left neighbour in the same row:
-// its scaled point fluxes come from xs (written by that neighbour), bitwise
-// what the cell would compute itself, and only the lift is done here.
-template <int NB, int QP, int NQ>
-__device__ __forceinline__ void x_lift_shared(const double* __restrict__ xs, const Grid& g, const CellPos& cp,
-                                              double (&rhs)[NQ][NB]) {
-    constexpr int NF = QP * QP;
-    const auto& T = face_tab<NB>();
-    const int il = cp.i == 0 ? g.nx - 1 : cp.i - 1;
-#pragma unroll 1
-    for (int p = 0; p < NF; p++) {
-#pragma unroll
-        for (int f = 0; f < NQ; f++) {
-            const double v = xs[(long)(p * NQ + f) * g.nx + il];
-#pragma unroll
-            for (int r = 0; r < NB; r++) rhs[f][r] += T.cf[0][0][p][r] * v;
-        }
-    }
 }
 
 // ----------------------------------------------------------- limiter -------
@@ -616,171 +392,6 @@ __global__ __launch_bounds__(256, (NB == 4 ? 4 : (NB == 8 ? 2 : 1))) void k_limi
 
 // ------------------------------------------------------------ kernel -------
 __device__ __forceinline__ void fence() { asm volatile("" ::: "memory"); }
-
-// advance_time_level and the SSP combination of one cell (src/integrator.f90:
-// 62-86, 210-232): rhs becomes m + dt*rhs (the stress fields scaled by faci
-// under ivis 1), combined with the step-start state qn by COMB (0: none,
-// 1: RK2 (qn+v)/2, 2: RK3 3qn/4 + v/4, 3: RK3 qn/3 + 2v/3).  Returns whether a
-// mean value came out NaN.
-template <int NB, int NQ, int COMB>
-__device__ __forceinline__ bool advance(const double (&m)[NQ][NB], double (&rhs)[NQ][NB],
-                                        const double* __restrict__ qn, long N, long c, double dt, double faci,
-                                        bool relax) {
-    double q0[COMB ? NQ : 1][COMB ? NB : 1];
-    if constexpr (COMB != 0) load_modes<NB, NQ>(qn, N, c, q0);
-    bool bad = false;
-#pragma unroll
-    for (int f = 0; f < NQ; f++)
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            double v = m[f][r] + dt * rhs[f][r];
-            if (f >= PXX && relax) v = faci * v;
-            if (r == 0 && v != v) bad = true;
-            if constexpr (COMB == 1) v = 0.5 * (q0[f][r] + v);
-            if constexpr (COMB == 2) v = 0.75 * q0[f][r] + 0.25 * v;
-            if constexpr (COMB == 3) v = (1. / 3.) * q0[f][r] + (2. / 3.) * v;
-            rhs[f][r] = v;  // reuse the accumulator as the output cell
-        }
-    return bad;
-}
-
-// One cell of one stage; `bad_id` is the index reported when mode 1 of the
-// output is NaN.
-// XS: the workgroup is one periodic row of cells (k_stage_xs); each x face is
-// evaluated once, by its left cell, and shared through xs (LDS).
-template <int NB, int QP, int NQ, int RM, bool NZ, bool XS = false>
-__device__ __forceinline__ void stage_cell(const double* __restrict__ qin, const double* __restrict__ qn,
-                                           double* __restrict__ qout, const Grid& g, const Phys& ph,
-                                           const StageParams& sp, const CellPos& cp, long bad_id,
-                                           double* xs = nullptr) {
-    const long c = cp.c;
-    double m[NQ][NB];
-    load_modes<NB, NQ>(qin, g, c, m);
-    double rhs[NQ][NB];
-#pragma unroll
-    for (int f = 0; f < NQ; f++)
-#pragma unroll
-        for (int r = 0; r < NB; r++) rhs[f][r] = 0.;
-    // The fences keep each section's loads inside it, so the compiler does not
-    // hoist all six neighbours' modes at once (which would spill).  The first
-    // face's neighbour is loaded ahead of the volume term, whose arithmetic
-    // covers that load's latency.
-    double nm0[NQ][NB];
-    if constexpr (XS) {
-        load_neighbor<NB, NQ, 0, 1>(qin, g, cp, nm0);
-    } else {
-        if (!(cp.i == 0 && g.bc[0] != BC_PERIODIC)) load_neighbor<NB, NQ, 0, 0>(qin, g, cp, nm0);
-    }
-    volume_term<NB, QP, NQ, NZ>(m, rhs, ph, g.dxi, g.dyi, g.dzi, sp, c, g.N);
-    fence();
-    if constexpr (XS) {
-        face_term<NB, QP, NQ, RM, NZ, 0, 1, true, true>(qin, g, cp, m, rhs, ph, g.dxi, sp, xs, nm0);
-        __syncthreads();
-        x_lift_shared<NB, QP, NQ>(xs, g, cp, rhs);
-    } else {
-        face_term<NB, QP, NQ, RM, NZ, 0, 0, false, true>(qin, g, cp, m, rhs, ph, g.dxi, sp, nullptr, nm0);
-        fence();
-        face_term<NB, QP, NQ, RM, NZ, 0, 1>(qin, g, cp, m, rhs, ph, g.dxi, sp);
-    }
-    fence();
-    face_term<NB, QP, NQ, RM, NZ, 1, 0>(qin, g, cp, m, rhs, ph, g.dyi, sp);
-    fence();
-    face_term<NB, QP, NQ, RM, NZ, 1, 1>(qin, g, cp, m, rhs, ph, g.dyi, sp);
-    fence();
-    face_term<NB, QP, NQ, RM, NZ, 2, 0>(qin, g, cp, m, rhs, ph, g.dzi, sp);
-    fence();
-    face_term<NB, QP, NQ, RM, NZ, 2, 1>(qin, g, cp, m, rhs, ph, g.dzi, sp);
-    fence();
-    // sources (src/sources.f90:12-84): ivis 0 relaxes the stress explicitly
-    // (-coll*P, projected exactly in modal space); body force rho*g, m.g
-    if constexpr (NQ >= 11) {
-        if (sp.ivis == 0 && sp.coll != 0.)
-#pragma unroll
-            for (int f = PXX; f <= PYZ; f++)
-#pragma unroll
-                for (int r = 0; r < NB; r++) rhs[f][r] += -sp.coll * m[f][r];
-    }
-    if (sp.bf[0] != 0. || sp.bf[1] != 0. || sp.bf[2] != 0.) {
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            rhs[MX][r] += sp.bf[0] * m[RH][r];
-            rhs[MY][r] += sp.bf[1] * m[RH][r];
-            rhs[MZ][r] += sp.bf[2] * m[RH][r];
-            rhs[EN][r] += sp.bf[0] * m[MX][r] + sp.bf[1] * m[MY][r] + sp.bf[2] * m[MZ][r];
-        }
-    }
-    // advance_time_level + SSP combination
-    const double dt = *sp.dt;
-    const double faci = 1. / (1. + dt * sp.coll);
-    bool bad = false;
-    if (sp.mode == 1) {
-#pragma unroll
-        for (int f = 0; f < NQ; f++)
-#pragma unroll
-            for (int r = 0; r < NB; r++) qout[((long)r * NQ + f) * g.N + c] = rhs[f][r];
-        return;
-    }
-    // one branch per combination, outside the element loop, so that the
-    // step-start values are loaded together rather than one per branch
-    const bool relax = NQ >= 11 && sp.ivis == 1;
-    switch (sp.combine) {
-        case 1: bad = advance<NB, NQ, 1>(m, rhs, qn, g.N, c, dt, faci, relax); break;
-        case 2: bad = advance<NB, NQ, 2>(m, rhs, qn, g.N, c, dt, faci, relax); break;
-        case 3: bad = advance<NB, NQ, 3>(m, rhs, qn, g.N, c, dt, faci, relax); break;
-        default: bad = advance<NB, NQ, 0>(m, rhs, qn, g.N, c, dt, faci, relax); break;
-    }
-    // When this output is the next stage's input, apply that stage's limiter
-    // here: the reference limits the stage input in place before anything
-    // reads it (src/integrator.f90:106-113), so the stored values are the same.
-    if (sp.limit_out) limit_cell<NB, QP, NQ>(rhs, sp.lp);
-#pragma unroll
-    for (int f = 0; f < NQ; f++)
-#pragma unroll
-        for (int r = 0; r < NB; r++) qout[((long)r * NQ + f) * g.N + c] = rhs[f][r];
-    if (bad) {
-        atomicOr(sp.err, 1);
-        atomicMin(sp.bad, (unsigned long long)bad_id);
-    }
-}
-
-
-template <int NB, int QP, int NQ, int RM, bool NZ>
-__global__ __launch_bounds__(256) void k_stage(const double* __restrict__ qin, const double* __restrict__ qn,
-                                               double* __restrict__ qout, Grid g, Phys ph, StageParams sp) {
-    const long c = (long)xcd_block() * blockDim.x + threadIdx.x;
-    if (c >= g.N) return;
-    CellPos cp;
-    cp.c = c;
-    cp.i = (int)(c % g.nx);
-    cp.j = (int)((c / g.nx) % g.ny);
-    cp.k = (int)(c / ((long)g.nx * g.ny));
-    stage_cell<NB, QP, NQ, RM, NZ>(qin, qn, qout, g, ph, sp, cp, c);
-}
-
-// One periodic row of nx cells per workgroup (nx a multiple of 64, at most
-// 256): the x faces are evaluated once and shared through LDS
-// (NF*NQ*nx doubles of dynamic shared memory).  The grid covers the rows
-// exactly, so every thread reaches the barrier.  Each XCD takes a contiguous
-// range of workgroups; with rows_zfast the rows run with z fastest, so that
-// a row's z neighbours are the adjacent workgroups and its y neighbours nz
-// workgroups away, both inside the window of rows in flight on that XCD
-// (whose L2 then serves the neighbour modes); otherwise y runs fastest.
-template <int NB, int QP, int NQ, int RM, bool NZ>
-__global__ __launch_bounds__(256) void k_stage_xs(const double* __restrict__ qin, const double* __restrict__ qn,
-                                                  double* __restrict__ qout, Grid g, Phys ph, StageParams sp) {
-    extern __shared__ double xs[];
-    const long r = (long)xcd_block();
-    const int j = sp.rows_zfast ? (int)(r / g.nz) : (int)(r % g.ny);
-    const int k = sp.rows_zfast ? (int)(r % g.nz) : (int)(r / g.ny);
-    const long row = (long)j + (long)g.ny * k;
-    const long c = row * g.nx + threadIdx.x;
-    CellPos cp;
-    cp.c = c;
-    cp.i = (int)threadIdx.x;
-    cp.j = j;
-    cp.k = k;
-    stage_cell<NB, QP, NQ, RM, NZ, true>(qin, qn, qout, g, ph, sp, cp, c, xs);
-}
 
 // Face fluxes of the 13-moment model on a grid periodic in every direction,
 // as face moments fl[((f*NK + k)*nfaces) + face] (lift13_mom).  A workgroup

@@ -2,6 +2,9 @@
 // configuration; included by the instantiation units only.
 #pragma once
 #include "hd_ctx.h"
+#include "hd_stage.h"
+
+#include <algorithm>
 
 namespace hd {
 
@@ -53,47 +56,56 @@ struct Impl {
                            c->fl[1], c->fl[2], c->dtab, c->grid, c->ph, sp);
     }
     static void fused(hd_ctx* c, const double* qin, const double* qn, double* qout, const StageParams& sp, hipStream_t s) {
-        const int bs = c->stage_bs;
-        if (c->xs_bytes) {
-            // one periodic row per workgroup, x faces shared through LDS
-            const unsigned rows = (unsigned)(c->N / c->grid.nx);
-            if constexpr (NQ >= 11) {
-                if (sp.noise[0]) {
-                    hipLaunchKernelGGL((fz::k_stage_xs<NB, QP, NQ, RM, true>), dim3(rows), dim3(c->grid.nx),
-                                       c->xs_bytes, s, qin, qn, qout, c->grid, c->ph, sp);
-                    return;
+        const Grid& g = c->grid;
+        const unsigned tiles = sg::stage_tiles(g);
+        const int planes = c->stage_planes == STAGE_AUTO
+                               ? sg::stage_planes<NB, NQ>((long)tiles, g.nz, c->num_cus)
+                               : c->stage_planes;
+        if constexpr (!(NB == 10 && NQ >= 11)) {  // its five waves would not have the registers
+            if (planes < 0) {
+                const unsigned n = tiles * (unsigned)g.nz, grid = (n + 7) / 8 * 8;
+                if constexpr (NQ >= 11) {
+                    if (sp.noise[0]) {
+                        hipLaunchKernelGGL((sg::k_stage_wide<NB, QP, NQ, RM, true>), dim3(grid), dim3(320), 0, s, qin,
+                                           qn, qout, g, c->ph, sp, tiles, n);
+                        return;
+                    }
                 }
-            }
-            hipLaunchKernelGGL((fz::k_stage_xs<NB, QP, NQ, RM, false>), dim3(rows), dim3(c->grid.nx), c->xs_bytes, s,
-                               qin, qn, qout, c->grid, c->ph, sp);
-            return;
-        }
-        if constexpr (NQ >= 11) {
-            if (sp.noise[0]) {
-                hipLaunchKernelGGL((fz::k_stage<NB, QP, NQ, RM, true>), dim3(blocks_for(c->N, bs)), dim3(bs), 0, s,
-                                   qin, qn, qout, c->grid, c->ph, sp);
+                hipLaunchKernelGGL((sg::k_stage_wide<NB, QP, NQ, RM, false>), dim3(grid), dim3(320), 0, s, qin, qn,
+                                   qout, g, c->ph, sp, tiles, n);
                 return;
             }
         }
-        hipLaunchKernelGGL((fz::k_stage<NB, QP, NQ, RM, false>), dim3(blocks_for(c->N, bs)), dim3(bs), 0, s, qin, qn,
-                           qout, c->grid, c->ph, sp);
+        const int zc = planes > 0 ? planes : 0;
+        const long n = zc ? (long)tiles * ((g.nz + zc - 1) / zc)
+                          : std::min((long)tiles * g.nz, (long)c->num_cus * sg::occupancy<NB, NQ>());
+        const unsigned grid = (unsigned)((n + 7) / 8 * 8);
+        if constexpr (NQ >= 11) {
+            if (sp.noise[0]) {
+                hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, true>), dim3(grid), dim3(256), 0, s, qin, qn, qout, g,
+                                   c->ph, sp, tiles, zc);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, false>), dim3(grid), dim3(256), 0, s, qin, qn, qout, g, c->ph,
+                           sp, tiles, zc);
     }
     static void ens_limit(hd_ens* e, double* q, hipStream_t s) {
-        hipLaunchKernelGGL((ens::k_ens_limit<NB, QP>), dim3(e->grid), dim3(e->bs), 0, s, q, e->dreal, e->dwork,
-                           e->launch, e->lp);
+        hipLaunchKernelGGL((ens::k_ens_limit<NB, QP>), dim3(64, (unsigned)(e->nreal < 65535 ? e->nreal : 65535)),
+                           dim3(256), 0, s, q, e->dreal, e->nreal, e->lp);
     }
     static void ens_stage(hd_ens* e, const double* qin, const double* qn, double* qout, const StageParams& sp,
                           hipStream_t s) {
         if constexpr (NQ >= 11) {
             if (e->base.noise) {
-                hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, true>), dim3(e->grid), dim3(e->bs), 0, s, qin,
-                                   qn, qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr,
+                hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, true>), dim3(e->grid), dim3(256), 0, s, qin, qn,
+                                   qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr,
                                    e->noise_floats);
                 return;
             }
         }
-        hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, false>), dim3(e->grid), dim3(e->bs), 0, s, qin, qn,
-                           qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr, e->noise_floats);
+        hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, false>), dim3(e->grid), dim3(256), 0, s, qin, qn, qout,
+                           e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr, e->noise_floats);
     }
     // defined in hd_impl_vjp.h; the units that include it instantiate it
     // there, and hd_k4_vjp.hip holds the nbasis 4 instances, so that those

@@ -26,6 +26,7 @@ enum : int { RIEMANN_CENTRAL = 0, RIEMANN_HLLC = 1, RIEMANN_ROE = 2 };
 
 struct Phys {
     double gamma, gm1;       // aindex, aindm1
+    double gm1i;             // 1/(gamma - 1)
     double P_floor, rh_floor;
     double colvis, c2d3cv, c4d3cv;
     int ivis;                // 2: full 10-moment equations (table-driven kernels only)

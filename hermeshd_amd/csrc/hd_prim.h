@@ -88,55 +88,118 @@ __device__ __forceinline__ double contact_num(double aR, double uR, double aL, d
     return aR * uR - aL * uL + pL - pR;
 }
 
-// HLLC (Batten 1997 with Davis speeds) at one face point from primitives;
-// out[] holds the central flux on entry and keeps it when no branch applies.
-template <int DIR>
-__device__ __forceinline__ void hllc(const Phys& ph, const double* QL, const Prim& L, const double* QR, const Prim& R,
-                                     const double* FL, const double* FR, double* out) {
-    constexpr int IP = MX + DIR, I1 = MX + (DIR + 1) % 3, I2 = MX + (DIR + 2) % 3;
+// sqrt by the hardware estimate of 1/sqrt and two Goldschmidt steps, accurate
+// to an ulp; 0 for 0, NaN below 0.
+__device__ __forceinline__ double root(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x == 0.0 ? x : g;
+}
+
+// Flux through one face point from the two traces: rh..en by the Riemann
+// solver RM, and with stress (NQ >= 11, traces holding rh..en and row DIR of
+// the stress) the averaged velocity in F[5..7], to which the central fluxes
+// of the stress rows are proportional.  S: the row of the stochastic stress.
+// HLLC keeps density, velocity and pressure of both sides, selects one, and
+// forms the conserved values and the flux of that side only (few values are
+// live at a time; the momentum and energy come back to rounding).  HLLC after
+// Batten 1997 with Davis speeds, the order of the branches hllc_point's.
+template <int NQ, int DIR, int RM, bool NZ>
+__device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, const double* QR, const double* S,
+                                          double* F) {
+    constexpr int IP = MX + DIR;
     const double rL = QL[RH], rR = QR[RH];
-    const double uL = L.u[DIR], uR = R.u[DIR];
-    // HLLC pressure: gm1*(E - 0.5*rho*|v|^2), no floor (src/flux.f90:510-520)
-    const double pL = ph.gm1 * (QL[EN] - 0.5 * rL * (L.u[0] * L.u[0] + L.u[1] * L.u[1] + L.u[2] * L.u[2]));
-    const double pR = ph.gm1 * (QR[EN] - 0.5 * rR * (R.u[0] * R.u[0] + R.u[1] * R.u[1] + R.u[2] * R.u[2]));
-    const double cL = sqrt(ph.gamma * pL * L.ri), cR = sqrt(ph.gamma * pR * R.ri);
-    const double SL = fmin(uL - cL, uR - cR);
-    const double SR = fmax(uR + cR, uL + cL);
-    const double aR = rR * (SR - uR), aL = rL * (SL - uL);
+    const double riL = rcp(rL), riR = rcp(rR);
+    const double uL[3] = {QL[MX] * riL, QL[MY] * riL, QL[MZ] * riL};
+    const double uR[3] = {QR[MX] * riR, QR[MY] * riR, QR[MZ] * riR};
+    const double pL = ph.gm1 * fma(-0.5, fma(QL[MX], uL[0], fma(QL[MY], uL[1], QL[MZ] * uL[2])), QL[EN]);
+    const double pR = ph.gm1 * fma(-0.5, fma(QR[MX], uR[0], fma(QR[MY], uR[1], QR[MZ] * uR[2])), QR[EN]);
+    if constexpr (NQ >= 11) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) F[5 + a] = 0.5 * (uL[a] + uR[a]);
+    }
+    // physical flux of one side: floored pressure, stress row less the noise
+    auto side_flux = [&](const double* Q, const double* u, double p, const double* P3, double* f) {
+        const double pf = p < ph.P_floor ? ph.P_floor : p;
+        const double un = u[DIR];
+        f[RH] = Q[IP];
+        f[EN] = (Q[EN] + pf) * un;
+        if constexpr (NQ >= 11) {
+            double Pn[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                Pn[a] = P3[a];
+                if constexpr (NZ) Pn[a] -= S[a];
+                f[MX + a] = fma(Q[MX + a], un, a == DIR ? Pn[a] + pf : Pn[a]);
+            }
+            f[EN] += fma(Pn[0], u[0], fma(Pn[1], u[1], Pn[2] * u[2]));
+        } else {
+#pragma unroll
+            for (int a = 0; a < 3; a++) f[MX + a] = a == DIR ? fma(Q[MX + a], un, pf) : Q[MX + a] * un;
+        }
+    };
+    if constexpr (RM != RIEMANN_HLLC) {
+        double FL[5], FR[5];
+        side_flux(QL, uL, pL, QL + 5, FL);
+        side_flux(QR, uR, pR, QR + 5, FR);
+#pragma unroll
+        for (int f = 0; f < 5; f++) F[f] = 0.5 * (FL[f] + FR[f]);
+        if constexpr (RM == RIEMANN_ROE) roe_point<DIR>(ph, QL, QR, FL, FR, F);
+        return;
+    }
+    const double nL = uL[DIR], nR = uR[DIR];
+    const double cL = root(ph.gamma * pL * riL), cR = root(ph.gamma * pR * riR);
+    const double SL = fmin(nL - cL, nR - cR), SR = fmax(nR + cR, nL + cL);
+    const double aR = rR * (SR - nR), aL = rL * (SL - nL);
     double sm_den = aR - aL;
     if (sm_den == 0.0) sm_den = ph.rh_floor;
-    const double SM = divide(contact_num(aR, uR, aL, uL, pL, pR), sm_den);
-    int sel = -1;
-    if (SL > 0.0) sel = 0;
-    if (SL <= 0.0 && 0.0 < SM) sel = 1;
-    if (SM <= 0.0 && 0.0 <= SR) sel = 2;
-    if (SR < 0.0) sel = 3;
-    if (sel == 0) {
-        out[RH] = FL[RH]; out[MX] = FL[MX]; out[MY] = FL[MY]; out[MZ] = FL[MZ]; out[EN] = FL[EN];
-    } else if (sel == 3) {
-        out[RH] = FR[RH]; out[MX] = FR[MX]; out[MY] = FR[MY]; out[MZ] = FR[MZ]; out[EN] = FR[EN];
-    } else if (sel > 0) {
-        const bool left = (sel == 1);
-        const double* Qk = left ? QL : QR;
-        const double* Fk = left ? FL : FR;
-        const double Sk = left ? SL : SR;
-        const double uk = left ? uL : uR, pk = left ? pL : pR;
-        const double pstar = rL * (uL - SL) * (uL - SM) + pL;  // Eq. (36)
-        double den = Sk - SM;
-        if (den == 0.0) den = ph.rh_floor;
-        const double slrm_i = rcp(den);
-        const double sq = Sk - uk;
-        const double s0 = Qk[RH] * sq * slrm_i;
-        const double s1 = (sq * Qk[IP] + pstar - pk) * slrm_i;
-        const double s2 = sq * Qk[I1] * slrm_i;
-        const double s3 = sq * Qk[I2] * slrm_i;
-        const double s4 = (sq * Qk[EN] - pk * uk + pstar * SM) * slrm_i;
-        out[RH] = Fk[RH] + Sk * (s0 - Qk[RH]);
-        out[IP] = Fk[IP] + Sk * (s1 - Qk[IP]);
-        out[I1] = Fk[I1] + Sk * (s2 - Qk[I1]);
-        out[I2] = Fk[I2] + Sk * (s3 - Qk[I2]);
-        out[EN] = Fk[EN] + Sk * (s4 - Qk[EN]);
+    const double SM = divide(contact_num(aR, nR, aL, nL, pL, pR), sm_den);
+    const double pstar = fma(-aL, nL - SM, pL);  // Eq. (36)
+    // the last true of: SL > 0 (left), SL <= 0 < SM (left star),
+    // SM <= 0 <= SR (right star), SR < 0 (right)
+    const bool s3 = SR < 0.0, s2 = SM <= 0.0 && 0.0 <= SR, s1 = SL <= 0.0 && 0.0 < SM, s0 = SL > 0.0;
+    // NaN speeds: the central flux (the reference's default), before the
+    // selection so that only one side's values are live after it
+    const bool none = !(s0 || s1 || s2 || s3);
+    if (__builtin_expect(none, 0)) {
+        double FL[5], FR[5];
+        side_flux(QL, uL, pL, QL + 5, FL);
+        side_flux(QR, uR, pR, QR + 5, FR);
+#pragma unroll
+        for (int e = 0; e < 5; e++) F[e] = 0.5 * (FL[e] + FR[e]);
     }
+    const bool right = s3 || s2;
+    const double r = right ? rR : rL, p = right ? pR : pL, Sk = right ? SR : SL;
+    double u[3], P3[3] = {0., 0., 0.}, Q[5], f[5];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        u[a] = right ? uR[a] : uL[a];
+        if constexpr (NQ >= 11) P3[a] = right ? QR[5 + a] : QL[5 + a];
+    }
+    if (none) return;
+    Q[RH] = r;
+#pragma unroll
+    for (int a = 0; a < 3; a++) Q[MX + a] = r * u[a];
+    Q[EN] = fma(0.5, fma(Q[MX], u[0], fma(Q[MY], u[1], Q[MZ] * u[2])), p * ph.gm1i);
+    side_flux(Q, u, p, P3, f);
+    if (s3 || !(s2 || s1)) {  // supersonic: the side's own flux
+#pragma unroll
+        for (int e = 0; e < 5; e++) F[e] = f[e];
+        return;
+    }
+    double den = Sk - SM;
+    if (den == 0.0) den = ph.rh_floor;
+    const double sr = Sk * rcp(den);
+    // F + Sk*(Q* - Q) with Q* = (Sk - un)/(Sk - SM) Q + pressure terms
+    const double ga = fma(sr, Sk - u[DIR], -Sk);
+#pragma unroll
+    for (int e = 0; e < 5; e++) F[e] = fma(ga, Q[e], f[e]);
+    F[IP] = fma(sr, pstar - p, F[IP]);
+    F[EN] = fma(sr, fma(pstar, SM, -(p * u[DIR])), F[EN]);
 }
 
 }  // namespace pr

@@ -1,0 +1,1059 @@
+// hd_stage.h -- one RK stage of the fused path: a workgroup of waves per run
+// of cells, the stage's parts spread over the waves.
+//
+// The operator is that of hd_fused.h (volume integral, Riemann fluxes on six
+// faces, lifts, sources, update, SSP combination, the next stage's limiter).
+// A tile is 64 consecutive positions of a plane's row lattice (nx+1 positions
+// per row: the faces across x), one per lane; it updates the cells of its
+// first 63 positions, so that the face above a cell in x is always the next
+// lane's.  A workgroup steps its tile through planes of z:
+//   part 0: the face below every cell in y, and the first third (half, with
+//           two Gauss points) of the volume integral;
+//   part 1: the face above in y, and the second third (half);
+//   part 2: the faces in x, and the rest of the volume integral (with two
+//           points: the terms of the modes and of the step-start state);
+//   part 3: the face above in z (the one below is the last plane's), then the
+//           sum of all parts, the limiter and the stores.
+// Every face is evaluated once, but for the faces in y (by the tiles on both
+// sides) and the first one of a workgroup in z.  The parts are equally long,
+// and meet once per plane.  Which wave takes which part rotates with the
+// workgroup, so that what inequality there is does not always meet one SIMD.
+//
+// Fields of a face: the stress fields' flux is linear in the velocity, and a
+// face of direction d carries only row d of the stress.  With stress a face
+// therefore has eight values (rh..en and the row) and eight fluxes (rh..en
+// and the velocity, from which the six stress rows follow), not eleven.
+#pragma once
+#include "hd_fused.h"
+
+namespace hd {
+namespace sg {
+
+using fz::CellPos;
+
+// values and moments of a face
+HD_DEV constexpr int face_nm(int nq) { return nq >= 11 ? 8 : 5; }
+// field of value e of a face of direction d
+HD_DEV constexpr int face_field(int nq, int d, int e) {
+    return e < 5 ? e
+         : d == 0 ? (e == 5 ? PXX : (e == 6 ? PXY : PXZ))
+         : d == 1 ? (e == 5 ? PXY : (e == 6 ? PYY : PYZ))
+                  : (e == 5 ? PXZ : (e == 6 ? PYZ : PZZ));
+}
+// stochastic stress component of row d, column a
+HD_DEV constexpr int noise_comp(int d, int a) {
+    return d == a ? d : (d + a == 1 ? 3 : (d + a == 2 ? 4 : 5));
+}
+
+// Pointer to cell c of plane `plane`, stepped plane by plane.  The empty asm
+// hides where it came from, so that the compiler neither keeps the addresses
+// of every plane alive nor shares them between the parts of the kernel.
+typedef const __attribute__((address_space(1))) double* gptr;
+typedef __attribute__((address_space(1))) double* gptr_w;
+__device__ __forceinline__ gptr plane_ptr(const double* q, long N, int plane, long c) {
+    asm volatile("" : "+v"(c));
+    return (gptr)(q + (long)plane * N + c);
+}
+template <typename P>
+__device__ __forceinline__ void step(P& p, long st) {
+    p += st;
+    asm volatile("" : "+v"(p));
+}
+// end of a section: no load or computation moves across
+__device__ __forceinline__ void section() {
+    fz::fence();
+    fz::point_barrier();
+}
+
+// Values that are complete here: the compiler may not move their last
+// operations to where they are used (it would keep the operands alive
+// instead, hundreds of registers).
+template <int A, int B>
+__device__ __forceinline__ void pin(double (&v)[A][B]) {
+#pragma unroll
+    for (int a = 0; a < A; a++)
+#pragma unroll
+        for (int b = 0; b < B; b++) asm volatile("" : "+v"(v[a][b]));
+}
+
+template <int B>
+__device__ __forceinline__ void pin(double (&v)[B]) {
+#pragma unroll
+    for (int b = 0; b < B; b++) asm volatile("" : "+v"(v[b]));
+}
+
+// LDS of a workgroup: two partial sums of a cell's output, one face's moments
+template <int NB, int NQ>
+HD_DEV constexpr int lds_doubles() { return (2 * NB * NQ + face_nm(NQ) * fz::face_nk<NB>()) * 64; }
+
+// ------------------------------------------------------------- faces -------
+// The modes that a DIR face needs of cell c.
+template <int NB, int NQ, int DIR>
+__device__ __forceinline__ void load_side(const double* __restrict__ q, long N, long c, double (&m)[face_nm(NQ)][NB]) {
+    constexpr int NM = face_nm(NQ);
+    gptr p = plane_ptr(q, N, 0, c);
+#pragma unroll
+    for (int r = 0; r < NB; r++)
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+#pragma unroll
+            for (int e = 0; e < NM; e++)
+                if (face_field(NQ, DIR, e) == f) m[e][r] = *p;
+            step(p, N);
+        }
+}
+
+// The face basis b_k at point (ii, jj), selected in scalar registers: a table
+// in memory costs a wait on the scalar cache at every point.
+template <int NB, int QP>
+struct FacePoint {
+    double b[fz::face_nk<NB>()], w;
+    __device__ __forceinline__ FacePoint(int ii, int jj) {
+        constexpr double s = fz::Rule<QP>::x(QP - 1);
+        if constexpr (QP == 2) {
+            b[1] = ii ? s : -s;
+            b[2] = jj ? s : -s;
+            if constexpr (NB == 8) b[3] = ii == jj ? s * s : -(s * s);
+            w = 1.0;
+        } else {
+            constexpr double w0 = fz::Rule<3>::w(0), w1 = fz::Rule<3>::w(1);
+            b[1] = ii == 1 ? 0.0 : (ii == 0 ? -s : s);
+            b[2] = jj == 1 ? 0.0 : (jj == 0 ? -s : s);
+            b[3] = (ii == 1 || jj == 1) ? 0.0 : (ii == jj ? s * s : -(s * s));
+            b[4] = ii == 1 ? fz::Rule<3>::p2(1) : fz::Rule<3>::p2(0);
+            b[5] = jj == 1 ? fz::Rule<3>::p2(1) : fz::Rule<3>::p2(0);
+            w = (ii == 1) != (jj == 1) ? w0 * w1 : (ii == 1 ? w1 * w1 : w0 * w0);
+        }
+        b[0] = 1.0;
+    }
+};
+template <int NM, int NK>
+__device__ __forceinline__ void eval_point(const double (&K)[NM][NK], const double (&b)[NK], double* out) {
+#pragma unroll
+    for (int e = 0; e < NM; e++) {
+        double s = K[e][0];
+#pragma unroll
+        for (int k = 1; k < NK; k++) s = fma(K[e][k], b[k], s);
+        out[e] = s;
+    }
+}
+
+// Face-polynomial coefficients of a DIR face from a cell's modes: the modes
+// odd along DIR enter with sign sgn (+1 above the cell, -1 below).
+template <int NB, int NM, int DIR, int NK>
+__device__ __forceinline__ void signed_coeffs(const double (&m)[NM][NB], double sgn, double (&K)[NM][NK]) {
+#pragma unroll
+    for (int e = 0; e < NM; e++)
+#pragma unroll
+        for (int k = 0; k < NK; k++) {
+            double s = 0., odd = 0.;
+            bool has = false, hodd = false;
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                if (fz::lift_k<NB, DIR>(r) != k) continue;
+                if (fz::deg<NB>(r, DIR) == 1) {
+                    odd = m[e][r];
+                    hodd = true;
+                } else {
+                    s = has ? s + m[e][r] : m[e][r];
+                    has = true;
+                }
+            }
+            K[e][k] = hodd ? fma(sgn, odd, s) : s;
+        }
+}
+
+// The face of direction DIR between cells cL and cR: its NM*NK moments, times
+// dxi_d, in M.  extL/extR: that side is outside the grid
+// (boundary kind bc) and follows from the other side's trace.
+template <int NB, int QP, int NQ, int RM, bool NZ, int DIR>
+__device__ __forceinline__ void face_moments(const double* __restrict__ q, const Grid& g, long cL, long cR, bool extL,
+                                             bool extR, int bc, const CellPos& cp, long fid, const Phys& ph,
+                                             double dxi_d, const StageParams& sp,
+                                             double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
+    constexpr int NF = QP * QP, NM = face_nm(NQ), NK = fz::face_nk<NB>();
+    double KL[NM][NK], KR[NM][NK];
+    {
+        // both sides' loads before the first use
+        double mL[NM][NB], mR[NM][NB];
+        load_side<NB, NQ, DIR>(q, g.N, cL, mL);
+        load_side<NB, NQ, DIR>(q, g.N, cR, mR);
+        // a side outside the grid starts as a copy of the other side's trace
+        signed_coeffs<NB, NM, DIR, NK>(mL, extL ? -1.0 : 1.0, KL);
+        signed_coeffs<NB, NM, DIR, NK>(mR, extR ? 1.0 : -1.0, KR);
+        pin(KL);
+        pin(KR);
+        section();
+    }
+    const bool ext = extL || extR;
+    bool zero_normal = false;
+    if (ext) {
+        // outflow boundaries decide on the whole face (src/boundary.f90:213-338)
+        if (bc == BC_OUTFLOW && !(DIR == 0 && extR)) {
+            double v = 0.;
+            for (int p = 0; p < NF; p++) {
+                const FacePoint<NB, QP> fp(p / QP, p % QP);
+                double s = KL[MX + DIR][0];
+#pragma unroll
+                for (int k = 1; k < NK; k++) s = fma(KL[MX + DIR][k], fp.b[k], s);
+                v = (p == 0) ? s : (extR ? fmin(v, s) : fmax(v, s));
+            }
+            zero_normal = extR ? (v < 0.0) : (v > 0.0);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < NM; e++)
+#pragma unroll
+        for (int k = 0; k < NK; k++) M[e][k] = 0.;
+    // the row of the stochastic stress, one point ahead of its use
+    float Sn[3];
+    if constexpr (NZ) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) Sn[a] = sp.noise[DIR][((long)noise_comp(DIR, a) * NF) * sp.nfb + fid];
+    }
+    int ii = 0, jj = 0;
+#pragma unroll 1
+    for (int p = 0; p < NF; p++) {
+        const FacePoint<NB, QP> fp(ii, jj);
+        if (++jj == QP) {
+            jj = 0;
+            ii++;
+        }
+        double QL[NM], QR[NM], F[NM];
+        eval_point<NM, NK>(KL, fp.b, QL);
+        eval_point<NM, NK>(KR, fp.b, QR);
+        if (ext) {
+            if (bc == BC_NOSLIP) {
+                if (extL) QL[MX] = QL[MY] = QL[MZ] = 0.0;
+                else QR[MX] = QR[MY] = QR[MZ] = 0.0;
+            } else if (bc == BC_WALL || (bc == BC_OUTFLOW && zero_normal)) {
+                if (extL) QL[MX + DIR] = 0.0;
+                else QR[MX + DIR] = 0.0;
+            } else if (bc == BC_OUTFLOW && DIR == 0 && extR) {
+                if (QR[MX] > 0.0) QR[MX] = -QL[MX];
+            }
+            if constexpr (DIR == 0) {
+                // x_bc_inflow (src/boundary.f90:571-592): prescribed rh, mx, en;
+                // no transverse momentum; the stress fields from the interior
+                if (bc == BC_INFLOW && extL) fz::inflow_ghost<NQ>(sp.inflow, g, cp, p, NF, QL);
+            }
+        }
+        double S[3] = {0., 0., 0.};
+        if constexpr (NZ) {
+            const int pn = p + 1 < NF ? p + 1 : p;
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                S[a] = Sn[a];
+                Sn[a] = sp.noise[DIR][((long)noise_comp(DIR, a) * NF + pn) * sp.nfb + fid];
+            }
+        }
+        pr::face_flux<NQ, DIR, RM, NZ>(ph, QL, QR, S, F);
+        const double wd = QP == 2 ? dxi_d : fp.w * dxi_d;
+#pragma unroll
+        for (int e = 0; e < NM; e++) {
+            F[e] *= wd;
+            M[e][0] += F[e];
+#pragma unroll
+            for (int k = 1; k < NK; k++) M[e][k] = fma(fp.b[k], F[e], M[e][k]);
+        }
+    }
+    pin(M);
+}
+template <int NM, int NK>
+__device__ __forceinline__ void store_moments(const double (&M)[NM][NK], double* __restrict__ mom) {
+#pragma unroll
+    for (int e = 0; e < NM; e++)
+#pragma unroll
+        for (int k = 0; k < NK; k++) mom[(e * NK + k) * 64] = M[e][k];
+}
+
+// ------------------------------------------------------------ volume -------
+// Index of mode r among the modes with degree >= 1 along d
+template <int NB>
+HD_DEV constexpr int ndeg() { return NB == 4 ? 1 : 4; }
+template <int NB>
+HD_DEV constexpr int deg_index(int d, int r) {
+    int n = 0;
+    for (int s = 0; s < r; s++)
+        if (fz::deg<NB>(s, d) > 0) n++;
+    return n;
+}
+
+// A uniform value in scalar registers.
+__device__ __forceinline__ double scalar(double x) {
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Fluxes at volume point (i,j,k) from the point's fields Q, projected onto
+// the modes' derivatives; the products are written as fma so that the
+// compiler does not share scaled modes between points (which would keep
+// hundreds of them alive).  HYD: rh..en into rhs; VEL: the velocity into au.
+template <int NB, int QP, int NQ, bool NZ, bool HYD, bool VEL>
+__device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], int i, int j, int k, double (&rhs)[5][NB],
+                                             double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()], const Phys& ph,
+                                             const double (&di)[3], const StageParams& sp, long c, long N) {
+    float S[6];
+    if constexpr (NZ && HYD) {
+        constexpr long npg = QP * QP * QP;
+#pragma unroll
+        for (int e = 0; e < 6; e++) S[e] = sp.noise[3][((long)e * npg + (i * QP + j) * QP + k) * N + c];
+    }
+    const double ri = pr::rcp(Q[RH]);
+    const double u[3] = {Q[MX] * ri, Q[MY] * ri, Q[MZ] * ri};
+    double P = 0.;
+    if constexpr (HYD) {
+        P = ph.gm1 * (Q[EN] - 0.5 * (Q[MX] * u[0] + Q[MY] * u[1] + Q[MZ] * u[2]));
+        P = P < ph.P_floor ? ph.P_floor : P;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double wd = QP == 2 ? di[d] : scalar(fz::Rule<QP>::w3(i, j, k) * di[d]);
+        const double ud = wd * u[d];
+        double F[5];
+        if constexpr (HYD) {
+            F[RH] = wd * Q[MX + d];
+            F[EN] = (Q[EN] + P) * ud;
+        }
+        if constexpr (HYD && NQ >= 11) {
+            double Pn[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                Pn[a] = Q[face_field(NQ, d, 5 + a)];
+                if constexpr (NZ) Pn[a] -= (double)S[noise_comp(d, a)];
+                F[MX + a] = fma(Q[MX + a], ud, wd * (a == d ? Pn[a] + P : Pn[a]));
+            }
+            F[EN] = fma(wd, fma(Pn[0], u[0], fma(Pn[1], u[1], Pn[2] * u[2])), F[EN]);
+        } else if constexpr (HYD) {
+#pragma unroll
+            for (int a = 0; a < 3; a++) F[MX + a] = a == d ? fma(Q[MX + a], ud, wd * P) : Q[MX + a] * ud;
+        }
+        // dphi_r/dxi_d at the point: 1, other coordinates, or 3 x_d
+#pragma unroll
+        for (int r = 1; r < NB; r++) {
+            if (fz::deg<NB>(r, d) == 0) continue;
+            const double cf = fz::dphi<NB, QP>(d, r, i, j, k);
+            if (cf == 0.0) continue;
+            if constexpr (HYD) {
+#pragma unroll
+                for (int f = 0; f < 5; f++) rhs[f][r] = fma(cf, F[f], rhs[f][r]);
+            }
+            if constexpr (VEL) {
+#pragma unroll
+                for (int a = 0; a < 3; a++)
+                    au[a][d][deg_index<NB>(d, r)] = fma(cf, a == d ? ud : wd * u[a], au[a][d][deg_index<NB>(d, r)]);
+            }
+        }
+    }
+    fz::point_barrier();
+}
+
+// innerintegral2 (src/flux.f90:751-928) of cell c without its 0.25 cb_r; with
+// stress, the stress rows' fluxes are carried by the velocity's projections
+// au[a][d][.] onto the modes that vary along d.  nbasis 10 holds one x plane
+// of the cell at a time (its polynomial in y and z, six coefficients a
+// field) and reads the modes once per plane, since modes and accumulators
+// together do not fit 256 registers.  I0, I1: the x planes of the rule to take.
+template <int NB, int QP, int NQ, bool NZ, bool HYD, bool VEL, int I0, int I1>
+__device__ __forceinline__ void volume_moments(const double* __restrict__ q, const Grid& g, long c,
+                                               double (&rhs)[5][NB], double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()],
+                                               const Phys& ph, const StageParams& sp) {
+    const double di[3] = {g.dxi, g.dyi, g.dzi};
+    constexpr int NV = HYD ? NQ : 4;  // fields read
+    if constexpr (NB == 10) {
+#pragma unroll
+        for (int i = I0; i < I1; i++) {
+            const double x = fz::Rule<QP>::x(i), p2 = fz::Rule<QP>::p2(i);
+            double a0[NV], ay[NV], az[NV], ayz[NV], ayy[NV], azz[NV];
+#pragma unroll
+            for (int f = 0; f < NV; f++) {
+                gptr p = plane_ptr(q, g.N, f, c);
+                double m[NB];
+#pragma unroll
+                for (int r = 0; r < NB; r++) {
+                    m[r] = *p;
+                    step(p, (long)NQ * g.N);
+                }
+                a0[f] = fma(p2, m[KXX], m[0]);
+                if (x != 0.0) a0[f] = fma(x, m[KX], a0[f]);
+                ay[f] = x != 0.0 ? fma(x, m[KXY], m[KY]) : m[KY];
+                az[f] = x != 0.0 ? fma(x, m[KZX], m[KZ]) : m[KZ];
+                ayz[f] = m[KYZ];
+                ayy[f] = m[KYY];
+                azz[f] = m[KZZ];
+                if (f % 3 == 2 || f == NV - 1) section();
+            }
+#pragma unroll
+            for (int j = 0; j < QP; j++) {
+                const double y = fz::Rule<QP>::x(j), q2 = fz::Rule<QP>::p2(j);
+#pragma unroll
+                for (int k = 0; k < QP; k++) {
+                    const double z = fz::Rule<QP>::x(k), r2 = fz::Rule<QP>::p2(k);
+                    double Q[NV];
+#pragma unroll
+                    for (int f = 0; f < NV; f++) {
+                        double s = fma(q2, ayy[f], a0[f]);
+                        if (y != 0.0) s = fma(y, ay[f], s);
+                        s = fma(r2, azz[f], s);
+                        if (z != 0.0) s = fma(z, az[f], s);
+                        if (y * z != 0.0) s = fma(y * z, ayz[f], s);
+                        Q[f] = s;
+                    }
+                    volume_point<NB, QP, NQ, NZ, HYD, VEL>(Q, i, j, k, rhs, au, ph, di, sp, c, g.N);
+                }
+            }
+        }
+    } else {
+        double m[NQ][NB];
+        fz::load_modes<NB, NQ>(q, g, c, m);
+#pragma unroll
+        for (int i = I0; i < I1; i++)
+#pragma unroll
+            for (int j = 0; j < QP; j++)
+#pragma unroll
+                for (int k = 0; k < QP; k++) {
+                    double Q[NQ];
+#pragma unroll
+                    for (int f = 0; f < NQ; f++) {
+                        double s = m[f][0];
+#pragma unroll
+                        for (int r = 1; r < NB; r++) s = fma(fz::phi_int<NB, QP>(r, i, j, k), m[f][r], s);
+                        Q[f] = s;
+                    }
+                    volume_point<NB, QP, NQ, NZ, HYD, VEL>(Q, i, j, k, rhs, au, ph, di, sp, c, g.N);
+                }
+    }
+}
+
+// The output of one stage is linear in the right-hand side: with
+// v = wn q_n + wv fac (m + dt (volume + sources)), each face adds
+// wv fac dt 0.25 cb_r times its lift (advance_time_level and the SSP
+// combination, src/integrator.f90:62-86,210-232).
+struct Weights {
+    double wm, wn, ws, wsf;  // of m, q_n, the right-hand side and (with relaxation) the stress fields'
+    double wmf;
+};
+__device__ __forceinline__ Weights stage_weights(const StageParams& sp) {
+    Weights w;
+    const double* pdt = sp.dt;
+    asm volatile("" : "+s"(pdt));  // read where it is used, not kept in registers across the planes
+    if (sp.mode == 1) {
+        w.wm = 0.;
+        w.wn = 0.;
+        w.ws = w.wsf = 1.;
+        w.wmf = 0.;
+        return w;
+    }
+    const double dt = *pdt;
+    const double wv = sp.combine == 0 ? 1. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.25 : 2. / 3.));
+    w.wn = sp.combine == 0 ? 0. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.75 : 1. / 3.));
+    const double faci = sp.ivis == 1 ? 1. / (1. + dt * sp.coll) : 1.;
+    w.wm = wv;
+    w.ws = wv * dt;
+    w.wmf = wv * faci;
+    w.wsf = w.wmf * dt;
+    return w;
+}
+
+template <int NB, int NQ>
+__device__ __forceinline__ void load_start(const double* __restrict__ qin, const double* __restrict__ qn,
+                                           const Grid& g, const Weights& w, long c, int f, double (&m)[NB],
+                                           double (&q0)[NB]) {
+    const long st = (long)NQ * g.N;
+    gptr p = plane_ptr(qin, g.N, f, c);
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        m[r] = *p;
+        step(p, st);
+    }
+    if (w.wn != 0.) {
+        p = plane_ptr(qn, g.N, f, c);
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            q0[r] = *p;
+            step(p, st);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < NB; r++) q0[r] = 0.;
+    }
+}
+// t (without 0.25 cb_r) becomes wn q_n + wm m + ws (t + sources)
+template <int NB, int NQ>
+__device__ __forceinline__ void start_field(const double* __restrict__ qin, const Grid& g, const StageParams& sp,
+                                            const Weights& w, long c, int f, const double (&m)[NB],
+                                            const double (&q0)[NB], double (&t)[NB]) {
+    const long st = (long)NQ * g.N;
+#pragma unroll
+    for (int r = 0; r < NB; r++) t[r] *= 0.25 * fz::cbasis<NB>(r);
+    // sources (src/sources.f90:12-84): ivis 0 relaxes the stress explicitly
+    // (-coll*P, projected exactly in modal space); body force rho*g, m.g
+    if constexpr (NQ >= 11) {
+        if (f >= PXX && sp.ivis == 0 && sp.coll != 0.)
+#pragma unroll
+            for (int r = 0; r < NB; r++) t[r] = fma(-sp.coll, m[r], t[r]);
+    }
+    if (f >= MX && f <= MZ && sp.bf[f - MX] != 0.) {
+        gptr p = plane_ptr(qin, g.N, RH, c);
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            t[r] = fma(sp.bf[f - MX], *p, t[r]);
+            step(p, st);
+        }
+    }
+    if (f == EN && (sp.bf[0] != 0. || sp.bf[1] != 0. || sp.bf[2] != 0.)) {
+        gptr p = plane_ptr(qin, g.N, MX, c);
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            t[r] = fma(sp.bf[0], p[0], fma(sp.bf[1], p[g.N], fma(sp.bf[2], p[2 * g.N], t[r])));
+            step(p, st);
+        }
+    }
+    const double wm = f >= PXX ? w.wmf : w.wm, ws = f >= PXX ? w.wsf : w.ws;
+#pragma unroll
+    for (int r = 0; r < NB; r++) t[r] = fma(ws, t[r], fma(wm, m[r], w.wn * q0[r]));
+}
+
+// t[r] += the lift of a face's moments in direction D, without 0.25 cb_r: the
+// face below (LO) or above the cell.
+template <int NB, int NK, int D, bool LO>
+__device__ __forceinline__ void lift(const double (&m)[NK], double (&t)[NB]) {
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        const double x = m[fz::lift_k<NB, D>(r)];
+        t[r] += LO && fz::deg<NB>(r, D) != 1 ? x : -x;
+    }
+}
+// The stress field that the flux of u_a in direction d drives (a != d)
+HD_DEV constexpr int shear_field(int a, int d) { return a + d == 1 ? PXY : (a + d == 2 ? PXZ : PYZ); }
+
+// The volume part of field f's right-hand side (without 0.25 cb_r) from the
+// projections of the velocity's fluxes, for the stress fields.
+template <int NB>
+__device__ __forceinline__ void stress_volume(const Phys& ph, const double (&au)[3][3][ndeg<NB>()], int f,
+                                              double (&t)[NB]) {
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        double s = 0.;
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                if (fz::deg<NB>(r, d) == 0) continue;
+                const double x = au[a][d][deg_index<NB>(d, r)];
+                if (f <= PZZ && a == d) s = fma(f - PXX == a ? ph.c4d3cv : -ph.c2d3cv, x, s);
+                if (f >= PXY && a != d && f == (a + d == 1 ? PXY : (a + d == 2 ? PXZ : PYZ)))
+                    s = fma(ph.colvis, x, s);
+            }
+        t[r] = s;
+    }
+}
+
+// Field f's share of a part, without 0.25 cb_r: t (rh..en) or, for the stress
+// fields, what the velocity's lifts tu in direction D and its volume
+// projections au (VOL) drive.
+template <int NB, int NQ, int D, bool VOL>
+__device__ __forceinline__ void part_field(const Phys& ph, const double (&t)[5][NB],
+                                           const double (&tu)[NQ >= 11 ? 3 : 1][NB],
+                                           const double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()], int f,
+                                           double (&o)[NB]) {
+    if (f < 5) {
+#pragma unroll
+        for (int r = 0; r < NB; r++) o[r] = t[f][r];
+        return;
+    }
+    if constexpr (NQ >= 11) {
+        if constexpr (VOL) {
+            stress_volume<NB>(ph, au, f, o);
+        } else {
+#pragma unroll
+            for (int r = 0; r < NB; r++) o[r] = 0.;
+        }
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            if (a == D ? f > PZZ : f != shear_field(a, D)) continue;
+            const double cf = a != D ? ph.colvis : (f - PXX == a ? ph.c4d3cv : -ph.c2d3cv);
+#pragma unroll
+            for (int r = 0; r < NB; r++) o[r] = fma(cf, tu[a][r], o[r]);
+        }
+    }
+}
+
+// The output of one cell: NaN check, the next stage's limiter, stores.
+template <int NB, int QP, int NQ>
+__device__ __forceinline__ void store_cell(double* __restrict__ qout, const Grid& g, const StageParams& sp, long c,
+                                           long bad_id, bool live, double (&v)[NQ][NB]) {
+    bool bad = false;
+    if (sp.mode != 1) {
+#pragma unroll
+        for (int f = 0; f < NQ; f++) bad |= v[f][0] != v[f][0];
+        // When this output is the next stage's input, apply that stage's limiter
+        // here: the reference limits the stage input in place before anything
+        // reads it (src/integrator.f90:106-113), so the stored values are the same.
+        if (sp.limit_out) fz::limit_cell<NB, QP, NQ>(v, sp.lp);
+    }
+    if (!live) return;
+    gptr_w p = (gptr_w)plane_ptr(qout, g.N, 0, c);
+#pragma unroll
+    for (int r = 0; r < NB; r++)
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+            *p = v[f][r];
+            step(p, g.N);
+        }
+    if (bad) {
+        atomicOr(sp.err, 1);
+        atomicMin(sp.bad, (unsigned long long)bad_id);
+    }
+}
+
+// ------------------------------------------------------------- waves -------
+// A lane's column of cells: position pi of the row lattice at row j, planes
+// stepped by the caller.
+struct Column {
+    int pi, i, j;     // lattice position 0..nx (the face below cell pi in x), cell, row
+    bool live;        // the lane updates the cell
+    long row0;        // offset of the row within a plane
+};
+__device__ __forceinline__ Column column(const Grid& g, unsigned tile, int lane) {
+    // 32-bit position arithmetic: a plane of 2^31 cells would not fit the device.
+    // Worked out where it is used: kept across the planes it would cost registers
+    // that the faces need.
+    asm volatile("" : "+s"(tile));
+    const unsigned pitch = (unsigned)g.nx + 1u, npos = pitch * (unsigned)g.ny;
+    unsigned pos = tile * 63u + (unsigned)lane;
+    const bool in = pos < npos;
+    if (!in) pos = npos - 1u;
+    const unsigned row = pos / pitch;
+    Column o;
+    o.pi = (int)(pos - row * pitch);
+    o.i = o.pi < g.nx ? o.pi : g.nx - 1;
+    o.j = (int)row;
+    o.live = in && o.pi < g.nx && lane < 63;
+    o.row0 = (long)g.nx * o.j;
+    return o;
+}
+
+// Face s (0 below, 1 above) in direction DIR of the column's cell at plane k
+// (DIR 0: the face below lattice position pi, s = 0).
+template <int NB, int QP, int NQ, int RM, bool NZ, int DIR>
+__device__ __forceinline__ void column_face(const double* __restrict__ qin, const Grid& g, const Phys& ph,
+                                            const StageParams& sp, const Column& o, int k, int s,
+                                            double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
+    const long plane = (long)g.nx * g.ny;
+    const int n = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
+    const int af = DIR == 0 ? o.pi : (DIR == 1 ? o.j : k) + s;  // the face below cell af
+    const bool per = g.bc[2 * DIR] == BC_PERIODIC;
+    const bool extL = !per && af == 0, extR = !per && af == n;
+    const int aL = af == 0 ? (per ? n - 1 : 0) : af - 1, aR = af == n ? (per ? 0 : n - 1) : af;
+    const int bc = extL ? g.bc[2 * DIR] : g.bc[2 * DIR + 1];
+    long base, st;
+    if (DIR == 0) base = o.row0 + plane * k, st = 1;
+    else if (DIR == 1) base = o.i + plane * k, st = g.nx;
+    else base = o.row0 + o.i, st = plane;
+    const long nfx = g.nx + 1, nfxy = nfx * (g.ny + 1);
+    const int an = per && af == n ? 0 : af;
+    const long fid = (DIR == 0 ? an : o.i) + nfx * (DIR == 1 ? an : o.j) + nfxy * (DIR == 2 ? an : k);
+    CellPos cp;
+    cp.i = o.i;
+    cp.j = o.j;
+    cp.k = k;
+    cp.c = 0;
+    face_moments<NB, QP, NQ, RM, NZ, DIR>(qin, g, base + aL * st, base + aR * st, extL, extR, bc, cp, fid, ph,
+                                          DIR == 0 ? g.dxi : DIR == 1 ? g.dyi : g.dzi, sp, M);
+}
+
+// Waves per SIMD that the registers are held to.
+template <int NB, int NQ>
+HD_DEV constexpr int occupancy() { return NB == 4 && NQ == 5 ? 3 : (NB == 10 && NQ >= 11 ? 1 : 2); }
+
+inline int stage_occupancy(int nb, int nq) { return nb == 4 && nq == 5 ? 3 : (nb == 10 && nq >= 11 ? 1 : 2); }
+
+// Cost of items of zc planes on `resident` workgroups, in planes: rounds times
+// an item's length, its start (the first face below in z and the first loads)
+// worth 0.6 planes.
+inline double march_cost(long items, int zc, long resident) {
+    return (double)((items + resident - 1) / resident) * (zc + 0.6);
+}
+
+// How a grid of `tiles` tiles a plane and nz planes is run: -1 by k_stage_wide,
+// 0 in equal runs, n > 0 in items of n planes.
+//  * Up to two tiles per CU k_stage_wide: latency decides (Sod tube of 256
+//    cells 22 us a step in five waves against 26, channel 64x128 24 against 31).
+//  * Up to 8 planes per resident workgroup in equal runs: whole rounds of items
+//    would leave part of the chip idle (nbasis 10, 75x61x27: 330 us a step
+//    against 446 in items of 4).
+//  * Above, the items of least cost: neighbouring tiles at the same plane share
+//    L2, which equal runs lose (nbasis 4, 256x256x128: 4.0 ms a step in items
+//    of 8 or 16 against 4.8; nbasis 8, 120x80x64: 576 us against 640).
+template <int NB, int NQ>
+inline int stage_planes(long tiles, int nz, long cus) {
+    const long work = tiles * nz, resident = cus * occupancy<NB, NQ>();
+    if (work <= 2 * cus && !(NB == 10 && NQ >= 11)) return -1;
+    if (work < 8 * resident) return 0;
+    int best = 1;
+    for (int zc = 2; zc <= nz && zc <= 16; zc++)
+        if (march_cost(tiles * ((nz + zc - 1) / zc), zc, resident) <
+            march_cost(tiles * ((nz + best - 1) / best), best, resident))
+            best = zc;
+    return best;
+}
+
+// What the waves of a workgroup share.
+struct Shared {
+    double *r0, *r1;  // partial sums of the outputs: parts 2 and 0, part 1
+    double* z;        // moments of the face below in z
+    int* flags;       // planes whose sums part 3 has read; planes that part 2 has written
+};
+__device__ __forceinline__ void raise(int* flag, int n) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __hip_atomic_store(flag, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// The waves of a workgroup are resident together, and the one waited for
+// never waits for this one before it raises the flag.
+__device__ __forceinline__ void await(int* flag, int n) {
+    while (__hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < n) __builtin_amdgcn_s_sleep(1);
+}
+
+// value of the next lane
+__device__ __forceinline__ double next_lane(double x, int addr) {
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Which part adds field f's terms of the modes and the step-start state: part
+// 2, which has no share of the two-point volume rule, or parts 0 and 1.
+template <int QP>
+HD_DEV constexpr bool starts(int part, int f) { return QP == 2 ? part == 2 : part == (f & 1); }
+
+// Parts 0-2 of plane k (p planes after the workgroup's first): one direction's
+// face, a share of the volume integral, and some fields' terms of the modes
+// and the step-start state; the sum to LDS.
+template <int NB, int QP, int NQ, int RM, bool NZ, int PART>
+__device__ __forceinline__ void sum_part(const double* __restrict__ qin, const double* __restrict__ qn, const Grid& g,
+                                         const Phys& ph, const StageParams& sp, unsigned tile, int k, int p,
+                                         const Shared& sh, int lane) {
+    constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
+    constexpr int D = PART == 2 ? 0 : 1;
+    constexpr bool VOL = PART < QP;
+    const Column o = column(g, tile, lane);
+    const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
+    double t[5][NB], tu[NQ >= 11 ? 3 : 1][NB], au[NQ >= 11 ? 3 : 1][3][ndeg<NB>()];
+    {
+        double M[NM][NK];
+        column_face<NB, QP, NQ, RM, NZ, D>(qin, g, ph, sp, o, k, PART == 1 ? 1 : 0, M);
+#pragma unroll
+        for (int e = 0; e < NM; e++) {
+            double s[NB];
+#pragma unroll
+            for (int r = 0; r < NB; r++) s[r] = 0.;
+            if constexpr (PART == 0) {
+                lift<NB, NK, 1, true>(M[e], s);
+            } else if constexpr (PART == 1) {
+                lift<NB, NK, 1, false>(M[e], s);
+            } else {
+                double h[NK];
+                const int addr = ((lane + 1) & 63) * 4;
+#pragma unroll
+                for (int n = 0; n < NK; n++) h[n] = next_lane(M[e][n], addr);
+                lift<NB, NK, 0, true>(M[e], s);
+                lift<NB, NK, 0, false>(h, s);
+            }
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                if (e < 5) t[e < 5 ? e : 0][r] = s[r];
+                else tu[e < 5 ? 0 : e - 5][r] = s[r];
+            }
+        }
+        pin(t);
+        if constexpr (NQ >= 11) pin(tu);
+        section();
+    }
+#pragma unroll
+    for (int a = 0; a < (NQ >= 11 ? 3 : 1); a++)
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int r = 0; r < ndeg<NB>(); r++) au[a][d][r] = 0.;
+    if constexpr (VOL) {
+        if constexpr (NB == 10 && NQ >= 11) {
+            // in two passes over the points: their accumulators do not fit together
+            volume_moments<NB, QP, NQ, NZ, true, false, PART, PART + 1>(qin, g, c, t, au, ph, sp);
+            pin(t);
+            section();
+            volume_moments<NB, QP, NQ, NZ, false, true, PART, PART + 1>(qin, g, c, t, au, ph, sp);
+        } else {
+            volume_moments<NB, QP, NQ, NZ, true, (NQ >= 11), PART, PART + 1>(qin, g, c, t, au, ph, sp);
+        }
+        pin(t);
+        if constexpr (NQ >= 11) {
+#pragma unroll
+            for (int a = 0; a < 3; a++) pin(au[a]);
+        }
+        section();
+    }
+    const Weights w = stage_weights(sp);
+    double* const R = (PART == 1 ? sh.r1 : sh.r0) + lane;
+    // a batch of fields at a time: the loads of its modes and step-start
+    // values together, the first batch's before the wait
+    constexpr int BATCH = NB == 10 && NQ >= 11 ? 4 : (NQ >= 11 ? 6 : 5);
+#pragma unroll
+    for (int f0 = 0; f0 < NQ; f0 += BATCH) {
+        double m[BATCH][NB], q0[BATCH][NB];
+#pragma unroll
+        for (int b = 0; b < BATCH; b++)
+            if (f0 + b < NQ && starts<QP>(PART, f0 + b))
+                load_start<NB, NQ>(qin, qn, g, w, c, f0 + b, m[b], q0[b]);
+        if (f0 == 0) {
+            // part 2 is done first: it writes, part 0 adds
+            if (PART == 0) await(sh.flags + 1, p + 1);
+            else await(sh.flags, p);
+        }
+#pragma unroll
+        for (int b = 0; b < BATCH; b++) {
+            const int f = f0 + b;
+            if (f >= NQ) continue;
+            double v[NB];
+            part_field<NB, NQ, D, VOL>(ph, t, tu, au, f, v);
+            if (starts<QP>(PART, f)) {
+                start_field<NB, NQ>(qin, g, sp, w, c, f, m[b], q0[b], v);
+            } else {
+#pragma unroll
+                for (int r = 0; r < NB; r++) v[r] *= (f < 5 ? w.ws : w.wsf) * (0.25 * fz::cbasis<NB>(r));
+            }
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                double* const x = R + (f * NB + r) * 64;
+                *x = PART == 0 ? *x + v[r] : v[r];
+            }
+        }
+        section();
+    }
+    if (PART == 2) raise(sh.flags + 1, p + 1);
+}
+
+// Part 3 of plane k after its face above in z (moments M, the next plane's
+// face below): once all parts have met, the sum, the next stage's limiter and
+// the stores.
+template <int NB, int QP, int NQ>
+__device__ __forceinline__ void finish_part(double* __restrict__ qout, const Grid& g, const Phys& ph, const StageParams& sp,
+                                            unsigned tile, int k, int p, long cell0,
+                                            const Shared& sh, int lane, bool same,
+                                            double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
+    constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
+    const Column o = column(g, tile, lane);
+    const Weights w = stage_weights(sp);
+    const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
+    double v[NQ][NB];
+#pragma unroll
+    for (int f = 0; f < NQ; f++)
+#pragma unroll
+        for (int r = 0; r < NB; r++) v[f][r] = 0.;
+    __syncthreads();
+    double* const z = sh.z + lane;
+    // same: the faces below and above are one (a periodic axis of one cell)
+    double tu[NQ >= 11 ? 3 : 1][NB];
+#pragma unroll
+    for (int e = 0; e < NM; e++) {
+        double lo[NK], s[NB];
+#pragma unroll
+        for (int n = 0; n < NK; n++) {
+            lo[n] = z[(e * NK + n) * 64];
+            if (same) M[e][n] = lo[n];
+        }
+#pragma unroll
+        for (int r = 0; r < NB; r++) s[r] = 0.;
+        lift<NB, NK, 2, true>(lo, s);
+        lift<NB, NK, 2, false>(M[e], s);
+#pragma unroll
+        for (int n = 0; n < NK; n++) z[(e * NK + n) * 64] = M[e][n];
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            if (e < 5) v[e < 5 ? e : 0][r] = fma(w.ws * (0.25 * fz::cbasis<NB>(r)), s[r], v[e < 5 ? e : 0][r]);
+            else tu[e < 5 ? 0 : e - 5][r] = s[r];
+        }
+        if (NB > 4 && e % 2 == 1) section();
+    }
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        if constexpr (NQ >= 11) {
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                if (f < 5 || (a == 2 ? f > PZZ : f != shear_field(a, 2))) continue;
+                const double cf = w.wsf * (a != 2 ? ph.colvis : (f == PZZ ? ph.c4d3cv : -ph.c2d3cv));
+#pragma unroll
+                for (int r = 0; r < NB; r++) v[f][r] = fma(cf * (0.25 * fz::cbasis<NB>(r)), tu[a][r], v[f][r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            const int x = (f * NB + r) * 64 + lane;
+            // the sum that holds the modes last: one rounding at their size
+            if (starts<QP>(1, f)) v[f][r] = (v[f][r] + sh.r0[x]) + sh.r1[x];
+            else v[f][r] = (v[f][r] + sh.r1[x]) + sh.r0[x];
+        }
+        if (f % (NB > 4 ? 2 : 4) == 1) section();
+    }
+    pin(v);
+    raise(sh.flags, p + 1);
+    store_cell<NB, QP, NQ>(qout, g, sp, c, cell0 + c, o.live, v);
+}
+
+// One tile over planes [k0, k1), after p0 planes of this workgroup: four waves.
+template <int NB, int QP, int NQ, int RM, bool NZ>
+__device__ __forceinline__ void stage_march(const double* __restrict__ qin, const double* __restrict__ qn,
+                                            double* __restrict__ qout, const Grid& g, const Phys& ph,
+                                            const StageParams& sp, unsigned tile, int k0, int k1, int p0, int part,
+                                            long cell0, const Shared& sh) {
+    constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
+    const int lane = (int)(threadIdx.x & 63u);
+    if (part == 0) {
+#pragma unroll 1
+        for (int k = k0; k < k1; k++) {
+            sum_part<NB, QP, NQ, RM, NZ, 0>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            __syncthreads();
+        }
+    } else if (part == 1) {
+#pragma unroll 1
+        for (int k = k0; k < k1; k++) {
+            sum_part<NB, QP, NQ, RM, NZ, 1>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            __syncthreads();
+        }
+    } else if (part == 2) {
+#pragma unroll 1
+        for (int k = k0; k < k1; k++) {
+            sum_part<NB, QP, NQ, RM, NZ, 2>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            __syncthreads();
+        }
+    } else {
+        const bool one_z = g.nz == 1 && g.bc[4] == BC_PERIODIC;
+#pragma unroll 1
+        for (int k = k0; k <= k1; k++) {  // the face below plane k
+            double M[NM][NK];
+            if (k > k0 && one_z) {
+#pragma unroll
+                for (int e = 0; e < NM; e++)
+#pragma unroll
+                    for (int n = 0; n < NK; n++) M[e][n] = 0.;
+            } else column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, column(g, tile, lane), k, 0, M);
+            if (k == k0) {
+#pragma unroll
+                for (int e = 0; e < NM; e++)
+#pragma unroll
+                    for (int n = 0; n < NK; n++) sh.z[(e * NK + n) * 64 + lane] = M[e][n];
+            } else {
+                finish_part<NB, QP, NQ>(qout, g, ph, sp, tile, k - 1, p0 + k - 1 - k0, cell0, sh, lane, one_z, M);
+            }
+        }
+    }
+}
+
+// One tile of one plane by five waves, for grids of few tiles (latency): the
+// face below in z has a wave of its own.
+template <int NB, int QP, int NQ, int RM, bool NZ>
+__device__ __forceinline__ void stage_wide(const double* __restrict__ qin, const double* __restrict__ qn,
+                                           double* __restrict__ qout, const Grid& g, const Phys& ph,
+                                           const StageParams& sp, unsigned tile, int k, int part, long cell0,
+                                           const Shared& sh) {
+    constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
+    const int lane = (int)(threadIdx.x & 63u);
+    if (part == 0) {
+        sum_part<NB, QP, NQ, RM, NZ, 0>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+    } else if (part == 1) {
+        sum_part<NB, QP, NQ, RM, NZ, 1>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+    } else if (part == 2) {
+        sum_part<NB, QP, NQ, RM, NZ, 2>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+    } else {
+        const bool one_z = g.nz == 1 && g.bc[4] == BC_PERIODIC;
+        double M[NM][NK];
+        if (part == 4 || !one_z) column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, column(g, tile, lane), k, part == 3 ? 1 : 0, M);
+        if (part == 3) {
+            finish_part<NB, QP, NQ>(qout, g, ph, sp, tile, k, 0, cell0, sh, lane, one_z, M);
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < NM; e++)
+#pragma unroll
+            for (int n = 0; n < NK; n++) sh.z[(e * NK + n) * 64 + lane] = M[e][n];
+    }
+    __syncthreads();
+}
+
+// The workgroup's LDS, flags cleared.
+template <int NB, int NQ>
+__device__ __forceinline__ Shared share(double* lds, int* flags) {
+    Shared sh;
+    sh.r0 = lds;
+    sh.r1 = lds + NB * NQ * 64;
+    sh.z = lds + 2 * NB * NQ * 64;
+    sh.flags = flags;
+    if (threadIdx.x < 2) flags[threadIdx.x] = 0;
+    __syncthreads();
+    return sh;
+}
+
+// tiles of a plane: the last position of its lattice has no cell
+inline unsigned stage_tiles(const Grid& g) { return (unsigned)(((long)(g.nx + 1) * g.ny - 1 + 62) / 63); }
+
+// The grid's work is ntile tiles of nz planes.  With zc > 0 a workgroup takes
+// zc planes of one tile, tiles first, so that neighbouring tiles are at the
+// same planes at the same time and find each other's modes in L2.  With zc = 0
+// it takes an equal run of the whole work, z fastest, in a launch of as many
+// workgroups as are resident: they start and end together.  Workgroup b runs
+// on XCD b mod 8: each XCD takes a contiguous eighth (the grid is a multiple
+// of 8).
+template <int NB, int QP, int NQ, int RM, bool NZ>
+__global__ __launch_bounds__(256, (occupancy<NB, NQ>())) void k_stage(
+    const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout, Grid g, Phys ph,
+    StageParams sp, unsigned ntile, int zc) {
+    __shared__ double lds[lds_doubles<NB, NQ>()];
+    __shared__ int flags[2];
+    const unsigned b = blockIdx.x >> 3, w = (blockIdx.x & 7u) * (gridDim.x >> 3) + b;
+    unsigned tile, left;
+    int k0, p = 0;
+    if (zc > 0) {
+        const unsigned ch = w / ntile;
+        tile = w - ch * ntile;
+        k0 = (int)ch * zc;
+        if (k0 >= g.nz) return;
+        left = (unsigned)(k0 + zc < g.nz ? zc : g.nz - k0);
+    } else {
+        const unsigned long long work = (unsigned long long)ntile * (unsigned)g.nz;
+        const unsigned long long u = work * w / gridDim.x;
+        left = (unsigned)(work * (w + 1) / gridDim.x - u);
+        tile = (unsigned)(u / (unsigned)g.nz);
+        k0 = (int)(u - (unsigned long long)tile * (unsigned)g.nz);
+    }
+    const Shared sh = share<NB, NQ>(lds, flags);
+    const int part = __builtin_amdgcn_readfirstlane((int)(((threadIdx.x >> 6) + b) & 3u));
+#pragma unroll 1
+    while (left > 0) {
+        const int n = (unsigned)(g.nz - k0) < left ? g.nz - k0 : (int)left;
+        stage_march<NB, QP, NQ, RM, NZ>(qin, qn, qout, g, ph, sp, tile, k0, k0 + n, p, part, 0, sh);
+        left -= (unsigned)n;
+        p += n;
+        k0 = 0;
+        tile++;
+    }
+}
+
+template <int NB, int QP, int NQ, int RM, bool NZ>
+__global__ __launch_bounds__(320) void k_stage_wide(
+    const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout, Grid g, Phys ph,
+    StageParams sp, unsigned ntile, unsigned nwork) {
+    __shared__ double lds[lds_doubles<NB, NQ>()];
+    __shared__ int flags[2];
+    const unsigned t = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (t >= nwork) return;
+    const Shared sh = share<NB, NQ>(lds, flags);
+    const unsigned k = t / ntile;
+    const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    stage_wide<NB, QP, NQ, RM, NZ>(qin, qn, qout, g, ph, sp, t - k * ntile, (int)k, part, 0, sh);
+}
+
+}  // namespace sg
+}  // namespace hd

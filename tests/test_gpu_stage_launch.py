@@ -1,0 +1,68 @@
+"""The fused stage's ways of taking a grid (five waves a tile, equal runs of
+planes, items of n planes) at the edges of its 63-cell tiles, against the C
+oracle (GPU).
+
+Tolerance 1e-12 relative per physical quantity, as in test_gpu_parity.py: both
+sides compute in FP64 and differ by contraction and summation order only."""
+import os
+
+import numpy as np
+import pytest
+
+from hermeshd_amd.config import HDConfig
+from test_gpu_parity import TOL, field_rel_err, smooth_state
+
+pytestmark = pytest.mark.gpu
+
+PERIODIC = ("periodic",) * 6
+MIXED = ("outflow", "outflow", "noslip", "wall", "periodic", "periodic")
+CASES = {
+    "nb4": dict(nbasis=4, iquad=2, nQ=5, riemann="hllc", integrator="heun"),
+    "nb8": dict(nbasis=8, iquad=2, nQ=5, riemann="roe", integrator="heun"),
+    "nb10": dict(nbasis=10, iquad=3, nQ=5, riemann="hllc", integrator="shu-osher"),
+    "nb4_stress": dict(nbasis=4, iquad=2, nQ=11, ivis=1, coll=20.0, colvis=0.5, riemann="hllc", integrator="heun",
+                       body_force=(0.02, -0.01, 0.03)),
+    "nb4_noise": dict(nbasis=4, iquad=2, nQ=11, ivis=0, coll=3.0, colvis=0.5, riemann="hllc", integrator="heun",
+                      noise=True, eta_sd=0.02),
+    "nb10_stress": dict(nbasis=10, iquad=3, nQ=11, ivis=1, coll=30.0, colvis=0.4, riemann="central",
+                        integrator="shu-osher"),
+}
+# one cell; a tile exactly, one short and one over; several tiles; planes that
+# the items do not divide
+SIZES = [(1, 1, 1), (62, 1, 3), (63, 2, 4), (64, 1, 5), (20, 13, 7)]
+
+
+@pytest.fixture(scope="module")
+def torch_mod():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a ROCm device"
+    return torch
+
+
+@pytest.mark.parametrize("bc", [PERIODIC, MIXED], ids=["periodic", "mixed"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_launch_forms_match_oracle(torch_mod, oracle_mod, name, bc):
+    from hermeshd_amd.solver import Solver
+    for n in SIZES:
+        cfg = HDConfig(nx=n[0], ny=n[1], nz=n[2], lx=0.1 * n[0], ly=0.1 * n[1], lz=0.1 * n[2], bc=bc, T_floor=1e-4,
+                       limiter=True, **CASES[name])
+        q0 = smooth_state(cfg, seed=3)
+        o = oracle_mod.Oracle(cfg.as_ints())
+        ref, r1, r2 = q0.copy(), np.zeros_like(q0), np.zeros_like(q0)
+        t, dt = np.array(0.0), np.array(0.0)
+        o.step(ref, r1, r2, t, dt)
+        for planes in ("-1", "0", "1", "3"):
+            print(f"[stage_launch] {name} {n} planes {planes}", flush=True)
+            old = os.environ.get("HD_STAGE_PLANES")
+            os.environ["HD_STAGE_PLANES"] = planes
+            try:
+                s = Solver(cfg)
+            finally:
+                if old is None:
+                    del os.environ["HD_STAGE_PLANES"]
+                else:
+                    os.environ["HD_STAGE_PLANES"] = old
+            q = torch_mod.from_numpy(q0.copy()).cuda()
+            s.step(q, torch_mod.zeros_like(q))
+            s.check()
+            assert field_rel_err(q.cpu().numpy(), ref) < TOL, (n, planes)
