@@ -864,7 +864,7 @@ __global__ __launch_bounds__(256) void k_stage_vjp_split(const double* __restric
 
 // ------------------------------------------------- 13-moment transpose ----
 // The transpose of a 13-moment stage on a grid periodic in every direction,
-// split as the forward stage is (fz::k_face13 + k_cell13), so that no lane
+// split into a face and a cell kernel, so that no lane
 // holds a whole cell: the face kernel writes, per face point, the cotangents
 // that the face flux sends to the traces of its two cells; the cell kernel,
 // one field per wave, adds the volume transpose and gathers those face
@@ -872,7 +872,7 @@ __global__ __launch_bounds__(256) void k_stage_vjp_split(const double* __restric
 // in another order.
 
 // One wave per face point over 64 consecutive faces of direction DIR (as
-// fz::k_face13): phase 1 stages both sides' trace coefficients (face_coeffs
+// one wave per face point): phase 1 stages both sides' trace coefficients (face_coeffs
 // of the limited modes q) and lifted-cotangent coefficients (lift_coeffs of
 // b*lam through the relaxation factors) in LDS; phase 2 forms the face
 // flux's cotangent mu at point p, reverses the Riemann solver and the

@@ -262,12 +262,9 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
                  nfz = (size_t)g.nx * g.ny * (g.nz + 1);
     c->npart = 1024;
     // the full 10-moment equations (ivis 2) and the water EOS (ieos 2) run on the
-    // table-driven kernels only, and the 13-moment model on the same face/cell
-    // split with its own kernels; HD_KERNELS=generic selects the table-driven
-    // kernels for any configuration
+    // table-driven kernels only; HD_KERNELS=generic selects those for any configuration
     const char* kern = std::getenv("HD_KERNELS");
-    c->generic = (kern && std::strcmp(kern, "generic") == 0) || cfg->ivis == 2 || cfg->ieos == 2 ||
-                 cfg->nQ == 13;
+    c->generic = (kern && std::strcmp(kern, "generic") == 0) || cfg->ivis == 2 || cfg->ieos == 2;
     if (c->generic && cfg->noise) {
         hd_destroy(c);
         return fail(HD_ERR_UNSUPPORTED, "the table-driven kernels (HD_KERNELS=generic) carry no stochastic stress");
@@ -317,7 +314,6 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
         return fail(HD_ERR_HIP, "initialising context buffers failed");
     }
     if (const char* lm = std::getenv("HD_LIMITER")) c->table_limiter = std::strcmp(lm, "table") == 0;
-    if (const char* fc = std::getenv("HD_FACES")) c->table_faces = std::strcmp(fc, "table") == 0;
     if (const char* vj = std::getenv("HD_VJP")) c->fused_vjp = std::strcmp(vj, "fused") == 0;
     if (hipDeviceGetAttribute(&c->num_cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) c->num_cus = 256;
     if (const char* sp = std::getenv("HD_STAGE_PLANES")) c->stage_planes = std::max(-1, std::atoi(sp));
@@ -489,7 +485,8 @@ int hd_apply_mask(hd_ctx* c, double* q, void* stream) {
 }
 
 // The split 13-moment transpose (periodic grids) writes the left cells' face
-// cotangents into fl and the right cells' into bq2, allocated here once.
+// cotangents into fl and the right cells' into bq2, allocated here once (fl is
+// there already where the table-driven kernels run).
 static int ensure_vjp13_buffers(hd_ctx* c) {
     if (c->cfg.nQ != 13 || c->fused_vjp || c->bq2[0]) return HD_OK;
     for (int b = 0; b < 6; b++)
@@ -498,8 +495,10 @@ static int ensure_vjp13_buffers(hd_ctx* c) {
     const size_t nf = (size_t)c->nface * c->nQ;
     const size_t nfd[3] = {(size_t)(g.nx + 1) * g.ny * g.nz, (size_t)g.nx * (g.ny + 1) * g.nz,
                            (size_t)g.nx * g.ny * (g.nz + 1)};
-    for (int d = 0; d < 3; d++) {
-        const int r = alloc(c, (void**)&c->bq2[d], nf * nfd[d] * sizeof(double));
+    for (int d = 2; d >= 0; d--) {  // bq2[0] last: it says that all are there
+        int r = HD_OK;
+        if (!c->fl[d]) r = alloc(c, (void**)&c->fl[d], nf * nfd[d] * sizeof(double));
+        if (r == HD_OK && !c->bq2[d]) r = alloc(c, (void**)&c->bq2[d], nf * nfd[d] * sizeof(double));
         if (r) return r;
     }
     return HD_OK;

@@ -62,8 +62,6 @@ struct hd_ctx {
     int stage_planes = hd::STAGE_AUTO;
     // table-driven limiter kernel instead of fz::k_limit (HD_LIMITER=table)
     int table_limiter = 0;
-    // one-thread-per-face k_face_flux for periodic 13-moment grids too (HD_FACES=table)
-    int table_faces = 0;
     // fused per-cell transpose for periodic 13-moment grids too (HD_VJP=fused)
     int fused_vjp = 0;
     int64_t bytes = 0;

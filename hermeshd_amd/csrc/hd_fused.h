@@ -1,6 +1,6 @@
 // hd_fused.h -- what the fused kernels share: the basis and quadrature rules as
 // compile-time constants, face polynomials, mode loads, the limiter; and the
-// 13-moment face and cell kernels.
+// 13-moment cell kernel of the table-driven path.
 //
 // Operator (the reference's glflux + innerintegral2 + source_calc +
 // advance_time_level, src/flux.f90:751-1022, src/sources.f90:12-84,
@@ -393,144 +393,18 @@ __global__ __launch_bounds__(256, (NB == 4 ? 4 : (NB == 8 ? 2 : 1))) void k_limi
 // ------------------------------------------------------------ kernel -------
 __device__ __forceinline__ void fence() { asm volatile("" ::: "memory"); }
 
-// Face fluxes of the 13-moment model on a grid periodic in every direction,
-// as face moments fl[((f*NK + k)*nfaces) + face] (lift13_mom).  A workgroup
-// owns 64 consecutive faces of direction DIR, one wave per face point, so no
-// lane holds more than one point's states.  Phase 1 turns the modes of the
-// cells on both sides into face-polynomial coefficients (face_coeffs, NK per
-// field and side) in LDS, one (side, field, face) item per thread.  Phase 2
-// evaluates point p of every face on wave p (face_eval), then the physical
-// fluxes and the Riemann solver of k_face_flux.  Phase 3 reduces the points
-// of each (field, face) to the NK face moments.  Lanes past the last face
-// reuse the last face and store nothing.
-template <int NB, int QP, int RM, int DIR>
-__global__ __launch_bounds__(QP * QP * 64) void k_face13(const double* __restrict__ q, double* __restrict__ fl,
-                                                        Grid g, Phys ph) {
-    constexpr int NQ = 13, NF = QP * QP, NK = face_nk<NB>();
-    __shared__ double ks[2][NQ][NK][64];
-    const int ni = g.nx + (DIR == 0), nj = g.ny + (DIR == 1);
-    const long nfaces = (long)ni * nj * (g.nz + (DIR == 2));
-    const long f0 = (long)xcd_block() * 64;  // XCD-contiguous ranges of faces
-    // phase 1: NIT (side, field) items per thread, all their loads issued
-    // before the first is used
-    constexpr int NIT = (2 * NQ * 64 + NF * 64 - 1) / (NF * 64);
-    // the item stride NF*64 is a multiple of 64, so every item of a thread
-    // belongs to its lane's face: the two cells are found once per lane, in
-    // 32-bit arithmetic (hd_create bounds the faces per direction by 2^31)
-    long cell2[2];
-    {
-        const long fl64 = f0 + (long)(threadIdx.x & 63);
-        const unsigned fid = (unsigned)(fl64 < nfaces ? fl64 : nfaces - 1);
-        const unsigned fq = fid / (unsigned)ni;
-        int ci = (int)(fid - fq * (unsigned)ni), cj = (int)(fq % (unsigned)nj), ck = (int)(fq / (unsigned)nj);
-        int& a = DIR == 0 ? ci : DIR == 1 ? cj : ck;
-        const int n_ax = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
-        // side 0: the cell below the face (index a - 1, wrapped), side 1: above (index a, wrapped)
-        const int a_lo = a == 0 ? n_ax - 1 : a - 1, a_hi = a == n_ax ? 0 : a;
-        a = a_lo;
-        cell2[0] = (long)(unsigned)(ci + g.nx * (cj + g.ny * ck));
-        a = a_hi;
-        cell2[1] = (long)(unsigned)(ci + g.nx * (cj + g.ny * ck));
-    }
-    double m1[NIT][1][NB];
-#pragma unroll
-    for (int u = 0; u < NIT; u++) {
-        const int it = (int)threadIdx.x + u * NF * 64;
-        if (it < 2 * NQ * 64) {
-            const int side = (it >> 6) / NQ, fld = (it >> 6) % NQ;
-            const long cell = side == 0 ? cell2[0] : cell2[1];
-#pragma unroll
-            for (int r = 0; r < NB; r++) m1[u][0][r] = q[((long)r * NQ + fld) * g.N + cell];
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < NIT; u++) {
-        const int it = (int)threadIdx.x + u * NF * 64;
-        if (it < 2 * NQ * 64) {
-            const int l = it & 63, side = (it >> 6) / NQ, fld = (it >> 6) % NQ;
-            double K1[1][NK];
-            if (side == 0) face_coeffs<NB, 1, DIR, 1, NK>(m1[u], K1);
-            else face_coeffs<NB, 1, DIR, 0, NK>(m1[u], K1);
-#pragma unroll
-            for (int k = 0; k < NK; k++) ks[side][fld][k][l] = K1[0][k];
-        }
-    }
-    __syncthreads();
-    // lanes past the last face evaluate the last face again and store nothing
-    const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int l = (int)(threadIdx.x & 63);
-    const auto& FP = face_poly<NB>();
-    double QL[NQ], QR[NQ];
-#pragma unroll
-    for (int f = 0; f < NQ; f++) {
-        double sl = ks[0][f][0][l], sr = ks[1][f][0][l];
-#pragma unroll
-        for (int k = 1; k < NK; k++) {
-            sl += ks[0][f][k][l] * FP.b[p][k];
-            sr += ks[1][f][k][l] * FP.b[p][k];
-        }
-        QL[f] = sl;
-        QR[f] = sr;
-    }
-    double FL[NQ], FR[NQ], out[NQ];
-    gflux<NQ, DIR>(ph, QL, FL);
-    gflux<NQ, DIR>(ph, QR, FR);
-#pragma unroll
-    for (int f = 0; f < NQ; f++) out[f] = 0.5 * (FL[f] + FR[f]);
-    if constexpr (RM == RIEMANN_HLLC) hllc_point<DIR>(ph, QL, QR, FL, FR, out);  // ideal gas: no last-state speed
-    if constexpr (RM == RIEMANN_ROE) roe_point<DIR, NQ>(ph, QL, QR, FL, FR, out);
-    // phase 3: the face moments M_k = sum_p wb_p[k] F_p of each field, the
-    // point fluxes exchanged through ks once every wave has read it
-    static_assert(NF <= 2 * NK, "the point fluxes fit in ks");
-    double* vs = &ks[0][0][0][0];
-    __syncthreads();
-#pragma unroll
-    for (int f = 0; f < NQ; f++) vs[(f * NF + p) * 64 + l] = out[f];
-    __syncthreads();
-    for (int it = (int)threadIdx.x; it < NQ * NK * 64; it += NF * 64) {
-        const int lf = it & 63;
-        const int fk = __builtin_amdgcn_readfirstlane(it >> 6);
-        const int f = fk / NK, k = fk - f * NK;
-        double s = 0.;
-#pragma unroll
-        for (int pp = 0; pp < NF; pp++) s += FP.wb[pp][k] * vs[(f * NF + pp) * 64 + lf];
-        if (f0 + lf < nfaces) fl[((long)f * NK + k) * nfaces + f0 + lf] = s;
-    }
-}
-
-// Face lift of one field in direction D from the face moments of k_face13:
-// sum_p w2_p phi_r(p) F_p on a face is Lface(deg_D(r), side) M_{k(r)}, with
-// k(r) the mode's face-polynomial pair, so the sums of lift13_dir become
-// t[r] += di (M+_{k(r)} - Lface(deg_D(r), 0) M-_{k(r)}), M+ of the cell's
-// high face and M- of its low face.
+// A face's lift onto mode r in direction D is Lface(deg_D(r), side) times one
+// face moment, sum_p w2_p b_k(p) F_p, k the mode's face-polynomial pair:
 template <int NB, int D>
 HD_DEV constexpr int lift_k(int r) {
     return pair_index(deg<NB>(r, row_axis(D)), deg<NB>(r, col_axis(D)));
 }
-template <int NB, int D>
-__device__ __forceinline__ void lift13_mom(const double* __restrict__ fl, long nfl, long fm, long fp, double di,
-                                           int f, double (&t)[NB]) {
-    constexpr int NK = face_nk<NB>();
-    double mm[NK], mp[NK];
-#pragma unroll
-    for (int k = 0; k < NK; k++) {
-        mm[k] = fl[((long)f * NK + k) * nfl + fm];
-        mp[k] = fl[((long)f * NK + k) * nfl + fp];
-    }
-#pragma unroll
-    for (int r = 0; r < NB; r++) {
-        const int k = lift_k<NB, D>(r);
-        const double s = deg<NB>(r, D) == 1 ? mp[k] + mm[k] : mp[k] - mm[k];
-        t[r] = D == 0 ? di * s : t[r] + di * s;
-    }
-}
-
 }  // namespace fz
 
 
-// MOM: the face arrays hold the face moments of fz::k_face13 (periodic
-// grids); otherwise the point fluxes of k_face_flux.
-template <int NB, int QP, bool MOM>
+// The 13-moment cell kernel of the table-driven path: the face arrays hold the
+// point fluxes of k_face_flux.
+template <int NB, int QP>
 __global__ __launch_bounds__(CELL13_WAVES * 64) void k_cell13(
     const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout,
     const double* __restrict__ flx, const double* __restrict__ fly, const double* __restrict__ flz,
@@ -562,15 +436,9 @@ __global__ __launch_bounds__(CELL13_WAVES * 64) void k_cell13(
     const long nfx = (long)(g.nx + 1) * g.ny * g.nz, nfy = (long)g.nx * (g.ny + 1) * g.nz,
                nfz = (long)g.nx * g.ny * (g.nz + 1);
     double t[NB];
-    if constexpr (MOM) {
-        fz::lift13_mom<NB, 0>(flx, nfx, fxm, fxm + 1, dxi, f, t);
-        fz::lift13_mom<NB, 1>(fly, nfy, fym, fym + g.nx, dyi, f, t);
-        fz::lift13_mom<NB, 2>(flz, nfz, fzm, fzm + (long)g.nx * g.ny, dzi, f, t);
-    } else {
-        lift13_dir<NB, NF, 0>(flx, nfx, fxm, fxm + 1, dxi, f, T, t);
-        lift13_dir<NB, NF, 1>(fly, nfy, fym, fym + g.nx, dyi, f, T, t);
-        lift13_dir<NB, NF, 2>(flz, nfz, fzm, fzm + (long)g.nx * g.ny, dzi, f, T, t);
-    }
+    lift13_dir<NB, NF, 0>(flx, nfx, fxm, fxm + 1, dxi, f, T, t);
+    lift13_dir<NB, NF, 1>(fly, nfy, fym, fym + g.nx, dyi, f, T, t);
+    lift13_dir<NB, NF, 2>(flz, nfz, fzm, fzm + (long)g.nx * g.ny, dzi, f, T, t);
     // ---- volume integral: every wave reaches every barrier ----
     // glf[r] = 0.25 cb[r] (t[r] - sum_d di acc_d[r]) for r >= 1, so each
     // accumulator starts at -t[r] over its grid factor and t[1..] need not

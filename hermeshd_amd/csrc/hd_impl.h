@@ -21,18 +21,6 @@ struct Impl {
     static void faces(hd_ctx* c, const double* q, hipStream_t s) {
         const Grid& g = c->grid;
         long nfx = (long)(g.nx + 1) * g.ny * g.nz, nfy = (long)g.nx * (g.ny + 1) * g.nz, nfz = (long)g.nx * g.ny * (g.nz + 1);
-        if constexpr (NQ == 13) {
-            // all-periodic grids: one wave per face point (fz::k_face13)
-            bool periodic = !c->table_faces;
-            for (int b = 0; b < 6; b++) periodic = periodic && g.bc[b] == BC_PERIODIC;
-            if (periodic) {
-                constexpr int NT = QP * QP * 64;
-                hipLaunchKernelGGL((fz::k_face13<NB, QP, RM, 0>), dim3(blocks_for(nfx, 64)), dim3(NT), 0, s, q, c->fl[0], g, c->ph);
-                hipLaunchKernelGGL((fz::k_face13<NB, QP, RM, 1>), dim3(blocks_for(nfy, 64)), dim3(NT), 0, s, q, c->fl[1], g, c->ph);
-                hipLaunchKernelGGL((fz::k_face13<NB, QP, RM, 2>), dim3(blocks_for(nfz, 64)), dim3(NT), 0, s, q, c->fl[2], g, c->ph);
-                return;
-            }
-        }
         hipLaunchKernelGGL((k_face_flux<NB, QP, NQ, RM, 0>), dim3(blocks_for(nfx, 128)), dim3(128), 0, s, q, c->fl[0], c->dtab, g, c->ph, c->inflow);
         hipLaunchKernelGGL((k_face_flux<NB, QP, NQ, RM, 1>), dim3(blocks_for(nfy, 128)), dim3(128), 0, s, q, c->fl[1], c->dtab, g, c->ph, c->inflow);
         hipLaunchKernelGGL((k_face_flux<NB, QP, NQ, RM, 2>), dim3(blocks_for(nfz, 128)), dim3(128), 0, s, q, c->fl[2], c->dtab, g, c->ph, c->inflow);
@@ -40,16 +28,9 @@ struct Impl {
     static void cell(hd_ctx* c, const double* qin, const double* qn, double* qout, const StageParams& sp, hipStream_t s) {
         if constexpr (NQ == 13) {
             // one field per wave, 64 cells per workgroup (every wave of a
-            // workgroup reaches its barriers: the grid is padded, not clipped);
-            // face moments from k_face13 on all-periodic grids (as faces())
-            bool periodic = !c->table_faces;
-            for (int b = 0; b < 6; b++) periodic = periodic && c->grid.bc[b] == BC_PERIODIC;
-            if (periodic)
-                hipLaunchKernelGGL((k_cell13<NB, QP, true>), dim3(blocks_for(c->N, 64)), dim3(CELL13_WAVES * 64), 0,
-                                   s, qin, qn, qout, c->fl[0], c->fl[1], c->fl[2], c->dtab, c->grid, c->ph, sp);
-            else
-                hipLaunchKernelGGL((k_cell13<NB, QP, false>), dim3(blocks_for(c->N, 64)), dim3(CELL13_WAVES * 64), 0,
-                                   s, qin, qn, qout, c->fl[0], c->fl[1], c->fl[2], c->dtab, c->grid, c->ph, sp);
+            // workgroup reaches its barriers: the grid is padded, not clipped)
+            hipLaunchKernelGGL((k_cell13<NB, QP>), dim3(blocks_for(c->N, 64)), dim3(CELL13_WAVES * 64), 0, s, qin, qn,
+                               qout, c->fl[0], c->fl[1], c->fl[2], c->dtab, c->grid, c->ph, sp);
             return;
         }
         hipLaunchKernelGGL((k_cell<NB, QP, NQ>), dim3(blocks_for(c->N, 128)), dim3(128), 0, s, qin, qn, qout, c->fl[0],
@@ -64,7 +45,7 @@ struct Impl {
         if constexpr (!(NB == 10 && NQ >= 11)) {  // its five waves would not have the registers
             if (planes < 0) {
                 const unsigned n = tiles * (unsigned)g.nz, grid = (n + 7) / 8 * 8;
-                if constexpr (NQ >= 11) {
+                if constexpr (NQ == 11) {
                     if (sp.noise[0]) {
                         hipLaunchKernelGGL((sg::k_stage_wide<NB, QP, NQ, RM, true>), dim3(grid), dim3(320), 0, s, qin,
                                            qn, qout, g, c->ph, sp, tiles, n);
@@ -80,7 +61,7 @@ struct Impl {
         const long n = zc ? (long)tiles * ((g.nz + zc - 1) / zc)
                           : std::min((long)tiles * g.nz, (long)c->num_cus * sg::occupancy<NB, NQ>());
         const unsigned grid = (unsigned)((n + 7) / 8 * 8);
-        if constexpr (NQ >= 11) {
+        if constexpr (NQ == 11) {
             if (sp.noise[0]) {
                 hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, true>), dim3(grid), dim3(256), 0, s, qin, qn, qout, g,
                                    c->ph, sp, tiles, zc);
@@ -113,9 +94,8 @@ struct Impl {
     static void stage_vjp(hd_ctx* c, const double* q, const double* lam, double* lam_in, const adj::AdjParams& ap,
                           hipStream_t s);
     static Ops ops() {
-        // the 13-moment model runs on its own face and cell kernels (no fused
-        // stage, no ensembles); its transpose is split on periodic grids
-        if constexpr (NQ == 13) return Ops{&limiter, &faces, &cell, nullptr, nullptr, nullptr, &stage_vjp};
+        // no ensembles of the 13-moment model; its transpose is split on periodic grids
+        if constexpr (NQ == 13) return Ops{&limiter, &faces, &cell, &fused, nullptr, nullptr, &stage_vjp};
         else return Ops{&limiter, &faces, &cell, &fused, &ens_limit, &ens_stage, &stage_vjp};
     }
 };

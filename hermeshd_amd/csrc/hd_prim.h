@@ -100,10 +100,52 @@ __device__ __forceinline__ double root(double x) {
     return x == 0.0 ? x : g;
 }
 
+// Roe flux (roe_point: Eulderink and Mellema, half the thermal enthalpy) from
+// the traces' velocities, pressures and 1/rho, with refined reciprocals and
+// roots; out holds 0.5 (FL + FR) on entry.
+template <int DIR>
+__device__ __forceinline__ void roe_diss(const Phys& ph, const double* QL, const double* QR, double riL, double riR,
+                                         const double* uL, const double* uR, double pL, double pR, double* out) {
+    constexpr int IP = MX + DIR, I1 = MX + (DIR + 1) % 3, I2 = MX + (DIR + 2) % 3;
+    constexpr int A = DIR, B = (DIR + 1) % 3, C = (DIR + 2) % 3;
+    const double cp = ph.gamma * ph.gm1i;
+    const double kL = root(QL[RH]), kR = root(QR[RH]), ki = rcp(kL + kR);
+    const double hL = fma(uL[0], uL[0], fma(uL[1], uL[1], fma(uL[2], uL[2], cp * (pL * riL))));
+    const double hR = fma(uR[0], uR[0], fma(uR[1], uR[1], fma(uR[2], uR[2], cp * (pR * riR))));
+    const double v0 = fma(kL, uL[A], kR * uR[A]) * ki, v1 = fma(kL, uL[B], kR * uR[B]) * ki,
+                 v2 = fma(kL, uL[C], kR * uR[C]) * ki, h = 0.5 * (fma(kL, hL, kR * hR) * ki);
+    const double hv = 0.5 * fma(v0, v0, fma(v1, v1, v2 * v2));
+    const double asq = ph.gm1 * (h - hv);
+    if (__builtin_expect(!(asq > 0.0), 0)) {
+        // no Roe sound speed: local Lax-Friedrichs, as the legacy code
+        const double cw = fmax(fabs(uL[A]) + root(ph.gamma * pL * riL), fabs(uR[A]) + root(ph.gamma * pR * riR));
+#pragma unroll
+        for (int f = 0; f < 5; f++) out[f] -= 0.5 * cw * (QR[f] - QL[f]);
+        return;
+    }
+    const double ai = rcp(asq), a = root(asq);
+    const double dr = fma(QR[RH], riL, -1.), de = (QR[EN] - QL[EN]) * riL, dn = (QR[IP] - QL[IP]) * riL,
+                 d1 = (QR[I1] - QL[I1]) * riL, d2 = (QR[I2] - QL[I2]) * riL;
+    const double ea = ph.gm1 * ai;
+    const double vd = fma(v0, dn, fma(v1, d1, fma(v2, d2, -de)));
+    const double ev = 0.5 * ea * fma(hv, dr, -vd), od = 0.5 * fma(-v0, dr, dn) * (a * ai);
+    const double l2 = fabs(v0);
+    const double t0 = (ev - od) * fabs(v0 - a), t1 = (ev + od) * fabs(v0 + a);
+    const double t2 = ea * fma(h - 2. * hv, dr, vd) * l2, t3 = fma(-v1, dr, d1) * l2, t4 = fma(-v2, dr, d2) * l2;
+    const double sr = t0 + t1 + t2, hl = -0.5 * QL[RH];
+    out[RH] = fma(hl, sr, out[RH]);
+    out[IP] = fma(hl, fma(v0, sr, a * (t1 - t0)), out[IP]);
+    out[I1] = fma(hl, fma(v1, sr, t3), out[I1]);
+    out[I2] = fma(hl, fma(v2, sr, t4), out[I2]);
+    out[EN] = fma(hl, fma(h, t0 + t1, fma(a * v0, t1 - t0, fma(hv, t2, fma(v1, t3, v2 * t4)))), out[EN]);
+}
+
 // Flux through one face point from the two traces: rh..en by the Riemann
 // solver RM, and with stress (NQ >= 11, traces holding rh..en and row DIR of
 // the stress) the averaged velocity in F[5..7], to which the central fluxes
-// of the stress rows are proportional.  S: the row of the stochastic stress.
+// of the stress rows are proportional; with 13 moments (traces holding also
+// the heat flux along DIR) the averaged temperature in F[8].  S: the row of
+// the stochastic stress.
 // HLLC keeps density, velocity and pressure of both sides, selects one, and
 // forms the conserved values and the flux of that side only (few values are
 // live at a time; the momentum and energy come back to rounding).  HLLC after
@@ -122,6 +164,8 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
 #pragma unroll
         for (int a = 0; a < 3; a++) F[5 + a] = 0.5 * (uL[a] + uR[a]);
     }
+    if constexpr (NQ == 13)
+        F[8] = 0.5 * ((pL < ph.P_floor ? ph.P_floor : pL) * riL + (pR < ph.P_floor ? ph.P_floor : pR) * riR);
     // physical flux of one side: floored pressure, stress row less the noise
     auto side_flux = [&](const double* Q, const double* u, double p, const double* P3, double* f) {
         const double pf = p < ph.P_floor ? ph.P_floor : p;
@@ -137,6 +181,7 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
                 f[MX + a] = fma(Q[MX + a], un, a == DIR ? Pn[a] + pf : Pn[a]);
             }
             f[EN] += fma(Pn[0], u[0], fma(Pn[1], u[1], Pn[2] * u[2]));
+            if constexpr (NQ == 13) f[EN] += P3[3];
         } else {
 #pragma unroll
             for (int a = 0; a < 3; a++) f[MX + a] = a == DIR ? fma(Q[MX + a], un, pf) : Q[MX + a] * un;
@@ -148,7 +193,7 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
         side_flux(QR, uR, pR, QR + 5, FR);
 #pragma unroll
         for (int f = 0; f < 5; f++) F[f] = 0.5 * (FL[f] + FR[f]);
-        if constexpr (RM == RIEMANN_ROE) roe_point<DIR>(ph, QL, QR, FL, FR, F);
+        if constexpr (RM == RIEMANN_ROE) roe_diss<DIR>(ph, QL, QR, riL, riR, uL, uR, pL, pR, F);
         return;
     }
     const double nL = uL[DIR], nR = uR[DIR];
@@ -174,12 +219,13 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
     }
     const bool right = s3 || s2;
     const double r = right ? rR : rL, p = right ? pR : pL, Sk = right ? SR : SL;
-    double u[3], P3[3] = {0., 0., 0.}, Q[5], f[5];
+    double u[3], P3[4] = {0., 0., 0., 0.}, Q[5], f[5];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         u[a] = right ? uR[a] : uL[a];
         if constexpr (NQ >= 11) P3[a] = right ? QR[5 + a] : QL[5 + a];
     }
+    if constexpr (NQ == 13) P3[3] = right ? QR[8] : QL[8];
     if (none) return;
     Q[RH] = r;
 #pragma unroll

@@ -22,7 +22,8 @@
 // Fields of a face: the stress fields' flux is linear in the velocity, and a
 // face of direction d carries only row d of the stress.  With stress a face
 // therefore has eight values (rh..en and the row) and eight fluxes (rh..en
-// and the velocity, from which the six stress rows follow), not eleven.
+// and the velocity, from which the six stress rows follow), not eleven; with
+// 13 moments also the heat flux along d and, for its flux, the temperature.
 #pragma once
 #include "hd_fused.h"
 
@@ -32,17 +33,48 @@ namespace sg {
 using fz::CellPos;
 
 // values and moments of a face
-HD_DEV constexpr int face_nm(int nq) { return nq >= 11 ? 8 : 5; }
-// field of value e of a face of direction d
+HD_DEV constexpr int face_nm(int nq) { return nq == 13 ? 9 : (nq >= 11 ? 8 : 5); }
+// Field of value e of a face of direction d: rh..en, the row of the stress,
+// with 13 moments the heat flux along d.  The 13-moment pzz = -pxx - pyy has
+// no field of its own (face_pzz): its value starts from pxx.
 HD_DEV constexpr int face_field(int nq, int d, int e) {
     return e < 5 ? e
+         : e == 8 ? T_QX + d
+         : nq == 13 ? (d == 0 ? (e == 5 ? T_PXX : (e == 6 ? T_PXY : T_PXZ))
+                     : d == 1 ? (e == 5 ? T_PXY : (e == 6 ? T_PYY : T_PYZ))
+                              : (e == 5 ? T_PXZ : (e == 6 ? T_PYZ : T_PXX)))
          : d == 0 ? (e == 5 ? PXX : (e == 6 ? PXY : PXZ))
          : d == 1 ? (e == 5 ? PXY : (e == 6 ? PYY : PYZ))
                   : (e == 5 ? PXZ : (e == 6 ? PYZ : PZZ));
 }
+HD_DEV constexpr bool face_pzz(int nq, int d, int e) { return nq == 13 && d == 2 && e == 7; }
+// stress P_da at a point with fields Q
+template <int NQ>
+__device__ __forceinline__ double stress_value(const double* Q, int d, int a) {
+    if (NQ == 13 && d == 2 && a == 2) return -(Q[T_PXX] + Q[T_PYY]);
+    return Q[face_field(NQ, d, 5 + a)];
+}
 // stochastic stress component of row d, column a
 HD_DEV constexpr int noise_comp(int d, int a) {
     return d == a ? d : (d + a == 1 ? 3 : (d + a == 2 ? 4 : 5));
+}
+// Scalars whose fluxes drive the fields past en: the velocity, with 13 moments
+// also the temperature.
+HD_DEV constexpr int nscal(int nq) { return nq == 13 ? 4 : (nq >= 11 ? 3 : 1); }
+// Factor of field f's flux in direction d from scalar a: colvis (4/3, -2/3 or
+// 1) times u_a for the stress, col_q T along d for the heat flux; 0 if none.
+HD_DEV constexpr bool drives(int nq, int f, int a, int d) {
+    if (nq == 13 && f >= T_QX) return a == 3 && f - T_QX == d;
+    if (a > 2 || f < 5) return false;
+    const int ndiag = nq == 13 ? 2 : 3;
+    if (f < 5 + ndiag) return a == d;
+    const int off = f - 5 - ndiag;  // xy, xz, yz
+    return a != d && off == (a + d == 1 ? 0 : (a + d == 2 ? 1 : 2));
+}
+__device__ __forceinline__ double drive_factor(const Phys& ph, int nq, int f, int a) {
+    if (a == 3) return ph.colq;
+    if (f < 5 + (nq == 13 ? 2 : 3)) return f - 5 == a ? ph.c4d3cv : -ph.c2d3cv;
+    return ph.colvis;
 }
 
 // Pointer to cell c of plane `plane`, stepped plane by plane.  The empty asm
@@ -97,8 +129,10 @@ __device__ __forceinline__ void load_side(const double* __restrict__ q, long N, 
 #pragma unroll
         for (int f = 0; f < NQ; f++) {
 #pragma unroll
-            for (int e = 0; e < NM; e++)
-                if (face_field(NQ, DIR, e) == f) m[e][r] = *p;
+            for (int e = 0; e < NM; e++) {
+                if (face_field(NQ, DIR, e) == f) m[e][r] = face_pzz(NQ, DIR, e) ? -*p : *p;
+                else if (face_pzz(NQ, DIR, e) && f == T_PYY) m[e][r] -= *p;
+            }
             step(p, N);
         }
 }
@@ -290,10 +324,10 @@ __device__ __forceinline__ double scalar(double x) {
 // Fluxes at volume point (i,j,k) from the point's fields Q, projected onto
 // the modes' derivatives; the products are written as fma so that the
 // compiler does not share scaled modes between points (which would keep
-// hundreds of them alive).  HYD: rh..en into rhs; VEL: the velocity into au.
+// hundreds of them alive).  HYD: rh..en into rhs; VEL: the scalars into au.
 template <int NB, int QP, int NQ, bool NZ, bool HYD, bool VEL>
-__device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], int i, int j, int k, double (&rhs)[5][NB],
-                                             double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()], const Phys& ph,
+__device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : (NQ == 13 ? 5 : 4)], int i, int j, int k, double (&rhs)[5][NB],
+                                             double (&au)[nscal(NQ)][3][ndeg<NB>()], const Phys& ph,
                                              const double (&di)[3], const StageParams& sp, long c, long N) {
     float S[6];
     if constexpr (NZ && HYD) {
@@ -304,7 +338,7 @@ __device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], in
     const double ri = pr::rcp(Q[RH]);
     const double u[3] = {Q[MX] * ri, Q[MY] * ri, Q[MZ] * ri};
     double P = 0.;
-    if constexpr (HYD) {
+    if constexpr (HYD || NQ == 13) {
         P = ph.gm1 * (Q[EN] - 0.5 * (Q[MX] * u[0] + Q[MY] * u[1] + Q[MZ] * u[2]));
         P = P < ph.P_floor ? ph.P_floor : P;
     }
@@ -321,11 +355,13 @@ __device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], in
             double Pn[3];
 #pragma unroll
             for (int a = 0; a < 3; a++) {
-                Pn[a] = Q[face_field(NQ, d, 5 + a)];
+                Pn[a] = stress_value<NQ>(Q, d, a);
                 if constexpr (NZ) Pn[a] -= (double)S[noise_comp(d, a)];
                 F[MX + a] = fma(Q[MX + a], ud, wd * (a == d ? Pn[a] + P : Pn[a]));
             }
-            F[EN] = fma(wd, fma(Pn[0], u[0], fma(Pn[1], u[1], Pn[2] * u[2])), F[EN]);
+            double pu = fma(Pn[0], u[0], fma(Pn[1], u[1], Pn[2] * u[2]));
+            if constexpr (NQ == 13) pu += Q[T_QX + d];
+            F[EN] = fma(wd, pu, F[EN]);
         } else if constexpr (HYD) {
 #pragma unroll
             for (int a = 0; a < 3; a++) F[MX + a] = a == d ? fma(Q[MX + a], ud, wd * P) : Q[MX + a] * ud;
@@ -344,6 +380,8 @@ __device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], in
 #pragma unroll
                 for (int a = 0; a < 3; a++)
                     au[a][d][deg_index<NB>(d, r)] = fma(cf, a == d ? ud : wd * u[a], au[a][d][deg_index<NB>(d, r)]);
+                if constexpr (NQ == 13)
+                    au[3][d][deg_index<NB>(d, r)] = fma(cf, wd * (P * ri), au[3][d][deg_index<NB>(d, r)]);
             }
         }
     }
@@ -351,17 +389,17 @@ __device__ __forceinline__ void volume_point(const double (&Q)[HYD ? NQ : 4], in
 }
 
 // innerintegral2 (src/flux.f90:751-928) of cell c without its 0.25 cb_r; with
-// stress, the stress rows' fluxes are carried by the velocity's projections
-// au[a][d][.] onto the modes that vary along d.  nbasis 10 holds one x plane
+// stress, the fluxes of the fields past en are carried by their scalars'
+// projections au[a][d][.] onto the modes that vary along d.  nbasis 10 holds one x plane
 // of the cell at a time (its polynomial in y and z, six coefficients a
 // field) and reads the modes once per plane, since modes and accumulators
 // together do not fit 256 registers.  I0, I1: the x planes of the rule to take.
 template <int NB, int QP, int NQ, bool NZ, bool HYD, bool VEL, int I0, int I1>
 __device__ __forceinline__ void volume_moments(const double* __restrict__ q, const Grid& g, long c,
-                                               double (&rhs)[5][NB], double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()],
+                                               double (&rhs)[5][NB], double (&au)[nscal(NQ)][3][ndeg<NB>()],
                                                const Phys& ph, const StageParams& sp) {
     const double di[3] = {g.dxi, g.dyi, g.dzi};
-    constexpr int NV = HYD ? NQ : 4;  // fields read
+    constexpr int NV = HYD ? NQ : (NQ == 13 ? 5 : 4);  // fields read
     if constexpr (NB == 10) {
 #pragma unroll
         for (int i = I0; i < I1; i++) {
@@ -432,28 +470,37 @@ __device__ __forceinline__ void volume_moments(const double* __restrict__ q, con
 // wv fac dt 0.25 cb_r times its lift (advance_time_level and the SSP
 // combination, src/integrator.f90:62-86,210-232).
 struct Weights {
-    double wm, wn, ws, wsf;  // of m, q_n, the right-hand side and (with relaxation) the stress fields'
-    double wmf;
+    double wn;        // of q_n
+    double wm[3], ws[3];  // of m and of the right-hand side: rh..en, stress, heat flux
 };
+template <int NQ>
+HD_DEV constexpr int field_class(int f) { return f < 5 ? 0 : (NQ == 13 && f >= T_QX ? 2 : 1); }
+template <int NQ>
 __device__ __forceinline__ Weights stage_weights(const StageParams& sp) {
     Weights w;
     const double* pdt = sp.dt;
     asm volatile("" : "+s"(pdt));  // read where it is used, not kept in registers across the planes
     if (sp.mode == 1) {
-        w.wm = 0.;
         w.wn = 0.;
-        w.ws = w.wsf = 1.;
-        w.wmf = 0.;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            w.wm[i] = 0.;
+            w.ws[i] = 1.;
+        }
         return w;
     }
     const double dt = *pdt;
     const double wv = sp.combine == 0 ? 1. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.25 : 2. / 3.));
     w.wn = sp.combine == 0 ? 0. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.75 : 1. / 3.));
-    const double faci = sp.ivis == 1 ? 1. / (1. + dt * sp.coll) : 1.;
-    w.wm = wv;
-    w.ws = wv * dt;
-    w.wmf = wv * faci;
-    w.wsf = w.wmf * dt;
+    w.wm[0] = w.wm[1] = w.wm[2] = wv;
+    if constexpr (NQ >= 11) {
+        if (sp.ivis == 1) {
+            w.wm[1] = wv * (1. / (1. + dt * sp.coll));
+            if constexpr (NQ == 13) w.wm[2] = wv * (1. / (1. + dt * sp.coll_q));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) w.ws[i] = w.wm[i] * dt;
     return w;
 }
 
@@ -491,9 +538,10 @@ __device__ __forceinline__ void start_field(const double* __restrict__ qin, cons
     // sources (src/sources.f90:12-84): ivis 0 relaxes the stress explicitly
     // (-coll*P, projected exactly in modal space); body force rho*g, m.g
     if constexpr (NQ >= 11) {
-        if (f >= PXX && sp.ivis == 0 && sp.coll != 0.)
+        const double rate = field_class<NQ>(f) == 2 ? sp.coll_q : sp.coll;
+        if (f >= 5 && sp.ivis == 0 && rate != 0.)
 #pragma unroll
-            for (int r = 0; r < NB; r++) t[r] = fma(-sp.coll, m[r], t[r]);
+            for (int r = 0; r < NB; r++) t[r] = fma(-rate, m[r], t[r]);
     }
     if (f >= MX && f <= MZ && sp.bf[f - MX] != 0.) {
         gptr p = plane_ptr(qin, g.N, RH, c);
@@ -511,7 +559,7 @@ __device__ __forceinline__ void start_field(const double* __restrict__ qin, cons
             step(p, st);
         }
     }
-    const double wm = f >= PXX ? w.wmf : w.wm, ws = f >= PXX ? w.wsf : w.ws;
+    const double wm = w.wm[field_class<NQ>(f)], ws = w.ws[field_class<NQ>(f)];
 #pragma unroll
     for (int r = 0; r < NB; r++) t[r] = fma(ws, t[r], fma(wm, m[r], w.wn * q0[r]));
 }
@@ -526,58 +574,35 @@ __device__ __forceinline__ void lift(const double (&m)[NK], double (&t)[NB]) {
         t[r] += LO && fz::deg<NB>(r, D) != 1 ? x : -x;
     }
 }
-// The stress field that the flux of u_a in direction d drives (a != d)
-HD_DEV constexpr int shear_field(int a, int d) { return a + d == 1 ? PXY : (a + d == 2 ? PXZ : PYZ); }
-
-// The volume part of field f's right-hand side (without 0.25 cb_r) from the
-// projections of the velocity's fluxes, for the stress fields.
-template <int NB>
-__device__ __forceinline__ void stress_volume(const Phys& ph, const double (&au)[3][3][ndeg<NB>()], int f,
-                                              double (&t)[NB]) {
-#pragma unroll
-    for (int r = 0; r < NB; r++) {
-        double s = 0.;
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                if (fz::deg<NB>(r, d) == 0) continue;
-                const double x = au[a][d][deg_index<NB>(d, r)];
-                if (f <= PZZ && a == d) s = fma(f - PXX == a ? ph.c4d3cv : -ph.c2d3cv, x, s);
-                if (f >= PXY && a != d && f == (a + d == 1 ? PXY : (a + d == 2 ? PXZ : PYZ)))
-                    s = fma(ph.colvis, x, s);
-            }
-        t[r] = s;
-    }
-}
-
-// Field f's share of a part, without 0.25 cb_r: t (rh..en) or, for the stress
-// fields, what the velocity's lifts tu in direction D and its volume
+// Field f's share of a part, without 0.25 cb_r: t (rh..en) or, for the fields
+// past en, what the scalars' lifts tu in direction D and their volume
 // projections au (VOL) drive.
 template <int NB, int NQ, int D, bool VOL>
-__device__ __forceinline__ void part_field(const Phys& ph, const double (&t)[5][NB],
-                                           const double (&tu)[NQ >= 11 ? 3 : 1][NB],
-                                           const double (&au)[NQ >= 11 ? 3 : 1][3][ndeg<NB>()], int f,
-                                           double (&o)[NB]) {
+__device__ __forceinline__ void part_field(const Phys& ph, const double (&t)[5][NB], const double (&tu)[nscal(NQ)][NB],
+                                           const double (&au)[nscal(NQ)][3][ndeg<NB>()], int f, double (&o)[NB]) {
     if (f < 5) {
 #pragma unroll
         for (int r = 0; r < NB; r++) o[r] = t[f][r];
         return;
     }
+#pragma unroll
+    for (int r = 0; r < NB; r++) o[r] = 0.;
     if constexpr (NQ >= 11) {
-        if constexpr (VOL) {
-            stress_volume<NB>(ph, au, f, o);
-        } else {
 #pragma unroll
-            for (int r = 0; r < NB; r++) o[r] = 0.;
-        }
+        for (int a = 0; a < nscal(NQ); a++)
 #pragma unroll
-        for (int a = 0; a < 3; a++) {
-            if (a == D ? f > PZZ : f != shear_field(a, D)) continue;
-            const double cf = a != D ? ph.colvis : (f - PXX == a ? ph.c4d3cv : -ph.c2d3cv);
+            for (int d = 0; d < 3; d++) {
+                if (!drives(NQ, f, a, d)) continue;
+                const double cf = drive_factor(ph, NQ, f, a);
+                if constexpr (VOL) {
 #pragma unroll
-            for (int r = 0; r < NB; r++) o[r] = fma(cf, tu[a][r], o[r]);
-        }
+                    for (int r = 0; r < NB; r++)
+                        if (fz::deg<NB>(r, d) > 0) o[r] = fma(cf, au[a][d][deg_index<NB>(d, r)], o[r]);
+                }
+                if (d == D)
+#pragma unroll
+                    for (int r = 0; r < NB; r++) o[r] = fma(cf, tu[a][r], o[r]);
+            }
     }
 }
 
@@ -742,7 +767,7 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const d
     constexpr bool VOL = PART < QP;
     const Column o = column(g, tile, lane);
     const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
-    double t[5][NB], tu[NQ >= 11 ? 3 : 1][NB], au[NQ >= 11 ? 3 : 1][3][ndeg<NB>()];
+    double t[5][NB], tu[nscal(NQ)][NB], au[nscal(NQ)][3][ndeg<NB>()];
     {
         double M[NM][NK];
         column_face<NB, QP, NQ, RM, NZ, D>(qin, g, ph, sp, o, k, PART == 1 ? 1 : 0, M);
@@ -774,7 +799,7 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const d
         section();
     }
 #pragma unroll
-    for (int a = 0; a < (NQ >= 11 ? 3 : 1); a++)
+    for (int a = 0; a < nscal(NQ); a++)
 #pragma unroll
         for (int d = 0; d < 3; d++)
 #pragma unroll
@@ -792,11 +817,11 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const d
         pin(t);
         if constexpr (NQ >= 11) {
 #pragma unroll
-            for (int a = 0; a < 3; a++) pin(au[a]);
+            for (int a = 0; a < nscal(NQ); a++) pin(au[a]);
         }
         section();
     }
-    const Weights w = stage_weights(sp);
+    const Weights w = stage_weights<NQ>(sp);
     double* const R = (PART == 1 ? sh.r1 : sh.r0) + lane;
     // a batch of fields at a time: the loads of its modes and step-start
     // values together, the first batch's before the wait
@@ -823,7 +848,7 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const d
                 start_field<NB, NQ>(qin, g, sp, w, c, f, m[b], q0[b], v);
             } else {
 #pragma unroll
-                for (int r = 0; r < NB; r++) v[r] *= (f < 5 ? w.ws : w.wsf) * (0.25 * fz::cbasis<NB>(r));
+                for (int r = 0; r < NB; r++) v[r] *= w.ws[field_class<NQ>(f)] * (0.25 * fz::cbasis<NB>(r));
             }
 #pragma unroll
             for (int r = 0; r < NB; r++) {
@@ -846,7 +871,7 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
                                             double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     const Column o = column(g, tile, lane);
-    const Weights w = stage_weights(sp);
+    const Weights w = stage_weights<NQ>(sp);
     const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
     double v[NQ][NB];
 #pragma unroll
@@ -856,7 +881,7 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
     __syncthreads();
     double* const z = sh.z + lane;
     // same: the faces below and above are one (a periodic axis of one cell)
-    double tu[NQ >= 11 ? 3 : 1][NB];
+    double tu[nscal(NQ)][NB];
 #pragma unroll
     for (int e = 0; e < NM; e++) {
         double lo[NK], s[NB];
@@ -873,7 +898,7 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
         for (int n = 0; n < NK; n++) z[(e * NK + n) * 64] = M[e][n];
 #pragma unroll
         for (int r = 0; r < NB; r++) {
-            if (e < 5) v[e < 5 ? e : 0][r] = fma(w.ws * (0.25 * fz::cbasis<NB>(r)), s[r], v[e < 5 ? e : 0][r]);
+            if (e < 5) v[e < 5 ? e : 0][r] = fma(w.ws[0] * (0.25 * fz::cbasis<NB>(r)), s[r], v[e < 5 ? e : 0][r]);
             else tu[e < 5 ? 0 : e - 5][r] = s[r];
         }
         if (NB > 4 && e % 2 == 1) section();
@@ -882,9 +907,9 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
     for (int f = 0; f < NQ; f++) {
         if constexpr (NQ >= 11) {
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                if (f < 5 || (a == 2 ? f > PZZ : f != shear_field(a, 2))) continue;
-                const double cf = w.wsf * (a != 2 ? ph.colvis : (f == PZZ ? ph.c4d3cv : -ph.c2d3cv));
+            for (int a = 0; a < nscal(NQ); a++) {
+                if (!drives(NQ, f, a, 2)) continue;
+                const double cf = w.ws[field_class<NQ>(f)] * drive_factor(ph, NQ, f, a);
 #pragma unroll
                 for (int r = 0; r < NB; r++) v[f][r] = fma(cf * (0.25 * fz::cbasis<NB>(r)), tu[a][r], v[f][r]);
             }

@@ -26,6 +26,10 @@ CASES = {
                       noise=True, eta_sd=0.02),
     "nb10_stress": dict(nbasis=10, iquad=3, nQ=11, ivis=1, coll=30.0, colvis=0.4, riemann="central",
                         integrator="shu-osher"),
+    "nb4_13": dict(nbasis=4, iquad=2, nQ=13, ivis=0, coll=3.0, colvis=0.2, coll_q=2.0, col_q=0.3, riemann="hllc",
+                   integrator="heun"),
+    "nb10_13": dict(nbasis=10, iquad=3, nQ=13, ivis=1, coll=30.0, colvis=0.4, coll_q=12.0, col_q=0.6, riemann="roe",
+                    integrator="shu-osher"),
 }
 # one cell; a tile exactly, one short and one over; several tiles; planes that
 # the items do not divide
