@@ -290,12 +290,12 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
         return fail(r, msg);
     }
     if (cfg->noise) {
-        // the step's stress field: 6 components at every point of the three
-        // face lattices and of the volume rule
+        // the step's stress field: a row (3 components) at every point of the three
+        // face lattices, 6 components at those of the volume rule
         c->nfb = (long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
         c->kap_f = rule_kappa(c->htab, 2);
         c->kap_v = rule_kappa(c->htab, 3);
-        const size_t nfw = (size_t)6 * c->nface * c->nfb, nvw = (size_t)6 * c->htab.npg * c->N;
+        const size_t nfw = (size_t)3 * c->nface * c->nfb, nvw = (size_t)6 * c->htab.npg * c->N;
         for (int d = 0; d < 3 && r == HD_OK; d++) r = alloc(c, (void**)&c->noise_f[d], nfw * sizeof(float));
         if (r == HD_OK) r = alloc(c, (void**)&c->noise_v, nvw * sizeof(float));
         if (r) {

@@ -82,13 +82,13 @@ struct hd_ens {
     hd::LimParams lp;
     double dxi = 0., dyi = 0., dzi = 0., kap_f = 0., kap_v = 0.;
     std::vector<hd::ens::EnsReal> hreal;
-    std::vector<long> hpts;             // noise point prefix sums (nreal+1)
+    std::vector<long> hpts;             // noise point prefix sums (4*nreal+1)
     std::vector<int2> hwork;
     hd::ens::EnsReal* dreal = nullptr;
     long* dpts = nullptr;
     int2* dwork = nullptr;
     size_t work_cap = 0;
-    long state_doubles = 0, cells = 0, noise_floats = 0;
+    long state_doubles = 0, cells = 0;
     float* noise = nullptr;
     double* one_dt = nullptr;          // 1.0: the noise time step of hd_ens_rhs
     double* stage_buf = nullptr;       // RK3 third array when the caller passes none
@@ -100,10 +100,6 @@ struct hd_ens {
     hd::ens::Launch launch{};
     // captured step (hd_ens_run)
     hipStream_t cap_stream = nullptr;
-    // the next step's noise is drawn on side_stream while the captured
-    // step's stages run (fork/join events inside the capture)
-    hipStream_t side_stream = nullptr;
-    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     hipGraphExec_t gexec = nullptr;
     const void* gkey[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     int gchoice = -1;

@@ -21,7 +21,7 @@ namespace ens {
 struct EnsReal {
     Grid g;
     long qoff;     // offset of the realization's state in a packed array (doubles)
-    long noff;     // offset of its noise block: 3 face families of 6*nface*nfb, then 6*npg*N volume
+    long noff;     // offset of its noise block: 3 face families of 3*nface*nfb, then 6*npg*N volume
     long nfb;      // (nx+1)(ny+1)(nz+1)
     long cell0;    // first cell of the realization in the packed cell numbering
     int ntile;     // tiles of a plane
@@ -38,7 +38,7 @@ template <int NB, int QP, int NQ, int RM, bool NZ>
 __global__ __launch_bounds__(256, (sg::occupancy<NB, NQ>())) void k_ens_stage(
     const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout,
     const EnsReal* __restrict__ reals, const int2* __restrict__ work, Launch L, Phys ph, StageParams sp,
-    const float* __restrict__ noise, const unsigned long long* __restrict__ step, long nfloats) {
+    const float* __restrict__ noise) {
     constexpr int NF = QP * QP;
     __shared__ double lds[sg::lds_doubles<NB, NQ>()];
     __shared__ int flags[2];
@@ -50,9 +50,8 @@ __global__ __launch_bounds__(256, (sg::occupancy<NB, NQ>())) void k_ens_stage(
     const EnsReal& R = reals[wk.x];
     const Grid g = R.g;
     if constexpr (NZ) {
-        const long fsz = 6L * NF * R.nfb;
-        // the field of the current step: buffer (step & 1)
-        const float* base = noise + ((*step & 1ull) ? nfloats : 0L) + R.noff;
+        const long fsz = 3L * NF * R.nfb;
+        const float* base = noise + R.noff;
         sp.noise[0] = base;
         sp.noise[1] = base + fsz;
         sp.noise[2] = base + 2 * fsz;
@@ -90,16 +89,15 @@ __global__ __launch_bounds__(256) void k_ens_limit(double* __restrict__ q, const
     }
 }
 
-// Noise of every realization for the current step: flat over all points;
-// `pts` holds the prefix sums of the per-realization point counts
-// (3*nface*nfb + npg*N), each rounded up to a whole number of 256-thread
-// blocks so that a block lies in one realization (nreal+1 entries).
-constexpr long NOISE_BLOCK = 256;
+// Noise of every realization for the current step: flat over all points of
+// the realizations' families (three of faces, nface*nfb points each, and
+// npg*N volume points); `pts` holds the prefix sums of the families' counts,
+// each rounded up to whole chunks of 256 points so that a chunk lies in one
+// family (4*nreal+1 entries).
+constexpr long NOISE_CHUNK = 256;
 struct EnsNoise {
     unsigned long long seed;
     const unsigned long long* step;
-    int ahead;       // draws step *step + ahead
-    long nfloats;    // floats of one step's field; step s lives in buffer s & 1
     const double* dt;
     double eta_sd, zeta_sd, dVi, kap_f, kap_v;
     int nface, npg, nreal;
@@ -108,54 +106,42 @@ struct EnsNoise {
     float* out;
 };
 
-// One chunk of NOISE_BLOCK points (chunk b covers points b*NOISE_BLOCK ...).
-__device__ __forceinline__ void ens_noise_chunk(const EnsNoise& np, long b) {
-    // the chunk's realization: a search on its first point, uniform over the
-    // block
-    const long t0 = b * NOISE_BLOCK;
-    if (t0 >= np.pts[np.nreal]) return;
-    int lo = 0, hi = np.nreal;  // pts[lo] <= t0 < pts[hi]
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (np.pts[mid] <= t0) lo = mid; else hi = mid;
-    }
-    const EnsReal& R = np.reals[lo];
-    const long u = t0 - np.pts[lo] + threadIdx.x;
-    const long nf = (long)np.nface * R.nfb, nv = (long)np.npg * R.g.N;
-    if (u >= 3 * nf + nv) return;  // the padding of the last block
+// Each block takes an equal run of chunks: the amplitude is worked out and the
+// first family searched for once per block, not once per chunk.  The draw is
+// bound by vector instructions, as the stages are, so it runs before them, on
+// the whole device: beside them on a second stream, one block a CU, it slowed
+// them by more than it saved (96 boxes of 16^3 cells, 96 of 24^3 and 64 of
+// 32^3, one step: 5.7 ms beside the stages, 4.9 ms before them with the same
+// draw, 4.7 ms with this one).
+static __global__ __launch_bounds__(NOISE_CHUNK) void k_ens_noise(EnsNoise np) {
+    const long nchunk = np.pts[4 * np.nreal] / NOISE_CHUNK;
+    long b = nchunk * blockIdx.x / gridDim.x;
+    const long b1 = nchunk * (blockIdx.x + 1) / gridDim.x;
+    if (b >= b1) return;
     const double sq = sqrt(np.dVi / *np.dt);
-    const unsigned long long st = *np.step + (unsigned long long)np.ahead;
-    long id, count;
-    unsigned int stream;
-    float* out = np.out + ((st & 1ull) ? np.nfloats : 0L) + R.noff;
-    double kap;
-    if (u < 3 * nf) {
-        const int d = (u >= nf) + (u >= 2 * nf);
-        id = u - (long)d * nf;
-        count = nf;
-        stream = (unsigned int)(d + 1);
-        out += (long)d * 6 * nf;
-        kap = np.kap_f;
-    } else {
-        id = u - 3 * nf;
-        count = nv;
-        stream = 4u;
-        out += 3L * 6 * nf;
-        kap = np.kap_v;
+    const double ef = np.eta_sd * sq * np.kap_f, zf = np.zeta_sd * sq * np.kap_f;
+    const double ev = np.eta_sd * sq * np.kap_v, zv = np.zeta_sd * sq * np.kap_v;
+    const unsigned long long st = *np.step;
+    int s = 0, hi = 4 * np.nreal;  // pts[s] <= the chunk's first point < pts[hi]
+    while (hi - s > 1) {
+        const int mid = (s + hi) >> 1;
+        if (np.pts[mid] <= b * NOISE_CHUNK) s = mid; else hi = mid;
     }
-    double S[6];
-    noise::stress(np.seed, R.realization, st, stream, (unsigned long long)id, np.eta_sd * sq * kap,
-                  np.zeta_sd * sq * kap, S);
-#pragma unroll
-    for (int e = 0; e < 6; e++) out[(long)e * count + id] = (float)S[e];  // single precision, as k_noise
-}
-
-// Blocks stride over the chunks: one chunk per block when the grid covers
-// them all, or a small grid (one block per CU) that stays beside a running
-// stage kernel and draws the next step's field in the stage's shadow.
-static __global__ __launch_bounds__(NOISE_BLOCK) void k_ens_noise(EnsNoise np) {
-    const long nchunk = np.pts[np.nreal] / NOISE_BLOCK;
-    for (long b = blockIdx.x; b < nchunk; b += gridDim.x) ens_noise_chunk(np, b);
+    while (b < b1) {
+        const EnsReal& R = np.reals[s >> 2];
+        const int fam = s & 3;
+        const long nf = (long)np.nface * R.nfb, nv = (long)np.npg * R.g.N, count = fam < 3 ? nf : nv;
+        const long p0 = np.pts[s], p1 = np.pts[s + 1];
+        const long e = b1 < p1 / NOISE_CHUNK ? b1 : p1 / NOISE_CHUNK;
+        float* const out = np.out + R.noff + (long)fam * 3 * nf;
+        const double ae = fam < 3 ? ef : ev, az = fam < 3 ? zf : zv;
+        const unsigned realization = R.realization;
+        for (; b < e; b++) {
+            const long id = b * NOISE_CHUNK - p0 + threadIdx.x;
+            if (id < count) noise::draw(np.seed, realization, st, fam, id, count, ae, az, out);
+        }
+        s++;
+    }
 }
 
 }  // namespace ens

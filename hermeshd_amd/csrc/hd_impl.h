@@ -80,13 +80,12 @@ struct Impl {
         if constexpr (NQ >= 11) {
             if (e->base.noise) {
                 hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, true>), dim3(e->grid), dim3(256), 0, s, qin, qn,
-                                   qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr,
-                                   e->noise_floats);
+                                   qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
                 return;
             }
         }
         hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, false>), dim3(e->grid), dim3(256), 0, s, qin, qn, qout,
-                           e->dreal, e->dwork, e->launch, e->ph, sp, e->noise, e->step_ctr, e->noise_floats);
+                           e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
     }
     // defined in hd_impl_vjp.h; the units that include it instantiate it
     // there, and hd_k4_vjp.hip holds the nbasis 4 instances, so that those

@@ -17,7 +17,8 @@
 // face families (stream 1..3, id = p*NFB + fid, fid = i + (nx+1)(j + (ny+1)k)
 // over the (nx+1)(ny+1)(nz+1) face lattice) and every volume point (stream 4,
 // id = p*N + cell).  Each point is drawn once and read by every stage of the
-// step and by both cells of a face.  Layout: component-major,
+// step and by both cells of a face.  A face keeps the three components that
+// its flux takes, a volume point all six.  Layout: component-major,
 // out[e*count + id], so that neighbouring cells read neighbouring words.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -31,8 +32,9 @@ __device__ __forceinline__ void philox4x32_10(uint32_t& c0, uint32_t& c1, uint32
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
 #pragma unroll
     for (int r = 0; r < 10; r++) {
-        const uint32_t hi0 = __umulhi(M0, c0), lo0 = M0 * c0;
-        const uint32_t hi1 = __umulhi(M1, c2), lo1 = M1 * c2;
+        // both halves of each product from one 64-bit multiply-add
+        const uint64_t p0 = (uint64_t)M0 * c0, p1 = (uint64_t)M1 * c2;
+        const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0, hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
         const uint32_t n0 = hi1 ^ c1 ^ k0, n2 = hi0 ^ c3 ^ k1;
         c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
         k0 += W0; k1 += W1;
@@ -113,22 +115,66 @@ __device__ __forceinline__ void normals4(uint64_t seed, uint32_t realization, ui
     }
 }
 
-// stress (xx, yy, zz, xy, xz, yz) at point id of a stream
-__device__ __forceinline__ void stress(uint64_t seed, uint32_t realization, uint64_t step, uint32_t stream, uint64_t id,
-                                       double ae, double az, double S[6]) {
-    double g[8];
-    normals4(seed, realization, step, stream, 2 * id, g);
-    normals4(seed, realization, step, stream, 2 * id + 1, g + 4);
+// x / 3, correctly rounded: the quotient by the rounded reciprocal, corrected
+// once with its exact remainder (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990)
+__device__ __forceinline__ double third(double x) {
+    const double y = 1. / 3., q = x * y;
+    return fma(fma(-3., q, x), y, q);
+}
+
+// stress at point id of a stream: row d (0, 1, 2: the components that the flux
+// along d takes, xx xy xz / xy yy yz / xz yz zz) for faces, or all of xx, yy,
+// zz, xy, xz, yz for volume points
+__device__ __forceinline__ void stress_diag(const double* g, double ae, double az, double (&S)[3]) {
     const double s2 = 1.4142135623730951;
     const double dxx = s2 * g[0], dyy = s2 * g[1], dzz = s2 * g[2];
-    const double tr = (dxx + dyy + dzz) / 3.0;
+    const double tr = third(dxx + dyy + dzz);
     const double trW = g[0] + g[1] + g[2];
     S[0] = ae * (dxx - tr) + az * trW;
     S[1] = ae * (dyy - tr) + az * trW;
     S[2] = ae * (dzz - tr) + az * trW;
+}
+__device__ __forceinline__ void stress_row(uint64_t seed, uint32_t realization, uint64_t step, int d, uint64_t id,
+                                           double ae, double az, double (&S)[3]) {
+    double g[8], D[3];
+    normals4(seed, realization, step, (uint32_t)(d + 1), 2 * id, g);
+    normals4(seed, realization, step, (uint32_t)(d + 1), 2 * id + 1, g + 4);
+    stress_diag(g, ae, az, D);
+    const double xy = ae * g[3], xz = ae * g[4], yz = ae * g[5];
+    S[0] = d == 0 ? D[0] : (d == 1 ? xy : xz);
+    S[1] = d == 0 ? xy : (d == 1 ? D[1] : yz);
+    S[2] = d == 0 ? xz : (d == 1 ? yz : D[2]);
+}
+__device__ __forceinline__ void stress(uint64_t seed, uint32_t realization, uint64_t step, uint64_t id, double ae,
+                                       double az, double (&S)[6]) {
+    double g[8], D[3];
+    normals4(seed, realization, step, 4u, 2 * id, g);
+    normals4(seed, realization, step, 4u, 2 * id + 1, g + 4);
+    stress_diag(g, ae, az, D);
+    S[0] = D[0]; S[1] = D[1]; S[2] = D[2];
     S[3] = ae * g[3];
     S[4] = ae * g[4];
     S[5] = ae * g[5];
+}
+// Draws point id of family fam (0-2: faces of `count` points, 3: volume) into
+// out, component-major, in single precision, the reference's precision for its
+// Gaussian draws (vsRngGaussian, src/random.f90:61,87).  Bound by its vector
+// instructions (two Philox calls, three Box-Muller pairs); storing a face's
+// row instead of all six components halves what it writes there.
+__device__ __forceinline__ void draw(uint64_t seed, uint32_t realization, uint64_t step, int fam, long id, long count,
+                                     double ae, double az, float* __restrict__ out) {
+    if (fam < 3) {
+        double S[3];
+        stress_row(seed, realization, step, fam, (uint64_t)id, ae, az, S);
+#pragma unroll
+        for (int e = 0; e < 3; e++) out[(long)e * count + id] = (float)S[e];
+    } else {
+        double S[6];
+        stress(seed, realization, step, (uint64_t)id, ae, az, S);
+#pragma unroll
+        for (int e = 0; e < 6; e++) out[(long)e * count + id] = (float)S[e];
+    }
 }
 
 struct NoiseParams {
@@ -139,7 +185,7 @@ struct NoiseParams {
     const double* dt;                // device time step
     double eta_sd, zeta_sd, dVi, kap_f, kap_v;
     long nfb, N;                     // face lattice size, cells
-    float* face[3];                  // [6][nface][nfb] per face family
+    float* face[3];                  // [3][nface][nfb] per face family: the stress row of its direction
     float* vol;                      // [6][npg][N]
 };
 
@@ -149,30 +195,11 @@ static __global__ __launch_bounds__(256) void k_noise(NoiseParams np) {
     if (t >= 3 * nf + nv) return;
     const double sq = sqrt(np.dVi / *np.dt);
     const uint64_t step = *np.step;
-    long id, count;
-    uint32_t stream;
-    float* out;
-    double kap;
-    if (t < 3 * nf) {
-        const int d = (t >= nf) + (t >= 2 * nf);
-        id = t - (long)d * nf;
-        count = nf;
-        stream = (uint32_t)(d + 1);
-        out = np.face[d];
-        kap = np.kap_f;
-    } else {
-        id = t - 3 * nf;
-        count = nv;
-        stream = 4u;
-        out = np.vol;
-        kap = np.kap_v;
-    }
-    double S[6];
-    stress(np.seed, np.realization, step, stream, (uint64_t)id, np.eta_sd * sq * kap, np.zeta_sd * sq * kap, S);
-    // stored in single precision, the reference's precision for its
-    // Gaussian draws (vsRngGaussian, src/random.f90:61,87)
-#pragma unroll
-    for (int e = 0; e < 6; e++) out[(long)e * count + id] = (float)S[e];
+    const int fam = (t >= nf) + (t >= 2 * nf) + (t >= 3 * nf);
+    const double kap = fam < 3 ? np.kap_f : np.kap_v;
+    float* out = fam == 0 ? np.face[0] : (fam == 1 ? np.face[1] : (fam == 2 ? np.face[2] : np.vol));
+    draw(np.seed, np.realization, step, fam, t - (long)fam * nf, fam < 3 ? nf : nv, np.eta_sd * sq * kap,
+         np.zeta_sd * sq * kap, out);
 }
 
 static __global__ void k_set_step(unsigned long long* step, unsigned long long value, int advance) {

@@ -243,7 +243,7 @@ __device__ __forceinline__ void face_moments(const double* __restrict__ q, const
     float Sn[3];
     if constexpr (NZ) {
 #pragma unroll
-        for (int a = 0; a < 3; a++) Sn[a] = sp.noise[DIR][((long)noise_comp(DIR, a) * NF) * sp.nfb + fid];
+        for (int a = 0; a < 3; a++) Sn[a] = sp.noise[DIR][((long)a * NF) * sp.nfb + fid];
     }
     int ii = 0, jj = 0;
 #pragma unroll 1
@@ -278,7 +278,7 @@ __device__ __forceinline__ void face_moments(const double* __restrict__ q, const
 #pragma unroll
             for (int a = 0; a < 3; a++) {
                 S[a] = Sn[a];
-                Sn[a] = sp.noise[DIR][((long)noise_comp(DIR, a) * NF + pn) * sp.nfb + fid];
+                Sn[a] = sp.noise[DIR][((long)a * NF + pn) * sp.nfb + fid];
             }
         }
         pr::face_flux<NQ, DIR, RM, NZ>(ph, QL, QR, S, F);

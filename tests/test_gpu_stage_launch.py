@@ -70,3 +70,24 @@ def test_launch_forms_match_oracle(torch_mod, oracle_mod, name, bc):
             s.step(q, torch_mod.zeros_like(q))
             s.check()
             assert field_rel_err(q.cpu().numpy(), ref) < TOL, (n, planes)
+
+
+@pytest.mark.parametrize("dims", [[(1, 1, 1), (3, 1, 2)], [(23, 30, 29), (2, 3, 1), (31, 24, 27)]],
+                         ids=["few_chunks", "runs_of_chunks"])
+def test_ensemble_draw_equals_single(dims):
+    """The ensemble's draw, fewer chunks than blocks and blocks that cross
+    from one family or realization to the next: bitwise each context's own."""
+    import torch
+    from hermeshd_amd.ensemble import Ensemble
+    from hermeshd_amd.solver import Solver
+    nx, ny, nz = dims[0]
+    base = HDConfig(nx=nx, ny=ny, nz=nz, lx=1. * nx, ly=1. * ny, lz=1. * nz, nbasis=4, iquad=2, nQ=11, ivis=0,
+                    coll=3.0, colvis=0.5, riemann="hllc", integrator="heun", noise=True, eta_sd=0.02, seed=5,
+                    realization=3, T_floor=1e-4)
+    cfgs = [base.replace(nx=d[0], ny=d[1], nz=d[2], lx=1. * d[0], ly=1. * d[1], lz=1. * d[2],
+                         realization=base.realization + r) for r, d in enumerate(dims)]
+    ens = Ensemble(base, dims)
+    qs = [smooth_state(c, seed=9 + r) for r, c in enumerate(cfgs)]
+    out = ens.views(ens.rhs(ens.pack(qs)))
+    for r, c in enumerate(cfgs):
+        assert torch.equal(Solver(c).rhs(torch.from_numpy(qs[r]).cuda()), out[r]), f"realization {r}"
