@@ -25,7 +25,7 @@
 // are those of the forward evaluation at the same state.  The stochastic
 // stress and the Roe solver have no adjoint here.
 #pragma once
-#include "hd_fused.h"
+#include "hd_stage.h"
 
 namespace hd {
 namespace adj {
@@ -287,17 +287,18 @@ __device__ __forceinline__ bool hllc_vjp(const Phys& ph, const double* QL, const
     return true;
 }
 
-// face flux reverse: mu (cotangent of the face flux, all fields) -> bQL, bQR (+=)
-template <int NQ, int RM, int DIR>
-__device__ __forceinline__ void face_vjp(const Phys& ph, const double* QL, const double* QR, const double* mu,
-                                         double* bQL, double* bQR) {
-    const pr::Prim sL = pr::prim<NQ>(ph, QL), sR = pr::prim<NQ>(ph, QR);
-    double bFL[NQ], bFR[NQ];
+// The Euler fields of the face flux reversed to the cotangents of both sides'
+// physical fluxes (bFL, bFR, set) and of their states through the solver
+// (bQL, bQR, +=).  L, R: the sides' velocities and densities.
+template <int RM, int DIR>
+__device__ __forceinline__ void riemann_vjp(const Phys& ph, const double* QL, const pr::Prim& L, const double* QR,
+                                            const pr::Prim& R, const double* mu, double* bQL, double* bQR,
+                                            double* bFL, double* bFR) {
 #pragma unroll
-    for (int f = 0; f < NQ; f++) { bFL[f] = 0.5 * mu[f]; bFR[f] = 0.5 * mu[f]; }
+    for (int f = 0; f < 5; f++) { bFL[f] = 0.5 * mu[f]; bFR[f] = 0.5 * mu[f]; }
     if constexpr (RM == RIEMANN_HLLC) {
         double zL[5] = {0., 0., 0., 0., 0.}, zR[5] = {0., 0., 0., 0., 0.};
-        if (hllc_vjp<DIR>(ph, QL, sL, QR, sR, mu, bQL, bQR, zL, zR)) {
+        if (hllc_vjp<DIR>(ph, QL, L, QR, R, mu, bQL, bQR, zL, zR)) {
             // HLLC replaced the central flux of rh..en
 #pragma unroll
             for (int f = 0; f < 5; f++) { bFL[f] = zL[f]; bFR[f] = zR[f]; }
@@ -310,6 +311,17 @@ __device__ __forceinline__ void face_vjp(const Phys& ph, const double* QL, const
         for (int f = 0; f < 5; f++) { bFL[f] = 0.; bFR[f] = 0.; }
         roe_point_vjp<DIR>(ph, QL, QR, mu, bQL, bQR, bFL, bFR);
     }
+}
+
+// face flux reverse: mu (cotangent of the face flux, all fields) -> bQL, bQR (+=)
+template <int NQ, int RM, int DIR>
+__device__ __forceinline__ void face_vjp(const Phys& ph, const double* QL, const double* QR, const double* mu,
+                                         double* bQL, double* bQR) {
+    const pr::Prim sL = pr::prim<NQ>(ph, QL), sR = pr::prim<NQ>(ph, QR);
+    double bFL[NQ], bFR[NQ];
+#pragma unroll
+    for (int f = 5; f < NQ; f++) { bFL[f] = 0.5 * mu[f]; bFR[f] = 0.5 * mu[f]; }
+    riemann_vjp<RM, DIR>(ph, QL, sL, QR, sR, mu, bQL, bQR, bFL, bFR);
     flux_vjp<NQ, DIR>(ph, QL, sL, bFL, bQL);
     flux_vjp<NQ, DIR>(ph, QR, sR, bFR, bQR);
 }
@@ -864,246 +876,344 @@ __global__ __launch_bounds__(256) void k_stage_vjp_split(const double* __restric
 
 // ------------------------------------------------- 13-moment transpose ----
 // The transpose of a 13-moment stage on a grid periodic in every direction,
-// split into a face and a cell kernel, so that no lane
-// holds a whole cell: the face kernel writes, per face point, the cotangents
-// that the face flux sends to the traces of its two cells; the cell kernel,
-// one field per wave, adds the volume transpose and gathers those face
-// cotangents.  The sum over the terms is the fused k_stage_vjp's, evaluated
-// in another order.
+// split into a face and a cell kernel, so that no lane holds a whole cell.
+// Both take a workgroup's quadrature points side by side, one point of one
+// face or cell a lane: the modes wait in LDS, where each lane reads what its
+// point needs, and the points' cotangents go back through LDS to be summed.
+// The face kernel writes, for each side of a face, the moments
+// M_k = sum_p b_k(p) v(p) of the cotangents v of that side's trace (NK values
+// a field instead of QP^2); the cell kernel adds the volume transpose and
+// gathers its six faces.  The sum over the terms is k_stage_vjp's, evaluated
+// in another order.  A periodic grid has as many faces a direction as cells:
+// face c is the low face of cell c.
+// nbasis 10, Roe, 40^3 cells, a stage: 252 us the faces (three directions in
+// one launch, 51 KB of LDS: three workgroups a CU) and 214 us the cells,
+// against 840 and 429 us for a wave per face point over 64 faces (156 KB of
+// LDS, one workgroup a CU, waiting for its loads two thirds of the time, and
+// a last round of one workgroup) and a field per wave (three of thirteen
+// waves at the points).  Bound by the arithmetic of the points at three or
+// four waves a SIMD, then by L2: 0.6 GB a stage.
 
-// One wave per face point over 64 consecutive faces of direction DIR (as
-// one wave per face point): phase 1 stages both sides' trace coefficients (face_coeffs
-// of the limited modes q) and lifted-cotangent coefficients (lift_coeffs of
-// b*lam through the relaxation factors) in LDS; phase 2 forms the face
-// flux's cotangent mu at point p, reverses the Riemann solver and the
-// physical fluxes (face_vjp), and writes the left cell's trace cotangent to
-// bql and the right cell's to bqr, laid out as the forward face fluxes.
+// Faces of a workgroup of 256: as many as give every lane a face point.
+template <int QP>
+constexpr int face13_faces() { return 256 / (QP * QP); }
+template <int NB, int QP>
+constexpr int face13_doubles() {
+    const int modes = 3 * 13 * fz::face_nk<NB>() * face13_faces<QP>(), points = 2 * 13 * QP * QP * face13_faces<QP>();
+    return modes > points ? modes : points;
+}
+
+// The faces f0.. of direction DIR: each field's trace coefficients of both
+// sides and the sum of their lifted-cotangent coefficients (of b*lam through
+// the relaxation factors) to LDS; then at each point the cotangent mu of the
+// flux, reversed through the Riemann solver and the physical fluxes; then the
+// moments of both sides' trace cotangents.
 template <int NB, int QP, int RM, int DIR>
-__global__ __launch_bounds__(QP * QP * 64) void k_face13_vjp(const double* __restrict__ q,
-                                                            const double* __restrict__ lam, double* __restrict__ bql,
-                                                            double* __restrict__ bqr, Grid g, Phys ph, AdjParams ap) {
-    constexpr int NQ = 13, NF = QP * QP, NK = fz::face_nk<NB>();
-    __shared__ double ks[2][NQ][NK][64];
-    __shared__ double ls[2][NQ][NK][64];
+__device__ __forceinline__ void face13_vjp(double* __restrict__ lds, const double* __restrict__ q,
+                                           const double* __restrict__ lam, double* __restrict__ ml,
+                                           double* __restrict__ mr, long f0, const Grid& g, const Phys& ph,
+                                           const AdjParams& ap) {
+    constexpr int NQ = 13, NF = QP * QP, NK = fz::face_nk<NB>(), F = face13_faces<QP>();
     const double dt = *ap.dt;
     const double faci = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll) : 1.0;
     const double faciq = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll_q) : 1.0;
-    const int ni = g.nx + (DIR == 0), nj = g.ny + (DIR == 1);
-    const long nfaces = (long)ni * nj * (g.nz + (DIR == 2));
-    const long f0 = (long)xcd_block() * 64;
-    for (int it = (int)threadIdx.x; it < 2 * NQ * 64; it += NF * 64) {
-        const int l = it & 63, side = (it >> 6) / NQ, fld = (it >> 6) % NQ;
-        const long fid = f0 + l < nfaces ? f0 + l : nfaces - 1;
-        int ci = (int)(fid % ni), cj = (int)((fid / ni) % nj), ck = (int)(fid / ((long)ni * nj));
-        int& a = DIR == 0 ? ci : DIR == 1 ? cj : ck;
+    const auto& FP = fz::face_poly<NB>();
+    const int t = (int)threadIdx.x;
+    for (int it = t; it < NQ * F; it += 256) {
+        const int l = it % F, fld = it / F;
+        const long cr = f0 + l < g.N ? f0 + l : g.N - 1;
+        const long sd = DIR == 0 ? 1 : DIR == 1 ? g.nx : (long)g.nx * g.ny;
         const int n_ax = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
-        if (side == 0) a = a == 0 ? n_ax - 1 : a - 1;
-        else if (a == n_ax) a = 0;
-        const long cell = (long)ci + (long)g.nx * ((long)cj + (long)g.ny * ck);
-        const double fac = fld >= T_QX ? faciq : (fld >= PXX ? faci : 1.0);
-        double m1[1][NB], l1[1][NB], K1[1][NK], L1[1][NK];
+        const int a = (int)(DIR == 0 ? cr % g.nx : DIR == 1 ? (cr / g.nx) % g.ny : cr / ((long)g.nx * g.ny));
+        const long cl = a == 0 ? cr + (n_ax - 1) * sd : cr - sd;
+        const double fac = ap.b * (fld >= T_QX ? faciq : (fld >= PXX ? faci : 1.0));
+        double m0[1][NB], m1[1][NB], l0[1][NB], l1[1][NB], K0[1][NK], K1[1][NK], L0[1][NK], L1[1][NK];
 #pragma unroll
         for (int r = 0; r < NB; r++) {
-            const long o = ((long)r * NQ + fld) * g.N + cell;
-            m1[0][r] = q[o];
-            l1[0][r] = ap.b * lam[o] * fac;
+            const long o = ((long)r * NQ + fld) * g.N;
+            m0[0][r] = q[o + cl];
+            m1[0][r] = q[o + cr];
+            l0[0][r] = lam[o + cl];
+            l1[0][r] = lam[o + cr];
         }
-        if (side == 0) {
-            fz::face_coeffs<NB, 1, DIR, 1, NK>(m1, K1);
-            lift_coeffs<NB, 1, DIR, 1, NK>(l1, L1);
-        } else {
-            fz::face_coeffs<NB, 1, DIR, 0, NK>(m1, K1);
-            lift_coeffs<NB, 1, DIR, 0, NK>(l1, L1);
-        }
+        fz::face_coeffs<NB, 1, DIR, 1, NK>(m0, K0);
+        fz::face_coeffs<NB, 1, DIR, 0, NK>(m1, K1);
+        lift_coeffs<NB, 1, DIR, 1, NK>(l0, L0);
+        lift_coeffs<NB, 1, DIR, 0, NK>(l1, L1);
+        double* const k = lds + it * NK;
 #pragma unroll
-        for (int k = 0; k < NK; k++) {
-            ks[side][fld][k][l] = K1[0][k];
-            ls[side][fld][k][l] = L1[0][k];
+        for (int e = 0; e < NK; e++) {
+            k[e] = K0[0][e];
+            k[NQ * F * NK + e] = K1[0][e];
+            k[2 * NQ * F * NK + e] = fac * (L0[0][e] + L1[0][e]);
         }
     }
     __syncthreads();
-    const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int l = (int)(threadIdx.x & 63);
-    const long fid = f0 + l;
-    if (fid >= nfaces) return;
-    const auto& FP = fz::face_poly<NB>();
-    const double dxi_d = DIR == 0 ? g.dxi : DIR == 1 ? g.dyi : g.dzi;
-    double QL[NQ], QR[NQ], mu[NQ];
-#pragma unroll
-    for (int f = 0; f < NQ; f++) {
-        double sl = ks[0][f][0][l], sr = ks[1][f][0][l];
-        double tl = ls[0][f][0][l] * FP.wb[p][0], tr = ls[1][f][0][l] * FP.wb[p][0];
-#pragma unroll
-        for (int k = 1; k < NK; k++) {
-            sl += ks[0][f][k][l] * FP.b[p][k];
-            sr += ks[1][f][k][l] * FP.b[p][k];
-            tl += ls[0][f][k][l] * FP.wb[p][k];
-            tr += ls[1][f][k][l] * FP.wb[p][k];
-        }
-        QL[f] = sl;
-        QR[f] = sr;
-        mu[f] = dxi_d * (tl + tr);
-    }
+    const bool point = t < NF * F;
     double bL[NQ], bR[NQ];
+    if (point) {
+        const int p = t / F, l = t % F;
+        const double dxi_d = DIR == 0 ? g.dxi : DIR == 1 ? g.dyi : g.dzi;
+        double b[NK], wb[NK];
 #pragma unroll
-    for (int f = 0; f < NQ; f++) { bL[f] = 0.; bR[f] = 0.; }
-    face_vjp<NQ, RM, DIR>(ph, QL, QR, mu, bL, bR);
+        for (int e = 0; e < NK; e++) {
+            b[e] = FP.b[p][e];
+            wb[e] = dxi_d * FP.wb[p][e];
+        }
+        // field f of a side's state, or (side 2, with wb) of the flux's cotangent
+        auto value = [&](int side, int f, const double (&w)[NK]) {
+            const double* const k = lds + ((side * NQ + f) * F + l) * NK;
+            double s = k[0] * w[0];
 #pragma unroll
-    for (int f = 0; f < NQ; f++) {
-        const long o = ((long)f * NF + p) * nfaces + fid;
-        bql[o] = bL[f];
-        bqr[o] = bR[f];
+            for (int e = 1; e < NK; e++) s += k[e] * w[e];
+            return s;
+        };
+        // face_vjp in three parts (the Riemann solver's Euler fields, the
+        // left flux, the right flux), so that no part holds all that the
+        // point has: 13 fields of two states and of their cotangents at once
+        // spilled 480 registers
+        double QL[NQ], QR[NQ], mu[NQ], bFL[NQ], bFR[NQ];
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+            bL[f] = 0.;
+            bR[f] = 0.;
+        }
+#pragma unroll
+        for (int f = 0; f < 5; f++) {
+            QL[f] = value(0, f, b);
+            QR[f] = value(1, f, b);
+            mu[f] = value(2, f, wb);
+        }
+        riemann_vjp<RM, DIR>(ph, QL, pr::prim<5>(ph, QL), QR, pr::prim<5>(ph, QR), mu, bL, bR, bFL, bFR);
+        sg::section();
+#pragma unroll
+        for (int f = 5; f < NQ; f++) {
+            QL[f] = value(0, f, b);
+            bFL[f] = 0.5 * value(2, f, wb);
+        }
+        flux_vjp<NQ, DIR>(ph, QL, pr::prim<NQ>(ph, QL), bFL, bL);
+        sg::section();
+#pragma unroll
+        for (int f = 5; f < NQ; f++) {
+            QR[f] = value(1, f, b);
+            bFR[f] = 0.5 * value(2, f, wb);
+        }
+        flux_vjp<NQ, DIR>(ph, QR, pr::prim<NQ>(ph, QR), bFR, bR);
+    }
+    __syncthreads();  // the points' cotangents overwrite the coefficients
+    if (point) {
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+            lds[f * NF * F + t] = bL[f];
+            lds[(NQ + f) * NF * F + t] = bR[f];
+        }
+    }
+    __syncthreads();
+    for (int it = t; it < 2 * NQ * F; it += 256) {
+        const int l = it % F, row = it / F;  // row: side, field
+        double M[NK];
+#pragma unroll
+        for (int p = 0; p < NF; p++) {
+            const double v = lds[(row * NF + p) * F + l];
+#pragma unroll
+            for (int e = 0; e < NK; e++) M[e] = p == 0 ? v * FP.b[p][e] : M[e] + v * FP.b[p][e];
+        }
+        if (f0 + l < g.N) {
+            double* const out = row < NQ ? ml + (long)row * NK * g.N : mr + (long)(row - NQ) * NK * g.N;
+#pragma unroll
+            for (int e = 0; e < NK; e++) out[e * g.N + f0 + l] = M[e];
+        }
     }
 }
 
-// per-block partial of d(lam.out)/dcoll for workgroups of 13 waves
+// All three directions in one launch, a tile's directions next to each other
+// and each XCD a contiguous eighth of the tiles (L2 serves the cells that
+// several faces share).
+template <int NB, int QP, int RM>
+__global__ __launch_bounds__(256, (NB == 10 ? 3 : 2)) void k_face13_vjp(
+    const double* __restrict__ q, const double* __restrict__ lam, double* __restrict__ ml0,
+    double* __restrict__ ml1, double* __restrict__ ml2, double* __restrict__ mr0, double* __restrict__ mr1,
+    double* __restrict__ mr2, Grid g, Phys ph, AdjParams ap) {
+    __shared__ __attribute__((aligned(16))) double lds[face13_doubles<NB, QP>()];
+    const unsigned b = xcd_block();  // the grid is a multiple of 8
+    const unsigned tile = b / 3, d = b % 3;
+    const long f0 = (long)tile * face13_faces<QP>();
+    if (f0 >= g.N) return;
+    if (d == 0) face13_vjp<NB, QP, RM, 0>(lds, q, lam, ml0, mr0, f0, g, ph, ap);
+    else if (d == 1) face13_vjp<NB, QP, RM, 1>(lds, q, lam, ml1, mr1, f0, g, ph, ap);
+    else face13_vjp<NB, QP, RM, 2>(lds, q, lam, ml2, mr2, f0, g, ph, ap);
+}
+
+// Cells of a workgroup of k_cell13_vjp, and its lanes: a volume point each,
+// and one more wave for the limiter's factors.
+template <int QP>
+constexpr int cell13_cells() { return QP == 3 ? 16 : 32; }
+template <int QP>
+constexpr int cell13_threads() { return (QP * QP * QP * cell13_cells<QP>() + 63) / 64 * 64 + 64; }
+
+// per-block partial of d(lam.out)/dcoll for workgroups of W waves
+template <int W>
 __device__ __forceinline__ void block_partial13(double v, double* partial) {
-    __shared__ double red[CELL13_WAVES];
+    __shared__ double red[W];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0.;
-        for (int w = 0; w < CELL13_WAVES; w++) s += red[w];
+        for (int w = 0; w < W; w++) s += red[w];
         partial[blockIdx.x] = s;
     }
 }
 
-// One field per wave over 64 consecutive cells (as k_cell13).  The faces
-// come first (their loads beside the modes'): bfc^T of the cotangents written
-// by k_face13_vjp.  The volume transpose then takes one row of the rule (QP
-// points) per exchange: each wave writes its field's point value and the
-// cotangents of its three point fluxes (the transposes of k_cell's volume
-// sums); one wave per point reverses the point's physical fluxes (flux_vjp)
-// and shares the state cotangent, which each wave projects onto its field's
-// modes.  Then the sources, the stage map (lo + dt*rt, the accumulated terms)
-// and the frozen limiter, as cell_vjp_finish; d/dcoll as cell_vjp_parts.
+// The cells' modes and cotangents to LDS; then a volume point a lane: its
+// state, the cotangents of its three fluxes (the transposes of the volume
+// sums), the fluxes reversed (flux_vjp) and the state cotangent to LDS; then
+// a field of a cell a lane: the points' sum, the face moments (the cell is
+// the right side of its low faces and the left side of its high faces), the
+// sources, the stage map (lo + dt*rt, the accumulated terms) and the frozen
+// limiter, as cell_vjp_finish; d/dcoll as cell_vjp_parts.
 template <int NB, int QP, int RM>
-__global__ __launch_bounds__(CELL13_WAVES * 64) void k_cell13_vjp(
+__global__ __launch_bounds__(cell13_threads<QP>(), 4) void k_cell13_vjp(
     const double* __restrict__ q, const double* __restrict__ lam, double* __restrict__ lam_in,
-    const double* __restrict__ bql0, const double* __restrict__ bql1, const double* __restrict__ bql2,
-    const double* __restrict__ bqr0, const double* __restrict__ bqr1, const double* __restrict__ bqr2,
+    const double* __restrict__ ml0, const double* __restrict__ ml1, const double* __restrict__ ml2,
+    const double* __restrict__ mr0, const double* __restrict__ mr1, const double* __restrict__ mr2,
     const Tables* __restrict__ T, Grid g, Phys ph, AdjParams ap) {
-    constexpr int NQ = 13, NF = QP * QP, NPG = QP * QP * QP, NCH = QP;
-    __shared__ double qp_s[NQ][NCH][64];
-    __shared__ double bf_s[NQ][3][NCH][64];
-    __shared__ double bq_s[NQ][NCH][64];
-    const int f = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
-    const long c = (long)xcd_block() * 64 + lane;
-    const bool live = c < g.N;
-    const long cc = live ? c : g.N - 1;  // lanes past the grid compute a copy of the last cell and store nothing
-    const int i = (int)(cc % g.nx), j = (int)((cc / g.nx) % g.ny), k = (int)(cc / ((long)g.nx * g.ny));
+    constexpr int NQ = 13, NPG = QP * QP * QP, NK = fz::face_nk<NB>(), C = cell13_cells<QP>();
+    constexpr int NT = cell13_threads<QP>();
+    __shared__ __attribute__((aligned(16))) double m_s[NQ][C][NB], lo_s[NQ][C][NB];
+    __shared__ double bq_s[NQ][NPG * C];
+    __shared__ double th_s[2][C];
+    __shared__ int lim_s[C];
+    const int t = (int)threadIdx.x;
+    const long c0 = (long)xcd_block() * C;
     const double dt = *ap.dt;
     const double faci = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll) : 1.0;
     const double faciq = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll_q) : 1.0;
-    const double fac = f >= T_QX ? faciq : (f >= PXX ? faci : 1.0);
-    const double dxi = g.dxi, dyi = g.dyi, dzi = g.dzi;
-    double mf[NB], lof[NB], rt[NB];
 #pragma unroll
-    for (int r = 0; r < NB; r++) {
-        const long o = qoff(g, cc, f, r);
-        mf[r] = q[o];
-        lof[r] = ap.b * lam[o] * fac;
-        rt[r] = 0.;
+    for (int n = 0; n < (NQ * NB * C + NT - 1) / NT; n++) {
+        const int it = t + n * NT;
+        if (it < NQ * NB * C) {
+            const int c = it % C, row = it / C, r = row / NQ, f = row % NQ;
+            // lanes past the grid take a copy of the last cell and store nothing
+            const long o = (long)row * g.N + (c0 + c < g.N ? c0 + c : g.N - 1);
+            m_s[f][c][r] = q[o];
+            lo_s[f][c][r] = ap.b * lam[o] * (f >= T_QX ? faciq : (f >= PXX ? faci : 1.0));
+        }
     }
-    // ---- faces first, their loads beside those of the modes: the cell is
-    // the right side of its low faces and the left side of its high faces ----
-    {
-        const long nfl[3] = {(long)(g.nx + 1) * g.ny * g.nz, (long)g.nx * (g.ny + 1) * g.nz,
-                             (long)g.nx * g.ny * (g.nz + 1)};
-        const long fm[3] = {(long)i + (long)(g.nx + 1) * ((long)j + (long)g.ny * k),
-                            (long)i + (long)g.nx * ((long)j + (long)(g.ny + 1) * k),
-                            (long)i + (long)g.nx * ((long)j + (long)g.ny * k)};
-        const long fp[3] = {fm[0] + 1, fm[1] + g.nx, fm[2] + (long)g.nx * g.ny};
-        const double* const bqr[3] = {bqr0, bqr1, bqr2};
-        const double* const bql[3] = {bql0, bql1, bql2};
+    __syncthreads();
+    if (t < NPG * C) {
+        const int p = t / C, c = t % C;
+        double b[NB], Qp[NQ], bF[NQ], bQ[NQ];
+#pragma unroll
+        for (int r = 0; r < NB; r++) b[r] = T->bint[p][r];
+        const double w = 0.25 * T->w3[p];
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+            double v = m_s[f][c][0];
+#pragma unroll
+            for (int r = 1; r < NB; r++) v += b[r] * m_s[f][c][r];
+            Qp[f] = v;
+            bQ[f] = 0.;
+        }
+        const pr::Prim st = pr::prim<NQ>(ph, Qp);
+        // cotangent of a field's flux: sum_r cb_r d(phi_r) lo_r
+        {
+            const double h = g.dxi * w;
+#pragma unroll
+            for (int f = 0; f < NQ; f++) {
+                const double* const l = lo_s[f][c];
+                double s = 3. * l[KX];
+                if constexpr (NB == 10) s += 9. * b[KZ] * l[KZX] + 9. * b[KY] * l[KXY] + 15. * b[KX] * l[KXX];
+                bF[f] = h * s;
+            }
+            flux_vjp<NQ, 0>(ph, Qp, st, bF, bQ);
+        }
+        {
+            const double h = g.dyi * w;
+#pragma unroll
+            for (int f = 0; f < NQ; f++) {
+                const double* const l = lo_s[f][c];
+                double s = 3. * l[KY];
+                if constexpr (NB == 10) s += 9. * b[KZ] * l[KYZ] + 9. * b[KX] * l[KXY] + 15. * b[KY] * l[KYY];
+                bF[f] = h * s;
+            }
+            flux_vjp<NQ, 1>(ph, Qp, st, bF, bQ);
+        }
+        {
+            const double h = g.dzi * w;
+#pragma unroll
+            for (int f = 0; f < NQ; f++) {
+                const double* const l = lo_s[f][c];
+                double s = 3. * l[KZ];
+                if constexpr (NB == 10) s += 9. * b[KY] * l[KYZ] + 9. * b[KX] * l[KZX] + 15. * b[KZ] * l[KZZ];
+                bF[f] = h * s;
+            }
+            flux_vjp<NQ, 2>(ph, Qp, st, bF, bQ);
+        }
+#pragma unroll
+        for (int f = 0; f < NQ; f++) bq_s[f][t] = bQ[f];
+    } else if (ap.q_raw && t >= NT - 64 && t < NT - 64 + C) {
+        const int c = t - (NT - 64);
+        const long cc = c0 + c < g.N ? c0 + c : g.N - 1;
+        double raw[5][NB];
+#pragma unroll
+        for (int e = 0; e < 5; e++)
+#pragma unroll
+            for (int r = 0; r < NB; r++) raw[e][r] = ap.q_raw[qoff(g, cc, e, r)];
+        const LimFactors L = limit_factors<NB, QP, 5>(raw, ap.lp);
+        th_s[0][c] = L.th_rho;
+        th_s[1][c] = L.th_p;
+        lim_s[c] = (L.zero ? 1 : 0) + (L.floor ? 2 : 0);
+    }
+    __syncthreads();
+    double dcoll = 0.;
+    for (int it = t; it < NQ * C; it += NT) {
+        const int f = it / C, lc = it % C;
+        const long c = c0 + lc;
+        if (c >= g.N) continue;
+        double rt[NB];
+#pragma unroll
+        for (int r = 0; r < NB; r++) rt[r] = 0.;
+#pragma unroll
+        for (int p = 0; p < NPG; p++) {
+            const double v = bq_s[f][p * C + lc];
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const double b = fz::phi_int<NB, QP>(r, p / (QP * QP), (p / QP) % QP, p % QP);
+                if (b != 0.) rt[r] += b * v;
+            }
+        }
+        const int i = (int)(c % g.nx), j = (int)((c / g.nx) % g.ny), k = (int)(c / ((long)g.nx * g.ny));
+        const long nxy = (long)g.nx * g.ny;
+        const long ch[3] = {i == g.nx - 1 ? c - i : c + 1, j == g.ny - 1 ? c - (long)j * g.nx : c + g.nx,
+                            k == g.nz - 1 ? c - k * nxy : c + nxy};
+        const double* const ml[3] = {ml0, ml1, ml2};
+        const double* const mr[3] = {mr0, mr1, mr2};
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-#pragma unroll 1
-            for (int p = 0; p < NF; p++) {
-                const long o = (long)f * NF + p;
-                const double vR = bqr[d][o * nfl[d] + fm[d]];  // this cell is the right side of its low face
-                const double vL = bql[d][o * nfl[d] + fp[d]];  // and the left side of its high face
+            double ML[NK], MR[NK];
 #pragma unroll
-                for (int r = 0; r < NB; r++) rt[r] += T->bfc[2 * d][p][r] * vR + T->bfc[2 * d + 1][p][r] * vL;
+            for (int e = 0; e < NK; e++) {
+                MR[e] = mr[d][((long)f * NK + e) * g.N + c];
+                ML[e] = ml[d][((long)f * NK + e) * g.N + ch[d]];
+            }
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const int e = fz::pair_index(fz::deg<NB>(r, fz::row_axis(d)), fz::deg<NB>(r, fz::col_axis(d)));
+                rt[r] += fz::Lface(fz::deg<NB>(r, d), 0) * MR[e] + ML[e];
             }
         }
-    }
-    // ---- volume transpose; every wave reaches every barrier ----
-#pragma unroll 1
-    for (int p0 = 0; p0 < NPG; p0 += NCH) {
+        double lof[NB];
 #pragma unroll
-        for (int qq = 0; qq < NCH; qq++) {
-            const int p = p0 + qq;
-            const double* b = T->bint[p];
-            double v = 0.;
-#pragma unroll
-            for (int r = 0; r < NB; r++) v += b[r] * mf[r];
-            qp_s[f][qq][lane] = v;
-            // cotangents of F_x, F_y, F_z of field f at point p: the
-            // transposes of k_cell's volume sums acc[*] and intr[*]
-            double bx = T->cb[KX] * lof[KX], by = T->cb[KY] * lof[KY], bz = T->cb[KZ] * lof[KZ];
-            if constexpr (NB > 4) {
-                by += T->cb[KYZ] * b[KZ] * lof[KYZ];
-                bz += T->cb[KYZ] * b[KY] * lof[KYZ];
-                bx += T->cb[KZX] * b[KZ] * lof[KZX];
-                bz += T->cb[KZX] * b[KX] * lof[KZX];
-                bx += T->cb[KXY] * b[KY] * lof[KXY];
-                by += T->cb[KXY] * b[KX] * lof[KXY];
-                if constexpr (NB == 10) {
-                    bx += T->cb[KXX] * 3. * b[KX] * lof[KXX];
-                    by += T->cb[KYY] * 3. * b[KY] * lof[KYY];
-                    bz += T->cb[KZZ] * 3. * b[KZ] * lof[KZZ];
-                } else {
-                    bx += T->cb[KXYZ] * b[KYZ] * lof[KXYZ];
-                    by += T->cb[KXYZ] * b[KZX] * lof[KXYZ];
-                    bz += T->cb[KXYZ] * b[KXY] * lof[KXYZ];
-                }
-            }
-            const double w = 0.25 * T->w3[p];
-            bf_s[f][0][qq][lane] = dxi * w * bx;
-            bf_s[f][1][qq][lane] = dyi * w * by;
-            bf_s[f][2][qq][lane] = dzi * w * bz;
-        }
-        __syncthreads();
-        if (f < NCH) {
-            double Qp[NQ], bx[NQ], by[NQ], bz[NQ], bQ[NQ];
-#pragma unroll
-            for (int e = 0; e < NQ; e++) {
-                Qp[e] = qp_s[e][f][lane];
-                bx[e] = bf_s[e][0][f][lane];
-                by[e] = bf_s[e][1][f][lane];
-                bz[e] = bf_s[e][2][f][lane];
-                bQ[e] = 0.;
-            }
-            const pr::Prim st = pr::prim<NQ>(ph, Qp);
-            flux_vjp<NQ, 0>(ph, Qp, st, bx, bQ);
-            flux_vjp<NQ, 1>(ph, Qp, st, by, bQ);
-            flux_vjp<NQ, 2>(ph, Qp, st, bz, bQ);
-#pragma unroll
-            for (int e = 0; e < NQ; e++) bq_s[e][f][lane] = bQ[e];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int qq = 0; qq < NCH; qq++) {
-            const double bQf = bq_s[f][qq][lane];
-            const double* b = T->bint[p0 + qq];
-#pragma unroll
-            for (int r = 0; r < NB; r++) rt[r] += b[r] * bQf;
-        }
-        __syncthreads();  // the next row overwrites the exchange arrays
-    }
-    double dcoll = 0.;
-    if (live) {
+        for (int r = 0; r < NB; r++) lof[r] = lo_s[f][lc][r];
         // ---- sources (as cell_vjp_parts) ----
         if (ap.ivis == 0) {
             if (f >= PXX && f <= T_PYZ && ap.coll != 0.)
 #pragma unroll
                 for (int r = 0; r < NB; r++) {
                     rt[r] += -ap.coll * lof[r];
-                    dcoll += -dt * lof[r] * mf[r];
+                    dcoll += -dt * lof[r] * m_s[f][lc][r];
                 }
             if (f >= T_QX && ap.coll_q != 0.)
 #pragma unroll
@@ -1125,46 +1235,38 @@ __global__ __launch_bounds__(CELL13_WAVES * 64) void k_cell13_vjp(
             if (f == RH)
 #pragma unroll
                 for (int r = 0; r < NB; r++)
-                    rt[r] += ap.bf[0] * ap.b * lam[qoff(g, c, MX, r)] + ap.bf[1] * ap.b * lam[qoff(g, c, MY, r)] +
-                             ap.bf[2] * ap.b * lam[qoff(g, c, MZ, r)];
-            if (f >= MX && f <= MZ)
+                    rt[r] += ap.bf[0] * lo_s[MX][lc][r] + ap.bf[1] * lo_s[MY][lc][r] + ap.bf[2] * lo_s[MZ][lc][r];
+            if (f >= MX && f <= MZ) {
+                const double bf = f == MX ? ap.bf[0] : (f == MY ? ap.bf[1] : ap.bf[2]);
 #pragma unroll
-                for (int r = 0; r < NB; r++) rt[r] += ap.bf[f - MX] * ap.b * lam[qoff(g, c, EN, r)];
+                for (int r = 0; r < NB; r++) rt[r] += bf * lo_s[EN][lc][r];
+            }
         }
         // ---- finish (as cell_vjp_finish) ----
-        if (ap.rhs_only) {
-#pragma unroll
-            for (int r = 0; r < NB; r++) lam_in[qoff(g, c, f, r)] = rt[r];
-        } else {
+        if (!ap.rhs_only) {
 #pragma unroll
             for (int r = 0; r < NB; r++) rt[r] = lof[r] + dt * rt[r];
 #pragma unroll
-            for (int t = 0; t < 2; t++)
-                if (ap.acc[t])
+            for (int e = 0; e < 2; e++)
+                if (ap.acc[e])
 #pragma unroll
-                    for (int r = 0; r < NB; r++) rt[r] += ap.w[t] * ap.acc[t][qoff(g, c, f, r)];
+                    for (int r = 0; r < NB; r++) rt[r] += ap.w[e] * ap.acc[e][qoff(g, c, f, r)];
             if (ap.q_raw && f <= EN) {
-                double raw[5][NB];
-#pragma unroll
-                for (int e = 0; e < 5; e++)
-#pragma unroll
-                    for (int r = 0; r < NB; r++) raw[e][r] = ap.q_raw[qoff(g, c, e, r)];
-                const LimFactors F = limit_factors<NB, QP, 5>(raw, ap.lp);
-                if (F.zero) {
+                if (lim_s[lc] & 1) {
 #pragma unroll
                     for (int r = 1; r < NB; r++) rt[r] = 0.0;
-                    if (F.floor && f == RH) rt[0] = 0.0;
+                    if ((lim_s[lc] & 2) && f == RH) rt[0] = 0.0;
                 } else {
-                    const double th = f == RH ? F.th_rho * F.th_p : F.th_p;
+                    const double th = f == RH ? th_s[0][lc] * th_s[1][lc] : th_s[1][lc];
 #pragma unroll
                     for (int r = 1; r < NB; r++) rt[r] *= th;
                 }
             }
-#pragma unroll
-            for (int r = 0; r < NB; r++) lam_in[qoff(g, c, f, r)] = rt[r];
         }
+#pragma unroll
+        for (int r = 0; r < NB; r++) lam_in[qoff(g, c, f, r)] = rt[r];
     }
-    if (ap.partial) block_partial13(dcoll, ap.partial);
+    if (ap.partial) block_partial13<NT / 64>(dcoll, ap.partial);
 }
 
 // adds the block partials to *acc (one block, fixed order)

@@ -280,7 +280,7 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
         (r = alloc(c, (void**)&c->bad, sizeof(unsigned long long))) ||
         (r = alloc(c, (void**)&c->scratch_dt, sizeof(double))) ||
         (r = alloc(c, (void**)&c->step_ctr, sizeof(unsigned long long))) ||
-        (r = alloc(c, (void**)&c->vjp_partial, blocks_for(c->N, 64) * sizeof(double))) ||
+        (r = alloc(c, (void**)&c->vjp_partial, blocks_for(c->N, 16) * sizeof(double))) ||
         (cfg->bc[0] == HD_BC_INFLOW &&
          (r = alloc(c, (void**)&c->inflow, (size_t)g.ny * g.nz * c->nface * c->nQ * sizeof(double)))) ||
         (cfg->integrator == 3 &&
@@ -484,21 +484,20 @@ int hd_apply_mask(hd_ctx* c, double* q, void* stream) {
     return apply_mask(c, q, (hipStream_t)stream);
 }
 
-// The split 13-moment transpose (periodic grids) writes the left cells' face
-// cotangents into fl and the right cells' into bq2, allocated here once (fl is
-// there already where the table-driven kernels run).
+// The split 13-moment transpose (periodic grids) writes the moments of the
+// left cells' face cotangents into fl and of the right cells' into bq2,
+// allocated here once (fl is there already, and larger, where the table-driven
+// kernels run).
 static int ensure_vjp13_buffers(hd_ctx* c) {
     if (c->cfg.nQ != 13 || c->fused_vjp || c->bq2[0]) return HD_OK;
     for (int b = 0; b < 6; b++)
         if (c->cfg.bc[b] != HD_BC_PERIODIC) return HD_OK;
-    const Grid& g = c->grid;
-    const size_t nf = (size_t)c->nface * c->nQ;
-    const size_t nfd[3] = {(size_t)(g.nx + 1) * g.ny * g.nz, (size_t)g.nx * (g.ny + 1) * g.nz,
-                           (size_t)g.nx * g.ny * (g.nz + 1)};
+    const size_t nk = c->nb == 10 ? 6 : 3;  // fz::face_nk
+    const size_t bytes = nk * 13 * (size_t)c->N * sizeof(double);
     for (int d = 2; d >= 0; d--) {  // bq2[0] last: it says that all are there
         int r = HD_OK;
-        if (!c->fl[d]) r = alloc(c, (void**)&c->fl[d], nf * nfd[d] * sizeof(double));
-        if (r == HD_OK && !c->bq2[d]) r = alloc(c, (void**)&c->bq2[d], nf * nfd[d] * sizeof(double));
+        if (!c->fl[d]) r = alloc(c, (void**)&c->fl[d], bytes);
+        if (r == HD_OK && !c->bq2[d]) r = alloc(c, (void**)&c->bq2[d], bytes);
         if (r) return r;
     }
     return HD_OK;

@@ -9,22 +9,16 @@ template <int NB, int QP, int NQ, int RM>
 void Impl<NB, QP, NQ, RM>::stage_vjp(hd_ctx* c, const double* q, const double* lam, double* lam_in,
                                      const adj::AdjParams& ap, hipStream_t s) {
     if constexpr (NQ == 13) {
-        // periodic grids: the split transpose (one wave per face point,
-        // then one field per wave); bq2 exists only for those
+        // periodic grids: the split transpose (a face point, then a volume
+        // point a lane); bq2 exists only for those
         if (c->bq2[0]) {
             const Grid& g = c->grid;
-            const long nfd[3] = {(long)(g.nx + 1) * g.ny * g.nz, (long)g.nx * (g.ny + 1) * g.nz,
-                                 (long)g.nx * g.ny * (g.nz + 1)};
-            constexpr int NT = QP * QP * 64;
-            hipLaunchKernelGGL((adj::k_face13_vjp<NB, QP, RM, 0>), dim3(blocks_for(nfd[0], 64)), dim3(NT), 0, s, q,
-                               lam, c->fl[0], c->bq2[0], g, c->ph, ap);
-            hipLaunchKernelGGL((adj::k_face13_vjp<NB, QP, RM, 1>), dim3(blocks_for(nfd[1], 64)), dim3(NT), 0, s, q,
-                               lam, c->fl[1], c->bq2[1], g, c->ph, ap);
-            hipLaunchKernelGGL((adj::k_face13_vjp<NB, QP, RM, 2>), dim3(blocks_for(nfd[2], 64)), dim3(NT), 0, s, q,
-                               lam, c->fl[2], c->bq2[2], g, c->ph, ap);
-            c->vjp_blocks = (int)blocks_for(c->N, 64);
-            hipLaunchKernelGGL((adj::k_cell13_vjp<NB, QP, RM>), dim3(c->vjp_blocks), dim3(CELL13_WAVES * 64), 0, s,
-                               q, lam, lam_in, c->fl[0], c->fl[1], c->fl[2], c->bq2[0], c->bq2[1], c->bq2[2],
+            const unsigned nf = 3 * blocks_for(g.N, adj::face13_faces<QP>());
+            hipLaunchKernelGGL((adj::k_face13_vjp<NB, QP, RM>), dim3((nf + 7) / 8 * 8), dim3(256), 0, s, q, lam,
+                               c->fl[0], c->fl[1], c->fl[2], c->bq2[0], c->bq2[1], c->bq2[2], g, c->ph, ap);
+            c->vjp_blocks = (int)blocks_for(c->N, adj::cell13_cells<QP>());
+            hipLaunchKernelGGL((adj::k_cell13_vjp<NB, QP, RM>), dim3(c->vjp_blocks), dim3(adj::cell13_threads<QP>()),
+                               0, s, q, lam, lam_in, c->fl[0], c->fl[1], c->fl[2], c->bq2[0], c->bq2[1], c->bq2[2],
                                c->dtab, g, c->ph, ap);
             return;
         }
