@@ -417,8 +417,8 @@ __device__ __forceinline__ void limit_vjp(double (&lam)[MQ][NB], const LimFactor
 }
 
 // ------------------------------------------------------------- stage -----
-// grids up to this many cells use the four-wave split of the transpose (when
-// its three 64-cell partial sums fit the 160 KB of LDS)
+// three-point rules: grids up to this many cells use the four-wave split of
+// the transpose (when its three 64-cell partial sums fit the 160 KB of LDS)
 constexpr long kSplitCells = 1L << 17;
 template <int NB, int NQ>
 constexpr bool split_fits() { return 3L * NQ * NB * 64 * 8 <= 150L * 1024; }
@@ -874,6 +874,450 @@ __global__ __launch_bounds__(256) void k_stage_vjp_split(const double* __restric
     if (ap.partial) block_partial(dcoll, ap.partial);
 }
 
+// ------------------------------------------- a point, then a field a lane ----
+// One volume point of a cell whose modes and cotangents lie in LDS (field f at
+// m + f*fs, lo + f*fs): its state, the cotangents of its three fluxes (the
+// transposes of the volume sums; b: the basis there, w: 0.25 times its weight)
+// and the fluxes reversed to the state's cotangent bQ.
+template <int NB, int NQ>
+__device__ __forceinline__ void volume_point_vjp(const double* m, const double* lo, int fs,
+                                                 const double* __restrict__ bp, double w, const Grid& g,
+                                                 const Phys& ph, double (&bQ)[NQ]) {
+    double b[NB], Qp[NQ], bF[NQ];
+#pragma unroll
+    for (int r = 0; r < NB; r++) b[r] = bp[r];
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        double v = m[f * fs];
+#pragma unroll
+        for (int r = 1; r < NB; r++) v += b[r] * m[f * fs + r];
+        Qp[f] = v;
+        bQ[f] = 0.;
+    }
+    const pr::Prim st = pr::prim<NQ>(ph, Qp);
+    const double h[3] = {g.dxi * w, g.dyi * w, g.dzi * w};
+    // cotangent of a field's flux: sum_r cb_r d(phi_r) lo_r
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        const double* const l = lo + f * fs;
+        double s = 3. * l[KX];
+        if constexpr (NB > 4) s += 9. * b[KZ] * l[KZX] + 9. * b[KY] * l[KXY];
+        if constexpr (NB == 10) s += 15. * b[KX] * l[KXX];
+        if constexpr (NB == 8) s += 27. * b[KYZ] * l[KXYZ];
+        bF[f] = h[0] * s;
+    }
+    flux_vjp<NQ, 0>(ph, Qp, st, bF, bQ);
+    sg::section();
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        const double* const l = lo + f * fs;
+        double s = 3. * l[KY];
+        if constexpr (NB > 4) s += 9. * b[KZ] * l[KYZ] + 9. * b[KX] * l[KXY];
+        if constexpr (NB == 10) s += 15. * b[KY] * l[KYY];
+        if constexpr (NB == 8) s += 27. * b[KZX] * l[KXYZ];
+        bF[f] = h[1] * s;
+    }
+    flux_vjp<NQ, 1>(ph, Qp, st, bF, bQ);
+    sg::section();
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        const double* const l = lo + f * fs;
+        double s = 3. * l[KZ];
+        if constexpr (NB > 4) s += 9. * b[KY] * l[KYZ] + 9. * b[KX] * l[KZX];
+        if constexpr (NB == 10) s += 15. * b[KZ] * l[KZZ];
+        if constexpr (NB == 8) s += 27. * b[KXY] * l[KXYZ];
+        bF[f] = h[2] * s;
+    }
+    flux_vjp<NQ, 2>(ph, Qp, st, bF, bQ);
+}
+
+// Field f of cell c from the sum rt of its face and volume terms: the sources,
+// the stage map (lo + dt*rt, the accumulated terms) and the frozen limiter
+// (zero, floor: bits of `lim`), as cell_vjp_parts and cell_vjp_finish, stored;
+// returns the field's share of d/dcoll.  m: this field's modes, lo: the cell's
+// cotangents, field e at lo + e*fs.
+template <int NB, int NQ>
+__device__ __forceinline__ double field_finish(const double* __restrict__ lam, double* __restrict__ lam_in,
+                                               const Grid& g, const AdjParams& ap, int f, long c, double dt,
+                                               double faci, const double* m, const double* lo, int fs, int lim,
+                                               double th_rho, double th_p, double (&rt)[NB]) {
+    double dcoll = 0.;
+    double lof[NB];
+#pragma unroll
+    for (int r = 0; r < NB; r++) lof[r] = lo[f * fs + r];
+    if constexpr (NQ >= 11) {
+        constexpr int SLAST = NQ == 13 ? T_PYZ : PYZ;
+        if (ap.ivis == 0) {
+            if (f >= PXX && f <= SLAST && ap.coll != 0.)
+#pragma unroll
+                for (int r = 0; r < NB; r++) {
+                    rt[r] += -ap.coll * lof[r];
+                    dcoll += -dt * lof[r] * m[r];
+                }
+            if (NQ == 13 && f >= T_QX && ap.coll_q != 0.)
+#pragma unroll
+                for (int r = 0; r < NB; r++) rt[r] += -ap.coll_q * lof[r];
+        }
+        if (ap.ivis == 1 && ap.coll != 0. && ap.out && f >= PXX && f <= SLAST) {
+            // qn is read only when its weight a is nonzero (callers pass no
+            // qn for the first stage)
+            const bool with_qn = ap.a != 0.;
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const long o = qoff(g, c, f, r);
+                const double bv = with_qn ? ap.out[o] - ap.a * ap.qn[o] : ap.out[o];
+                dcoll += -dt * faci * lam[o] * bv;
+            }
+        }
+    }
+    if (ap.bf[0] != 0. || ap.bf[1] != 0. || ap.bf[2] != 0.) {
+        // lo of the Euler fields (relaxation factor 1)
+        if (f == RH)
+#pragma unroll
+            for (int r = 0; r < NB; r++)
+                rt[r] += ap.bf[0] * lo[MX * fs + r] + ap.bf[1] * lo[MY * fs + r] + ap.bf[2] * lo[MZ * fs + r];
+        if (f >= MX && f <= MZ) {
+            const double bf = f == MX ? ap.bf[0] : (f == MY ? ap.bf[1] : ap.bf[2]);
+#pragma unroll
+            for (int r = 0; r < NB; r++) rt[r] += bf * lo[EN * fs + r];
+        }
+    }
+    if (!ap.rhs_only) {
+#pragma unroll
+        for (int r = 0; r < NB; r++) rt[r] = lof[r] + dt * rt[r];
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+            if (ap.acc[e])
+#pragma unroll
+                for (int r = 0; r < NB; r++) rt[r] += ap.w[e] * ap.acc[e][qoff(g, c, f, r)];
+        if (ap.q_raw && f <= EN) {
+            if (lim & 1) {
+#pragma unroll
+                for (int r = 1; r < NB; r++) rt[r] = 0.0;
+                if ((lim & 2) && f == RH) rt[0] = 0.0;
+            } else {
+                const double th = f == RH ? th_rho * th_p : th_p;
+#pragma unroll
+                for (int r = 1; r < NB; r++) rt[r] *= th;
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < NB; r++) lam_in[qoff(g, c, f, r)] = rt[r];
+    return dcoll;
+}
+
+// the limiter's factors of cell c, for field_finish
+template <int NB, int QP>
+__device__ __forceinline__ void limit_terms(const AdjParams& ap, const Grid& g, long c, int& lim, double& th_rho,
+                                            double& th_p) {
+    double raw[5][NB];
+#pragma unroll
+    for (int e = 0; e < 5; e++)
+#pragma unroll
+        for (int r = 0; r < NB; r++) raw[e][r] = ap.q_raw[qoff(g, c, e, r)];
+    const LimFactors L = limit_factors<NB, QP, 5>(raw, ap.lp);
+    th_rho = L.th_rho;
+    th_p = L.th_p;
+    lim = (L.zero ? 1 : 0) + (L.floor ? 2 : 0);
+}
+
+// per-block partial of d(lam.out)/dcoll for workgroups of W waves
+template <int W>
+__device__ __forceinline__ void block_partial_of(double v, double* partial) {
+    __shared__ double red[W];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.;
+        for (int w = 0; w < W; w++) s += red[w];
+        partial[blockIdx.x] = s;
+    }
+}
+
+// Two-point rules (nbasis 4 and 8): a workgroup of eight waves takes 16 cells,
+// each of its first six waves one face of each (a lane a face point: 16 cells
+// by 4 points), the last two the volume points.  The cells' own modes and
+// cotangents lie in LDS for all; a face wave adds its neighbours' face
+// coefficients.  Then a field of a cell a lane sums the points and finishes.
+// Bound by latency (a chain of loads, one point, the sums) on the grids it is
+// for; five fields run as fast in 128 registers, two workgroups a CU (64,000
+// cells: 71 us against 96 with 256), more fields spill there (8,192 cells, 11
+// fields: 22.4 us against 20.8 with 256).
+constexpr int kPointCells = 16;
+
+template <int NB, int NQ, int DIR, int SIDE>
+__device__ __forceinline__ bool face_neighbour(const Grid& g, long c, long& cn) {
+    const long sd = DIR == 0 ? 1 : DIR == 1 ? g.nx : (long)g.nx * g.ny;
+    const int n_ax = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
+    const int a = (int)(DIR == 0 ? c % g.nx : DIR == 1 ? (c / g.nx) % g.ny : c / ((long)g.nx * g.ny));
+    const bool edge = SIDE ? a == n_ax - 1 : a == 0;
+    cn = SIDE ? (edge ? c - (n_ax - 1) * sd : c + sd) : (edge ? c + (n_ax - 1) * sd : c - sd);
+    return edge && g.bc[2 * DIR + SIDE] != BC_PERIODIC;  // a boundary face: cn is not its neighbour
+}
+
+// trace and lifted-cotangent coefficients of the neighbours, to kn
+template <int NB, int NQ, int DIR, int SIDE>
+__device__ __forceinline__ void load_neighbours(double* kn, const double* __restrict__ q,
+                                                const double* __restrict__ lam, long c0, const Grid& g,
+                                                double b, double faci, double faciq) {
+    constexpr int NK = fz::face_nk<NB>(), C = kPointCells;
+    const int lane = (int)(threadIdx.x & 63);
+    const long c = c0 + lane % C < g.N ? c0 + lane % C : g.N - 1;
+    long cn;
+    if (face_neighbour<NB, NQ, DIR, SIDE>(g, c, cn)) return;
+#pragma unroll
+    for (int n = 0; n < (NQ * C + 63) / 64; n++) {
+        const int it = lane + 64 * n, f = it / C;
+        if (it < NQ * C) {
+            double m[1][NB], l[1][NB], K[1][NK], L[1][NK];
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const long o = ((long)r * NQ + f) * g.N + cn;
+                m[0][r] = q[o];
+                l[0][r] = lam[o];
+            }
+            fz::face_coeffs<NB, 1, DIR, 1 - SIDE, NK>(m, K);
+            lift_coeffs<NB, 1, DIR, 1 - SIDE, NK>(l, L);
+            const double fac = b * (NQ == 13 && f >= T_QX ? faciq : (f >= PXX ? faci : 1.0));
+#pragma unroll
+            for (int k = 0; k < NK; k++) {
+                kn[it * NK + k] = K[0][k];
+                kn[(NQ * C + it) * NK + k] = fac * L[0][k];
+            }
+        }
+    }
+}
+
+// One face point of a cell: the cotangent of the cell's trace to the wave's
+// part of LDS (kn, its neighbours' coefficients until then).
+template <int NB, int QP, int NQ, int RM, int DIR, int SIDE>
+__device__ __forceinline__ void face_point_vjp(double* kn, const double* m_s, const double* lo_s, long c0,
+                                               const Grid& g, const Phys& ph, const double* __restrict__ inflow) {
+    constexpr int NF = QP * QP, NK = fz::face_nk<NB>(), C = kPointCells;
+    static_assert(NF * C == 64, "a wave is 16 cells by 4 points");
+    const auto& FP = fz::face_poly<NB>();
+    const int lane = (int)(threadIdx.x & 63), p = lane / C, lc = lane % C;
+    const long c = c0 + lc < g.N ? c0 + lc : g.N - 1;
+    long cn;
+    const bool ext = face_neighbour<NB, NQ, DIR, SIDE>(g, c, cn);
+    const int bc = g.bc[2 * DIR + SIDE];
+    const double dxi_d = DIR == 0 ? g.dxi : DIR == 1 ? g.dyi : g.dzi;
+    double b[NK], wb[NK];
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+        b[k] = FP.b[p][k];
+        wb[k] = dxi_d * FP.wb[p][k];
+    }
+    // field f of the cell's trace (with the forward kernel's arithmetic, so
+    // that every Riemann branch is taken as in the forward stage), of the
+    // neighbour's, and of the flux's cotangent
+    auto own_at = [&](int f) {
+        double m[1][NB], K[1][NK];
+#pragma unroll
+        for (int r = 0; r < NB; r++) m[0][r] = m_s[(f * C + lc) * NB + r];
+        fz::face_coeffs<NB, 1, DIR, SIDE, NK>(m, K);
+        double s = K[0][0];
+#pragma unroll
+        for (int k = 1; k < NK; k++) s += K[0][k] * b[k];
+        return s;
+    };
+    auto other_at = [&](int f) {
+        const double* const k = kn + (f * C + lc) * NK;
+        double s = k[0];
+#pragma unroll
+        for (int e = 1; e < NK; e++) s += k[e] * b[e];
+        return s;
+    };
+    auto mu_at = [&](int f) {
+        double l[1][NB], L[1][NK];
+#pragma unroll
+        for (int r = 0; r < NB; r++) l[0][r] = lo_s[(f * C + lc) * NB + r];
+        lift_coeffs<NB, 1, DIR, SIDE, NK>(l, L);
+        const double* const k = kn + (NQ * C + f * C + lc) * NK;
+        double s = 0.;
+#pragma unroll
+        for (int e = 0; e < NK; e++) s += (ext ? L[0][e] : L[0][e] + k[e]) * wb[e];
+        return s;
+    };
+    double own[NQ], oth[NQ], mu[NQ], bo[NQ], bt[NQ], bFo[NQ], bFt[NQ];
+#pragma unroll
+    for (int f = 0; f < NQ; f++) {
+        bo[f] = 0.;
+        bt[f] = 0.;
+    }
+#pragma unroll
+    for (int f = 0; f < 5; f++) {
+        own[f] = own_at(f);
+        mu[f] = mu_at(f);
+    }
+    bool zero_normal = false, flip_mx = false;
+    if (ext) {
+#pragma unroll
+        for (int f = 0; f < 5; f++) oth[f] = own[f];
+        if (bc == BC_NOSLIP) {
+            oth[MX] = oth[MY] = oth[MZ] = 0.0;
+        } else if (bc == BC_WALL) {
+            oth[MX + DIR] = 0.0;
+        } else if (bc == BC_OUTFLOW) {
+            if (DIR == 0 && SIDE == 1) {
+                if (oth[MX] > 0.0) { oth[MX] = -own[MX]; flip_mx = true; }
+            } else {
+                // the face's extreme normal momentum decides for all its points
+                double v = own[MX + DIR];
+#pragma unroll
+                for (int o = C; o < 64; o <<= 1) {
+                    const double w = __shfl_xor(v, o, 64);
+                    v = SIDE ? fmin(v, w) : fmax(v, w);
+                }
+                zero_normal = SIDE ? (v < 0.0) : (v > 0.0);
+                if (zero_normal) oth[MX + DIR] = 0.0;
+            }
+        }
+        if constexpr (DIR == 0 && SIDE == 0) {
+            if (bc == BC_INFLOW) {
+                fz::CellPos cp;
+                cp.c = c;
+                cp.i = 0;
+                cp.j = (int)((c / g.nx) % g.ny);
+                cp.k = (int)(c / ((long)g.nx * g.ny));
+                fz::inflow_ghost<NQ>(inflow, g, cp, p, NF, oth);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int f = 0; f < 5; f++) oth[f] = other_at(f);
+    }
+    // face_vjp in parts (the Riemann solver's Euler fields, the cell's own
+    // flux, at a boundary the ghost's), so that no part holds all that the
+    // point has
+    {
+        const pr::Prim so = pr::prim<5>(ph, own), st = pr::prim<5>(ph, oth);
+        riemann_vjp<RM, DIR>(ph, SIDE ? own : oth, SIDE ? so : st, SIDE ? oth : own, SIDE ? st : so, mu,
+                             SIDE ? bo : bt, SIDE ? bt : bo, SIDE ? bFo : bFt, SIDE ? bFt : bFo);
+    }
+    sg::section();
+#pragma unroll
+    for (int f = 5; f < NQ; f++) {
+        own[f] = own_at(f);
+        bFo[f] = 0.5 * mu_at(f);
+    }
+    flux_vjp<NQ, DIR>(ph, own, pr::prim<NQ>(ph, own), bFo, bo);
+    sg::section();
+    if (ext) {
+        // ghost = G(own): add G^T of the ghost's cotangent
+#pragma unroll
+        for (int f = 5; f < NQ; f++) {
+            oth[f] = own_at(f);
+            bFt[f] = 0.5 * mu_at(f);
+        }
+        flux_vjp<NQ, DIR>(ph, oth, pr::prim<NQ>(ph, oth), bFt, bt);
+#pragma unroll
+        for (int f = 0; f < NQ; f++) {
+            double gcoef = 1.0;
+            if (bc == BC_NOSLIP && (f == MX || f == MY || f == MZ)) gcoef = 0.0;
+            if (bc == BC_WALL && f == MX + DIR) gcoef = 0.0;
+            if (bc == BC_INFLOW && f <= EN) gcoef = 0.0;  // prescribed: no dependence on the interior
+            if (bc == BC_OUTFLOW) {
+                if (DIR == 0 && SIDE == 1) {
+                    if (f == MX && flip_mx) gcoef = -1.0;
+                } else if (zero_normal && f == MX + DIR) {
+                    gcoef = 0.0;
+                }
+            }
+            bo[f] += gcoef * bt[f];
+        }
+    }
+    sg::section();  // the wave has read its neighbours' coefficients
+#pragma unroll
+    for (int f = 0; f < NQ; f++) kn[f * 64 + lane] = bo[f];
+}
+
+template <int NB, int QP, int NQ, int RM>
+__global__ __launch_bounds__(512, (NQ == 5 ? 4 : 2)) void k_points_vjp(const double* __restrict__ q, const double* __restrict__ lam,
+                                                       double* __restrict__ lam_in, const Tables* __restrict__ T,
+                                                       Grid g, Phys ph, AdjParams ap) {
+    constexpr int NK = fz::face_nk<NB>(), C = kPointCells, NPG = QP * QP * QP, NF = QP * QP;
+    static_assert(NPG * C == 128, "two waves of volume points");
+    __shared__ __attribute__((aligned(16))) double m_s[NQ * C * NB], lo_s[NQ * C * NB];
+    __shared__ __attribute__((aligned(16))) double kn_s[6][2 * NQ * C * NK];
+    __shared__ double bq_s[NQ][NPG * C];
+    __shared__ double th_s[2][C];
+    __shared__ int lim_s[C];
+    const int t = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const long c0 = (long)xcd_block() * C;
+    const double dt = *ap.dt;
+    const double faci = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll) : 1.0;
+    const double faciq = (ap.ivis == 1 && !ap.rhs_only) ? 1. / (1. + dt * ap.coll_q) : 1.0;
+#pragma unroll
+    for (int n = 0; n < (NQ * NB * C + 511) / 512; n++) {
+        const int it = t + n * 512;
+        if (it < NQ * NB * C) {
+            const int c = it % C, row = it / C, r = row / NQ, f = row % NQ;
+            // lanes past the grid take a copy of the last cell and store nothing
+            const long o = (long)row * g.N + (c0 + c < g.N ? c0 + c : g.N - 1);
+            m_s[(f * C + c) * NB + r] = q[o];
+            lo_s[(f * C + c) * NB + r] = ap.b * lam[o] * (NQ == 13 && f >= T_QX ? faciq : (f >= PXX ? faci : 1.0));
+        }
+    }
+    double* const kn = kn_s[wave < 6 ? wave : 0];
+    switch (wave) {
+    case 0: load_neighbours<NB, NQ, 0, 0>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    case 1: load_neighbours<NB, NQ, 0, 1>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    case 2: load_neighbours<NB, NQ, 1, 0>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    case 3: load_neighbours<NB, NQ, 1, 1>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    case 4: load_neighbours<NB, NQ, 2, 0>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    case 5: load_neighbours<NB, NQ, 2, 1>(kn, q, lam, c0, g, ap.b, faci, faciq); break;
+    }
+    __syncthreads();
+    switch (wave) {
+    case 0: face_point_vjp<NB, QP, NQ, RM, 0, 0>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    case 1: face_point_vjp<NB, QP, NQ, RM, 0, 1>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    case 2: face_point_vjp<NB, QP, NQ, RM, 1, 0>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    case 3: face_point_vjp<NB, QP, NQ, RM, 1, 1>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    case 4: face_point_vjp<NB, QP, NQ, RM, 2, 0>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    case 5: face_point_vjp<NB, QP, NQ, RM, 2, 1>(kn, m_s, lo_s, c0, g, ph, ap.inflow); break;
+    default: {
+        const int v = t - 384, p = v / C, c = v % C;
+        double bQ[NQ];
+        volume_point_vjp<NB, NQ>(m_s + c * NB, lo_s + c * NB, C * NB, T->bint[p], 0.25 * T->w3[p], g, ph, bQ);
+#pragma unroll
+        for (int f = 0; f < NQ; f++) bq_s[f][v] = bQ[f];
+        if (ap.q_raw && v >= 64 && v < 64 + C)
+            limit_terms<NB, QP>(ap, g, c0 + c < g.N ? c0 + c : g.N - 1, lim_s[c], th_s[0][c], th_s[1][c]);
+    }
+    }
+    __syncthreads();
+    double dcoll = 0.;
+    for (int it = t; it < NQ * C; it += 512) {
+        const int f = it / C, lc = it % C;
+        const long c = c0 + lc;
+        if (c >= g.N) continue;
+        double rt[NB];
+#pragma unroll
+        for (int r = 0; r < NB; r++) rt[r] = 0.;
+#pragma unroll
+        for (int p = 0; p < NPG; p++) {
+            const double v = bq_s[f][p * C + lc];
+#pragma unroll
+            for (int r = 0; r < NB; r++) rt[r] += fz::phi_int<NB, QP>(r, p / (QP * QP), (p / QP) % QP, p % QP) * v;
+        }
+#pragma unroll
+        for (int w = 0; w < 6; w++)
+#pragma unroll
+            for (int p = 0; p < NF; p++) {
+                const double v = kn_s[w][f * 64 + p * C + lc];
+#pragma unroll
+                for (int r = 0; r < NB; r++) rt[r] += fz::phi_face<NB, QP>(w / 2, w % 2, r, p / QP, p % QP) * v;
+            }
+        dcoll += field_finish<NB, NQ>(lam, lam_in, g, ap, f, c, dt, faci, m_s + (f * C + lc) * NB, lo_s + lc * NB,
+                                      C * NB, lim_s[lc], th_s[0][lc], th_s[1][lc], rt);
+    }
+    if (ap.partial) block_partial_of<8>(dcoll, ap.partial);
+}
+
 // ------------------------------------------------- 13-moment transpose ----
 // The transpose of a 13-moment stage on a grid periodic in every direction,
 // split into a face and a cell kernel, so that no lane holds a whole cell.
@@ -1051,21 +1495,6 @@ constexpr int cell13_cells() { return QP == 3 ? 16 : 32; }
 template <int QP>
 constexpr int cell13_threads() { return (QP * QP * QP * cell13_cells<QP>() + 63) / 64 * 64 + 64; }
 
-// per-block partial of d(lam.out)/dcoll for workgroups of W waves
-template <int W>
-__device__ __forceinline__ void block_partial13(double v, double* partial) {
-    __shared__ double red[W];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.;
-        for (int w = 0; w < W; w++) s += red[w];
-        partial[blockIdx.x] = s;
-    }
-}
-
 // The cells' modes and cotangents to LDS; then a volume point a lane: its
 // state, the cotangents of its three fluxes (the transposes of the volume
 // sums), the fluxes reversed (flux_vjp) and the state cotangent to LDS; then
@@ -1104,67 +1533,14 @@ __global__ __launch_bounds__(cell13_threads<QP>(), 4) void k_cell13_vjp(
     __syncthreads();
     if (t < NPG * C) {
         const int p = t / C, c = t % C;
-        double b[NB], Qp[NQ], bF[NQ], bQ[NQ];
-#pragma unroll
-        for (int r = 0; r < NB; r++) b[r] = T->bint[p][r];
-        const double w = 0.25 * T->w3[p];
-#pragma unroll
-        for (int f = 0; f < NQ; f++) {
-            double v = m_s[f][c][0];
-#pragma unroll
-            for (int r = 1; r < NB; r++) v += b[r] * m_s[f][c][r];
-            Qp[f] = v;
-            bQ[f] = 0.;
-        }
-        const pr::Prim st = pr::prim<NQ>(ph, Qp);
-        // cotangent of a field's flux: sum_r cb_r d(phi_r) lo_r
-        {
-            const double h = g.dxi * w;
-#pragma unroll
-            for (int f = 0; f < NQ; f++) {
-                const double* const l = lo_s[f][c];
-                double s = 3. * l[KX];
-                if constexpr (NB == 10) s += 9. * b[KZ] * l[KZX] + 9. * b[KY] * l[KXY] + 15. * b[KX] * l[KXX];
-                bF[f] = h * s;
-            }
-            flux_vjp<NQ, 0>(ph, Qp, st, bF, bQ);
-        }
-        {
-            const double h = g.dyi * w;
-#pragma unroll
-            for (int f = 0; f < NQ; f++) {
-                const double* const l = lo_s[f][c];
-                double s = 3. * l[KY];
-                if constexpr (NB == 10) s += 9. * b[KZ] * l[KYZ] + 9. * b[KX] * l[KXY] + 15. * b[KY] * l[KYY];
-                bF[f] = h * s;
-            }
-            flux_vjp<NQ, 1>(ph, Qp, st, bF, bQ);
-        }
-        {
-            const double h = g.dzi * w;
-#pragma unroll
-            for (int f = 0; f < NQ; f++) {
-                const double* const l = lo_s[f][c];
-                double s = 3. * l[KZ];
-                if constexpr (NB == 10) s += 9. * b[KY] * l[KYZ] + 9. * b[KX] * l[KZX] + 15. * b[KZ] * l[KZZ];
-                bF[f] = h * s;
-            }
-            flux_vjp<NQ, 2>(ph, Qp, st, bF, bQ);
-        }
+        double bQ[NQ];
+        volume_point_vjp<NB, NQ>(&m_s[0][c][0], &lo_s[0][c][0], C * NB, T->bint[p], 0.25 * T->w3[p], g, ph, bQ);
 #pragma unroll
         for (int f = 0; f < NQ; f++) bq_s[f][t] = bQ[f];
     } else if (ap.q_raw && t >= NT - 64 && t < NT - 64 + C) {
         const int c = t - (NT - 64);
         const long cc = c0 + c < g.N ? c0 + c : g.N - 1;
-        double raw[5][NB];
-#pragma unroll
-        for (int e = 0; e < 5; e++)
-#pragma unroll
-            for (int r = 0; r < NB; r++) raw[e][r] = ap.q_raw[qoff(g, cc, e, r)];
-        const LimFactors L = limit_factors<NB, QP, 5>(raw, ap.lp);
-        th_s[0][c] = L.th_rho;
-        th_s[1][c] = L.th_p;
-        lim_s[c] = (L.zero ? 1 : 0) + (L.floor ? 2 : 0);
+        limit_terms<NB, QP>(ap, g, cc, lim_s[c], th_s[0][c], th_s[1][c]);
     }
     __syncthreads();
     double dcoll = 0.;
@@ -1204,69 +1580,10 @@ __global__ __launch_bounds__(cell13_threads<QP>(), 4) void k_cell13_vjp(
                 rt[r] += fz::Lface(fz::deg<NB>(r, d), 0) * MR[e] + ML[e];
             }
         }
-        double lof[NB];
-#pragma unroll
-        for (int r = 0; r < NB; r++) lof[r] = lo_s[f][lc][r];
-        // ---- sources (as cell_vjp_parts) ----
-        if (ap.ivis == 0) {
-            if (f >= PXX && f <= T_PYZ && ap.coll != 0.)
-#pragma unroll
-                for (int r = 0; r < NB; r++) {
-                    rt[r] += -ap.coll * lof[r];
-                    dcoll += -dt * lof[r] * m_s[f][lc][r];
-                }
-            if (f >= T_QX && ap.coll_q != 0.)
-#pragma unroll
-                for (int r = 0; r < NB; r++) rt[r] += -ap.coll_q * lof[r];
-        }
-        if (ap.ivis == 1 && ap.coll != 0. && ap.out && f >= PXX && f <= T_PYZ) {
-            // qn is read only when its weight a is nonzero (callers pass no
-            // qn for the first stage)
-            const bool with_qn = ap.a != 0.;
-#pragma unroll
-            for (int r = 0; r < NB; r++) {
-                const long o = qoff(g, c, f, r);
-                const double bv = with_qn ? ap.out[o] - ap.a * ap.qn[o] : ap.out[o];
-                dcoll += -dt * faci * lam[o] * bv;
-            }
-        }
-        if (ap.bf[0] != 0. || ap.bf[1] != 0. || ap.bf[2] != 0.) {
-            // lo of the Euler fields (relaxation factor 1)
-            if (f == RH)
-#pragma unroll
-                for (int r = 0; r < NB; r++)
-                    rt[r] += ap.bf[0] * lo_s[MX][lc][r] + ap.bf[1] * lo_s[MY][lc][r] + ap.bf[2] * lo_s[MZ][lc][r];
-            if (f >= MX && f <= MZ) {
-                const double bf = f == MX ? ap.bf[0] : (f == MY ? ap.bf[1] : ap.bf[2]);
-#pragma unroll
-                for (int r = 0; r < NB; r++) rt[r] += bf * lo_s[EN][lc][r];
-            }
-        }
-        // ---- finish (as cell_vjp_finish) ----
-        if (!ap.rhs_only) {
-#pragma unroll
-            for (int r = 0; r < NB; r++) rt[r] = lof[r] + dt * rt[r];
-#pragma unroll
-            for (int e = 0; e < 2; e++)
-                if (ap.acc[e])
-#pragma unroll
-                    for (int r = 0; r < NB; r++) rt[r] += ap.w[e] * ap.acc[e][qoff(g, c, f, r)];
-            if (ap.q_raw && f <= EN) {
-                if (lim_s[lc] & 1) {
-#pragma unroll
-                    for (int r = 1; r < NB; r++) rt[r] = 0.0;
-                    if ((lim_s[lc] & 2) && f == RH) rt[0] = 0.0;
-                } else {
-                    const double th = f == RH ? th_s[0][lc] * th_s[1][lc] : th_s[1][lc];
-#pragma unroll
-                    for (int r = 1; r < NB; r++) rt[r] *= th;
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < NB; r++) lam_in[qoff(g, c, f, r)] = rt[r];
+        dcoll += field_finish<NB, NQ>(lam, lam_in, g, ap, f, c, dt, faci, &m_s[f][lc][0], &lo_s[0][lc][0], C * NB,
+                                      lim_s[lc], th_s[0][lc], th_s[1][lc], rt);
     }
-    if (ap.partial) block_partial13<NT / 64>(dcoll, ap.partial);
+    if (ap.partial) block_partial_of<NT / 64>(dcoll, ap.partial);
 }
 
 // adds the block partials to *acc (one block, fixed order)

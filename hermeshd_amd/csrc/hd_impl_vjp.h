@@ -23,7 +23,20 @@ void Impl<NB, QP, NQ, RM>::stage_vjp(hd_ctx* c, const double* q, const double* l
             return;
         }
     }
-    {
+    if constexpr (QP == 2) {
+        // A point a lane up to 7/8 of two rounds of the per-cell kernel's
+        // workgroups (256 cells, one a CU); past that a lane that holds its
+        // cell takes fewer steps in all.  nbasis 4, 11 fields: 21 us against
+        // 41 (8,192 cells, the per-cell kernel split over four waves, which
+        // this replaced), 133 against 133 (64,000, one round), 181 against 307
+        // (92,160, split), but 585 against 469 (262,144).
+        if (4 * c->N <= 7 * 256L * c->num_cus) {
+            c->vjp_blocks = (int)blocks_for(c->N, adj::kPointCells);
+            hipLaunchKernelGGL((adj::k_points_vjp<NB, QP, NQ, RM>), dim3(c->vjp_blocks), dim3(512), 0, s, q, lam,
+                               lam_in, c->dtab, c->grid, c->ph, ap);
+            return;
+        }
+    } else {
         // small grids are latency-bound: spread each cell over four waves
         if constexpr (adj::split_fits<NB, NQ>()) {
             if (c->N <= adj::kSplitCells) {
@@ -33,10 +46,10 @@ void Impl<NB, QP, NQ, RM>::stage_vjp(hd_ctx* c, const double* q, const double* l
                 return;
             }
         }
-        c->vjp_blocks = (int)blocks_for(c->N, 256);
-        hipLaunchKernelGGL((adj::k_stage_vjp<NB, QP, NQ, RM>), dim3(c->vjp_blocks), dim3(256), 0, s, q, lam,
-                           lam_in, c->grid, c->ph, ap);
     }
+    c->vjp_blocks = (int)blocks_for(c->N, 256);
+    hipLaunchKernelGGL((adj::k_stage_vjp<NB, QP, NQ, RM>), dim3(c->vjp_blocks), dim3(256), 0, s, q, lam, lam_in,
+                       c->grid, c->ph, ap);
 }
 
 }  // namespace hd
