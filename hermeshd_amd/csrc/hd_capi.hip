@@ -275,7 +275,7 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
         (c->generic && ((r = alloc(c, (void**)&c->fl[0], nf * nfx * sizeof(double))) ||
                         (r = alloc(c, (void**)&c->fl[1], nf * nfy * sizeof(double))) ||
                         (r = alloc(c, (void**)&c->fl[2], nf * nfz * sizeof(double))))) ||
-        (r = alloc(c, (void**)&c->partial, c->npart * sizeof(double))) ||
+        (r = alloc(c, (void**)&c->partial, (c->npart + 1) * sizeof(double))) ||
         (r = alloc(c, (void**)&c->err, sizeof(int))) ||
         (r = alloc(c, (void**)&c->bad, sizeof(unsigned long long))) ||
         (r = alloc(c, (void**)&c->scratch_dt, sizeof(double))) ||
@@ -404,13 +404,13 @@ int hd_min_dt(hd_ctx* c, const double* q, double* dt_dev, void* stream) {
     const int nblk = (int)std::min<long>(c->npart, (c->N + 255) / 256);
     hipLaunchKernelGGL(k_wavespeed, dim3(nblk), dim3(256), 0, s, q, c->grid, cfl_eos(c), 1.01 * c->cfg.rh_floor,
                        c->partial);
-    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q, c->grid, cfl_eos(c), c->partial, nblk, c->cfg.cflm,
-                       dt_dev, (double*)nullptr);
+    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q, c->grid, cfl_eos(c), c->partial, nblk,
+                       (const double*)nullptr, c->cfg.cflm, dt_dev, (double*)nullptr);
     HIPCHK(hipGetLastError());
     return HD_OK;
 }
 
-int hd_update(hd_ctx* c, double* q_io, double* q1, double* q2, const double* dt_dev, void* stream) {
+static int update(hd_ctx* c, double* q_io, double* q1, double* q2, const double* dt_dev, bool limited, void* stream) {
     if (!c || !q_io || !q1 || !dt_dev) return fail(HD_ERR_INVALID, "NULL argument");
     if (q_io == q1 || (q2 && (q2 == q_io || q2 == q1))) return fail(HD_ERR_INVALID, "q_io, q1 and q2 must differ");
     hipStream_t s = (hipStream_t)stream;
@@ -421,16 +421,20 @@ int hd_update(hd_ctx* c, double* q_io, double* q1, double* q2, const double* dt_
         // RK3 (src/integrator.f90:74-86): Q1 = E(Q0); Q2 = 3/4 Q0 + 1/4 E(Q1); Q0 = 1/3 Q0 + 2/3 E(Q2).
         // A stage never writes the array it reads neighbours from.
         double* q2b = q2 ? q2 : c->stage_buf;
-        if ((rc = stage(c, q_io, q_io, q1, dt_dev, 0, s, false, true))) return rc;
+        if ((rc = stage(c, q_io, q_io, q1, dt_dev, 0, s, limited, true))) return rc;
         if ((rc = stage(c, q1, q_io, q2b, dt_dev, 2, s, true, true))) return rc;
         if ((rc = stage(c, q2b, q_io, q_io, dt_dev, 3, s, true, false))) return rc;
     } else {
         // RK2 (src/integrator.f90:62-71): Q1 = E(Q0); Q0 = 1/2 (Q0 + E(Q1))
-        if ((rc = stage(c, q_io, q_io, q1, dt_dev, 0, s, false, true))) return rc;
+        if ((rc = stage(c, q_io, q_io, q1, dt_dev, 0, s, limited, true))) return rc;
         if ((rc = stage(c, q1, q_io, q_io, dt_dev, 1, s, true, false))) return rc;
     }
     if ((rc = apply_mask(c, q_io, s))) return rc;
     return advance_step(c, s);
+}
+
+int hd_update(hd_ctx* c, double* q_io, double* q1, double* q2, const double* dt_dev, void* stream) {
+    return update(c, q_io, q1, q2, dt_dev, false, stream);
 }
 
 int hd_stage(hd_ctx* c, int32_t rk_order, int32_t stage_index, double* q_in, const double* q_n, double* q_out,
@@ -585,13 +589,23 @@ int hd_set_step(hd_ctx* c, uint64_t step, void* stream) {
 int hd_step(hd_ctx* c, double* q_io, double* q1, double* q2, double* t_dev, double* dt_dev, void* stream) {
     if (!c || !q_io || !q1 || !dt_dev) return fail(HD_ERR_INVALID, "NULL argument");
     hipStream_t s = (hipStream_t)stream;
+    // in one pass with the first stage's limiter, unless the update is refused
+    const bool refused = q_io == q1 || (q2 && (q2 == q_io || q2 == q1)) ||
+                         (c->cfg.bc[0] == HD_BC_INFLOW && !c->inflow_set);
+    if (c->cfg.limiter && !c->generic && !refused && c->N <= START_CELLS) {
+        Ops o;
+        if (!pick_ops(c, &o)) return fail(HD_ERR_UNSUPPORTED, "configuration not built");
+        o.start(c, q_io, cfl_eos(c), dt_dev, t_dev, s);
+        HIPCHK(hipGetLastError());
+        return update(c, q_io, q1, q2, dt_dev, true, stream);
+    }
     const int nblk = (int)std::min<long>(c->npart, (c->N + 255) / 256);
     hipLaunchKernelGGL(k_wavespeed, dim3(nblk), dim3(256), 0, s, q_io, c->grid, cfl_eos(c), 1.01 * c->cfg.rh_floor,
                        c->partial);
     hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q_io, c->grid, cfl_eos(c), c->partial, nblk,
-                       c->cfg.cflm, dt_dev, t_dev);
+                       (const double*)nullptr, c->cfg.cflm, dt_dev, t_dev);
     HIPCHK(hipGetLastError());
-    return hd_update(c, q_io, q1, q2, dt_dev, stream);
+    return update(c, q_io, q1, q2, dt_dev, false, stream);
 }
 
 int hd_check(hd_ctx* c, void* stream, int64_t* bad_cell) {

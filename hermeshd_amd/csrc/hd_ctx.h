@@ -19,6 +19,12 @@
 
 namespace hd {
 constexpr int STAGE_AUTO = -2;
+// Grids whose step starts with one pass for dt and the limiter (fz::k_start):
+// there a launch costs more than the pass (us a step, two passes / one: 256
+// cells 26.4 / 22.0; nbasis 4, 4,096 cells 27.7 / 25.7, 16,384 cells 39.7 /
+// 38.4).  Past that two passes overlap their loads better (nbasis 4, 262,144
+// cells 145 / 150; nbasis 8, 524,288 cells 508 / 526; nbasis 10 equal).
+constexpr long START_CELLS = 32768;
 }
 
 struct hd_ctx {
@@ -34,7 +40,7 @@ struct hd_ctx {
     // periodic 13-moment transpose: the right cells' face cotangents (the left
     // cells' reuse fl); allocated at the first such transpose
     double* bq2[3] = {nullptr, nullptr, nullptr};
-    double* partial = nullptr;                    // wave-speed partial maxima
+    double* partial = nullptr;                    // wave-speed partial maxima (npart + 1)
     int npart = 0;
     int* err = nullptr;
     unsigned long long* bad = nullptr;
@@ -111,6 +117,8 @@ namespace hd {
 
 struct Ops {
     void (*limiter)(hd_ctx*, double*, hipStream_t);
+    // dt of the state (added to *t if t), and the limiter on it
+    void (*start)(hd_ctx*, double*, const CflEos&, double* dt, double* t, hipStream_t);
     void (*faces)(hd_ctx*, const double*, hipStream_t);
     void (*cell)(hd_ctx*, const double*, const double*, double*, const StageParams&, hipStream_t);
     void (*fused)(hd_ctx*, const double*, const double*, double*, const StageParams&, hipStream_t);

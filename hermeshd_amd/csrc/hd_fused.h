@@ -373,6 +373,44 @@ __device__ __forceinline__ bool limit_cell(double (&m)[MQ][NB], const LimParams&
     return changed;
 }
 
+// get_min_dt and the limiter of a step's first stage in one pass: the wave
+// speeds of the cells as they come, their modes as the limiter leaves them.
+// For grids whose step is bound by its launches.  One block stores dt itself;
+// several leave their maxima and, after them, the last cell's sound speed in
+// partial, for k_dt_finish.
+template <int NB, int QP>
+__global__ __launch_bounds__(256, (NB == 4 ? 4 : (NB == 8 ? 2 : 1))) void k_start(
+    double* __restrict__ q, Grid g, LimParams lp, CflEos eos, double dn_min, double cflm, double* __restrict__ partial,
+    double* __restrict__ dt_out, double* __restrict__ t_io) {
+    __shared__ double red[4];
+    __shared__ double last;
+    double vmag = 0.;
+    for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < g.N; c += (long)gridDim.x * blockDim.x) {
+        double m[5][NB], v0;
+#pragma unroll
+        for (int r = 0; r < NB; r++)
+#pragma unroll
+            for (int f = 0; f < 5; f++) m[f][r] = q[((long)r * g.nQ + f) * g.N + c];
+        const double cs = cell_sound_speed(q, g, c, eos, &v0);
+        if (v0 > vmag && m[RH][0] > dn_min) vmag = v0;
+        if (c == g.N - 1) {
+            if (gridDim.x == 1) last = cs;
+            else partial[gridDim.x] = cs;
+        }
+        if (limit_cell<NB, QP, 5>(m, lp)) {
+#pragma unroll
+            for (int r = 0; r < NB; r++)
+#pragma unroll
+                for (int f = 0; f < 5; f++) q[((long)r * g.nQ + f) * g.N + c] = m[f][r];
+        }
+    }
+    vmag = block_max(vmag, red);
+    if (threadIdx.x == 0) {
+        if (gridDim.x == 1) store_dt(vmag, last, g, cflm, dt_out, t_io);
+        else partial[blockIdx.x] = vmag;
+    }
+}
+
 template <int NB, int QP>
 __global__ __launch_bounds__(256, (NB == 4 ? 4 : (NB == 8 ? 2 : 1))) void k_limit(double* __restrict__ q, Grid g, LimParams lp) {
     const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;

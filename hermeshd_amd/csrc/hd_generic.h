@@ -676,6 +676,22 @@ __device__ __forceinline__ double wave_max(double v) {
     return v;
 }
 
+// The largest of the block's vmag (blocks of four waves), valid in thread 0.
+__device__ __forceinline__ double block_max(double v, double (&red)[4]) {
+    v = wave_max(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return fmax(fmax(fmax(red[0], red[1]), red[2]), red[3]);
+}
+
+__device__ __forceinline__ void store_dt(double vmag, double cs_last, const Grid& g, double cflm,
+                                         double* __restrict__ dt_out, double* __restrict__ t_io) {
+    const double vmax = (vmag + cs_last) * g.dxi;
+    const double dt = cflm / vmax;
+    *dt_out = dt;
+    if (t_io) *t_io = *t_io + dt;
+}
+
 static __global__ __launch_bounds__(256) void k_wavespeed(const double* __restrict__ q, Grid g, CflEos eos,
                                                    double dn_min, double* __restrict__ partial) {
     __shared__ double red[4];
@@ -686,34 +702,22 @@ static __global__ __launch_bounds__(256) void k_wavespeed(const double* __restri
         const double dn = q[qoff(g, c, RH, 0)];
         if (v0 > vmag && dn > dn_min) vmag = v0;
     }
-    vmag = wave_max(vmag);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = vmag;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double v = red[0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) v = fmax(v, red[w]);
-        partial[blockIdx.x] = v;
-    }
+    vmag = block_max(vmag, red);
+    if (threadIdx.x == 0) partial[blockIdx.x] = vmag;
 }
 
+// last: the last cell's sound speed, or nullptr to take it from q
 static __global__ __launch_bounds__(256) void k_dt_finish(const double* __restrict__ q, Grid g, CflEos eos,
-                                                   const double* __restrict__ partial, int npart, double cflm,
+                                                   const double* __restrict__ partial, int npart,
+                                                   const double* __restrict__ last, double cflm,
                                                    double* __restrict__ dt_out, double* __restrict__ t_io) {
     __shared__ double red[4];
     double v = 0.;
     for (int b = threadIdx.x; b < npart; b += blockDim.x) v = fmax(v, partial[b]);
-    v = wave_max(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
+    v = block_max(v, red);
     if (threadIdx.x == 0) {
-        double vmag = red[0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) vmag = fmax(vmag, red[w]);
         double v0;
-        const double cs_last = cell_sound_speed(q, g, g.N - 1, eos, &v0);
-        const double vmax = (vmag + cs_last) * g.dxi;
-        const double dt = cflm / vmax;
-        *dt_out = dt;
-        if (t_io) *t_io = *t_io + dt;
+        store_dt(v, last ? *last : cell_sound_speed(q, g, g.N - 1, eos, &v0), g, cflm, dt_out, t_io);
     }
 }
 

@@ -18,6 +18,16 @@ struct Impl {
         else
             hipLaunchKernelGGL((fz::k_limit<NB, QP>), dim3(blocks_for(c->N, 256)), dim3(256), 0, s, q, c->grid, c->lp);
     }
+    static void start(hd_ctx* c, double* q, const CflEos& eos, double* dt, double* t, hipStream_t s) {
+        // one block, and no second launch, while its two cells a thread cost less
+        // than that (512 cells 30.9 us a step, 513 in three blocks 32.0)
+        const long nblk = c->N <= 512 ? 1 : (c->N + 255) / 256;
+        hipLaunchKernelGGL((fz::k_start<NB, QP>), dim3((unsigned)nblk), dim3(256), 0, s, q, c->grid, c->lp, eos,
+                           1.01 * c->cfg.rh_floor, c->cfg.cflm, c->partial, dt, t);
+        if (nblk > 1)
+            hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q, c->grid, eos, c->partial, (int)nblk,
+                               c->partial + nblk, c->cfg.cflm, dt, t);
+    }
     static void faces(hd_ctx* c, const double* q, hipStream_t s) {
         const Grid& g = c->grid;
         long nfx = (long)(g.nx + 1) * g.ny * g.nz, nfy = (long)g.nx * (g.ny + 1) * g.nz, nfz = (long)g.nx * g.ny * (g.nz + 1);
@@ -94,8 +104,8 @@ struct Impl {
                           hipStream_t s);
     static Ops ops() {
         // no ensembles of the 13-moment model; its transpose is split on periodic grids
-        if constexpr (NQ == 13) return Ops{&limiter, &faces, &cell, &fused, nullptr, nullptr, &stage_vjp};
-        else return Ops{&limiter, &faces, &cell, &fused, &ens_limit, &ens_stage, &stage_vjp};
+        if constexpr (NQ == 13) return Ops{&limiter, &start, &faces, &cell, &fused, nullptr, nullptr, &stage_vjp};
+        else return Ops{&limiter, &start, &faces, &cell, &fused, &ens_limit, &ens_stage, &stage_vjp};
     }
 };
 

@@ -72,7 +72,8 @@ extern "C" int hd_min_dt_static(const hd_config* cfg, const double* q, double* d
     // one cell per thread: every workgroup writes its own partial, which the
     // finishing block reads back
     hipLaunchKernelGGL(k_wavespeed, dim3((unsigned)nblk), dim3(256), 0, s, q, g, e, 1.01 * cfg->rh_floor, partial);
-    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q, g, e, partial, (int)nblk, cfg->cflm, dt_dev,
+    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, q, g, e, partial, (int)nblk,
+                       (const double*)nullptr, cfg->cflm, dt_dev,
                        (double*)nullptr);
     HIPCHK(hipGetLastError());
     return HD_OK;

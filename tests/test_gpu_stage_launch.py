@@ -155,3 +155,31 @@ def test_transpose_of_a_point_a_lane(oracle_mod, name, bc, dims):
     (ref,) = torch.autograd.grad(dg.rhs(qt), qt, torch.from_numpy(lam))
     got = Solver(cfg).rhs_vjp(torch.from_numpy(q).cuda(), torch.from_numpy(lam).cuda()).cpu().numpy()
     assert field_rel_err(lam + got, lam + ref.numpy()) < VJP_TOL
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (255, 1, 1), (256, 2, 1), (27, 19, 1), (128, 16, 16), (331, 11, 9)],
+                         ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("name", ["nb4", "nb8", "nb10"])
+@pytest.mark.parametrize("low", ["steep", "mean"])
+def test_step_equals_min_dt_and_update(torch_mod, low, name, n):
+    """One pass for the time step and the first limiter, in one block (two cells
+    a thread), several, and in two passes again: bitwise min_dt and then
+    update, with steep cells or cells of a mean below the floor, the last one
+    (whose sound speed dt takes) among them."""
+    from hermeshd_amd.solver import Solver
+    cfg = HDConfig(nx=n[0], ny=n[1], nz=n[2], lx=0.1 * n[0], ly=0.1 * n[1], lz=0.1 * n[2], bc=PERIODIC, T_floor=1e-4,
+                   rh_floor=0.05, limiter=True, **CASES[name])
+    q = torch_mod.from_numpy(smooth_state(cfg, seed=6)).cuda()
+    cells = q[1:, :5].flatten(2) if low == "steep" else q.flatten(2)
+    cells[..., ::7] *= 12.0 if low == "steep" else 0.02
+    cells[..., -1] *= 12.0 if low == "steep" else 0.02
+    s, qa, qb = Solver(cfg), q.clone(), q.clone()
+    t, dt = torch_mod.full_like(s.t, 0.25), torch_mod.zeros_like(s.dt)
+    s.step(qa, torch_mod.zeros_like(q), t=t, dt=dt)
+    ref = s.min_dt(qb)
+    s.update(qb, torch_mod.zeros_like(q), None, ref)
+    lim = q.clone()
+    s.limit(lim)
+    assert low == "steep" or not torch_mod.equal(lim, q)
+    assert float(dt) == float(ref) and float(t) == 0.25 + float(ref)
+    assert torch_mod.equal(qa, qb)
