@@ -23,7 +23,7 @@ COMPILE_FLAGS = [
 ]
 LINK_FLAGS = ["-shared", "-fPIC", f"--offload-arch={ARCH}"]
 # per-unit scheduler choice, kept where it measured faster: the
-# memory-clause strategy speeds the nb 10 / nQ 5 row-shared stage kernel by
+# memory-clause strategy sped the nb 10 / nQ 5 stage kernel by
 # about 2 % and the nb 4 ensemble stage; it slowed the stage transposes, so
 # the nb 4 ones sit in hd_k4_vjp.hip with the default, and the 13-moment
 # units keep the default too
