@@ -690,11 +690,13 @@ __device__ __forceinline__ void column_face(const double* __restrict__ qin, cons
                                           DIR == 0 ? g.dxi : DIR == 1 ? g.dyi : g.dzi, sp, M);
 }
 
-// Waves per SIMD that the registers are held to.
+// Waves per SIMD that the registers are held to.  With more modes than four and
+// stress the sums' LDS leaves room for one workgroup a CU (nbasis 8, 11 fields,
+// 64x64x48 cells: 855 us a step held to two, 760 to one).
 template <int NB, int NQ>
-HD_DEV constexpr int occupancy() { return NB == 4 && NQ == 5 ? 3 : (NB == 10 && NQ >= 11 ? 1 : 2); }
+HD_DEV constexpr int occupancy() { return NB == 4 && NQ == 5 ? 3 : (NB > 4 && NQ >= 11 ? 1 : 2); }
 
-inline int stage_occupancy(int nb, int nq) { return nb == 4 && nq == 5 ? 3 : (nb == 10 && nq >= 11 ? 1 : 2); }
+inline int stage_occupancy(int nb, int nq) { return nb == 4 && nq == 5 ? 3 : (nb > 4 && nq >= 11 ? 1 : 2); }
 
 // Cost of items of zc planes on `resident` workgroups, in planes: rounds times
 // an item's length, its start (the first face below in z and the first loads)
