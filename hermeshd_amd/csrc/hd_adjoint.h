@@ -18,12 +18,18 @@
 // its active set and factors frozen at the forward values: the factors that
 // scaled the modes scale the cotangent.
 //
-// The point functions are differentiated by hand: pr::flux (physical flux
-// from primitives) and pr::hllc (Batten HLLC with Davis speeds), each
-// recomputing its forward intermediates and sweeping them backwards.  Branch
-// decisions (wave-speed selection, min/max, floors, boundary-ghost choices)
-// are those of the forward evaluation at the same state.  The stochastic
-// stress and the Roe solver have no adjoint here.
+// The point functions are differentiated by hand: the physical flux from
+// primitives, Batten's HLLC with Davis speeds and the Roe solver
+// (roe_point_vjp, hd_physics.h), each recomputing its forward intermediates and
+// sweeping them backwards.  The traces (sg::signed_coeffs, sg::eval_point) and
+// HLLC's speeds and branch (pr::side, pr::hllc_speeds) are the forward kernel's
+// own functions: with stress HLLC's flux jumps where the contact speed changes
+// sign, so the transpose must be of the branch that the forward stage took.
+// The pressure floor and Roe's |eigenvalues| switch continuously and follow the
+// transpose's own arithmetic (within rounding of the switch either one-sided
+// derivative may be taken), as does Roe's test for a sound speed at all, which
+// no state of positive pressure comes near.  The stochastic stress
+// has no adjoint here.
 #pragma once
 #include "hd_stage.h"
 
@@ -87,7 +93,7 @@ __device__ __forceinline__ void flux13_vjp(const Phys& ph, const double* Q, cons
     bQ[RH] += -s.ri * s.ri * bri;
 }
 
-// reverse of pr::prim + pr::flux<NQ,DIR>: bF (cotangent of F) -> bQ (+=)
+// reverse of pr::prim and the physical flux of direction DIR: bF (cotangent of F) -> bQ (+=)
 template <int NQ, int DIR>
 __device__ __forceinline__ void flux_vjp(const Phys& ph, const double* Q, const pr::Prim& s, const double* bF,
                                          double* bQ) {
@@ -147,32 +153,21 @@ __device__ __forceinline__ void flux_vjp(const Phys& ph, const double* Q, const 
 // -> bQL, bQR (+=, Euler fields), bFL, bFR (+=, Euler fields).  Returns false
 // when no branch applied (out kept the central flux).
 template <int DIR>
-__device__ __forceinline__ bool hllc_vjp(const Phys& ph, const double* QL, const pr::Prim& L, const double* QR,
-                                         const pr::Prim& R, const double* mu, double* bQL, double* bQR, double* bFL,
-                                         double* bFR) {
+__device__ __forceinline__ bool hllc_vjp(const Phys& ph, const double* QL, const double* QR, const double* mu,
+                                         double* bQL, double* bQR, double* bFL, double* bFR) {
     constexpr int IP = MX + DIR, I1 = MX + (DIR + 1) % 3, I2 = MX + (DIR + 2) % 3;
-    // ---- forward, as pr::face_flux
+    // the forward flux's own speeds and branch
     const double rL = QL[RH], rR = QR[RH];
-    const double uL = L.u[DIR], uR = R.u[DIR];
+    const pr::Side L = pr::side(ph, QL), R = pr::side(ph, QR);
+    const pr::HllcSpeeds w = pr::hllc_speeds<DIR>(ph, rL, L, rR, R);
+    const double uL = L.u[DIR], uR = R.u[DIR], pL = L.p, pR = R.p;
     const double v2L = L.u[0] * L.u[0] + L.u[1] * L.u[1] + L.u[2] * L.u[2];
     const double v2R = R.u[0] * R.u[0] + R.u[1] * R.u[1] + R.u[2] * R.u[2];
-    const double pL = ph.gm1 * (QL[EN] - 0.5 * rL * v2L);
-    const double pR = ph.gm1 * (QR[EN] - 0.5 * rR * v2R);
-    const double cL = sqrt(ph.gamma * pL * L.ri), cR = sqrt(ph.gamma * pR * R.ri);
+    const double cL = w.cL, cR = w.cR, SL = w.SL, SR = w.SR, SM = w.SM, aR = w.aR, aL = w.aL, sm_den = w.den;
     const bool sl_left = (uL - cL) <= (uR - cR);   // fmin picks uL - cL
     const bool sr_right = (uR + cR) >= (uL + cL);  // fmax picks uR + cR
-    const double SL = fmin(uL - cL, uR - cR);
-    const double SR = fmax(uR + cR, uL + cL);
-    const double aR = rR * (SR - uR), aL = rL * (SL - uL);
-    double sm_den = aR - aL;
-    const bool den_floor = (sm_den == 0.0);
-    if (den_floor) sm_den = ph.rh_floor;
-    const double SM = pr::divide(pr::contact_num(aR, uR, aL, uL, pL, pR), sm_den);
-    int sel = -1;
-    if (SL > 0.0) sel = 0;
-    if (SL <= 0.0 && 0.0 < SM) sel = 1;
-    if (SM <= 0.0 && 0.0 <= SR) sel = 2;
-    if (SR < 0.0) sel = 3;
+    const bool den_floor = w.den_floor;
+    const int sel = w.sel;
     if (sel < 0) return false;
     if (sel == 0) {
 #pragma unroll
@@ -289,16 +284,15 @@ __device__ __forceinline__ bool hllc_vjp(const Phys& ph, const double* QL, const
 
 // The Euler fields of the face flux reversed to the cotangents of both sides'
 // physical fluxes (bFL, bFR, set) and of their states through the solver
-// (bQL, bQR, +=).  L, R: the sides' velocities and densities.
+// (bQL, bQR, +=).
 template <int RM, int DIR>
-__device__ __forceinline__ void riemann_vjp(const Phys& ph, const double* QL, const pr::Prim& L, const double* QR,
-                                            const pr::Prim& R, const double* mu, double* bQL, double* bQR,
-                                            double* bFL, double* bFR) {
+__device__ __forceinline__ void riemann_vjp(const Phys& ph, const double* QL, const double* QR, const double* mu,
+                                            double* bQL, double* bQR, double* bFL, double* bFR) {
 #pragma unroll
     for (int f = 0; f < 5; f++) { bFL[f] = 0.5 * mu[f]; bFR[f] = 0.5 * mu[f]; }
     if constexpr (RM == RIEMANN_HLLC) {
         double zL[5] = {0., 0., 0., 0., 0.}, zR[5] = {0., 0., 0., 0., 0.};
-        if (hllc_vjp<DIR>(ph, QL, L, QR, R, mu, bQL, bQR, zL, zR)) {
+        if (hllc_vjp<DIR>(ph, QL, QR, mu, bQL, bQR, zL, zR)) {
             // HLLC replaced the central flux of rh..en
 #pragma unroll
             for (int f = 0; f < 5; f++) { bFL[f] = zL[f]; bFR[f] = zR[f]; }
@@ -317,13 +311,12 @@ __device__ __forceinline__ void riemann_vjp(const Phys& ph, const double* QL, co
 template <int NQ, int RM, int DIR>
 __device__ __forceinline__ void face_vjp(const Phys& ph, const double* QL, const double* QR, const double* mu,
                                          double* bQL, double* bQR) {
-    const pr::Prim sL = pr::prim<NQ>(ph, QL), sR = pr::prim<NQ>(ph, QR);
     double bFL[NQ], bFR[NQ];
 #pragma unroll
     for (int f = 5; f < NQ; f++) { bFL[f] = 0.5 * mu[f]; bFR[f] = 0.5 * mu[f]; }
-    riemann_vjp<RM, DIR>(ph, QL, sL, QR, sR, mu, bQL, bQR, bFL, bFR);
-    flux_vjp<NQ, DIR>(ph, QL, sL, bFL, bQL);
-    flux_vjp<NQ, DIR>(ph, QR, sR, bFR, bQR);
+    riemann_vjp<RM, DIR>(ph, QL, QR, mu, bQL, bQR, bFL, bFR);
+    flux_vjp<NQ, DIR>(ph, QL, pr::prim<NQ>(ph, QL), bFL, bQL);
+    flux_vjp<NQ, DIR>(ph, QR, pr::prim<NQ>(ph, QR), bFR, bQR);
 }
 
 // ------------------------------------------------------------ limiter ----
@@ -500,9 +493,9 @@ __device__ __forceinline__ void face_vjp_cell(const double* __restrict__ q, cons
     constexpr int NK = fz::face_nk<NB>();
     const auto& FP = fz::face_poly<NB>();
     double ko[NQ][NK], kn[NQ][NK], ln[NQ][NK];
-    // both sides' traces with the forward kernel's arithmetic, so that every
+    // both sides' traces by the forward kernel's functions, so that every
     // Riemann branch is taken as in the forward stage
-    fz::face_coeffs<NB, NQ, DIR, SIDE, NK>(m, ko);
+    sg::signed_coeffs<NB, NQ, DIR, NK>(m, SIDE ? 1.0 : -1.0, ko);
     if (!ext) {
         int an = SIDE ? a + 1 : a - 1;
         if (an < 0) an += n_ax;
@@ -512,7 +505,7 @@ __device__ __forceinline__ void face_vjp_cell(const double* __restrict__ q, cons
                                  : (cp.c + (long)(an - cp.k) * g.nx * g.ny);
         double nm[NQ][NB], nl[NQ][NB];
         fz::load_modes<NB, NQ>(q, g, cn, nm);
-        fz::face_coeffs<NB, NQ, DIR, 1 - SIDE, NK>(nm, kn);
+        sg::signed_coeffs<NB, NQ, DIR, NK>(nm, SIDE ? -1.0 : 1.0, kn);
         load_lp<NB, NQ>(lam, g, cn, scale, faci, faciq, nl);
         lift_coeffs<NB, NQ, DIR, 1 - SIDE, NK>(nl, ln);
     }
@@ -520,9 +513,7 @@ __device__ __forceinline__ void face_vjp_cell(const double* __restrict__ q, cons
     if (ext && bc == BC_OUTFLOW && !(DIR == 0 && SIDE == 1)) {
         double v = 0.;
         for (int p = 0; p < NF; p++) {
-            double s = 0.;
-#pragma unroll
-            for (int r = 0; r < NB; r++) s += T.bf[DIR][SIDE][p][r] * m[MX + DIR][r];
+            const double s = sg::eval_one<NK>(ko[MX + DIR], FP.b[p]);
             v = (p == 0) ? s : (SIDE ? fmin(v, s) : fmax(v, s));
         }
         zero_normal = SIDE ? (v < 0.0) : (v > 0.0);
@@ -530,7 +521,7 @@ __device__ __forceinline__ void face_vjp_cell(const double* __restrict__ q, cons
 #pragma unroll 1
     for (int p = 0; p < NF; p++) {
         double own[NQ], oth[NQ], mu[NQ];
-        fz::face_eval<NQ, NK>(ko, FP.b[p], own);
+        sg::eval_point<NQ, NK>(ko, FP.b[p], own);
 #pragma unroll
         for (int f = 0; f < NQ; f++) {
             double t = 0.;
@@ -540,7 +531,7 @@ __device__ __forceinline__ void face_vjp_cell(const double* __restrict__ q, cons
         }
         bool flip_mx = false;
         if (!ext) {
-            fz::face_eval<NQ, NK>(kn, FP.b[p], oth);
+            sg::eval_point<NQ, NK>(kn, FP.b[p], oth);
 #pragma unroll
             for (int f = 0; f < NQ; f++) {
                 double t = ln[f][0] * FP.wb[p][0];
@@ -1079,7 +1070,7 @@ __device__ __forceinline__ void load_neighbours(double* kn, const double* __rest
                 m[0][r] = q[o];
                 l[0][r] = lam[o];
             }
-            fz::face_coeffs<NB, 1, DIR, 1 - SIDE, NK>(m, K);
+            sg::signed_coeffs<NB, 1, DIR, NK>(m, SIDE ? -1.0 : 1.0, K);
             lift_coeffs<NB, 1, DIR, 1 - SIDE, NK>(l, L);
             const double fac = b * (NQ == 13 && f >= T_QX ? faciq : (f >= PXX ? faci : 1.0));
 #pragma unroll
@@ -1111,25 +1102,18 @@ __device__ __forceinline__ void face_point_vjp(double* kn, const double* m_s, co
         b[k] = FP.b[p][k];
         wb[k] = dxi_d * FP.wb[p][k];
     }
-    // field f of the cell's trace (with the forward kernel's arithmetic, so
-    // that every Riemann branch is taken as in the forward stage), of the
+    // field f of the cell's trace (by the forward kernel's functions, so that
+    // every Riemann branch is taken as in the forward stage), of the
     // neighbour's, and of the flux's cotangent
     auto own_at = [&](int f) {
         double m[1][NB], K[1][NK];
 #pragma unroll
         for (int r = 0; r < NB; r++) m[0][r] = m_s[(f * C + lc) * NB + r];
-        fz::face_coeffs<NB, 1, DIR, SIDE, NK>(m, K);
-        double s = K[0][0];
-#pragma unroll
-        for (int k = 1; k < NK; k++) s += K[0][k] * b[k];
-        return s;
+        sg::signed_coeffs<NB, 1, DIR, NK>(m, SIDE ? 1.0 : -1.0, K);
+        return sg::eval_one<NK>(K[0], b);
     };
     auto other_at = [&](int f) {
-        const double* const k = kn + (f * C + lc) * NK;
-        double s = k[0];
-#pragma unroll
-        for (int e = 1; e < NK; e++) s += k[e] * b[e];
-        return s;
+        return sg::eval_one<NK>(kn + (f * C + lc) * NK, b);
     };
     auto mu_at = [&](int f) {
         double l[1][NB], L[1][NK];
@@ -1193,11 +1177,8 @@ __device__ __forceinline__ void face_point_vjp(double* kn, const double* m_s, co
     // face_vjp in parts (the Riemann solver's Euler fields, the cell's own
     // flux, at a boundary the ghost's), so that no part holds all that the
     // point has
-    {
-        const pr::Prim so = pr::prim<5>(ph, own), st = pr::prim<5>(ph, oth);
-        riemann_vjp<RM, DIR>(ph, SIDE ? own : oth, SIDE ? so : st, SIDE ? oth : own, SIDE ? st : so, mu,
-                             SIDE ? bo : bt, SIDE ? bt : bo, SIDE ? bFo : bFt, SIDE ? bFt : bFo);
-    }
+    riemann_vjp<RM, DIR>(ph, SIDE ? own : oth, SIDE ? oth : own, mu, SIDE ? bo : bt, SIDE ? bt : bo,
+                         SIDE ? bFo : bFt, SIDE ? bFt : bFo);
     sg::section();
 #pragma unroll
     for (int f = 5; f < NQ; f++) {
@@ -1380,8 +1361,8 @@ __device__ __forceinline__ void face13_vjp(double* __restrict__ lds, const doubl
             l0[0][r] = lam[o + cl];
             l1[0][r] = lam[o + cr];
         }
-        fz::face_coeffs<NB, 1, DIR, 1, NK>(m0, K0);
-        fz::face_coeffs<NB, 1, DIR, 0, NK>(m1, K1);
+        sg::signed_coeffs<NB, 1, DIR, NK>(m0, 1.0, K0);
+        sg::signed_coeffs<NB, 1, DIR, NK>(m1, -1.0, K1);
         lift_coeffs<NB, 1, DIR, 1, NK>(l0, L0);
         lift_coeffs<NB, 1, DIR, 0, NK>(l1, L1);
         double* const k = lds + it * NK;
@@ -1404,9 +1385,12 @@ __device__ __forceinline__ void face13_vjp(double* __restrict__ lds, const doubl
             b[e] = FP.b[p][e];
             wb[e] = dxi_d * FP.wb[p][e];
         }
-        // field f of a side's state, or (side 2, with wb) of the flux's cotangent
+        // field f of a side's state (by the forward kernel's functions, so that
+        // every Riemann branch is taken as in the forward stage), or (side 2,
+        // with wb) of the flux's cotangent
         auto value = [&](int side, int f, const double (&w)[NK]) {
             const double* const k = lds + ((side * NQ + f) * F + l) * NK;
+            if (side < 2) return sg::eval_one<NK>(k, w);
             double s = k[0] * w[0];
 #pragma unroll
             for (int e = 1; e < NK; e++) s += k[e] * w[e];
@@ -1428,7 +1412,7 @@ __device__ __forceinline__ void face13_vjp(double* __restrict__ lds, const doubl
             QR[f] = value(1, f, b);
             mu[f] = value(2, f, wb);
         }
-        riemann_vjp<RM, DIR>(ph, QL, pr::prim<5>(ph, QL), QR, pr::prim<5>(ph, QR), mu, bL, bR, bFL, bFR);
+        riemann_vjp<RM, DIR>(ph, QL, QR, mu, bL, bR, bFL, bFR);
         sg::section();
 #pragma unroll
         for (int f = 5; f < NQ; f++) {

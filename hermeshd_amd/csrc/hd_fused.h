@@ -140,8 +140,9 @@ __device__ __forceinline__ const FaceTab<10, 3>& face_tab<10>() { return c_face_
 // with (dr, dc) in {(0,0), (1,0), (0,1), (1,1), (2,0), (0,2)}.  A side's
 // trace is therefore sum_k K_k b_k(p) with NK = 3 (nb 4), 4 (nb 8) or 6
 // (nb 10) coefficients K_k = sum of +-m_r over the modes of pair k: NK
-// products per point instead of NB.  Both cells of a face evaluate a side's
-// trace with this same arithmetic, so they still agree bitwise.
+// products per point instead of NB.  Coefficients and values come from
+// sg::signed_coeffs and sg::eval_point everywhere, so that all that evaluate a
+// side's trace agree bitwise.
 template <int NB>
 HD_DEV constexpr int face_nk() { return NB == 10 ? 6 : (NB == 8 ? 4 : 3); }
 HD_DEV constexpr int pair_index(int dr, int dc) {
@@ -181,39 +182,6 @@ template <>
 __device__ __forceinline__ const FacePoly<8, 2>& face_poly<8>() { return c_fpoly_8; }
 template <>
 __device__ __forceinline__ const FacePoly<10, 3>& face_poly<10>() { return c_fpoly_10; }
-
-// K[f][k] of the side SIDE (0: coordinate -1, 1: +1) of a DIR face of a cell with modes m
-template <int NB, int NQ, int DIR, int SIDE, int NK>
-__device__ __forceinline__ void face_coeffs(const double (&m)[NQ][NB], double (&K)[NQ][NK]) {
-#pragma unroll
-    for (int f = 0; f < NQ; f++) {
-#pragma unroll
-        for (int k = 0; k < NK; k++) {
-            double s = 0.;
-            bool first = true;
-#pragma unroll
-            for (int r = 0; r < NB; r++) {
-                if (pair_index(deg<NB>(r, row_axis(DIR)), deg<NB>(r, col_axis(DIR))) != k) continue;
-                const bool neg = Lface(deg<NB>(r, DIR), SIDE) < 0.0;
-                if (first) s = neg ? -m[f][r] : m[f][r];
-                else s = neg ? s - m[f][r] : s + m[f][r];
-                first = false;
-            }
-            K[f][k] = s;
-        }
-    }
-}
-
-template <int NQ, int NK>
-__device__ __forceinline__ void face_eval(const double (&K)[NQ][NK], const double* __restrict__ b, double* out) {
-#pragma unroll
-    for (int f = 0; f < NQ; f++) {
-        double s = K[f][0];
-#pragma unroll
-        for (int k = 1; k < NK; k++) s += K[f][k] * b[k];
-        out[f] = s;
-    }
-}
 
 // Keeps the scheduler from interleaving fully unrolled quadrature points,
 // which would stretch live ranges past the register file.

@@ -100,6 +100,56 @@ __device__ __forceinline__ double root(double x) {
     return x == 0.0 ? x : g;
 }
 
+// 1/rho, the velocity and the pressure (no floor) of one side of a face.  Shared
+// with the transpose, and rounded operation by operation, so that both see the
+// same values whatever the compiler makes of the code around them.
+struct Side {
+    double ri, u[3], p;
+};
+__device__ __forceinline__ Side side(const Phys& ph, const double* Q) {
+#pragma clang fp contract(off)
+    Side s;
+    s.ri = rcp(Q[RH]);
+#pragma unroll
+    for (int a = 0; a < 3; a++) s.u[a] = Q[MX + a] * s.ri;
+    s.p = ph.gm1 * fma(-0.5, fma(Q[MX], s.u[0], fma(Q[MY], s.u[1], Q[MZ] * s.u[2])), Q[EN]);
+    return s;
+}
+
+// HLLC's speeds and the branch they select (Batten 1997 with Davis speeds, the
+// order of the branches hllc_point's): the last true of SL > 0 (left), SL <= 0 <
+// SM (left star), SM <= 0 <= SR (right star), SR < 0 (right); none of them with
+// NaN speeds.  One function for the flux and its transpose: at rest the contact
+// speed is a difference of equal pressures, and with stress the flux jumps where
+// it changes sign.
+struct HllcSpeeds {
+    double cL, cR, SL, SR, SM, aL, aR, den;  // SM = contact_num / den
+    bool den_floor;
+    int sel;  // 0 left, 1 left star, 2 right star, 3 right, -1 none
+};
+template <int DIR>
+__device__ __forceinline__ HllcSpeeds hllc_speeds(const Phys& ph, double rL, const Side& L, double rR, const Side& R) {
+#pragma clang fp contract(off)
+    HllcSpeeds w;
+    const double nL = L.u[DIR], nR = R.u[DIR];
+    w.cL = root(ph.gamma * L.p * L.ri);
+    w.cR = root(ph.gamma * R.p * R.ri);
+    w.SL = fmin(nL - w.cL, nR - w.cR);
+    w.SR = fmax(nR + w.cR, nL + w.cL);
+    w.aR = rR * (w.SR - nR);
+    w.aL = rL * (w.SL - nL);
+    w.den = w.aR - w.aL;
+    w.den_floor = w.den == 0.0;
+    if (w.den_floor) w.den = ph.rh_floor;
+    w.SM = divide(contact_num(w.aR, nR, w.aL, nL, L.p, R.p), w.den);
+    w.sel = -1;
+    if (w.SL > 0.0) w.sel = 0;
+    if (w.SL <= 0.0 && 0.0 < w.SM) w.sel = 1;
+    if (w.SM <= 0.0 && 0.0 <= w.SR) w.sel = 2;
+    if (w.SR < 0.0) w.sel = 3;
+    return w;
+}
+
 // Roe flux (roe_point: Eulderink and Mellema, half the thermal enthalpy) from
 // the traces' velocities, pressures and 1/rho, with refined reciprocals and
 // roots; out holds 0.5 (FL + FR) on entry.
@@ -148,18 +198,15 @@ __device__ __forceinline__ void roe_diss(const Phys& ph, const double* QL, const
 // the stochastic stress.
 // HLLC keeps density, velocity and pressure of both sides, selects one, and
 // forms the conserved values and the flux of that side only (few values are
-// live at a time; the momentum and energy come back to rounding).  HLLC after
-// Batten 1997 with Davis speeds, the order of the branches hllc_point's.
+// live at a time; the momentum and energy come back to rounding).
 template <int NQ, int DIR, int RM, bool NZ>
 __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, const double* QR, const double* S,
                                           double* F) {
     constexpr int IP = MX + DIR;
     const double rL = QL[RH], rR = QR[RH];
-    const double riL = rcp(rL), riR = rcp(rR);
-    const double uL[3] = {QL[MX] * riL, QL[MY] * riL, QL[MZ] * riL};
-    const double uR[3] = {QR[MX] * riR, QR[MY] * riR, QR[MZ] * riR};
-    const double pL = ph.gm1 * fma(-0.5, fma(QL[MX], uL[0], fma(QL[MY], uL[1], QL[MZ] * uL[2])), QL[EN]);
-    const double pR = ph.gm1 * fma(-0.5, fma(QR[MX], uR[0], fma(QR[MY], uR[1], QR[MZ] * uR[2])), QR[EN]);
+    const Side L = side(ph, QL), R = side(ph, QR);
+    const double riL = L.ri, riR = R.ri, pL = L.p, pR = R.p;
+    const double (&uL)[3] = L.u, (&uR)[3] = R.u;
     if constexpr (NQ >= 11) {
 #pragma unroll
         for (int a = 0; a < 3; a++) F[5 + a] = 0.5 * (uL[a] + uR[a]);
@@ -196,20 +243,12 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
         if constexpr (RM == RIEMANN_ROE) roe_diss<DIR>(ph, QL, QR, riL, riR, uL, uR, pL, pR, F);
         return;
     }
-    const double nL = uL[DIR], nR = uR[DIR];
-    const double cL = root(ph.gamma * pL * riL), cR = root(ph.gamma * pR * riR);
-    const double SL = fmin(nL - cL, nR - cR), SR = fmax(nR + cR, nL + cL);
-    const double aR = rR * (SR - nR), aL = rL * (SL - nL);
-    double sm_den = aR - aL;
-    if (sm_den == 0.0) sm_den = ph.rh_floor;
-    const double SM = divide(contact_num(aR, nR, aL, nL, pL, pR), sm_den);
-    const double pstar = fma(-aL, nL - SM, pL);  // Eq. (36)
-    // the last true of: SL > 0 (left), SL <= 0 < SM (left star),
-    // SM <= 0 <= SR (right star), SR < 0 (right)
-    const bool s3 = SR < 0.0, s2 = SM <= 0.0 && 0.0 <= SR, s1 = SL <= 0.0 && 0.0 < SM, s0 = SL > 0.0;
+    const HllcSpeeds w = hllc_speeds<DIR>(ph, rL, L, rR, R);
+    const double SL = w.SL, SR = w.SR, SM = w.SM;
+    const double pstar = fma(-w.aL, uL[DIR] - SM, pL);  // Eq. (36)
     // NaN speeds: the central flux (the reference's default), before the
     // selection so that only one side's values are live after it
-    const bool none = !(s0 || s1 || s2 || s3);
+    const bool none = w.sel < 0;
     if (__builtin_expect(none, 0)) {
         double FL[5], FR[5];
         side_flux(QL, uL, pL, QL + 5, FL);
@@ -217,7 +256,7 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
 #pragma unroll
         for (int e = 0; e < 5; e++) F[e] = 0.5 * (FL[e] + FR[e]);
     }
-    const bool right = s3 || s2;
+    const bool right = w.sel >= 2;
     const double r = right ? rR : rL, p = right ? pR : pL, Sk = right ? SR : SL;
     double u[3], P3[4] = {0., 0., 0., 0.}, Q[5], f[5];
 #pragma unroll
@@ -232,7 +271,7 @@ __device__ __forceinline__ void face_flux(const Phys& ph, const double* QL, cons
     for (int a = 0; a < 3; a++) Q[MX + a] = r * u[a];
     Q[EN] = fma(0.5, fma(Q[MX], u[0], fma(Q[MY], u[1], Q[MZ] * u[2])), p * ph.gm1i);
     side_flux(Q, u, p, P3, f);
-    if (s3 || !(s2 || s1)) {  // supersonic: the side's own flux
+    if (w.sel == 0 || w.sel == 3) {  // supersonic: the side's own flux
 #pragma unroll
         for (int e = 0; e < 5; e++) F[e] = f[e];
         return;

@@ -161,19 +161,25 @@ struct FacePoint {
         b[0] = 1.0;
     }
 };
+// A face polynomial at a point.  The transposes evaluate theirs by these too
+// (fz::face_poly holds the same b_k): explicit fma, so that both sides of a
+// Riemann problem are bitwise the same there.
+template <int NK>
+__device__ __forceinline__ double eval_one(const double* K, const double* b) {
+    double s = K[0];
+#pragma unroll
+    for (int k = 1; k < NK; k++) s = fma(K[k], b[k], s);
+    return s;
+}
 template <int NM, int NK>
 __device__ __forceinline__ void eval_point(const double (&K)[NM][NK], const double (&b)[NK], double* out) {
 #pragma unroll
-    for (int e = 0; e < NM; e++) {
-        double s = K[e][0];
-#pragma unroll
-        for (int k = 1; k < NK; k++) s = fma(K[e][k], b[k], s);
-        out[e] = s;
-    }
+    for (int e = 0; e < NM; e++) out[e] = eval_one<NK>(K[e], b);
 }
 
 // Face-polynomial coefficients of a DIR face from a cell's modes: the modes
-// odd along DIR enter with sign sgn (+1 above the cell, -1 below).
+// odd along DIR enter with sign sgn (+1 above the cell, -1 below).  No product
+// but sgn's, so that nothing here can be contracted in two ways.
 template <int NB, int NM, int DIR, int NK>
 __device__ __forceinline__ void signed_coeffs(const double (&m)[NM][NB], double sgn, double (&K)[NM][NK]) {
 #pragma unroll
@@ -227,9 +233,7 @@ __device__ __forceinline__ void face_moments(const double* __restrict__ q, const
             double v = 0.;
             for (int p = 0; p < NF; p++) {
                 const FacePoint<NB, QP> fp(p / QP, p % QP);
-                double s = KL[MX + DIR][0];
-#pragma unroll
-                for (int k = 1; k < NK; k++) s = fma(KL[MX + DIR][k], fp.b[k], s);
+                const double s = eval_one<NK>(KL[MX + DIR], fp.b);
                 v = (p == 0) ? s : (extR ? fmin(v, s) : fmax(v, s));
             }
             zero_normal = extR ? (v < 0.0) : (v > 0.0);
