@@ -11,12 +11,17 @@
 //           two Gauss points) of the volume integral;
 //   part 1: the face above in y, and the second third (half);
 //   part 2: the faces in x, and the rest of the volume integral (with two
-//           points: the terms of the modes and of the step-start state);
+//           points: none);
 //   part 3: the face above in z (the one below is the last plane's), then the
-//           sum of all parts, the limiter and the stores.
+//           sum of all parts, the time step, the limiter and the stores.
 // Every face is evaluated once, but for the faces in y (by the tiles on both
-// sides) and the first one of a workgroup in z.  The parts are equally long,
-// and meet once per plane.  Which wave takes which part rotates with the
+// sides) and the first one of a workgroup in z.  The parts meet once per plane;
+// part 3 lets go of the others' sums before it takes the time step.
+// Part 3 alone holds terms of the state: with the state in one of the partial
+// sums each later addition rounded it once more (a step's error 1.3e-16 of the
+// state against 0.4e-16 to 0.8e-16), for 0 to 10 % less time (vortex 1363 us a
+// step against 1438, linear 3921 and 3950, 13 moments 6928 and 7052, channel
+// 23.2 and 25.7).  Which wave takes which part rotates with the
 // workgroup, so that what inequality there is does not always meet one SIMD.
 //
 // Fields of a face: the stress fields' flux is linear in the velocity, and a
@@ -114,9 +119,15 @@ __device__ __forceinline__ void pin(double (&v)[B]) {
     for (int b = 0; b < B; b++) asm volatile("" : "+v"(v[b]));
 }
 
-// LDS of a workgroup: two partial sums of a cell's output, one face's moments
+// LDS of a workgroup: two partial sums of a cell's right-hand side, one face's moments
 template <int NB, int NQ>
 HD_DEV constexpr int lds_doubles() { return (2 * NB * NQ + face_nm(NQ) * fz::face_nk<NB>()) * 64; }
+// k_stage_wide has a CU to itself: the cells' state and step start in its LDS
+// too, where they fit.
+template <int NB, int NQ>
+HD_DEV constexpr bool wide_staged() { return (lds_doubles<NB, NQ>() + 2 * NB * NQ * 64) * 8 <= 160 * 1024 - 64; }
+template <int NB, int NQ>
+HD_DEV constexpr int wide_lds_doubles() { return lds_doubles<NB, NQ>() + (wide_staged<NB, NQ>() ? 2 * NB * NQ * 64 : 0); }
 
 // ------------------------------------------------------------- faces -------
 // The modes that a DIR face needs of cell c.
@@ -469,76 +480,55 @@ __device__ __forceinline__ void volume_moments(const double* __restrict__ q, con
     }
 }
 
-// The output of one stage is linear in the right-hand side: with
-// v = wn q_n + wv fac (m + dt (volume + sources)), each face adds
-// wv fac dt 0.25 cb_r times its lift (advance_time_level and the SSP
-// combination, src/integrator.f90:62-86,210-232).
+// advance_time_level and the SSP combination (src/integrator.f90:62-86,
+// 210-232) of a value m of the stage's input, its right-hand side and the
+// step-start value q0: v = fac (m + dt rhs), out = wn q0 + wv v.  The sums of
+// the right-hand side hold no term of the state, so that the state is rounded
+// where the formula rounds it, and nowhere else: in v, in wn q0 and in the
+// combination.
 struct Weights {
-    double wn;        // of q_n
-    double wm[3], ws[3];  // of m and of the right-hand side: rh..en, stress, heat flux
+    double dt, fac[3];  // of rh..en, stress, heat flux
+    double wn, wv;
+    bool rhs;           // the right-hand side alone
 };
 template <int NQ>
 HD_DEV constexpr int field_class(int f) { return f < 5 ? 0 : (NQ == 13 && f >= T_QX ? 2 : 1); }
 template <int NQ>
 __device__ __forceinline__ Weights stage_weights(const StageParams& sp) {
     Weights w;
+    w.rhs = sp.mode == 1;
+    w.wv = sp.combine == 0 ? 1. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.25 : 2. / 3.));
+    w.wn = sp.combine == 0 ? 0. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.75 : 1. / 3.));
+    w.dt = 0.;
+    w.fac[0] = w.fac[1] = w.fac[2] = 1.;
+    if (w.rhs) return w;
     const double* pdt = sp.dt;
     asm volatile("" : "+s"(pdt));  // read where it is used, not kept in registers across the planes
-    if (sp.mode == 1) {
-        w.wn = 0.;
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            w.wm[i] = 0.;
-            w.ws[i] = 1.;
-        }
-        return w;
-    }
-    const double dt = *pdt;
-    const double wv = sp.combine == 0 ? 1. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.25 : 2. / 3.));
-    w.wn = sp.combine == 0 ? 0. : (sp.combine == 1 ? 0.5 : (sp.combine == 2 ? 0.75 : 1. / 3.));
-    w.wm[0] = w.wm[1] = w.wm[2] = wv;
+    w.dt = *pdt;
     if constexpr (NQ >= 11) {
         if (sp.ivis == 1) {
-            w.wm[1] = wv * (1. / (1. + dt * sp.coll));
-            if constexpr (NQ == 13) w.wm[2] = wv * (1. / (1. + dt * sp.coll_q));
+            w.fac[1] = 1. / (1. + w.dt * sp.coll);
+            if constexpr (NQ == 13) w.fac[2] = 1. / (1. + w.dt * sp.coll_q);
         }
     }
-#pragma unroll
-    for (int i = 0; i < 3; i++) w.ws[i] = w.wm[i] * dt;
     return w;
 }
-
 template <int NB, int NQ>
-__device__ __forceinline__ void load_start(const double* __restrict__ qin, const double* __restrict__ qn,
-                                           const Grid& g, const Weights& w, long c, int f, double (&m)[NB],
-                                           double (&q0)[NB]) {
-    const long st = (long)NQ * g.N;
-    gptr p = plane_ptr(qin, g.N, f, c);
+__device__ __forceinline__ void load_field(const double* __restrict__ q, const Grid& g, long c, int f, double (&m)[NB]) {
+    gptr p = plane_ptr(q, g.N, f, c);
 #pragma unroll
     for (int r = 0; r < NB; r++) {
         m[r] = *p;
-        step(p, st);
-    }
-    if (w.wn != 0.) {
-        p = plane_ptr(qn, g.N, f, c);
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            q0[r] = *p;
-            step(p, st);
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < NB; r++) q0[r] = 0.;
+        step(p, (long)NQ * g.N);
     }
 }
-// t (without 0.25 cb_r) becomes wn q_n + wm m + ws (t + sources)
+// The right-hand side t of field f becomes its output: sources, time step,
+// combination with the step-start values q0.
 template <int NB, int NQ>
-__device__ __forceinline__ void start_field(const double* __restrict__ qin, const Grid& g, const StageParams& sp,
-                                            const Weights& w, long c, int f, const double (&m)[NB],
-                                            const double (&q0)[NB], double (&t)[NB]) {
+__device__ __forceinline__ void advance_field(const double* __restrict__ qin, const Grid& g, const StageParams& sp,
+                                              const Weights& w, long c, int f, const double (&m)[NB],
+                                              const double (&q0)[NB], double (&t)[NB]) {
     const long st = (long)NQ * g.N;
-#pragma unroll
-    for (int r = 0; r < NB; r++) t[r] *= 0.25 * fz::cbasis<NB>(r);
     // sources (src/sources.f90:12-84): ivis 0 relaxes the stress explicitly
     // (-coll*P, projected exactly in modal space); body force rho*g, m.g
     if constexpr (NQ >= 11) {
@@ -563,13 +553,35 @@ __device__ __forceinline__ void start_field(const double* __restrict__ qin, cons
             step(p, st);
         }
     }
-    const double wm = w.wm[field_class<NQ>(f)], ws = w.ws[field_class<NQ>(f)];
+    if constexpr (NB == 10) {
+        // selects: branches would cost registers (13 moments, 96^3 cells: 7050 us
+        // a step against 7330)
+        const double fac = w.fac[field_class<NQ>(f)];
 #pragma unroll
-    for (int r = 0; r < NB; r++) t[r] = fma(ws, t[r], fma(wm, m[r], w.wn * q0[r]));
+        for (int r = 0; r < NB; r++) {
+            double v = fma(w.dt, t[r], m[r]);
+            if (f >= 5) v *= fac;
+            t[r] = w.rhs ? t[r] : (w.wn != 0. ? fma(w.wv, v, w.wn * q0[r]) : v);
+        }
+    } else {
+        // branches, which the empty asm keeps from becoming selects (channel of
+        // 64x128 cells: 25.7 us a step against 26.5)
+        if (w.rhs) return;
+#pragma unroll
+        for (int r = 0; r < NB; r++) t[r] = fma(w.dt, t[r], m[r]);
+        if (f >= 5 && sp.ivis == 1) {
+            asm volatile("");
+#pragma unroll
+            for (int r = 0; r < NB; r++) t[r] *= w.fac[field_class<NQ>(f)];
+        }
+        if (w.wn != 0.) {
+            asm volatile("");
+#pragma unroll
+            for (int r = 0; r < NB; r++) t[r] = fma(w.wv, t[r], w.wn * q0[r]);
+        }
+    }
 }
 
-// t[r] += the lift of a face's moments in direction D, without 0.25 cb_r: the
-// face below (LO) or above the cell.
 template <int NB, int NK, int D, bool LO>
 __device__ __forceinline__ void lift(const double (&m)[NK], double (&t)[NB]) {
 #pragma unroll
@@ -610,31 +622,14 @@ __device__ __forceinline__ void part_field(const Phys& ph, const double (&t)[5][
     }
 }
 
-// The output of one cell: NaN check, the next stage's limiter, stores.
-template <int NB, int QP, int NQ>
-__device__ __forceinline__ void store_cell(double* __restrict__ qout, const Grid& g, const StageParams& sp, long c,
-                                           long bad_id, bool live, double (&v)[NQ][NB]) {
-    bool bad = false;
-    if (sp.mode != 1) {
+template <int NB, int NQ>
+__device__ __forceinline__ void store_field(double* __restrict__ qout, const Grid& g, long c, int f,
+                                            const double (&v)[NB]) {
+    gptr_w p = (gptr_w)plane_ptr(qout, g.N, f, c);
 #pragma unroll
-        for (int f = 0; f < NQ; f++) bad |= v[f][0] != v[f][0];
-        // When this output is the next stage's input, apply that stage's limiter
-        // here: the reference limits the stage input in place before anything
-        // reads it (src/integrator.f90:106-113), so the stored values are the same.
-        if (sp.limit_out) fz::limit_cell<NB, QP, NQ>(v, sp.lp);
-    }
-    if (!live) return;
-    gptr_w p = (gptr_w)plane_ptr(qout, g.N, 0, c);
-#pragma unroll
-    for (int r = 0; r < NB; r++)
-#pragma unroll
-        for (int f = 0; f < NQ; f++) {
-            *p = v[f][r];
-            step(p, g.N);
-        }
-    if (bad) {
-        atomicOr(sp.err, 1);
-        atomicMin(sp.bad, (unsigned long long)bad_id);
+    for (int r = 0; r < NB; r++) {
+        *p = v[r];
+        step(p, (long)NQ * g.N);
     }
 }
 
@@ -734,8 +729,9 @@ inline int stage_planes(long tiles, int nz, long cus) {
 
 // What the waves of a workgroup share.
 struct Shared {
-    double *r0, *r1;  // partial sums of the outputs: parts 2 and 0, part 1
+    double *r0, *r1;  // partial sums of the right-hand sides: parts 2 and 0, part 1
     double* z;        // moments of the face below in z
+    double* m;        // k_stage_wide: the cells' state and step start
     int* flags;       // planes whose sums part 3 has read; planes that part 2 has written
 };
 __device__ __forceinline__ void raise(int* flag, int n) {
@@ -756,18 +752,11 @@ __device__ __forceinline__ double next_lane(double x, int addr) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Which part adds field f's terms of the modes and the step-start state: part
-// 2, which has no share of the two-point volume rule, or parts 0 and 1.
-template <int QP>
-HD_DEV constexpr bool starts(int part, int f) { return QP == 2 ? part == 2 : part == (f & 1); }
-
 // Parts 0-2 of plane k (p planes after the workgroup's first): one direction's
-// face, a share of the volume integral, and some fields' terms of the modes
-// and the step-start state; the sum to LDS.
+// face and a share of the volume integral; the sum to LDS.
 template <int NB, int QP, int NQ, int RM, bool NZ, int PART>
-__device__ __forceinline__ void sum_part(const double* __restrict__ qin, const double* __restrict__ qn, const Grid& g,
-                                         const Phys& ph, const StageParams& sp, unsigned tile, int k, int p,
-                                         const Shared& sh, int lane) {
+__device__ __forceinline__ void sum_part(const double* __restrict__ qin, const Grid& g, const Phys& ph,
+                                         const StageParams& sp, unsigned tile, int k, int p, const Shared& sh, int lane) {
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     constexpr int D = PART == 2 ? 0 : 1;
     constexpr bool VOL = PART < QP;
@@ -827,51 +816,32 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const d
         }
         section();
     }
-    const Weights w = stage_weights<NQ>(sp);
     double* const R = (PART == 1 ? sh.r1 : sh.r0) + lane;
-    // a batch of fields at a time: the loads of its modes and step-start
-    // values together, the first batch's before the wait
-    constexpr int BATCH = NB == 10 && NQ >= 11 ? 4 : (NQ >= 11 ? 6 : 5);
+    // part 2 is done first: it writes, part 0 adds
+    if (PART == 0) await(sh.flags + 1, p + 1);
+    else await(sh.flags, p);
 #pragma unroll
-    for (int f0 = 0; f0 < NQ; f0 += BATCH) {
-        double m[BATCH][NB], q0[BATCH][NB];
+    for (int f = 0; f < NQ; f++) {
+        double v[NB];
+        part_field<NB, NQ, D, VOL>(ph, t, tu, au, f, v);
 #pragma unroll
-        for (int b = 0; b < BATCH; b++)
-            if (f0 + b < NQ && starts<QP>(PART, f0 + b))
-                load_start<NB, NQ>(qin, qn, g, w, c, f0 + b, m[b], q0[b]);
-        if (f0 == 0) {
-            // part 2 is done first: it writes, part 0 adds
-            if (PART == 0) await(sh.flags + 1, p + 1);
-            else await(sh.flags, p);
+        for (int r = 0; r < NB; r++) {
+            double* const x = R + (f * NB + r) * 64;
+            v[r] *= 0.25 * fz::cbasis<NB>(r);
+            *x = PART == 0 ? *x + v[r] : v[r];
         }
-#pragma unroll
-        for (int b = 0; b < BATCH; b++) {
-            const int f = f0 + b;
-            if (f >= NQ) continue;
-            double v[NB];
-            part_field<NB, NQ, D, VOL>(ph, t, tu, au, f, v);
-            if (starts<QP>(PART, f)) {
-                start_field<NB, NQ>(qin, g, sp, w, c, f, m[b], q0[b], v);
-            } else {
-#pragma unroll
-                for (int r = 0; r < NB; r++) v[r] *= w.ws[field_class<NQ>(f)] * (0.25 * fz::cbasis<NB>(r));
-            }
-#pragma unroll
-            for (int r = 0; r < NB; r++) {
-                double* const x = R + (f * NB + r) * 64;
-                *x = PART == 0 ? *x + v[r] : v[r];
-            }
-        }
-        section();
+        if (f % 4 == 3) section();
     }
+    section();
     if (PART == 2) raise(sh.flags + 1, p + 1);
 }
 
 // Part 3 of plane k after its face above in z (moments M, the next plane's
-// face below): once all parts have met, the sum, the next stage's limiter and
-// the stores.
-template <int NB, int QP, int NQ>
-__device__ __forceinline__ void finish_part(double* __restrict__ qout, const Grid& g, const Phys& ph, const StageParams& sp,
+// face below): once all parts have met, the sum, the time step, the next
+// stage's limiter and the stores.
+template <int NB, int QP, int NQ, bool WIDE>
+__device__ __forceinline__ void finish_part(const double* __restrict__ qin, const double* __restrict__ qn,
+                                            double* __restrict__ qout, const Grid& g, const Phys& ph, const StageParams& sp,
                                             unsigned tile, int k, int p, long cell0,
                                             const Shared& sh, int lane, bool same,
                                             double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
@@ -879,11 +849,33 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
     const Column o = column(g, tile, lane);
     const Weights w = stage_weights<NQ>(sp);
     const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
+    // Values of the state and the step start are loaded AHEAD fields before they
+    // are used, the first ones before the parts meet.
+    constexpr bool STAGED = WIDE && wide_staged<NB, NQ>();
+    constexpr int AHEAD = NB == 4 ? 3 : (NB == 8 ? (NQ == 5 ? 2 : 3) : 1), RING = AHEAD + 1;
+    double m[RING][NB], q0[RING][NB];
+    const bool comb = sp.combine != 0 && sp.mode != 1;
+    const double* const q0p = comb ? qn : qin;
+    // the fields past en first: the limiter leaves them alone, so each is stored
+    // as it comes
+    auto load = [&](int i) {
+        if (i >= NQ) return;
+        const int f = (i + 5) % NQ;
+        if constexpr (STAGED) {
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                m[i % RING][r] = sh.m[(f * NB + r) * 64 + lane];
+                q0[i % RING][r] = sh.m[((NQ + f) * NB + r) * 64 + lane];
+            }
+        } else {
+            load_field<NB, NQ>(qin, g, c, f, m[i % RING]);
+            load_field<NB, NQ>(q0p, g, c, f, q0[i % RING]);
+        }
+    };
+    if constexpr (NB < 10 && !STAGED)
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) load(i);
     double v[NQ][NB];
-#pragma unroll
-    for (int f = 0; f < NQ; f++)
-#pragma unroll
-        for (int r = 0; r < NB; r++) v[f][r] = 0.;
     __syncthreads();
     double* const z = sh.z + lane;
     // same: the faces below and above are one (a periodic axis of one cell)
@@ -904,18 +896,28 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
         for (int n = 0; n < NK; n++) z[(e * NK + n) * 64] = M[e][n];
 #pragma unroll
         for (int r = 0; r < NB; r++) {
-            if (e < 5) v[e < 5 ? e : 0][r] = fma(w.ws[0] * (0.25 * fz::cbasis<NB>(r)), s[r], v[e < 5 ? e : 0][r]);
+            if (e < 5) v[e < 5 ? e : 0][r] = (0.25 * fz::cbasis<NB>(r)) * s[r];
             else tu[e < 5 ? 0 : e - 5][r] = s[r];
         }
         if (NB > 4 && e % 2 == 1) section();
     }
+    pin(tu);
+#pragma unroll
+    for (int f = 0; f < 5; f++) pin(v[f]);
+    if constexpr (NB == 10 || STAGED)
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) load(i);
 #pragma unroll
     for (int f = 0; f < NQ; f++) {
+        if (f >= 5) {
+#pragma unroll
+            for (int r = 0; r < NB; r++) v[f][r] = 0.;
+        }
         if constexpr (NQ >= 11) {
 #pragma unroll
             for (int a = 0; a < nscal(NQ); a++) {
                 if (!drives(NQ, f, a, 2)) continue;
-                const double cf = w.ws[field_class<NQ>(f)] * drive_factor(ph, NQ, f, a);
+                const double cf = drive_factor(ph, NQ, f, a);
 #pragma unroll
                 for (int r = 0; r < NB; r++) v[f][r] = fma(cf * (0.25 * fz::cbasis<NB>(r)), tu[a][r], v[f][r]);
             }
@@ -923,15 +925,35 @@ __device__ __forceinline__ void finish_part(double* __restrict__ qout, const Gri
 #pragma unroll
         for (int r = 0; r < NB; r++) {
             const int x = (f * NB + r) * 64 + lane;
-            // the sum that holds the modes last: one rounding at their size
-            if (starts<QP>(1, f)) v[f][r] = (v[f][r] + sh.r0[x]) + sh.r1[x];
-            else v[f][r] = (v[f][r] + sh.r1[x]) + sh.r0[x];
+            v[f][r] += sh.r0[x] + sh.r1[x];
         }
-        if (f % (NB > 4 ? 2 : 4) == 1) section();
+        if (!WIDE && f % (NB > 4 ? 2 : 4) == 1) section();
     }
     pin(v);
     raise(sh.flags, p + 1);
-    store_cell<NB, QP, NQ>(qout, g, sp, c, cell0 + c, o.live, v);
+    section();
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < NQ; i++) {
+        const int f = (i + 5) % NQ;
+        load(i + AHEAD);
+        advance_field<NB, NQ>(qin, g, sp, w, c, f, m[i % RING], q0[i % RING], v[f]);
+        pin(v[f]);
+        bad |= v[f][0] != v[f][0];
+        if (NB > 4 && f >= 5 && o.live) store_field<NB, NQ>(qout, g, c, f, v[f]);
+        if (!WIDE) section();
+    }
+    // When this output is the next stage's input, apply that stage's limiter
+    // here: the reference limits the stage input in place before anything
+    // reads it (src/integrator.f90:106-113), so the stored values are the same.
+    if (sp.limit_out) fz::limit_cell<NB, QP, NQ>(v, sp.lp);
+    if (!o.live) return;
+#pragma unroll
+    for (int f = 0; f < (NB > 4 ? 5 : NQ); f++) store_field<NB, NQ>(qout, g, c, f, v[f]);
+    if (bad && !w.rhs) {
+        atomicOr(sp.err, 1);
+        atomicMin(sp.bad, (unsigned long long)(cell0 + c));
+    }
 }
 
 // One tile over planes [k0, k1), after p0 planes of this workgroup: four waves.
@@ -945,19 +967,19 @@ __device__ __forceinline__ void stage_march(const double* __restrict__ qin, cons
     if (part == 0) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 0>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, 0>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else if (part == 1) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 1>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, 1>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else if (part == 2) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 2>(qin, qn, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else {
@@ -977,10 +999,36 @@ __device__ __forceinline__ void stage_march(const double* __restrict__ qin, cons
 #pragma unroll
                     for (int n = 0; n < NK; n++) sh.z[(e * NK + n) * 64 + lane] = M[e][n];
             } else {
-                finish_part<NB, QP, NQ>(qout, g, ph, sp, tile, k - 1, p0 + k - 1 - k0, cell0, sh, lane, one_z, M);
+                finish_part<NB, QP, NQ, false>(qin, qn, qout, g, ph, sp, tile, k - 1, p0 + k - 1 - k0, cell0, sh, lane, one_z, M);
             }
         }
     }
+}
+
+// k_stage_wide: a plane's state and step start to LDS for part 3, by the part
+// that has least to do: part 2 with two points (no volume), else part 4.
+template <int NB, int NQ>
+__device__ __forceinline__ void bring_state(const double* __restrict__ qin, const double* __restrict__ qn,
+                                            const Grid& g, const StageParams& sp, unsigned tile, int k,
+                                            const Shared& sh, int lane) {
+    const Column o = column(g, tile, lane);
+    const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
+    double m[NQ][NB];
+#pragma unroll
+    for (int f = 0; f < NQ; f++) load_field<NB, NQ>(qin, g, c, f, m[f]);
+    if (sp.combine != 0 && sp.mode != 1) {
+        double q0[NQ][NB];
+#pragma unroll
+        for (int f = 0; f < NQ; f++) load_field<NB, NQ>(qn, g, c, f, q0[f]);
+#pragma unroll
+        for (int f = 0; f < NQ; f++)
+#pragma unroll
+            for (int r = 0; r < NB; r++) sh.m[((NQ + f) * NB + r) * 64 + lane] = q0[f][r];
+    }
+#pragma unroll
+    for (int f = 0; f < NQ; f++)
+#pragma unroll
+        for (int r = 0; r < NB; r++) sh.m[(f * NB + r) * 64 + lane] = m[f][r];
 }
 
 // One tile of one plane by five waves, for grids of few tiles (latency): the
@@ -993,23 +1041,25 @@ __device__ __forceinline__ void stage_wide(const double* __restrict__ qin, const
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     const int lane = (int)(threadIdx.x & 63u);
     if (part == 0) {
-        sum_part<NB, QP, NQ, RM, NZ, 0>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, 0>(qin, g, ph, sp, tile, k, 0, sh, lane);
     } else if (part == 1) {
-        sum_part<NB, QP, NQ, RM, NZ, 1>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, 1>(qin, g, ph, sp, tile, k, 0, sh, lane);
     } else if (part == 2) {
-        sum_part<NB, QP, NQ, RM, NZ, 2>(qin, qn, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, tile, k, 0, sh, lane);
+        if constexpr (wide_staged<NB, NQ>() && QP == 2) bring_state<NB, NQ>(qin, qn, g, sp, tile, k, sh, lane);
     } else {
         const bool one_z = g.nz == 1 && g.bc[4] == BC_PERIODIC;
         double M[NM][NK];
         if (part == 4 || !one_z) column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, column(g, tile, lane), k, part == 3 ? 1 : 0, M);
         if (part == 3) {
-            finish_part<NB, QP, NQ>(qout, g, ph, sp, tile, k, 0, cell0, sh, lane, one_z, M);
+            finish_part<NB, QP, NQ, true>(qin, qn, qout, g, ph, sp, tile, k, 0, cell0, sh, lane, one_z, M);
             return;
         }
 #pragma unroll
         for (int e = 0; e < NM; e++)
 #pragma unroll
             for (int n = 0; n < NK; n++) sh.z[(e * NK + n) * 64 + lane] = M[e][n];
+        if constexpr (wide_staged<NB, NQ>() && QP == 3) bring_state<NB, NQ>(qin, qn, g, sp, tile, k, sh, lane);
     }
     __syncthreads();
 }
@@ -1021,6 +1071,7 @@ __device__ __forceinline__ Shared share(double* lds, int* flags) {
     sh.r0 = lds;
     sh.r1 = lds + NB * NQ * 64;
     sh.z = lds + 2 * NB * NQ * 64;
+    sh.m = lds + lds_doubles<NB, NQ>();
     sh.flags = flags;
     if (threadIdx.x < 2) flags[threadIdx.x] = 0;
     __syncthreads();
@@ -1076,7 +1127,7 @@ template <int NB, int QP, int NQ, int RM, bool NZ>
 __global__ __launch_bounds__(320) void k_stage_wide(
     const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout, Grid g, Phys ph,
     StageParams sp, unsigned ntile, unsigned nwork) {
-    __shared__ double lds[lds_doubles<NB, NQ>()];
+    __shared__ double lds[wide_lds_doubles<NB, NQ>()];
     __shared__ int flags[2];
     const unsigned t = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (t >= nwork) return;
