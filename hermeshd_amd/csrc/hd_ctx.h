@@ -37,8 +37,8 @@ struct hd_ctx {
     hd::Tables htab;
     hd::Tables* dtab = nullptr;
     double* fl[3] = {nullptr, nullptr, nullptr};  // face fluxes per direction (table-driven kernels)
-    // periodic 13-moment transpose: the right cells' face cotangents (the left
-    // cells' reuse fl); allocated at the first such transpose
+    // periodic 13-moment transpose: moments of the right cells' face cotangents
+    // (the left cells' in fl); allocated at the first such transpose
     double* bq2[3] = {nullptr, nullptr, nullptr};
     double* partial = nullptr;                    // wave-speed partial maxima (npart + 1)
     int npart = 0;

@@ -49,14 +49,24 @@ int set_launch(hd_ens* e, int choice) {
     const Candidate& k = kCandidates[choice];
     // planes per workgroup: the shape's, or those of least cost
     int zc = k.zc;
+    // folded if a quarter of the lanes would be idle otherwise, as stage_folds
+    long planes = 0, folded = 0;
+    for (const ens::EnsReal& R : e->hreal) {
+        planes += (long)R.ntile * R.g.nz;
+        folded += sg::fold_tiles(R.g, 1);
+    }
+    const bool fold = 3 * planes >= 4 * folded;
+    auto items_of = [&](const ens::EnsReal& R, int z) {
+        return fold ? sg::fold_tiles(R.g, std::min(z, R.g.nz)) : (long)R.ntile * ((R.g.nz + z - 1) / z);
+    };
     if (zc == 0) {
         int nz = 1;
         for (const ens::EnsReal& R : e->hreal) nz = std::max(nz, R.g.nz);
-        const long resident = (long)e->num_cus * sg::stage_occupancy(e->nb, e->nQ);
+        const long resident = (long)e->num_cus * sg::occupancy(e->nb, e->nQ);
         double best = 1e300;
         for (int z = 1; z <= nz && z <= 32; z++) {
             long items = 0;
-            for (const ens::EnsReal& R : e->hreal) items += (long)R.ntile * ((R.g.nz + z - 1) / z);
+            for (const ens::EnsReal& R : e->hreal) items += items_of(R, z);
             const double cost = sg::march_cost(items, z, resident);
             if (cost < best) {
                 best = cost;
@@ -67,7 +77,7 @@ int set_launch(hd_ens* e, int choice) {
     e->hwork.clear();
     for (int r = 0; r < e->nreal; r++) {
         const ens::EnsReal& R = e->hreal[r];
-        const long n = (long)R.ntile * ((R.g.nz + zc - 1) / zc);
+        const long n = items_of(R, zc);
         for (long t = 0; t < n; t++) e->hwork.push_back(make_int2(r, (int)t));
     }
     if (e->hwork.size() > (size_t)0x7fffffff) return fail(HD_ERR_INVALID, "work list too long");
@@ -83,6 +93,7 @@ int set_launch(hd_ens* e, int choice) {
     HIPCHK(hipMemcpy(e->dwork, e->hwork.data(), e->hwork.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(e->dreal, e->hreal.data(), e->hreal.size() * sizeof(ens::EnsReal), hipMemcpyHostToDevice));
     e->launch.zc = zc;
+    e->launch.fold = fold;
     e->launch.nwork = (int)e->hwork.size();
     e->launch.xcd_chunk = k.xcd;
     e->grid = (e->launch.nwork + 7) / 8 * 8;
@@ -227,7 +238,7 @@ int hd_ens_create(const hd_config* base, int32_t nreal, const int32_t* dims, con
         R.cell0 = cell0;
         R.nfb = (long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
         R.noff = noff;
-        R.ntile = (int)sg::stage_tiles(g);
+        R.ntile = (int)sg::plane_tiles(g);
         R.realization = realization_ids ? realization_ids[r] : base->realization + (uint32_t)r;
         qoff += g.N * e->nQ * e->nb;
         cell0 += g.N;

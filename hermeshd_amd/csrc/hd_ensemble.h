@@ -30,11 +30,12 @@ struct EnsReal {
 
 struct Launch {
     int zc;           // planes per item
+    int fold;         // items are tiles of segments of zc planes (sg::Rows)
     int xcd_chunk;    // 1: XCD-contiguous chunks of the work list
     int nwork;
 };
 
-template <int NB, int QP, int NQ, int RM, bool NZ>
+template <int NB, int QP, int NQ, int RM, bool NZ, bool FOLD>
 __global__ __launch_bounds__(256, (sg::occupancy<NB, NQ>())) void k_ens_stage(
     const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout,
     const EnsReal* __restrict__ reals, const int2* __restrict__ work, Launch L, Phys ph, StageParams sp,
@@ -58,10 +59,16 @@ __global__ __launch_bounds__(256, (sg::occupancy<NB, NQ>())) void k_ens_stage(
         sp.noise[3] = base + 3 * fsz;
         sp.nfb = R.nfb;
     }
-    const int ch = wk.y / R.ntile, k0 = ch * L.zc, k1 = k0 + L.zc < g.nz ? k0 + L.zc : g.nz;
     const int part = __builtin_amdgcn_readfirstlane(((int)(threadIdx.x >> 6) + b) & 3);
-    sg::stage_march<NB, QP, NQ, RM, NZ>(qin + R.qoff, qn + R.qoff, qout + R.qoff, g, ph, sp,
-                                        (unsigned)(wk.y - ch * R.ntile), k0, k1, 0, part, R.cell0, sh);
+    if constexpr (FOLD) {
+        const int zc = L.zc < g.nz ? L.zc : g.nz;
+        sg::stage_march<NB, QP, NQ, RM, NZ, true>(qin + R.qoff, qn + R.qoff, qout + R.qoff, g, ph, sp, (unsigned)wk.y,
+                                                  zc, 0, sg::fold_planes(g, (unsigned)wk.y, zc), 0, part, R.cell0, sh);
+    } else {
+        const int ch = wk.y / R.ntile, k0 = ch * L.zc, k1 = k0 + L.zc < g.nz ? k0 + L.zc : g.nz;
+        sg::stage_march<NB, QP, NQ, RM, NZ, false>(qin + R.qoff, qn + R.qoff, qout + R.qoff, g, ph, sp,
+                                                   (unsigned)(wk.y - ch * R.ntile), 0, k0, k1, 0, part, R.cell0, sh);
+    }
 }
 
 // The limiter, a cell a thread: realizations along y of the grid.

@@ -48,13 +48,10 @@ struct Impl {
     }
     static void fused(hd_ctx* c, const double* qin, const double* qn, double* qout, const StageParams& sp, hipStream_t s) {
         const Grid& g = c->grid;
-        const unsigned tiles = sg::stage_tiles(g);
-        const int planes = c->stage_planes == STAGE_AUTO
-                               ? sg::stage_planes<NB, NQ>((long)tiles, g.nz, c->num_cus)
-                               : c->stage_planes;
+        const int planes = c->stage_planes == STAGE_AUTO ? sg::stage_planes<NB, NQ>(g, c->num_cus) : c->stage_planes;
         if constexpr (!(NB == 10 && NQ >= 11)) {  // its five waves would not have the registers
             if (planes < 0) {
-                const unsigned n = tiles * (unsigned)g.nz, grid = (n + 7) / 8 * 8;
+                const unsigned tiles = (unsigned)sg::plane_tiles(g), n = tiles * (unsigned)g.nz, grid = (n + 7) / 8 * 8;
                 if constexpr (NQ == 11) {
                     if (sp.noise[0]) {
                         hipLaunchKernelGGL((sg::k_stage_wide<NB, QP, NQ, RM, true>), dim3(grid), dim3(320), 0, s, qin,
@@ -67,19 +64,30 @@ struct Impl {
                 return;
             }
         }
-        const int zc = planes > 0 ? planes : 0;
-        const long n = zc ? (long)tiles * ((g.nz + zc - 1) / zc)
-                          : std::min((long)tiles * g.nz, (long)c->num_cus * sg::occupancy<NB, NQ>());
-        const unsigned grid = (unsigned)((n + 7) / 8 * 8);
+        if (planes > 0 && sg::stage_folds(g)) {
+            const int zc = std::min(planes, g.nz);
+            const unsigned tiles = (unsigned)sg::fold_tiles(g, zc);
+            march<true>(c, qin, qn, qout, sp, (tiles + 7) / 8 * 8, tiles, zc, s);
+        } else {
+            const int zc = planes > 0 ? planes : 0;
+            const long tiles = sg::plane_tiles(g);
+            const long n = zc ? tiles * ((g.nz + zc - 1) / zc)
+                              : std::min(tiles * g.nz, (long)c->num_cus * sg::occupancy<NB, NQ>());
+            march<false>(c, qin, qn, qout, sp, (unsigned)((n + 7) / 8 * 8), (unsigned)tiles, zc, s);
+        }
+    }
+    template <bool FOLD>
+    static void march(hd_ctx* c, const double* qin, const double* qn, double* qout, const StageParams& sp, unsigned grid,
+                      unsigned tiles, int zc, hipStream_t s) {
         if constexpr (NQ == 11) {
             if (sp.noise[0]) {
-                hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, true>), dim3(grid), dim3(256), 0, s, qin, qn, qout, g,
-                                   c->ph, sp, tiles, zc);
+                hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, true, FOLD>), dim3(grid), dim3(256), 0, s, qin, qn,
+                                   qout, c->grid, c->ph, sp, tiles, zc);
                 return;
             }
         }
-        hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, false>), dim3(grid), dim3(256), 0, s, qin, qn, qout, g, c->ph,
-                           sp, tiles, zc);
+        hipLaunchKernelGGL((sg::k_stage<NB, QP, NQ, RM, false, FOLD>), dim3(grid), dim3(256), 0, s, qin, qn, qout,
+                           c->grid, c->ph, sp, tiles, zc);
     }
     static void ens_limit(hd_ens* e, double* q, hipStream_t s) {
         hipLaunchKernelGGL((ens::k_ens_limit<NB, QP>), dim3(64, (unsigned)(e->nreal < 65535 ? e->nreal : 65535)),
@@ -87,15 +95,21 @@ struct Impl {
     }
     static void ens_stage(hd_ens* e, const double* qin, const double* qn, double* qout, const StageParams& sp,
                           hipStream_t s) {
+        if (e->launch.fold) ens_march<true>(e, qin, qn, qout, sp, s);
+        else ens_march<false>(e, qin, qn, qout, sp, s);
+    }
+    template <bool FOLD>
+    static void ens_march(hd_ens* e, const double* qin, const double* qn, double* qout, const StageParams& sp,
+                          hipStream_t s) {
         if constexpr (NQ >= 11) {
             if (e->base.noise) {
-                hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, true>), dim3(e->grid), dim3(256), 0, s, qin, qn,
-                                   qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
+                hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, true, FOLD>), dim3(e->grid), dim3(256), 0, s, qin,
+                                   qn, qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
                 return;
             }
         }
-        hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, false>), dim3(e->grid), dim3(256), 0, s, qin, qn, qout,
-                           e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
+        hipLaunchKernelGGL((ens::k_ens_stage<NB, QP, NQ, RM, false, FOLD>), dim3(e->grid), dim3(256), 0, s, qin, qn,
+                           qout, e->dreal, e->dwork, e->launch, e->ph, sp, e->noise);
     }
     // defined in hd_impl_vjp.h; the units that include it instantiate it
     // there, and hd_k4_vjp.hip holds the nbasis 4 instances, so that those

@@ -6,7 +6,7 @@
 // A tile is 64 consecutive positions of a plane's row lattice (nx+1 positions
 // per row: the faces across x), one per lane; it updates the cells of its
 // first 63 positions, so that the face above a cell in x is always the next
-// lane's.  A workgroup steps its tile through planes of z:
+// lane's (thin grids: Rows below).  A workgroup steps its tile through planes of z:
 //   part 0: the face below every cell in y, and the first third (half, with
 //           two Gauss points) of the volume integral;
 //   part 1: the face above in y, and the second third (half);
@@ -634,30 +634,95 @@ __device__ __forceinline__ void store_field(double* __restrict__ qout, const Gri
 }
 
 // ------------------------------------------------------------- waves -------
-// A lane's column of cells: position pi of the row lattice at row j, planes
-// stepped by the caller.
+// How the cells are cut into tiles.  A tile is cut from the rows of one plane
+// and steps through planes, the same for all its lanes.  A grid that is thin
+// across x and y would leave lanes idle (a column of cells along z 63 of 64): it
+// is FOLDed.  The planes are then taken in segments of zc; the rows of all
+// segments (row j of segment n is row j + ny n) make one list, cut into tiles
+// whatever the segments, and a tile steps each lane through its own segment.
+// Rows have nx+1 positions, the last a face alone; folded rows that are periodic
+// and of up to eight cells are packed whole, without it: a row's last cell has
+// its face above in the row's first lane.
+// us a step of 65,536 cells, folded against cut from planes: 1x1x65536 cells
+// nbasis 4 52 / 1446, nbasis 10 216 / 7228; 4x4x4096 51 / 130, 194 / 533.
+// The lane's own plane costs registers: 256x256x128 cells nbasis 4 4.37 ms
+// folded, 3.95 ms cut from planes.
+struct Rows {
+    unsigned pitch, n;  // positions of a row, of a tile
+    bool whole;
+};
+template <bool FOLD>
+__host__ __device__ __forceinline__ Rows tile_rows(const Grid& g) {
+    Rows o;
+    o.whole = FOLD && g.nx <= 8 && g.bc[0] == BC_PERIODIC;
+    o.pitch = (unsigned)g.nx + (o.whole ? 0u : 1u);
+    o.n = o.whole ? 64u - 64u % (unsigned)g.nx : 63u;
+    return o;
+}
+// tiles of nrow rows: the last position has no cell where rows have an extra one
+template <bool FOLD>
+inline long row_tiles(const Grid& g, long nrow) {
+    const Rows o = tile_rows<FOLD>(g);
+    return (o.pitch * nrow - (o.whole ? 0 : 1) + o.n - 1) / o.n;
+}
+inline long plane_tiles(const Grid& g) { return row_tiles<false>(g, g.ny); }
+inline long fold_tiles(const Grid& g, int zc) { return row_tiles<true>(g, (long)g.ny * ((g.nz + zc - 1) / zc)); }
+// planes that a folded tile steps through: fewer than zc if all of its cells are
+// in the last segment
+__device__ __forceinline__ int fold_planes(const Grid& g, unsigned tile, int zc) {
+    const Rows o = tile_rows<true>(g);
+    const int k0 = (int)(tile * o.n / o.pitch / (unsigned)g.ny) * zc;
+    return g.nz - k0 < zc ? g.nz - k0 : zc;
+}
+
+// A lane's column of cells: position pi of its row at row j, planes stepped by
+// the caller: k, or folded the segment's k0 + 0, 1, ..
 struct Column {
-    int pi, i, j;     // lattice position 0..nx (the face below cell pi in x), cell, row
+    int pi, i, j;     // position 0..nx (the face below cell pi in x), cell, row
+    int k0, next;     // folded: first plane; the lane that has the face above in x
     bool live;        // the lane updates the cell
     long row0;        // offset of the row within a plane
 };
-__device__ __forceinline__ Column column(const Grid& g, unsigned tile, int lane) {
-    // 32-bit position arithmetic: a plane of 2^31 cells would not fit the device.
+template <bool FOLD>
+__device__ __forceinline__ Column column(const Grid& g, unsigned tile, int zc, int lane) {
+    // 32-bit position arithmetic: 2^31 cells would not fit the device.
     // Worked out where it is used: kept across the planes it would cost registers
     // that the faces need.
     asm volatile("" : "+s"(tile));
-    const unsigned pitch = (unsigned)g.nx + 1u, npos = pitch * (unsigned)g.ny;
-    unsigned pos = tile * 63u + (unsigned)lane;
-    const bool in = pos < npos;
-    if (!in) pos = npos - 1u;
-    const unsigned row = pos / pitch;
+    const Rows t = tile_rows<FOLD>(g);
     Column o;
-    o.pi = (int)(pos - row * pitch);
+    unsigned pos = tile * t.n + (unsigned)lane, row;
+    if constexpr (FOLD) {
+        const unsigned nrow = (unsigned)g.ny * (unsigned)((g.nz + zc - 1) / zc);
+        if (t.whole && (unsigned)lane >= t.n) pos = tile * t.n;
+        row = pos / t.pitch;
+        o.pi = (int)(pos - row * t.pitch);
+        o.live = row < nrow && o.pi < g.nx && (unsigned)lane < t.n;
+        if (row >= nrow) row = nrow - 1u;
+        const unsigned n = row / (unsigned)g.ny;
+        row -= n * (unsigned)g.ny;
+        o.k0 = (int)n * zc;
+        o.next = t.whole && o.pi == g.nx - 1 ? lane - o.pi : (lane + 1) & 63;
+    } else {
+        const unsigned npos = t.pitch * (unsigned)g.ny;
+        const bool in = pos < npos;
+        if (!in) pos = npos - 1u;
+        row = pos / t.pitch;
+        o.pi = (int)(pos - row * t.pitch);
+        o.live = in && o.pi < g.nx && lane < 63;
+        o.k0 = 0;
+        o.next = (lane + 1) & 63;
+    }
     o.i = o.pi < g.nx ? o.pi : g.nx - 1;
     o.j = (int)row;
-    o.live = in && o.pi < g.nx && lane < 63;
     o.row0 = (long)g.nx * o.j;
     return o;
+}
+// its plane kk, folded the last one past the grid's end
+template <bool FOLD>
+__device__ __forceinline__ int column_plane(const Grid& g, const Column& o, int kk) {
+    if constexpr (!FOLD) return kk;
+    return o.k0 + kk < g.nz ? o.k0 + kk : g.nz - 1;
 }
 
 // Face s (0 below, 1 above) in direction DIR of the column's cell at plane k
@@ -692,10 +757,9 @@ __device__ __forceinline__ void column_face(const double* __restrict__ qin, cons
 // Waves per SIMD that the registers are held to.  With more modes than four and
 // stress the sums' LDS leaves room for one workgroup a CU (nbasis 8, 11 fields,
 // 64x64x48 cells: 855 us a step held to two, 760 to one).
+HD_DEV constexpr int occupancy(int nb, int nq) { return nb == 4 && nq == 5 ? 3 : (nb > 4 && nq >= 11 ? 1 : 2); }
 template <int NB, int NQ>
-HD_DEV constexpr int occupancy() { return NB == 4 && NQ == 5 ? 3 : (NB > 4 && NQ >= 11 ? 1 : 2); }
-
-inline int stage_occupancy(int nb, int nq) { return nb == 4 && nq == 5 ? 3 : (nb > 4 && nq >= 11 ? 1 : 2); }
+HD_DEV constexpr int occupancy() { return occupancy(NB, NQ); }
 
 // Cost of items of zc planes on `resident` workgroups, in planes: rounds times
 // an item's length, its start (the first face below in z and the first loads)
@@ -704,26 +768,36 @@ inline double march_cost(long items, int zc, long resident) {
     return (double)((items + resident - 1) / resident) * (zc + 0.6);
 }
 
-// How a grid of `tiles` tiles a plane and nz planes is run: -1 by k_stage_wide,
-// 0 in equal runs, n > 0 in items of n planes.
+// A grid is folded if a quarter of the lanes would be idle otherwise.
+inline bool stage_folds(const Grid& g) { return 3 * plane_tiles(g) * g.nz >= 4 * fold_tiles(g, 1); }
+
+// How a grid is run: -1 by k_stage_wide, 0 in equal runs, n > 0 in items of n
+// planes.
+//  * Folded grids: the items of least cost; single planes where a plane is less
+//    than a 128-byte line of cells, so that neighbouring lanes' cells follow each
+//    other in memory (13 moments, 1x1x65536 cells: 650 us a step against 986 in
+//    items of 4).
 //  * Up to two tiles per CU k_stage_wide: latency decides (Sod tube of 256
-//    cells 22 us a step in five waves against 26, channel 64x128 24 against 31).
+//    cells 24 us a step in five waves against 26, channel 64x128 26 against 31).
 //  * Up to 8 planes per resident workgroup in equal runs: whole rounds of items
-//    would leave part of the chip idle (nbasis 10, 75x61x27: 330 us a step
+//    would leave part of the chip idle (nbasis 10, 75x61x27: 348 us a step
 //    against 446 in items of 4).
 //  * Above, the items of least cost: neighbouring tiles at the same plane share
 //    L2, which equal runs lose (nbasis 4, 256x256x128: 4.0 ms a step in items
 //    of 8 or 16 against 4.8; nbasis 8, 120x80x64: 576 us against 640).
 template <int NB, int NQ>
-inline int stage_planes(long tiles, int nz, long cus) {
-    const long work = tiles * nz, resident = cus * occupancy<NB, NQ>();
-    if (work <= 2 * cus && !(NB == 10 && NQ >= 11)) return -1;
-    if (work < 8 * resident) return 0;
+inline int stage_planes(const Grid& g, long cus) {
+    const bool fold = stage_folds(g);
+    const long tiles = plane_tiles(g), work = tiles * g.nz, resident = cus * occupancy<NB, NQ>();
+    if (!fold && work <= 2 * cus && !(NB == 10 && NQ >= 11)) return -1;
+    if (!fold && work < 8 * resident) return 0;
+    if (fold && (long)g.nx * g.ny < 16) return 1;
+    auto cost = [&](int zc) {
+        return march_cost(fold ? fold_tiles(g, zc) : tiles * ((g.nz + zc - 1) / zc), zc, resident);
+    };
     int best = 1;
-    for (int zc = 2; zc <= nz && zc <= 16; zc++)
-        if (march_cost(tiles * ((nz + zc - 1) / zc), zc, resident) <
-            march_cost(tiles * ((nz + best - 1) / best), best, resident))
-            best = zc;
+    for (int zc = 2; zc <= g.nz && zc <= 16; zc++)
+        if (cost(zc) < cost(best)) best = zc;
     return best;
 }
 
@@ -752,15 +826,17 @@ __device__ __forceinline__ double next_lane(double x, int addr) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Parts 0-2 of plane k (p planes after the workgroup's first): one direction's
+// Parts 0-2 of the tile's plane kk (p planes after the workgroup's first): one direction's
 // face and a share of the volume integral; the sum to LDS.
-template <int NB, int QP, int NQ, int RM, bool NZ, int PART>
+template <int NB, int QP, int NQ, int RM, bool NZ, bool FOLD, int PART>
 __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const Grid& g, const Phys& ph,
-                                         const StageParams& sp, unsigned tile, int k, int p, const Shared& sh, int lane) {
+                                         const StageParams& sp, unsigned tile, int zc, int kk, int p, const Shared& sh,
+                                         int lane) {
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     constexpr int D = PART == 2 ? 0 : 1;
     constexpr bool VOL = PART < QP;
-    const Column o = column(g, tile, lane);
+    const Column o = column<FOLD>(g, tile, zc, lane);
+    const int k = column_plane<FOLD>(g, o, kk);
     const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
     double t[5][NB], tu[nscal(NQ)][NB], au[nscal(NQ)][3][ndeg<NB>()];
     {
@@ -777,7 +853,7 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const G
                 lift<NB, NK, 1, false>(M[e], s);
             } else {
                 double h[NK];
-                const int addr = ((lane + 1) & 63) * 4;
+                const int addr = o.next * 4;
 #pragma unroll
                 for (int n = 0; n < NK; n++) h[n] = next_lane(M[e][n], addr);
                 lift<NB, NK, 0, true>(M[e], s);
@@ -836,19 +912,20 @@ __device__ __forceinline__ void sum_part(const double* __restrict__ qin, const G
     if (PART == 2) raise(sh.flags + 1, p + 1);
 }
 
-// Part 3 of plane k after its face above in z (moments M, the next plane's
+// Part 3 of the tile's plane kk after its face above in z (moments M, the next plane's
 // face below): once all parts have met, the sum, the time step, the next
 // stage's limiter and the stores.
-template <int NB, int QP, int NQ, bool WIDE>
+template <int NB, int QP, int NQ, bool FOLD, bool WIDE>
 __device__ __forceinline__ void finish_part(const double* __restrict__ qin, const double* __restrict__ qn,
                                             double* __restrict__ qout, const Grid& g, const Phys& ph, const StageParams& sp,
-                                            unsigned tile, int k, int p, long cell0,
+                                            unsigned tile, int zc, int kk, int p, long cell0,
                                             const Shared& sh, int lane, bool same,
                                             double (&M)[face_nm(NQ)][fz::face_nk<NB>()]) {
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
-    const Column o = column(g, tile, lane);
+    Column o = column<FOLD>(g, tile, zc, lane);
+    if constexpr (FOLD) o.live = o.live && o.k0 + kk < g.nz;
     const Weights w = stage_weights<NQ>(sp);
-    const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
+    const long c = o.row0 + o.i + (long)g.nx * g.ny * column_plane<FOLD>(g, o, kk);
     // Values of the state and the step start are loaded AHEAD fields before they
     // are used, the first ones before the parts meet.
     constexpr bool STAGED = WIDE && wide_staged<NB, NQ>();
@@ -956,30 +1033,31 @@ __device__ __forceinline__ void finish_part(const double* __restrict__ qin, cons
     }
 }
 
-// One tile over planes [k0, k1), after p0 planes of this workgroup: four waves.
-template <int NB, int QP, int NQ, int RM, bool NZ>
+// One tile over planes [k0, k1) (folded: of its segments, of zc planes), after p0
+// planes of this workgroup: four waves.
+template <int NB, int QP, int NQ, int RM, bool NZ, bool FOLD>
 __device__ __forceinline__ void stage_march(const double* __restrict__ qin, const double* __restrict__ qn,
                                             double* __restrict__ qout, const Grid& g, const Phys& ph,
-                                            const StageParams& sp, unsigned tile, int k0, int k1, int p0, int part,
+                                            const StageParams& sp, unsigned tile, int zc, int k0, int k1, int p0, int part,
                                             long cell0, const Shared& sh) {
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     const int lane = (int)(threadIdx.x & 63u);
     if (part == 0) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 0>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, FOLD, 0>(qin, g, ph, sp, tile, zc, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else if (part == 1) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 1>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, FOLD, 1>(qin, g, ph, sp, tile, zc, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else if (part == 2) {
 #pragma unroll 1
         for (int k = k0; k < k1; k++) {
-            sum_part<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, tile, k, p0 + k - k0, sh, lane);
+            sum_part<NB, QP, NQ, RM, NZ, FOLD, 2>(qin, g, ph, sp, tile, zc, k, p0 + k - k0, sh, lane);
             __syncthreads();
         }
     } else {
@@ -992,14 +1070,19 @@ __device__ __forceinline__ void stage_march(const double* __restrict__ qin, cons
                 for (int e = 0; e < NM; e++)
 #pragma unroll
                     for (int n = 0; n < NK; n++) M[e][n] = 0.;
-            } else column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, column(g, tile, lane), k, 0, M);
+            } else {
+                const Column o = column<FOLD>(g, tile, zc, lane);
+                const int kf = !FOLD ? k : (o.k0 + k < g.nz ? o.k0 + k : g.nz);
+                column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, o, kf, 0, M);
+            }
             if (k == k0) {
 #pragma unroll
                 for (int e = 0; e < NM; e++)
 #pragma unroll
                     for (int n = 0; n < NK; n++) sh.z[(e * NK + n) * 64 + lane] = M[e][n];
             } else {
-                finish_part<NB, QP, NQ, false>(qin, qn, qout, g, ph, sp, tile, k - 1, p0 + k - 1 - k0, cell0, sh, lane, one_z, M);
+                finish_part<NB, QP, NQ, FOLD, false>(qin, qn, qout, g, ph, sp, tile, zc, k - 1, p0 + k - 1 - k0, cell0, sh, lane,
+                                               one_z, M);
             }
         }
     }
@@ -1011,7 +1094,7 @@ template <int NB, int NQ>
 __device__ __forceinline__ void bring_state(const double* __restrict__ qin, const double* __restrict__ qn,
                                             const Grid& g, const StageParams& sp, unsigned tile, int k,
                                             const Shared& sh, int lane) {
-    const Column o = column(g, tile, lane);
+    const Column o = column<false>(g, tile, 1, lane);
     const long c = o.row0 + o.i + (long)g.nx * g.ny * k;
     double m[NQ][NB];
 #pragma unroll
@@ -1041,18 +1124,21 @@ __device__ __forceinline__ void stage_wide(const double* __restrict__ qin, const
     constexpr int NM = face_nm(NQ), NK = fz::face_nk<NB>();
     const int lane = (int)(threadIdx.x & 63u);
     if (part == 0) {
-        sum_part<NB, QP, NQ, RM, NZ, 0>(qin, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, false, 0>(qin, g, ph, sp, tile, 1, k, 0, sh, lane);
     } else if (part == 1) {
-        sum_part<NB, QP, NQ, RM, NZ, 1>(qin, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, false, 1>(qin, g, ph, sp, tile, 1, k, 0, sh, lane);
     } else if (part == 2) {
-        sum_part<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, tile, k, 0, sh, lane);
+        sum_part<NB, QP, NQ, RM, NZ, false, 2>(qin, g, ph, sp, tile, 1, k, 0, sh, lane);
         if constexpr (wide_staged<NB, NQ>() && QP == 2) bring_state<NB, NQ>(qin, qn, g, sp, tile, k, sh, lane);
     } else {
         const bool one_z = g.nz == 1 && g.bc[4] == BC_PERIODIC;
         double M[NM][NK];
-        if (part == 4 || !one_z) column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, column(g, tile, lane), k, part == 3 ? 1 : 0, M);
+        if (part == 4 || !one_z) {
+            const Column o = column<false>(g, tile, 1, lane);
+            column_face<NB, QP, NQ, RM, NZ, 2>(qin, g, ph, sp, o, k, part == 3 ? 1 : 0, M);
+        }
         if (part == 3) {
-            finish_part<NB, QP, NQ, true>(qin, qn, qout, g, ph, sp, tile, k, 0, cell0, sh, lane, one_z, M);
+            finish_part<NB, QP, NQ, false, true>(qin, qn, qout, g, ph, sp, tile, 1, k, 0, cell0, sh, lane, one_z, M);
             return;
         }
 #pragma unroll
@@ -1078,23 +1164,27 @@ __device__ __forceinline__ Shared share(double* lds, int* flags) {
     return sh;
 }
 
-// tiles of a plane: the last position of its lattice has no cell
-inline unsigned stage_tiles(const Grid& g) { return (unsigned)(((long)(g.nx + 1) * g.ny - 1 + 62) / 63); }
-
 // The grid's work is ntile tiles of nz planes.  With zc > 0 a workgroup takes
 // zc planes of one tile, tiles first, so that neighbouring tiles are at the
-// same planes at the same time and find each other's modes in L2.  With zc = 0
-// it takes an equal run of the whole work, z fastest, in a launch of as many
-// workgroups as are resident: they start and end together.  Workgroup b runs
-// on XCD b mod 8: each XCD takes a contiguous eighth (the grid is a multiple
-// of 8).
-template <int NB, int QP, int NQ, int RM, bool NZ>
+// same planes at the same time and find each other's modes in L2 (folded: one of
+// the ntile tiles of segments of zc planes).  With zc = 0 it takes an equal run
+// of the whole work, z fastest, in a launch of as many workgroups as are
+// resident: they start and end together.  Workgroup b runs on XCD b mod 8: each
+// XCD takes a contiguous eighth (the grid is a multiple of 8).
+template <int NB, int QP, int NQ, int RM, bool NZ, bool FOLD>
 __global__ __launch_bounds__(256, (occupancy<NB, NQ>())) void k_stage(
     const double* __restrict__ qin, const double* __restrict__ qn, double* __restrict__ qout, Grid g, Phys ph,
     StageParams sp, unsigned ntile, int zc) {
     __shared__ double lds[lds_doubles<NB, NQ>()];
     __shared__ int flags[2];
     const unsigned b = blockIdx.x >> 3, w = (blockIdx.x & 7u) * (gridDim.x >> 3) + b;
+    if constexpr (FOLD) {
+        if (w >= ntile) return;
+        const Shared sh = share<NB, NQ>(lds, flags);
+        const int part = __builtin_amdgcn_readfirstlane((int)(((threadIdx.x >> 6) + b) & 3u));
+        stage_march<NB, QP, NQ, RM, NZ, true>(qin, qn, qout, g, ph, sp, w, zc, 0, fold_planes(g, w, zc), 0, part, 0, sh);
+        return;
+    }
     unsigned tile, left;
     int k0, p = 0;
     if (zc > 0) {
@@ -1115,7 +1205,7 @@ __global__ __launch_bounds__(256, (occupancy<NB, NQ>())) void k_stage(
 #pragma unroll 1
     while (left > 0) {
         const int n = (unsigned)(g.nz - k0) < left ? g.nz - k0 : (int)left;
-        stage_march<NB, QP, NQ, RM, NZ>(qin, qn, qout, g, ph, sp, tile, k0, k0 + n, p, part, 0, sh);
+        stage_march<NB, QP, NQ, RM, NZ, false>(qin, qn, qout, g, ph, sp, tile, 0, k0, k0 + n, p, part, 0, sh);
         left -= (unsigned)n;
         p += n;
         k0 = 0;
