@@ -94,7 +94,7 @@ struct hd_ens {
     long* dpts = nullptr;
     int2* dwork = nullptr;
     size_t work_cap = 0;
-    long state_doubles = 0, cells = 0;
+    long state_doubles = 0, cells = 0, max_cells = 0;  // max_cells: of the largest realization
     float* noise = nullptr;
     double* one_dt = nullptr;          // 1.0: the noise time step of hd_ens_rhs
     double* stage_buf = nullptr;       // RK3 third array when the caller passes none

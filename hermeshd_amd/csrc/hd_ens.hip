@@ -242,6 +242,7 @@ int hd_ens_create(const hd_config* base, int32_t nreal, const int32_t* dims, con
         R.realization = realization_ids ? realization_ids[r] : base->realization + (uint32_t)r;
         qoff += g.N * e->nQ * e->nb;
         cell0 += g.N;
+        e->max_cells = std::max(e->max_cells, g.N);
         if (base->noise) noff += 3L * 3 * e->nface * R.nfb + 6L * e->npg * g.N;
         for (int f = 0; f < 4; f++) {
             const long n = !base->noise ? 0 : (f < 3 ? (long)e->nface * R.nfb : (long)e->npg * g.N);

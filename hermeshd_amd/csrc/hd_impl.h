@@ -90,8 +90,12 @@ struct Impl {
                            c->grid, c->ph, sp, tiles, zc);
     }
     static void ens_limit(hd_ens* e, double* q, hipStream_t s) {
-        hipLaunchKernelGGL((ens::k_ens_limit<NB, QP>), dim3(64, (unsigned)(e->nreal < 65535 ? e->nreal : 65535)),
-                           dim3(256), 0, s, q, e->dreal, e->nreal, e->lp);
+        // a cell a thread of the largest realization, in a bounded launch (one
+        // box of 160^3 cells in 64 workgroups: 353 us, in 16,000: 108)
+        const long ny = std::min(e->nreal, 65535);
+        const long nx = std::min((e->max_cells + 255) / 256, std::max(64L, 65536 / ny));
+        hipLaunchKernelGGL((ens::k_ens_limit<NB, QP>), dim3((unsigned)nx, (unsigned)ny), dim3(256), 0, s, q, e->dreal,
+                           e->nreal, e->lp);
     }
     static void ens_stage(hd_ens* e, const double* qin, const double* qn, double* qout, const StageParams& sp,
                           hipStream_t s) {
