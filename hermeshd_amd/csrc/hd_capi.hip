@@ -262,9 +262,12 @@ int hd_create(const hd_config* cfg, hd_ctx** out) {
                  nfz = (size_t)g.nx * g.ny * (g.nz + 1);
     c->npart = 1024;
     // the full 10-moment equations (ivis 2) and the water EOS (ieos 2) run on the
-    // table-driven kernels only; HD_KERNELS=generic selects those for any configuration
+    // table-driven kernels only; HD_KERNELS=generic selects those for any
+    // configuration, HD_FACES=table for the 13-moment model
     const char* kern = std::getenv("HD_KERNELS");
-    c->generic = (kern && std::strcmp(kern, "generic") == 0) || cfg->ivis == 2 || cfg->ieos == 2;
+    const char* face = std::getenv("HD_FACES");
+    c->generic = (kern && std::strcmp(kern, "generic") == 0) || cfg->ivis == 2 || cfg->ieos == 2 ||
+                 (cfg->nQ == 13 && face && std::strcmp(face, "table") == 0);
     if (c->generic && cfg->noise) {
         hd_destroy(c);
         return fail(HD_ERR_UNSUPPORTED, "the table-driven kernels (HD_KERNELS=generic) carry no stochastic stress");
