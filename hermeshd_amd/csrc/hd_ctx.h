@@ -68,7 +68,7 @@ struct hd_ctx {
     int stage_planes = hd::STAGE_AUTO;
     // table-driven limiter kernel instead of fz::k_limit (HD_LIMITER=table)
     int table_limiter = 0;
-    // fused per-cell transpose for periodic 13-moment grids too (HD_VJP=fused)
+    // the per-cell transpose k_stage_vjp for every grid (HD_VJP=fused)
     int fused_vjp = 0;
     int64_t bytes = 0;
     int device = 0;

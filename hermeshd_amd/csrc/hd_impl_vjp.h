@@ -30,7 +30,7 @@ void Impl<NB, QP, NQ, RM>::stage_vjp(hd_ctx* c, const double* q, const double* l
         // 41 (8,192 cells, the per-cell kernel split over four waves, which
         // this replaced), 133 against 133 (64,000, one round), 181 against 307
         // (92,160, split), but 585 against 469 (262,144).
-        if (4 * c->N <= 7 * 256L * c->num_cus) {
+        if (!c->fused_vjp && 4 * c->N <= 7 * 256L * c->num_cus) {
             c->vjp_blocks = (int)blocks_for(c->N, adj::kPointCells);
             hipLaunchKernelGGL((adj::k_points_vjp<NB, QP, NQ, RM>), dim3(c->vjp_blocks), dim3(512), 0, s, q, lam,
                                lam_in, c->dtab, c->grid, c->ph, ap);
@@ -39,7 +39,7 @@ void Impl<NB, QP, NQ, RM>::stage_vjp(hd_ctx* c, const double* q, const double* l
     } else {
         // small grids are latency-bound: spread each cell over four waves
         if constexpr (adj::split_fits<NB, NQ>()) {
-            if (c->N <= adj::kSplitCells) {
+            if (!c->fused_vjp && c->N <= adj::kSplitCells) {
                 c->vjp_blocks = (int)blocks_for(c->N, 64);
                 hipLaunchKernelGGL((adj::k_stage_vjp_split<NB, QP, NQ, RM>), dim3(c->vjp_blocks), dim3(256), 0,
                                    s, q, lam, lam_in, c->grid, c->ph, ap);

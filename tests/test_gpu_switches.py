@@ -48,6 +48,42 @@ def test_table_driven_13_moments(oracle_mod, monkeypatch, name, env):
     assert field_rel_err(qd.cpu().numpy(), q) < TOL
 
 
+# ----------------------------------------------------- per-cell transposes ---
+def _two_point(names):
+    return [n for n in names if adjoint.CFGS[n].nbasis != 10]
+
+
+@pytest.mark.parametrize("name", _two_point(adjoint.CFGS))
+def test_per_cell_rhs_vjp(oracle_mod, monkeypatch, name):
+    monkeypatch.setenv("HD_VJP", "fused")
+    adjoint.test_rhs_vjp_matches_autograd(torch.device("cuda:0"), oracle_mod, name)
+
+
+@pytest.mark.parametrize("name,stage", [("nb4_nq11_hllc_noslip_ivis1", 2), ("nb4_nq11_hllc_walls_ivis0", 1),
+                                        ("nb4_nq11_hllc_inflow_ivis1", 3), ("nb8_nq5_central_outflow", 2),
+                                        ("nb4_nq11_roe_walls_ivis1", 2), ("nb4_nq13_roe_periodic_ivis1", 3)])
+def test_per_cell_stage_vjp(oracle_mod, monkeypatch, name, stage):
+    monkeypatch.setenv("HD_VJP", "fused")
+    adjoint.test_stage_vjp_matches_autograd(torch.device("cuda:0"), oracle_mod, name, stage)
+
+
+@pytest.mark.parametrize("nb,nq", [(4, 5), (4, 11), (8, 5), (8, 11), (4, 13), (10, 5), (10, 13)])
+def test_fused_selects_another_transpose(monkeypatch, nb, nq):
+    """The per-cell kernel sums in another order than the default of a small
+    grid: equal to rounding, in some of the values not bitwise."""
+    extra = dict(coll_q=2.0, col_q=0.3) if nq == 13 else {}
+    visc = dict(ivis=1, coll=3.0, colvis=0.2) if nq >= 11 else {}
+    cfg = HDConfig(nx=9, ny=7, nz=5, lx=0.9, ly=0.7, lz=0.5, nbasis=nb, iquad=3 if nb == 10 else 2, nQ=nq,
+                   riemann="hllc", bc=("periodic",) * 6, T_floor=1e-4, limiter=False, integrator="heun", **visc,
+                   **extra)
+    q = torch.from_numpy(smooth_state(cfg, seed=4)).cuda()
+    lam = torch.from_numpy(np.random.default_rng(3).standard_normal(q.shape)).cuda()
+    a = solver(cfg, monkeypatch).rhs_vjp(q, lam)
+    b = solver(cfg, monkeypatch, HD_VJP="fused").rhs_vjp(q, lam)
+    assert field_rel_err(a.cpu().numpy(), b.cpu().numpy()) < adjoint.VJP_TOL
+    assert not torch.equal(a, b)
+
+
 # ------------------------------------------------ ways of taking the stage ---
 @pytest.mark.parametrize("name", ["vortex_nb10_rows64", "relax_nq11_rows64", "vortex_nb10_hllc", "relax_nq11_bodyforce",
                                   "tm13_nb10_rows64"])
