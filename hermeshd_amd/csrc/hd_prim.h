@@ -44,40 +44,6 @@ __device__ __forceinline__ Prim prim(const Phys& ph, const double* Q) {
     return s;
 }
 
-// physical flux in direction DIR from primitives (flux_calc_pnts_r, ivis 0/1)
-template <int NQ, int DIR>
-__device__ __forceinline__ void flux(const Phys& ph, const double* Q, const Prim& s, double* F, const double* S) {
-    constexpr int ND = MX + DIR;
-    const double un = s.u[DIR];
-    const double P = s.pf;
-    double Pn[3] = {0., 0., 0.};  // stress row P_{DIR,*}
-    if constexpr (NQ >= 11) {
-        if (DIR == 0) { Pn[0] = Q[PXX]; Pn[1] = Q[PXY]; Pn[2] = Q[PXZ]; }
-        if (DIR == 1) { Pn[0] = Q[PXY]; Pn[1] = Q[PYY]; Pn[2] = Q[PYZ]; }
-        if (DIR == 2) { Pn[0] = Q[PXZ]; Pn[1] = Q[PYZ]; Pn[2] = Q[PZZ]; }
-    }
-    if (S) {
-        if (DIR == 0) { Pn[0] -= S[0]; Pn[1] -= S[3]; Pn[2] -= S[4]; }
-        if (DIR == 1) { Pn[0] -= S[3]; Pn[1] -= S[1]; Pn[2] -= S[5]; }
-        if (DIR == 2) { Pn[0] -= S[4]; Pn[1] -= S[5]; Pn[2] -= S[2]; }
-    }
-    F[RH] = Q[ND];
-    F[MX] = Q[MX] * un + Pn[0];
-    F[MY] = Q[MY] * un + Pn[1];
-    F[MZ] = Q[MZ] * un + Pn[2];
-    F[ND] += P;
-    F[EN] = (Q[EN] + P) * un + Pn[0] * s.u[0] + Pn[1] * s.u[1] + Pn[2] * s.u[2];
-    if constexpr (NQ >= 11) {
-        const double c4 = ph.c4d3cv * un, c2 = -ph.c2d3cv * un;
-        F[PXX] = DIR == 0 ? c4 : c2;
-        F[PYY] = DIR == 1 ? c4 : c2;
-        F[PZZ] = DIR == 2 ? c4 : c2;
-        F[PXY] = DIR == 0 ? ph.colvis * s.u[1] : (DIR == 1 ? ph.colvis * s.u[0] : 0.);
-        F[PXZ] = DIR == 0 ? ph.colvis * s.u[2] : (DIR == 2 ? ph.colvis * s.u[0] : 0.);
-        F[PYZ] = DIR == 1 ? ph.colvis * s.u[2] : (DIR == 2 ? ph.colvis * s.u[1] : 0.);
-    }
-}
-
 // Numerator of the HLLC contact speed, aR*uR - aL*uL + pL - pR, rounded
 // product by product: at a mirror state (the x-high outflow ghost reverses
 // the normal momentum) it is exactly zero, and a fused multiply-add would

@@ -20,7 +20,7 @@
 // Part 3 alone holds terms of the state: with the state in one of the partial
 // sums each later addition rounded it once more (a step's error 1.3e-16 of the
 // state against 0.4e-16 to 0.8e-16), for 0 to 10 % less time (vortex 1363 us a
-// step against 1438, linear 3921 and 3950, 13 moments 6928 and 7052, channel
+// step against 1438, linear 3950 and 4040, 13 moments 6935 and 7080, channel
 // 23.2 and 25.7).  Which wave takes which part rotates with the
 // workgroup, so that what inequality there is does not always meet one SIMD.
 //
@@ -778,13 +778,15 @@ inline bool stage_folds(const Grid& g) { return 3 * plane_tiles(g) * g.nz >= 4 *
 //    other in memory (13 moments, 1x1x65536 cells: 650 us a step against 986 in
 //    items of 4).
 //  * Up to two tiles per CU k_stage_wide: latency decides (Sod tube of 256
-//    cells 24 us a step in five waves against 26, channel 64x128 26 against 31).
+//    cells 23.4 us a step in five waves against 24.7, channel 64x128 25.7
+//    against 29.1).
 //  * Up to 8 planes per resident workgroup in equal runs: whole rounds of items
-//    would leave part of the chip idle (nbasis 10, 75x61x27: 348 us a step
-//    against 446 in items of 4).
+//    would leave part of the chip idle (nbasis 10, 75x61x27: 350 us a step
+//    against 461 in items of 4).
 //  * Above, the items of least cost: neighbouring tiles at the same plane share
-//    L2, which equal runs lose (nbasis 4, 256x256x128: 4.0 ms a step in items
-//    of 8 or 16 against 4.8; nbasis 8, 120x80x64: 576 us against 640).
+//    L2, which equal runs lose (nbasis 4, 256x256x128: 4.1 ms a step in items
+//    of 8 or 16 against 5.0; nbasis 8, 120x80x64: 593 us in items of 8 against
+//    637).
 template <int NB, int NQ>
 inline int stage_planes(const Grid& g, long cus) {
     const bool fold = stage_folds(g);

@@ -32,11 +32,12 @@ def _stream():
 
 @dataclass(frozen=True)
 class LaunchShape:
-    block: int
-    brick: tuple
-    linear: bool
-    wg_per_cu: int       # 0: one workgroup per tile
-    xcd_chunks: bool
+    """A way of cutting the stage's work into items of one workgroup each."""
+    block: int           # threads of a workgroup
+    brick: tuple         # cells of a tile along x and y; planes it steps through (0: those of least cost)
+    linear: bool         # tiles are runs of cells, over the ends of rows
+    wg_per_cu: int       # 0: one workgroup per item
+    xcd_chunks: bool     # each XCD takes a contiguous eighth of the items
 
 
 def launch_shapes() -> list[LaunchShape]:

@@ -146,9 +146,10 @@ int hd_stage(hd_ctx *ctx, int32_t rk_order, int32_t stage_index, double *q_in, c
    gradient of a run with respect to its initial state and the relaxation
    rate coll (used for the Poiseuille-channel sensitivity).  Central, HLLC and
    Roe face solvers; no noise.  On a 13-moment context periodic in every
-   direction, the first hd_rhs_vjp or hd_stage_vjp allocates the face
-   cotangents of the split transpose (3 arrays of nQ*iquad^2 doubles per face,
-   counted by hd_device_bytes) unless HD_VJP=fused was set at hd_create. */
+   direction, the first hd_rhs_vjp or hd_stage_vjp allocates the moments of the
+   face cotangents of the split transpose (6 arrays of 3*nQ, nbasis 4, or 6*nQ
+   doubles per cell, counted by hd_device_bytes) unless HD_VJP=fused was set at
+   hd_create. */
 
 /* out = (dR/dq)^T lam, R the right-hand side of hd_rhs at state q. */
 int hd_rhs_vjp(hd_ctx *ctx, const double *q, const double *lam, double *out, void *stream);
@@ -274,10 +275,12 @@ int hd_ens_set_step(hd_ens *ens, uint64_t step, void *stream);
 /* like hd_check; reports the realization and its cell */
 int hd_ens_check(hd_ens *ens, void *stream, int64_t *bad_realization, int64_t *bad_cell);
 
-/* Launch shapes of the stage kernel: tiles of consecutive cells or bricks,
-   one workgroup per tile or a persistent grid walking the (realization,
-   tile) list.  info: block size, brick bx,by,bz, linear flag, and
-   2*(workgroups per CU, 0 = one per tile) + (XCD-contiguous chunks).  */
+/* Launch shapes of the stage kernel: how many planes a workgroup steps its
+   tile of cells through, and whether each XCD takes a contiguous eighth of
+   the (realization, tile, planes) list.  info: block size, cells of a tile
+   along x and y, planes per item (0: those of least cost), linear flag (tiles
+   are runs of cells), and 2*(workgroups per CU, 0 = one per item) +
+   (XCD-contiguous eighths).  */
 int32_t hd_ens_launch_count(void);
 int hd_ens_launch_info(int32_t choice, int32_t info[6]);
 int hd_ens_set_launch(hd_ens *ens, int32_t choice);

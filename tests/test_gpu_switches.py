@@ -1,7 +1,5 @@
 """The switches that select a cross-check kernel (GPU): that they do, and that
 the kernels they select are right."""
-import os
-
 import numpy as np
 import pytest
 import torch
