@@ -1312,7 +1312,7 @@ __global__ __launch_bounds__(512, (NQ == 5 ? 4 : 2)) void k_points_vjp(const dou
 // in another order.  A periodic grid has as many faces a direction as cells:
 // face c is the low face of cell c.
 // nbasis 10, Roe, 40^3 cells, a stage: 217 us the faces (three directions in
-// one launch, 51 KB of LDS: three workgroups a CU) and 214 us the cells,
+// one launch, 51 KB of LDS: three workgroups a CU) and 201 us the cells,
 // against 840 and 429 us for a wave per face point over 64 faces (156 KB of
 // LDS, one workgroup a CU, waiting for its loads two thirds of the time, and
 // a last round of one workgroup) and a field per wave (three of thirteen
